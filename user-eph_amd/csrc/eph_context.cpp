@@ -85,13 +85,21 @@ int eph_grid::upload() {
 void eph_grid::refresh_minmax() {
   const size_t G = h.ntotal();
   cmin = h.C[0]; rmin = h.rho[0]; kmax = h.kappa[0];
-  for (size_t i = 1; i < G; ++i) {
-    if (h.flag[i] != CELL_CONSTANT) {
-      if (h.C[i] < cmin) cmin = h.C[i];
-      if (h.rho[i] < rmin) rmin = h.rho[i];
-      if (h.kappa[i] > kmax) kmax = h.kappa[i];
+  // one material in every cell, no walls: the solve reads no per-cell values
+  bool one = h.one_material;
+  if (!one) {
+    one = h.flag[0] == CELL_DYNAMIC && !h.tdyn[0];
+    for (size_t i = 1; i < G; ++i) {
+      if (h.flag[i] != CELL_CONSTANT) {
+        if (h.C[i] < cmin) cmin = h.C[i];
+        if (h.rho[i] < rmin) rmin = h.rho[i];
+        if (h.kappa[i] > kmax) kmax = h.kappa[i];
+      }
+      one = one && h.flag[i] == CELL_DYNAMIC && !h.tdyn[i] && h.kappa[i] == h.kappa[0] &&
+            h.S[i] == h.S[0] && h.rho[i] == h.rho[0] && h.C[i] == h.C[0];
     }
   }
+  uniform = one && std::isfinite(h.kappa[0]);
   minmax_valid = true;
 }
 
@@ -129,14 +137,11 @@ int eph_grid::solve(int* substeps_out) {
   unsigned new_steps = 0;
   substeps(&r, &new_steps, &inner_dt);
   last_r = r;
-  for (unsigned n = 0; n < new_steps; ++n) {
-    EPH_HIP(this, launch_fdm_substep(v, T.p, Tn.p, inner_dt, any_tdyn, stream));
-    std::swap(T.p, Tn.p);
-    v.T = T.p;
-    v.Tn = Tn.p;
-  }
-  EPH_HIP(this, launch_fill_double(dT.p, (long)h.ntotal(), 0.0, stream));
-  EPH_HIP(this, launch_nonfinite(T.p, (int)h.ntotal(), nonfinite.p, stream));
+  const FdmMaterial mat{h.kappa[0], h.S[0], h.rho[0], h.C[0]};
+  EPH_HIP(this, launch_fdm_solve(v, T.p, Tn.p, inner_dt, (int)new_steps,
+                                 !any_tdyn && uniform ? &mat : nullptr, any_tdyn, nonfinite.p, stream));
+  v.T = T.p;
+  v.Tn = Tn.p;
   last_steps = (int)new_steps;
   if (substeps_out) *substeps_out = (int)new_steps;
   return EPH_OK;
@@ -1599,6 +1604,7 @@ int eph_grid_set_cell(eph_grid* g, int i, int j, int k, double T, double S, doub
   const size_t c = i + j * g->h.nx + k * g->h.nx * g->h.ny;
   g->h.T[c] = T; g->h.S[c] = S; g->h.rho[c] = rho; g->h.C[c] = C; g->h.kappa[c] = kappa;
   g->h.flag[c] = (int8_t)flag; g->h.tdyn[c] = (int8_t)tdyn;
+  g->h.one_material = false;
   if ((rc = g->upload())) return rc;
   EPH_HIP(g, hipMemcpyAsync(g->dT.p, dTcur.data(), dTcur.size() * sizeof(double), hipMemcpyHostToDevice, g->stream));
   EPH_HIP(g, hipStreamSynchronize(g->stream));
@@ -1647,6 +1653,7 @@ int eph_grid_set(eph_grid* g, int which, const double* in) {
   std::vector<double>& dst = which == 0 ? g->h.T : which == 2 ? g->h.C : which == 3 ? g->h.rho
                            : which == 4 ? g->h.kappa : g->h.S;
   std::copy(in, in + G, dst.begin());
+  if (which != 0) g->h.one_material = false;
   if ((rc = g->upload())) return rc;
   EPH_HIP(g, hipMemcpyAsync(g->dT.p, dTcur.data(), G * sizeof(double), hipMemcpyHostToDevice, g->stream));
   EPH_HIP(g, hipStreamSynchronize(g->stream));

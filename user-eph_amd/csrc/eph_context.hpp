@@ -55,7 +55,8 @@ struct eph_grid {
   eph::DevArray<int> bcount, bitems, bqueue, bnq;
   int bucket_bytes_ok(size_t G);  // reserves the buckets; 0 when they are ready
   bool any_tdyn = false;
-  bool minmax_valid = false;
+  bool minmax_valid = false;  // cmin, rmin, kmax and uniform describe h
+  bool uniform = false;       // every cell dynamic and of one material
   double cmin = 0, rmin = 0, kmax = 0;
   double last_r = 0;
   int last_steps = 0;

@@ -250,6 +250,16 @@ hipError_t launch_grid_tdyn_update(const GridView& g, hipStream_t s);
 hipError_t launch_grid_minmax(const GridView& g, double* out3, double* scratch, hipStream_t s);
 hipError_t launch_fdm_substep(const GridView& g, const double* Tin, double* Tout, double inner_dt,
                               bool any_tdyn, hipStream_t s);
+// one material in every cell: kappa, S, rho_e, C_e
+struct FdmMaterial {
+  double kappa, S, rho, C;
+};
+// the nsub sub-steps of one solve (eph_fdm.hip): T holds the result on return
+// (T and Tn may have been swapped), dT is cleared, and bit 1 of *nonfinite is
+// set when T holds a non-finite value.  uniform: every cell is a dynamic cell
+// of this material (null: values per cell)
+hipError_t launch_fdm_solve(const GridView& g, double*& T, double*& Tn, double inner_dt, int nsub,
+                            const FdmMaterial* uniform, bool any_tdyn, int* nonfinite, hipStream_t s);
 hipError_t launch_grid_lookup(const GridView& g, int n, const double* x, const double* y,
                               const double* z, int* idx, double* T, hipStream_t s);
 hipError_t launch_sum(const double* v, int n, double* out, double* scratch, hipStream_t s);

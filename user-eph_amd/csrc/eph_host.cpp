@@ -253,6 +253,7 @@ bool make_grid_const(size_t nx, size_t ny, size_t nz, const double box[6], doubl
   g.dt = 1;
   g.param_file = "NULL";
   g.has_params = false;
+  g.one_material = true;
   return true;
 }
 

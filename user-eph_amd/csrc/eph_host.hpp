@@ -83,6 +83,7 @@ struct GridHost {
   std::vector<double> T, S, rho, C, kappa;
   std::vector<int8_t> flag, tdyn;
   bool has_params = false;
+  bool one_material = false;  // made of constants: dynamic cells, one S, rho, C, kappa
   Spline C_T, kappa_T;   // C_e(T), kappa(T) (eph_fdm.h:95-96)
   LinearTable E_T;       // E_e(T) cumulative table (eph_fdm.h:98-103)
   size_t ntotal() const { return nx * ny * nz; }

@@ -8,6 +8,7 @@
 // the cooperative forms a wavefront fetches its atoms' neighbour records
 // together through LDS; the sums themselves stay one thread per atom.
 #include "eph_devfn.hpp"
+#include "eph_fdm.hpp"
 #include "eph_rng.hpp"
 
 namespace eph {
@@ -1589,80 +1590,6 @@ __global__ __launch_bounds__(1024) void k_grid_minmax(GridView g, int n, double*
   if (threadIdx.x == 0) { out3[0] = s0[0]; out3[1] = s1[0]; out3[2] = s2[0]; }
 }
 
-// one dimension's two terms of the 7-point variable-kappa stencil
-// (eph_fdm.h:337-339, 350-352, 363-365), in the reference's order; p and q
-// are the cell's lower and upper neighbours after the wall rule
-static __device__ __forceinline__ double fdm_dim(double ddT, const double kr, const double Tr,
-                                                 const double kp, const double kq, const double Tp,
-                                                 const double Tq, const double d) {
-  ddT += (kq - kp) * (Tq - Tp) / d / d / 4.0;
-  ddT += kr * ((Tq + Tp - 2.0 * Tr) / d / d);
-  return ddT;
-}
-
-// the update of a cell from its stencil sum, then the clamp (eph_fdm.h:376-395)
-template <bool TDYN>
-static __device__ __forceinline__ double fdm_update(const GridView& g, const int r, const int fr,
-                                                    double T, const double ddT,
-                                                    const double inner_dt) {
-  if (fr == kCellDynamic) {
-    if (TDYN && g.tdyn[r] == 1) {
-      double E = linear_fwd(g, T);
-      E += (ddT + g.dT[r] + g.S[r]) / g.rho[r] * inner_dt;
-      T = linear_rev(g, E);
-    } else {
-      const double prescaler = g.rho[r] * g.C[r];
-      T += (ddT + g.dT[r] + g.S[r]) / prescaler * inner_dt;
-    }
-  }
-  if (T < 0.0) T = 0.0;
-  return T;
-}
-
-// one explicit sub-step of EPH_FDM::solve (eph_fdm.h:315-395): the 7-point
-// variable-kappa stencil on Tin, the update and the clamp, into Tout
-template <bool TDYN>
-__device__ __forceinline__ void fdm_cell(const GridView& g, const double* __restrict__ Tin,
-                                         double* __restrict__ Tout, const int r,
-                                         const double inner_dt) {
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const int i = r % nx, j = (r / nx) % ny, k = r / (nx * ny);
-  const int fr = g.flag[r];
-  double ddT = 0.0;
-  if (fr != kCellZeroDerivative) {
-    const double Tr = Tin[r], kr = g.kappa[r];
-    int p, q;
-    // x
-    p = i > 0 ? r - 1 : r + (nx - 1);
-    q = i < nx - 1 ? r + 1 : r - (nx - 1);
-    if (g.flag[q] == kCellZeroDerivative) q = r;
-    else if (g.flag[p] == kCellZeroDerivative) p = r;
-    ddT = fdm_dim(ddT, kr, Tr, g.kappa[p], g.kappa[q], Tin[p], Tin[q], g.dx);
-    // y
-    p = j > 0 ? r - nx : r + (ny - 1) * nx;
-    q = j < ny - 1 ? r + nx : r - (ny - 1) * nx;
-    if (g.flag[q] == kCellZeroDerivative) q = r;
-    else if (g.flag[p] == kCellZeroDerivative) p = r;
-    ddT = fdm_dim(ddT, kr, Tr, g.kappa[p], g.kappa[q], Tin[p], Tin[q], g.dy);
-    // z
-    const int pl = nx * ny;
-    p = k > 0 ? r - pl : r + (nz - 1) * pl;
-    q = k < nz - 1 ? r + pl : r - (nz - 1) * pl;
-    if (g.flag[q] == kCellZeroDerivative) q = r;
-    else if (g.flag[p] == kCellZeroDerivative) p = r;
-    ddT = fdm_dim(ddT, kr, Tr, g.kappa[p], g.kappa[q], Tin[p], Tin[q], g.dz);
-  }
-  Tout[r] = fdm_update<TDYN>(g, r, fr, Tin[r], ddT, inner_dt);
-}
-
-template <bool TDYN>
-__global__ __launch_bounds__(kBlock) void k_fdm_substep(GridView g, const double* __restrict__ Tin,
-                                                        double* __restrict__ Tout, double inner_dt) {
-  const int r = blockIdx.x * kBlock + threadIdx.x;
-  if (r >= g.nx * g.ny * g.nz) return;
-  fdm_cell<TDYN>(g, Tin, Tout, r, inner_dt);
-}
-
 __global__ __launch_bounds__(kBlock) void k_grid_lookup(GridView g, int n, const double* x,
                                                         const double* y, const double* z, int* idx,
                                                         double* T) {
@@ -2463,14 +2390,6 @@ hipError_t launch_grid_tdyn_update(const GridView& g, hipStream_t s) {
 
 hipError_t launch_grid_minmax(const GridView& g, double* out3, double*, hipStream_t s) {
   k_grid_minmax<<<1, 1024, 0, s>>>(g, g.nx * g.ny * g.nz, out3);
-  return hipGetLastError();
-}
-
-hipError_t launch_fdm_substep(const GridView& g, const double* Tin, double* Tout, double inner_dt,
-                              bool any_tdyn, hipStream_t s) {
-  const int n = g.nx * g.ny * g.nz;
-  if (any_tdyn) k_fdm_substep<true><<<nblk(n), kBlock, 0, s>>>(g, Tin, Tout, inner_dt);
-  else k_fdm_substep<false><<<nblk(n), kBlock, 0, s>>>(g, Tin, Tout, inner_dt);
   return hipGetLastError();
 }
 
