@@ -220,19 +220,9 @@ int eph_adjoint::step(long long n, Rec* r) {
   int rc;
   ctx->step = n;
   if ((rc = ctx->dev_initial_integrate())) return fail(rc, ctx->err);
-  const double lim = 0.25 * md->cfg.skin * md->cfg.skin;
-  EPH_HIP(this, launch_nb_check(nl, ctx->pos.p, md->xref.p, lim, md->nbw.go, s));
-  EPH_HIP(this, launch_nb_build(md->nbw, s));
-  EPH_HIP(this, hipMemcpyAsync(md->pinned, md->flags.p, 8 * sizeof(int), hipMemcpyDeviceToHost, s));
-  EPH_HIP(this, hipStreamSynchronize(s));
-  if (md->pinned[0]) {
-    if (md->pinned[1]) return fail(EPH_ERR_STATE, "neighbour capacity exceeded during the trajectory");
-    ctx->nghost = md->pinned[7];
-    md->nghost = ctx->nghost;
-  }
-  EPH_HIP(this, launch_ghost_xv(ctx->atoms_view(), ctx->ghost_owner.p, ctx->ghost_shift.p, s));
-  EPH_HIP(this, launch_lj(ctx->atoms_view(), md->lj_nbr.p, md->lj_nn.p, md->lj_stride, md->cfg.lj_eps,
-                          md->cfg.lj_sigma, md->cfg.cut_lj * md->cfg.cut_lj, s));
+  bool rebuilt = false, overflow = false;
+  if ((rc = md->neighbours_and_pair(ctx, false, nullptr, &rebuilt, &overflow))) return fail(rc, md->err);
+  if (overflow) return fail(EPH_ERR_STATE, "neighbour capacity exceeded during the trajectory");
   if ((rc = ctx->dev_post_force())) return fail(rc, ctx->err);
   if ((rc = ctx->dev_final_integrate())) return fail(rc, ctx->err);
   if (r) HCPY(r->TB.p, ctx->grid->T.p, G * sizeof(double));

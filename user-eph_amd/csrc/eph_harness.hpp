@@ -40,7 +40,8 @@ struct eph_md {
   eph::DevArray<int> rep, flags, cnt, start, bin_of, bcount, bstart, bfill, items, scan_tmp, nbi;
   eph::DevArray<double> box_d;
   eph::NbBuild nbw;
-  int* pinned = nullptr;  // go, nghost, overflow
+  int* pinned = nullptr;  // [0..7] copy of flags, [8] the neighbour check's answer
+  hipEvent_t checked = nullptr;
   std::vector<char> ckpt;  // eph_md_checkpoint_save(md, ctx, NULL) keeps it here
 
   int fail(int code, const std::string& m) { err = m; return code; }
@@ -50,6 +51,7 @@ struct eph_md {
   }
   ~eph_md() {
     if (pinned) (void)hipHostFree(pinned);
+    if (checked) (void)hipEventDestroy(checked);
   }
   void wrap();
   void build_ghosts();
@@ -61,4 +63,10 @@ struct eph_md {
     x_build.assign(x.begin(), x.begin() + 3 * (size_t)nlocal);
   }
   int upload(eph_context* ctx);
+  // Ghost update and pair force of one step on device lists, the lists rebuilt
+  // first where an atom moved more than skin/2 (or force).  ev (optional): ev[2],
+  // ev[3] recorded around ghost update and pair force.  *overflow: the rebuild
+  // does not fit and the host has to do it (no ghost update, no pair force then).
+  int neighbours_and_pair(eph_context* ctx, bool force, hipEvent_t* ev, bool* rebuilt, bool* overflow);
+  int ghosts_and_pair(eph_context* ctx, hipEvent_t* ev);
 };

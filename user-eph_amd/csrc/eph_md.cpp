@@ -243,7 +243,8 @@ int eph_md::upload(eph_context* ctx) {
   EPH_HIP(this, hipMemcpyAsync(box_d.p + 9, gl, sizeof gl, hipMemcpyHostToDevice, s));
   const int nbv[4] = {nb[0], nb[1], nb[2], 0};
   EPH_HIP(this, hipMemcpyAsync(nbi.p, nbv, sizeof nbv, hipMemcpyHostToDevice, s));
-  if (!pinned) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&pinned), 8 * sizeof(int)));
+  if (!pinned) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&pinned), 16 * sizeof(int)));
+  if (!checked) EPH_HIP(this, hipEventCreateWithFlags(&checked, hipEventDisableTiming));
   NbBuild& w = nbw;
   w.nlocal = nlocal; w.ghost_cap = ghost_cap; w.nbins = nbins;
   w.at.pos = ctx->pos.p; w.at.vel = ctx->vel.p; w.at.type = ctx->type.p; w.at.mask = ctx->mask.p;
@@ -263,6 +264,59 @@ int eph_md::upload(eph_context* ctx) {
   EPH_HIP(this, hipStreamSynchronize(s));
   if (pinned[0]) return fail(EPH_ERR_STATE, "pair list refused on the device (index or row width)");
   return EPH_OK;
+}
+
+int eph_md::ghosts_and_pair(eph_context* ctx, hipEvent_t* ev) {
+  hipStream_t s = ctx->stream;
+  if (ev) EPH_HIP(this, hipEventRecord(ev[2], s));
+  EPH_HIP(this, launch_ghost_xv(ctx->atoms_view(), ctx->ghost_owner.p, ctx->ghost_shift.p, s));
+  EPH_HIP(this, launch_lj(ctx->atoms_view(), lj_nbr.p, lj_nn.p, lj_stride, cfg.lj_eps, cfg.lj_sigma,
+                          cfg.cut_lj * cfg.cut_lj, s));
+  if (ev) EPH_HIP(this, hipEventRecord(ev[3], s));
+  return EPH_OK;
+}
+
+// Up to this many atoms the ghost update and the pair force are queued behind
+// the check before the host has its answer, so that the device has work while
+// the host waits (about 10 us); a rebuild then runs them again.  Above, the
+// pair force run in vain (37 us at 32,000 atoms, 145 at 256,000) costs more
+// than the waits it covers once lists are rebuilt every few steps.
+constexpr int kSpeculateAtoms = 65536;
+
+int eph_md::neighbours_and_pair(eph_context* ctx, bool force, hipEvent_t* ev, bool* rebuilt,
+                                bool* overflow) {
+  hipStream_t s = ctx->stream;
+  *rebuilt = *overflow = false;
+  volatile int* want = pinned + 8;
+  const bool ahead = !force && nlocal <= kSpeculateAtoms;
+  *want = force ? 1 : 0;
+  if (!force) {
+    const double lim = 0.25 * cfg.skin * cfg.skin;
+    EPH_HIP(this, launch_nb_want(nlocal, ctx->pos.p, xref.p, lim, pinned + 8, s));
+    if (ahead) {
+      EPH_HIP(this, hipEventRecord(checked, s));
+      if (int rc = ghosts_and_pair(ctx, ev)) return rc;
+      EPH_HIP(this, hipEventSynchronize(checked));
+    } else {
+      EPH_HIP(this, hipStreamSynchronize(s));
+    }
+  }
+  if (*want) {
+    EPH_HIP(this, launch_nb_force(nbw.go, s));
+    EPH_HIP(this, launch_nb_build(nbw, s));
+    EPH_HIP(this, hipMemcpyAsync(pinned, flags.p, 8 * sizeof(int), hipMemcpyDeviceToHost, s));
+    EPH_HIP(this, hipStreamSynchronize(s));
+    if (pinned[1]) {  // capacity exceeded
+      *overflow = true;
+      EPH_HIP(this, launch_fill_int(flags.p + 1, 1, 0, s));
+      return EPH_OK;
+    }
+    ctx->nghost = pinned[7];
+    nghost = ctx->nghost;
+    *rebuilt = true;
+  }
+  if (ahead && !*rebuilt) return EPH_OK;
+  return ghosts_and_pair(ctx, ev);
 }
 
 // copy the device-built system back into the host arrays (for checking)
@@ -567,7 +621,7 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
   for (auto& e : evs) EPH_HIP(md, hipEventCreate(&e));
   double t_fix = 0, t_total = 0, t_pair = 0, t_rebuild = 0;
   int nreb = 0;
-  const double lim = 0.25 * md->cfg.skin * md->cfg.skin;
+  const double lim = 0.25 * md->cfg.skin * md->cfg.skin;  // (host rebuilds)
   const int nbp = std::min(1024, std::max(1, (md->nlocal + kBlock - 1) / kBlock));
   std::vector<double> part(nbp);
   int rc = EPH_OK;
@@ -590,28 +644,17 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
       md->nbw.lists.ncand = cw.ncand;
       md->nbw.lists.cand2 = cw.rcand2;
       md->nbw.cref = cw.cref;
-      EPH_HIP(md, launch_nb_check(md->nlocal, ctx->pos.p, md->xref.p, lim, md->nbw.go, s));
-      if (md->force_next) EPH_HIP(md, launch_nb_force(md->nbw.go, s));
+      const bool force = md->force_next;
       md->force_next = false;
-      const hipError_t eb = launch_nb_build(md->nbw, s);
+      bool rebuilt = false;
+      rc = md->neighbours_and_pair(ctx, force, ev, &rebuilt, &host_rebuild);
       // the candidate buffers belong to this step's launch only (the
       // context may reallocate them before the next)
       md->nbw.lists.cand = nullptr;
       md->nbw.lists.ncand = nullptr;
       md->nbw.cref = nullptr;
-      EPH_HIP(md, eb);
-      EPH_HIP(md, hipMemcpyAsync(md->pinned, md->flags.p, 8 * sizeof(int), hipMemcpyDeviceToHost, s));
-      EPH_HIP(md, hipStreamSynchronize(s));
-      if (md->pinned[0]) {
-        if (md->pinned[1]) {
-          host_rebuild = true;  // capacity exceeded: rebuild through the host
-          EPH_HIP(md, launch_fill_int(md->flags.p + 1, 1, 0, s));
-        } else {
-          ctx->nghost = md->pinned[7];
-          md->nghost = ctx->nghost;
-          ++nreb;
-        }
-      }
+      if (rc) break;
+      if (rebuilt) ++nreb;
     } else {
       EPH_HIP(md, launch_max_disp2(ctx->atoms_view(), md->xref.p, md->partial.p, nbp, s));
       EPH_HIP(md, hipMemcpyAsync(part.data(), md->partial.p, nbp * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -630,11 +673,7 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
       ++nreb;
       t_rebuild += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
-    EPH_HIP(md, hipEventRecord(ev[2], s));
-    EPH_HIP(md, launch_ghost_xv(ctx->atoms_view(), ctx->ghost_owner.p, ctx->ghost_shift.p, s));
-    EPH_HIP(md, launch_lj(ctx->atoms_view(), md->lj_nbr.p, md->lj_nn.p, md->lj_stride, md->cfg.lj_eps,
-                          md->cfg.lj_sigma, md->cfg.cut_lj * md->cfg.cut_lj, s));
-    EPH_HIP(md, hipEventRecord(ev[3], s));
+    if ((!md->device_rebuild || host_rebuild) && (rc = md->ghosts_and_pair(ctx, ev))) break;
     if ((rc = ctx->dev_post_force())) break;
     // nothing runs between the two hooks here: one pass where the deposit allows
     if ((rc = ctx->dev_final_integrate_end_of_step(step))) break;

@@ -85,6 +85,9 @@ struct NbBuild {
 
 hipError_t launch_nb_check(int nlocal, const double4* pos, const double4* ref, double lim, int* go,
                            hipStream_t s);
+// *want (pinned host memory, cleared by the host) = 1 when an atom moved too far
+hipError_t launch_nb_want(int nlocal, const double4* pos, const double4* ref, double lim, int* want,
+                          hipStream_t s);
 hipError_t launch_nb_force(int* go, hipStream_t s);
 hipError_t launch_nb_build(const NbBuild& w, hipStream_t s);
 
