@@ -23,15 +23,15 @@ struct AdjStepView {
 
 // Adjoint accumulators (zeroed by the host where a step needs it).
 struct AdjBuffers {
-  double4* xb = nullptr;   // dL/dx' [nall]
-  double4* vhb = nullptr;  // dL/dvh [nall]
-  double4* wb = nullptr;   // dL/dw [nall]
+  double4* xb = nullptr;   // dL/dx' [nlocal]
+  double4* vhb = nullptr;  // dL/dvh [nlocal]
+  double4* wb = nullptr;   // dL/dw [nlocal]
   double4* vnb = nullptr;  // dL/dv' [nlocal]
-  double4* fEb = nullptr;  // dL/df_EPH from the deposit [nlocal]
-  double4* fRb = nullptr;  // dL/df_RNG from the deposit [nlocal]
+  double4* fEb = nullptr;  // dL/df_EPH: the deposit's part, then the whole [nlocal]
+  double4* fRb = nullptr;  // dL/df_RNG likewise, then times eta sqrt(T_e) [nlocal]
   double4* ftb = nullptr;  // dL/df_total [nlocal]
-  double* ab = nullptr;    // dL/dalpha [nall]
-  double* rb = nullptr;    // dL/drho [nall]
+  double* ab = nullptr;    // dL/dalpha [nlocal]
+  double* rb = nullptr;    // dL/drho [nlocal]
   double* Tb = nullptr;    // dL/dT_e at post_force [G]
   double* Gb = nullptr;    // dL/d(alpha table coefficients) [n_elem][n_beta][4]
 };
