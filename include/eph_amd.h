@@ -221,18 +221,18 @@ int eph_sync(eph_context* ctx);
 void* eph_stream(eph_context* ctx);
 
 /* Kernel forms of the two neighbour sweeps (no counterpart in the reference;
- * every form gives the same bits).  0: one 256-thread block per 256 atoms,
- * spline tables read through the caches (the force sweep's waves fetch their
- * neighbours' records together, 8 lanes per record, through LDS); 1, 2, 3:
+ * every form gives the same bits).  0: spline tables read through the caches,
+ * a wave's neighbour records fetched together through LDS; 16, 8 or 4 lanes
+ * per atom on smaller systems, one thread per atom (256 atoms per block) on
+ * larger ones; 1, 2, 3:
  * persistent blocks of 1024, 512 or 256 threads (one per CU: 4, 2 or 1 waves
  * per SIMD) with the rho(r^2) tables staged in LDS (only when they fit); -1:
- * chosen by system size (the default: form 1 for the density sweep of large
- * systems, form 0 otherwise).  eph_autotune times every form of each sweep on
+ * chosen by system size (the default: form 0).  eph_autotune times every form of each sweep on
  * the resident atoms (after eph_dev_post_force or the harness's attach) and
  * keeps the fastest; forms[2] receives the choice (density, force) and
  * ms[2 * EPH_SWEEP_FORMS] the times (density forms, then force forms; 0 for
- * a form the device cannot run).  f is not changed.  Forms 4, 5, 6 are form 0
- * held to 4, 3 or 2 blocks per CU (fewer neighbour records in flight per L2,
+ * a form the device cannot run).  f is not changed.  Forms 4, 5, 6 are form 0 with
+ * one thread per atom, held to 4, 3 or 2 blocks per CU (fewer neighbour records in flight per L2,
  * less latency hidden). */
 /* Candidate list of the density sweep (no counterpart in the reference; the
  * results are the same bits either way).  In form 0 (and 4-6) the rho loop of a

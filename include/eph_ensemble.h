@@ -58,9 +58,9 @@ int eph_ensemble_setup(eph_ensemble* e, long long first_step);
 int eph_ensemble_run(eph_ensemble* e, int nsteps, int use_graph, double* ms, int* rebuilt);
 
 /* Forms of the density and force sweeps, numbered as eph_set_sweep_forms
- * numbers them: 0 one chunk of a replica per 256-thread block, tables read
- * through the caches; 1, 2, 3 persistent blocks of 1024, 512, 256 threads with
- * the tables in LDS, walking tiles of 4, 2, 1 chunks; 4, 5, 6 form 0 held to
+ * numbers them: 0 tables read through the caches, 16, 8 or 4 lanes per atom
+ * in smaller batches and one chunk of a replica per 256-thread block in larger ones; 1, 2, 3 persistent blocks of 1024, 512, 256 threads with
+ * the tables in LDS, walking tiles of 4, 2, 1 chunks; 4, 5, 6 one chunk per block held to
  * 4, 3, 2 blocks per CU.  Every form gives the same bits. */
 #define EPH_ENSEMBLE_FORMS 7
 

@@ -431,6 +431,182 @@ __device__ __forceinline__ void density_w_atom_coop(const int i_lane, const bool
   if (valid) density_finish<XI>(i, grp, pi, rho, alpha, wx, wy, wz, a, p, w);
 }
 
+// ------------------------------------------------- several lanes per atom
+// The split forms of the sweeps, for systems that do not fill the chip at one
+// thread per atom (a list is then a serial chain of 20 to 40 gathers).  A wave
+// takes 64 / S atoms, S lanes each; the lanes of an atom compute S list entries
+// side by side and U such rows per round.  The terms go to LDS and are added
+// there in list order, one component per lane, so that each sum rounds as the
+// one-thread loop does; entries that do not count contribute +0, which leaves
+// a sum that started at +0 unchanged.  The records are fetched by the wave
+// together, as in the one-thread forms.  Bound by the latency of index, record
+// and table loads on small systems; the rounding of the lists to rows of S and
+// the sums through LDS make it slower than one thread per atom on large ones
+// (see split_density).
+// LDS per wave in 16-B units: the staged records, which the terms then overwrite
+constexpr int split_stage_w(int ur, int uw) { return ur * 128 > uw * 256 ? ur * 128 : uw * 256; }
+constexpr int split_stage_f(int u) { return u * kCoopStage; }
+constexpr int split_stage_lj(int u) { return u * 128; }
+
+// Lanes s < NC of each atom's 16 add component s of the round's U x 16 entries
+// to acc in order; the terms are laid out [atom][entry][NC].
+template <int S, int U, int NC>
+static __device__ __forceinline__ double split_add(double acc, const double* terms, int grp, int s) {
+  static_assert(NC <= S, "one lane per component");
+  if (s < NC) {
+    const double* t = terms + grp * (U * S * NC) + s;
+#pragma unroll
+    for (int m = 0; m < U * S; ++m) acc += t[m * NC];
+  }
+  return acc;
+}
+
+// the round's reads of LDS have returned: the next round's copies, which are
+// not ordered with them, may overwrite it
+static __device__ __forceinline__ void split_round_end() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  wave_lds_sync();
+}
+
+// density_w_atom in the split form.  first64: the first atom of the aligned 64
+// that form one wave of the other forms (the candidate test is theirs, so the
+// waves that scan their full lists are the same), n64: how many there are.
+template <int S, int UR, int UW, int XI, bool FRIC, bool MULTI>
+__device__ __forceinline__ void density_w_atom_split(const int i_atom, const bool valid,
+                                                     const int first64, const int n64,
+                                                     const AtomsView& a, const TablesView& t,
+                                                     const StepParams& p, const WorkView& w,
+                                                     double2* stage, const int rep = -1) {
+  const int i = valid ? i_atom : 0;
+  const int stride = a.stride;
+  const int lane = threadIdx.x & 63, s = lane & (S - 1), ga = lane / S;
+  const double4* __restrict__ rtab = t.rho_r2;
+  double* terms = reinterpret_cast<double*>(stage);
+  const double4 pi = a.pos[i];
+  const bool grp = valid && (a.mask[i] & a.groupbit) != 0;
+  const bool keep = w.rcand2 > 0.0;
+  bool use_cand = false, take = false;
+  if (keep) {
+    const int nm = w.cstate[2];
+    take = w.cstate[0] == 0;
+    use_cand = !take && nm <= w.moved_cap;
+    if (use_cand && nm > 0) {
+      const bool in = lane < n64;
+      use_cand = !wave_near_moved(in, a.pos[first64 + (in ? lane : 0)], w, nm, rep);
+    }
+    if (!use_cand && lane == 0 && i_atom == first64) atomicAdd(w.cstate + 1, 1);
+  }
+  const int* __restrict__ list = use_cand ? w.cand : w.nbr;
+  const int nn = grp ? (use_cand ? w.ncand[i] : w.nnbr[i]) : 0;
+  const int nnmax = wave_max(nn);
+  double rho = 0.0;
+  int na = 0, nc = 0;
+  {
+    constexpr int U = UR;
+    const double2* __restrict__ pos2 = reinterpret_cast<const double2*>(a.pos);
+    for (int k0 = 0; k0 < nnmax; k0 += U * S) {
+      int jj[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + S * u + s;
+        jj[u] = k < nn ? list[k * stride + i] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k0 + S * u < nnmax) coop_fetch_pos(pos2, jj[u], lane, stage + 128 * u);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      wave_lds_sync();
+      double v[U];
+      bool act[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + S * u + s;
+        v[u] = 0.0;
+        act[u] = false;
+        if (k0 + S * u < nnmax) {
+          const double4 pj = coop_read_pos(stage + 128 * u, lane);
+          const double ex = pj.x - pi.x, ey = pj.y - pi.y, ez = pj.z - pi.z;
+          const double r2 = ex * ex + ey * ey + ez * ez;
+          act[u] = k < nn && r2 < t.rc2;
+          if (act[u]) v[u] = rho_r2_at(rtab, t, MULTI ? static_cast<int>(pj.w) : 0, r2);
+          // the entries that count, in list order behind those of the rows before
+          const unsigned bits = static_cast<unsigned>(__ballot(act[u]) >> (S * ga)) & ((1u << S) - 1u);
+          if (act[u]) w.act[(na + __popc(bits & ((1u << s) - 1u))) * stride + i] = jj[u];
+          na += __popc(bits);
+          if (take) {
+            const bool in = k < nn && r2 < w.rcand2;
+            const unsigned cb = static_cast<unsigned>(__ballot(in) >> (S * ga)) & ((1u << S) - 1u);
+            if (in) w.cand[(nc + __popc(cb & ((1u << s) - 1u))) * stride + i] = jj[u];
+            nc += __popc(cb);
+          }
+        }
+      }
+      wave_lds_sync();
+#pragma unroll
+      for (int u = 0; u < U; ++u) terms[ga * (U * S) + S * u + s] = v[u];
+      wave_lds_sync();
+      // all 16 lanes keep the sum
+      const double* tm = terms + ga * (U * S);
+#pragma unroll
+      for (int m = 0; m < U * S; ++m) rho += tm[m];
+      split_round_end();
+    }
+  }
+  if (valid && s == 0) {
+    w.nact[i] = na;
+    if (take) w.ncand[i] = nc;
+  }
+  const double alpha = density_alpha<MULTI>(grp, rho, pi, t, w);
+  double wx = 0.0, wy = 0.0, wz = 0.0;
+  if (FRIC) {
+    constexpr int U = UW;
+    const int nw = (grp && rho > 0.0) ? na : 0;
+    const int nwmax = wave_max(nw);
+    const double4 vi = w.vw[i];
+    const double2* __restrict__ pv2 = reinterpret_cast<const double2*>(w.pv);
+    double acc = 0.0;
+    // (the active list was written by other lanes of this wave, whose memory
+    // operations stay in order)
+    for (int k0 = 0; k0 < nwmax; k0 += U * S) {
+      int jj[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + S * u + s;
+        jj[u] = k < nw ? w.act[k * stride + i] : 0;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k0 + S * u < nwmax) coop_fetch_pv(pv2, jj[u], lane, stage + 256 * u);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      wave_lds_sync();
+      double tx[U], ty[U], tz[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        tx[u] = ty[u] = tz[u] = 0.0;
+        if (k0 + S * u < nwmax) {
+          double4 pj, vj;
+          coop_read_pv(stage + 256 * u, lane, &pj, &vj);
+          if (k0 + S * u + s < nw)
+            density_w_pair<MULTI>(pi, vi, pj, vj, rho, alpha, t, rtab, &tx[u], &ty[u], &tz[u]);
+        }
+      }
+      wave_lds_sync();
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        double* q = terms + (ga * (U * S) + S * u + s) * 3;
+        q[0] = tx[u]; q[1] = ty[u]; q[2] = tz[u];
+      }
+      wave_lds_sync();
+      acc = split_add<S, U, 3>(acc, terms, ga, s);
+      split_round_end();
+    }
+    wx = __shfl(acc, ga * S);
+    wy = __shfl(acc, ga * S + 1);
+    wz = __shfl(acc, ga * S + 2);
+  }
+  if (valid && s == 0) density_finish<XI>(i, grp, pi, rho, alpha, wx, wy, wz, a, p, w);
+}
+
 // Before the sweep, over all nall = nlocal + nghost atoms: on a step that
 // retakes the candidates, the reference positions are the current ones;
 // otherwise every atom 0.45 delta or farther from its reference position (a
@@ -488,6 +664,20 @@ __global__ void k_cand_flags(int* cstate, int moved_cap) {
   cstate[0] = retake || cstate[2] <= moved_cap ? 1 : 0;
   cstate[1] = 0;
   cstate[2] = 0;
+}
+
+// the split form: 16 atoms per block
+template <int S, int UR, int UW, int XI, bool FRIC, bool MULTI>
+__global__ __launch_bounds__(kBlock) void k_density_w_split(AtomsView a, TablesView t, StepParams p,
+                                                            WorkView w) {
+  __shared__ double2 s_split[(kBlock / 64) * split_stage_w(UR, UW)];
+  const int wv = threadIdx.x >> 6;
+  const int base = xcd_block() * (kBlock / S) + wv * (64 / S);
+  if (base >= a.nlocal) return;
+  const int i = base + (threadIdx.x & 63) / S;
+  const int f64 = base & ~63;
+  density_w_atom_split<S, UR, UW, XI, FRIC, MULTI>(i, i < a.nlocal, f64, min(64, a.nlocal - f64), a, t, p, w,
+                                        s_split + wv * split_stage_w(UR, UW));
 }
 
 // 256 atoms per block, tables through the caches, cooperative gathers
@@ -910,6 +1100,88 @@ __device__ __forceinline__ void prl_forces_atom_coop(const int i_lane, const boo
   // the last copies land before the wave may leave
   __builtin_amdgcn_s_waitcnt(kWaitVm0);
   if (valid) prl_finish<FRIC, RAND>(i, on, pi, fe, fr, a, g, p, w);
+}
+
+// prl_forces_atom in the split form (see S)
+template <int S, int U, bool FRIC, bool RAND, bool MULTI>
+__device__ __forceinline__ void prl_forces_atom_split(const int i_atom, const bool valid,
+                                                      const AtomsView& a, const TablesView& t,
+                                                      const GridView& g, const StepParams& p,
+                                                      const WorkView& w, double2* stage) {
+  constexpr int NC = (FRIC ? 3 : 0) + (RAND ? 3 : 0);
+  const int i = valid ? i_atom : 0;
+  const int stride = a.stride;
+  const int lane = threadIdx.x & 63, s = lane & (S - 1), ga = lane / S;
+  const double4* __restrict__ rtab = t.rho_r2;
+  double* terms = reinterpret_cast<double*>(stage);
+  const bool grp = valid && (a.mask[i] & a.groupbit) != 0;
+  const double4 rwi = w.rec[i].rw, pi = w.rec[i].p, xai = w.rec[i].xa;
+  const bool on = grp && rwi.w > 0.0;
+  const int ei = MULTI ? static_cast<int>(pi.w) : 0;
+  const int na = on ? w.nact[i] : 0;
+  const int nmax = wave_max(na);
+  const double2* __restrict__ recs = reinterpret_cast<const double2*>(w.rec);
+  double acc = 0.0;
+  for (int k0 = 0; k0 < nmax; k0 += U * S) {
+    int jj[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + S * u + s;
+      jj[u] = k < na ? w.act[k * stride + i] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (k0 + S * u < nmax) coop_fetch6(recs, jj[u], lane, stage + kCoopStage * u);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    wave_lds_sync();
+    double te[U][3], tr[U][3];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) te[u][d] = tr[u][d] = 0.0;
+      if (k0 + S * u < nmax) {
+        const double2* m = stage + kCoopStage * u + 6 * lane;
+        const double4 pj = make_double4(m[0].x, m[0].y, m[1].x, m[1].y);
+        const double4 rwj = make_double4(m[2].x, m[2].y, m[3].x, m[3].y);
+        const double4 xaj = make_double4(m[4].x, m[4].y, m[5].x, m[5].y);
+        if (k0 + S * u + s < na && rwj.w > 0.0)
+          // 0 - t and 0 + t: the signs the sums take the terms with
+          prl_pair<FRIC, RAND, MULTI>(pi, rwi, xai, ei, pj, rwj, xaj, t, rtab, te[u], tr[u]);
+      }
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      double* q = terms + (ga * (U * S) + S * u + s) * NC;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        if (FRIC) q[d] = te[u][d];
+        if (RAND) q[NC - 3 + d] = tr[u][d];
+      }
+    }
+    wave_lds_sync();
+    acc = split_add<S, U, NC>(acc, terms, ga, s);
+    split_round_end();
+  }
+  double fe[3], fr[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    fe[d] = FRIC ? __shfl(acc, ga * S + d) : 0.0;
+    fr[d] = RAND ? __shfl(acc, ga * S + NC - 3 + d) : 0.0;
+  }
+  if (valid && s == 0) prl_finish<FRIC, RAND>(i, on, pi, fe, fr, a, g, p, w);
+}
+
+template <int S, int U, bool FRIC, bool RAND, bool MULTI>
+__global__ __launch_bounds__(kBlock) void k_prl_forces_split(AtomsView a, TablesView t, GridView g,
+                                                             StepParams p, WorkView w) {
+  __shared__ double2 s_split[(kBlock / 64) * split_stage_f(U)];
+  const int wv = threadIdx.x >> 6;
+  const int base = xcd_block() * (kBlock / S) + wv * (64 / S);
+  if (base >= a.nlocal) return;
+  const int i = base + (threadIdx.x & 63) / S;
+  prl_forces_atom_split<S, U, FRIC, RAND, MULTI>(i, i < a.nlocal, a, t, g, p, w,
+                                           s_split + wv * split_stage_f(U));
 }
 
 // 256 atoms per block, tables through the caches, cooperative gathers
@@ -1718,72 +1990,74 @@ __global__ __launch_bounds__(kBlock) void k_peratom(AtomsView a, TablesView t, W
 
 // ---------------------------------------------------------- harness
 // pair lj/cut, full list, Newton off: f_i = sum_j fpair (x_i - x_j), summed
-// in list order.  The neighbours' positions come through LDS as in the
-// density sweep's rho loop (coop_fetch_pos, kLjU entries per iteration, the
-// next entries' copies in flight while these are summed); the whole wave runs
-// to its longest list.
-constexpr int kLjU = 4;
+// in list order, S lanes per atom (see "several lanes per atom").  The next
+// round's indices travel while a round is summed.  One thread per atom took 42
+// us up to 32,000 atoms and 156 us for 256,000; with 16 lanes 14 us for 256
+// and 15 for 4000, with 8 lanes 26 for 32,000 and 135 for 256,000 (times with
+// the event pair around them).  Bound by latency, then by the vector memory
+// path (140 entries, 78 of them inside the cutoff).
+template <int S, int U>
 __global__ __launch_bounds__(kBlock) void k_lj(AtomsView a, const int* __restrict__ nbr,
-                                               const int* __restrict__ nn, int stride, double lj1,
-                                               double lj2, double rc2) {
-  __shared__ double2 s_lj[(kBlock / 64) * kLjU * 128];
-  const int base = xcd_block() * kBlock;
-  if (base + static_cast<int>(threadIdx.x & ~63u) >= a.nlocal) return;  // whole wave past the end
-  const int i_lane = base + threadIdx.x;
-  const bool valid = i_lane < a.nlocal;
-  const int i = valid ? i_lane : 0;
-  const int lane = threadIdx.x & 63;
-  double2* stage = s_lj + (threadIdx.x >> 6) * kLjU * 128;
+                                                     const int* __restrict__ nn, int stride,
+                                                     double lj1, double lj2, double rc2) {
+  __shared__ double2 s_split[(kBlock / 64) * split_stage_lj(U)];
+  const int wv = threadIdx.x >> 6;
+  double2* stage = s_split + wv * split_stage_lj(U);
+  double* terms = reinterpret_cast<double*>(stage);
+  const int base = xcd_block() * (kBlock / S) + wv * (64 / S);
+  if (base >= a.nlocal) return;
+  const int lane = threadIdx.x & 63, s = lane & (S - 1), ga = lane / S;
+  const bool valid = base + ga < a.nlocal;
+  const int i = valid ? base + ga : 0;
   const double2* __restrict__ pos2 = reinterpret_cast<const double2*>(a.pos);
   const double4 pi = a.pos[i];
-  double fx = 0.0, fy = 0.0, fz = 0.0;
   const int n = valid ? nn[i] : 0;
   const int nmax = wave_max(n);
-  constexpr int U = kLjU;
-  int jj[U], nx[U];
+  double acc = 0.0;
+  int jj[U];
 #pragma unroll
-  for (int e = 0; e < U; ++e) jj[e] = e < n ? nbr[e * stride + i] : 0;
+  for (int u = 0; u < U; ++u) jj[u] = S * u + s < n ? nbr[(S * u + s) * stride + i] : 0;
+  for (int k0 = 0; k0 < nmax; k0 += U * S) {
 #pragma unroll
-  for (int e = 0; e < U; ++e) nx[e] = U + e < n ? nbr[(U + e) * stride + i] : 0;
-  if (nmax > 0) {
-#pragma unroll
-    for (int e = 0; e < U; ++e) coop_fetch_pos(pos2, jj[e], lane, stage + 128 * e);
-  }
-  for (int k = 0; k < nmax; k += U) {
+    for (int u = 0; u < U; ++u)
+      if (k0 + S * u < nmax) coop_fetch_pos(pos2, jj[u], lane, stage + 128 * u);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     wave_lds_sync();
-    double4 pq[U];
+    // the next round's indices travel while this round is summed
 #pragma unroll
-    for (int e = 0; e < U; ++e) pq[e] = coop_read_pos(stage + 128 * e, lane);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wave_lds_sync();
-    if (k + U < nmax) {
-#pragma unroll
-      for (int e = 0; e < U; ++e) coop_fetch_pos(pos2, nx[e], lane, stage + 128 * e);
-#pragma unroll
-      for (int e = 0; e < U; ++e) nx[e] = k + 2 * U + e < n ? nbr[(k + 2 * U + e) * stride + i] : 0;
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + S * (U + u) + s;
+      jj[u] = k < n ? nbr[k * stride + i] : 0;
     }
+    double tx[U], ty[U], tz[U];
 #pragma unroll
-    for (int e = 0; e < U; ++e) {
-      if (k + e < n) {
-        const double dx = pi.x - pq[e].x, dy = pi.y - pq[e].y, dz = pi.z - pq[e].z;
+    for (int u = 0; u < U; ++u) {
+      tx[u] = ty[u] = tz[u] = 0.0;
+      if (k0 + S * u < nmax) {
+        const double4 q = coop_read_pos(stage + 128 * u, lane);
+        const double dx = pi.x - q.x, dy = pi.y - q.y, dz = pi.z - q.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
-        if (r2 < rc2) {
+        if (k0 + S * u + s < n && r2 < rc2) {
           const double r2inv = 1.0 / r2;
           const double r6inv = r2inv * r2inv * r2inv;
           const double fpair = r6inv * (lj1 * r6inv - lj2) * r2inv;
-          fx += dx * fpair;
-          fy += dy * fpair;
-          fz += dz * fpair;
+          tx[u] = dx * fpair;
+          ty[u] = dy * fpair;
+          tz[u] = dz * fpair;
         }
       }
     }
+    wave_lds_sync();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      double* q = terms + (ga * (U * S) + S * u + s) * 3;
+      q[0] = tx[u]; q[1] = ty[u]; q[2] = tz[u];
+    }
+    wave_lds_sync();
+    acc = split_add<S, U, 3>(acc, terms, ga, s);
+    split_round_end();
   }
-  if (!valid) return;
-  const int fs = a.fstride;
-  a.f[i] = fx;
-  a.f[fs + i] = fy;
-  a.f[2 * fs + i] = fz;
+  if (valid && s < 3) a.f[s * a.fstride + i] = acc;
 }
 
 __global__ __launch_bounds__(kBlock) void k_max_disp2(AtomsView a, const double4* ref,
@@ -1829,6 +2103,42 @@ __global__ __launch_bounds__(kBlock) void k_density_w_batch(AtomsView a, TablesV
   density_w_atom_coop<XI, FRIC, MULTI>(c.start + threadIdx.x, static_cast<int>(threadIdx.x) < c.count,
                                        a, t, t.rho_r2, pr, w, s_stage + (threadIdx.x >> 6) * kCoopStageW,
                                        c.rep);
+}
+
+// the forms with S lanes per atom: a chunk's kBlock atoms are S blocks
+template <int S, int UR, int UW, int XI, bool FRIC, bool MULTI>
+__global__ __launch_bounds__(kBlock) void k_density_w_batch_split(AtomsView a, TablesView t,
+                                                                  StepParams p, WorkView w,
+                                                                  const Chunk* __restrict__ chunks,
+                                                                  const uint32_t* __restrict__ seeds,
+                                                                  const uint64_t* __restrict__ step) {
+  __shared__ double2 s_split[(kBlock / 64) * split_stage_w(UR, UW)];
+  const Chunk c = chunks[blockIdx.x / S];
+  const int wv = threadIdx.x >> 6;
+  const int first = (blockIdx.x % S) * (kBlock / S) + wv * (64 / S);
+  if (first >= c.count) return;  // whole wave past the chunk
+  StepParams pr = p;
+  pr.seed = seeds[c.rep];
+  pr.step = *step;
+  const int at = first + (threadIdx.x & 63) / S, f64 = first & ~63;
+  density_w_atom_split<S, UR, UW, XI, FRIC, MULTI>(c.start + at, at < c.count, c.start + f64,
+                                                   min(64, c.count - f64), a, t, pr, w,
+                                                   s_split + wv * split_stage_w(UR, UW), c.rep);
+}
+
+template <int S, int U, bool FRIC, bool RAND, bool MULTI>
+__global__ __launch_bounds__(kBlock) void k_prl_forces_batch_split(AtomsView a, TablesView t,
+                                                                   const GridView* __restrict__ grids,
+                                                                   StepParams p, WorkView w,
+                                                                   const Chunk* __restrict__ chunks) {
+  __shared__ double2 s_split[(kBlock / 64) * split_stage_f(U)];
+  const Chunk c = chunks[blockIdx.x / S];
+  const int wv = threadIdx.x >> 6;
+  const int first = (blockIdx.x % S) * (kBlock / S) + wv * (64 / S);
+  if (first >= c.count) return;
+  const int at = first + (threadIdx.x & 63) / S;
+  prl_forces_atom_split<S, U, FRIC, RAND, MULTI>(c.start + at, at < c.count, a, t, grids[c.rep], p, w,
+                                                 s_split + wv * split_stage_f(U));
 }
 
 // start of a recorded step: step += 1
@@ -2132,6 +2442,19 @@ __global__ __launch_bounds__(kBlock) void k_d4_component(const double4* __restri
 // ================================================================ wrappers
 static inline int nblk(long n, int b = kBlock) { return static_cast<int>((n + b - 1) / b); }
 
+// Lanes per atom of the cache-table form (form 0) by system size, 0: one
+// thread per atom.  Measured on crystals of 42 pairs per atom, us per launch
+// (with the event pair around it), one thread / 4 / 8 / 16 lanes:
+//   density   4000 atoms 51 / 24 / 19 / 16, 16,384 56 / 28 / 25 / 30,
+//             32,000 59 / 34 / 35 / 46, 256,000 189 / 174 / 204 / 284,
+//             702,464 440 / 449 / 509 / -
+//   force     4000 atoms 31 / - / 13 / 11, 16,384 34 / - / 18 / 16,
+//             32,000 35 / - / 24 / 28, 55,296 37 / - / 39 / 44
+// The occupancy forms (4 to 6) keep one thread per atom.
+static int split_density(int nlocal) { return nlocal <= 8192 ? 16 : nlocal <= 400000 ? 4 : 0; }
+static int split_force(int nlocal) { return nlocal <= 20000 ? 16 : nlocal <= 50000 ? 8 : 0; }
+constexpr int kSplitLj16 = 16384;
+
 hipError_t launch_ghost_xv(const AtomsView& a, const int* owner, const double4* shift, hipStream_t s) {
   if (a.nghost == 0) return hipSuccess;
   k_ghost_xv<<<nblk(a.nghost), kBlock, 0, s>>>(a, owner, shift);
@@ -2242,15 +2565,19 @@ hipError_t launch_density_w(const AtomsView& a, const TablesView& t, const StepP
     if (ev) (void)hipEventRecord(ev[1], s);
     return hipGetLastError();
   }
-  const int g = nblk(a.nlocal);
+  const int sp = f == 0 ? split_density(a.nlocal) : 0;
+  const int g = nblk(a.nlocal, sp ? kBlock / sp : kBlock);
   const bool keep = w.rcand2 > 0.0 && w.cstate;
   WorkView wc = w;
   if (!keep) wc.rcand2 = 0.0;
   if (keep) k_cand_check<<<nblk(a.nlocal + a.nghost), kBlock, 0, s>>>(a.nlocal + a.nghost, a.pos, wc);
   if (ev) (void)hipEventRecord(ev[0], s);  // the sweep alone, without the candidate check
   const size_t dl = chunk_lds(f, kDensityStageBytes);
-#define EPH_DW(XI, F, M) k_density_w<XI, F, M><<<g, kBlock, dl, s>>>(a, t, p, wc)
-#define EPH_DW_M(XI, F) if (multi) EPH_DW(XI, F, true); else EPH_DW(XI, F, false)
+#define EPH_DW(XI, F, M)                                                                       \
+  if (sp == 16) k_density_w_split<16, 4, 3, XI, F, M><<<g, kBlock, 0, s>>>(a, t, p, wc);      \
+  else if (sp == 4) k_density_w_split<4, 4, 2, XI, F, M><<<g, kBlock, 0, s>>>(a, t, p, wc);   \
+  else k_density_w<XI, F, M><<<g, kBlock, dl, s>>>(a, t, p, wc)
+#define EPH_DW_M(XI, F) if (multi) { EPH_DW(XI, F, true); } else { EPH_DW(XI, F, false); }
 #define EPH_DW_F(XI) if (fric) { EPH_DW_M(XI, true); } else { EPH_DW_M(XI, false); }
   switch (p.xi_mode) {
     case 1: EPH_DW_F(1); break;
@@ -2321,10 +2648,14 @@ hipError_t launch_prl_forces(const AtomsView& a, const TablesView& t, const Grid
 #undef EPH_PFL_M
     return hipGetLastError();
   }
-  const int gr = nblk(a.nlocal);
+  const int sp = f == 0 ? split_force(a.nlocal) : 0;
+  const int gr = nblk(a.nlocal, sp ? kBlock / sp : kBlock);
   const size_t fl = chunk_lds(f, kForceStageBytes);
-#define EPH_PF(F, R, M) k_prl_forces<F, R, M><<<gr, kBlock, fl, s>>>(a, t, g, p, w)
-#define EPH_PF_M(F, R) if (multi) EPH_PF(F, R, true); else EPH_PF(F, R, false)
+#define EPH_PF(F, R, M)                                                                     \
+  if (sp == 16) k_prl_forces_split<16, 1, F, R, M><<<gr, kBlock, 0, s>>>(a, t, g, p, w);   \
+  else if (sp == 8) k_prl_forces_split<8, 1, F, R, M><<<gr, kBlock, 0, s>>>(a, t, g, p, w); \
+  else k_prl_forces<F, R, M><<<gr, kBlock, fl, s>>>(a, t, g, p, w)
+#define EPH_PF_M(F, R) if (multi) { EPH_PF(F, R, true); } else { EPH_PF(F, R, false); }
   if (fric && rnd) { EPH_PF_M(true, true); }
   else if (fric) { EPH_PF_M(true, false); }
   else { EPH_PF_M(false, true); }
@@ -2499,7 +2830,10 @@ hipError_t launch_lj(const AtomsView& a, const int* nbr, const int* nn, int stri
   if (a.nlocal == 0) return hipSuccess;
   const double s6 = sigma * sigma * sigma * sigma * sigma * sigma;
   const double lj1 = 48.0 * eps * s6 * s6, lj2 = 24.0 * eps * s6;
-  k_lj<<<nblk(a.nlocal), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2);
+  if (a.nlocal <= kSplitLj16)
+    k_lj<16, 3><<<nblk(a.nlocal, kBlock / 16), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2);
+  else
+    k_lj<8, 3><<<nblk(a.nlocal, kBlock / 8), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2);
   return hipGetLastError();
 }
 
@@ -2609,8 +2943,14 @@ hipError_t launch_density_w_batch(const AtomsView& a, const TablesView& t, const
   if (!keep) w.rcand2 = 0.0;
   if (keep) k_cand_check_dev<<<nblk(a.nlocal + a.nghost), kBlock, 0, s>>>(a.nlocal, ng, a.pos, rep, w);
   const size_t dl = chunk_lds(variant, kDensityStageBytes);
-#define EPH_DWB(XI, F, M) k_density_w_batch<XI, F, M><<<nchunks, kBlock, dl, s>>>(a, t, p, w, chunks, seeds, step)
-#define EPH_DWB_M(XI, F) if (multi) EPH_DWB(XI, F, true); else EPH_DWB(XI, F, false)
+  const int sp = variant == 0 ? split_density(a.nlocal) : 0;
+#define EPH_DWB_S(S, UR, UW, XI, F, M) \
+  k_density_w_batch_split<S, UR, UW, XI, F, M><<<nchunks * S, kBlock, 0, s>>>(a, t, p, w, chunks, seeds, step)
+#define EPH_DWB(XI, F, M)                             \
+  if (sp == 16) EPH_DWB_S(16, 4, 3, XI, F, M);        \
+  else if (sp == 4) EPH_DWB_S(4, 4, 2, XI, F, M);     \
+  else k_density_w_batch<XI, F, M><<<nchunks, kBlock, dl, s>>>(a, t, p, w, chunks, seeds, step)
+#define EPH_DWB_M(XI, F) if (multi) { EPH_DWB(XI, F, true); } else { EPH_DWB(XI, F, false); }
 #define EPH_DWB_F(XI) if (fric) { EPH_DWB_M(XI, true); } else { EPH_DWB_M(XI, false); }
   switch (p.xi_mode) {
     case 1: EPH_DWB_F(1); break;
@@ -2620,6 +2960,7 @@ hipError_t launch_density_w_batch(const AtomsView& a, const TablesView& t, const
 #undef EPH_DWB_F
 #undef EPH_DWB_M
 #undef EPH_DWB
+#undef EPH_DWB_S
   if (keep) k_cand_flags<<<1, 64, 0, s>>>(w.cstate, w.moved_cap);
   return hipGetLastError();
 }
@@ -2650,13 +2991,20 @@ hipError_t launch_prl_forces_batch(const AtomsView& a, const TablesView& t, cons
     return hipGetLastError();
   }
   const size_t fl = chunk_lds(variant, kForceStageBytes);
-#define EPH_PFB(F, R, M) k_prl_forces_batch<F, R, M><<<nchunks, kBlock, fl, s>>>(a, t, grids, p, w, chunks)
-#define EPH_PFB_M(F, R) if (multi) EPH_PFB(F, R, true); else EPH_PFB(F, R, false)
+  const int sp = variant == 0 ? split_force(a.nlocal) : 0;
+#define EPH_PFB_S(S, F, R, M) \
+  k_prl_forces_batch_split<S, 1, F, R, M><<<nchunks * S, kBlock, 0, s>>>(a, t, grids, p, w, chunks)
+#define EPH_PFB(F, R, M)                  \
+  if (sp == 16) EPH_PFB_S(16, F, R, M);   \
+  else if (sp == 8) EPH_PFB_S(8, F, R, M); \
+  else k_prl_forces_batch<F, R, M><<<nchunks, kBlock, fl, s>>>(a, t, grids, p, w, chunks)
+#define EPH_PFB_M(F, R) if (multi) { EPH_PFB(F, R, true); } else { EPH_PFB(F, R, false); }
   if (fric && rnd) { EPH_PFB_M(true, true); }
   else if (fric) { EPH_PFB_M(true, false); }
   else { EPH_PFB_M(false, true); }
 #undef EPH_PFB_M
 #undef EPH_PFB
+#undef EPH_PFB_S
   return hipGetLastError();
 }
 
