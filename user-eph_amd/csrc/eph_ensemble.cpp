@@ -48,7 +48,7 @@ struct eph_ensemble {
   DevArray<int> rep, flags, cnt, start, bin_of, bcount, bstart, bfill, items, scan_tmp, nbi,
       lj_nbr, lj_nn, rlog;
   DevArray<double> box_d;
-  DevArray<double4> xref;
+  DevArray<double4> xref, bpos;
   NbBuild nbw;
   // fix batching
   DevArray<Chunk> chunks;
@@ -194,6 +194,7 @@ int eph_ensemble::setup(long long first) {
   EPH_HIP(this, start.reserve(cap + 1));
   EPH_HIP(this, bin_of.reserve(cap));
   EPH_HIP(this, items.reserve(cap));
+  EPH_HIP(this, bpos.reserve(cap));
   EPH_HIP(this, bcount.reserve(nbins + 1));
   EPH_HIP(this, bstart.reserve(nbins + 1));
   EPH_HIP(this, bfill.reserve(nbins + 1));
@@ -210,7 +211,7 @@ int eph_ensemble::setup(long long first) {
   w.lists.stride = st;
   w.go = flags.p; w.overflow = flags.p + 1; w.nrebuild = flags.p + 2; w.nghost = flags.p + 4;
   w.cnt = cnt.p; w.start = start.p; w.bin_of = bin_of.p; w.bcount = bcount.p; w.bstart = bstart.p;
-  w.bfill = bfill.p; w.items = items.p; w.scan_tmp = scan_tmp.p; w.xref = xref.p;
+  w.bfill = bfill.p; w.items = items.p; w.bpos = bpos.p; w.scan_tmp = scan_tmp.p; w.xref = xref.p;
   // each rebuild also writes the density sweep's candidate lists, valid at
   // the rebuild's positions (the buffers keep their size for the ensemble's life)
   {

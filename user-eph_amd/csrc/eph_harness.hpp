@@ -30,7 +30,7 @@ struct eph_md {
   eph::CSR fix, lj;
   // device side
   eph::DevArray<int> lj_nbr, lj_nn, lj_off, lj_idx;
-  eph::DevArray<double4> xref;
+  eph::DevArray<double4> xref, bpos;
   eph::DevArray<double> partial;
   int lj_stride = 0;
   // device rebuild (eph_nbuild.hip)

@@ -231,6 +231,7 @@ int eph_md::upload(eph_context* ctx) {
   EPH_HIP(this, start.reserve(cap + 1));
   EPH_HIP(this, bin_of.reserve(cap));
   EPH_HIP(this, items.reserve(cap));
+  EPH_HIP(this, bpos.reserve(cap));
   EPH_HIP(this, bcount.reserve(nbins + 1));
   EPH_HIP(this, bstart.reserve(nbins + 1));
   EPH_HIP(this, bfill.reserve(nbins + 1));
@@ -259,7 +260,7 @@ int eph_md::upload(eph_context* ctx) {
   w.go = flags.p; w.overflow = flags.p + 1; w.nrebuild = flags.p + 2; w.nghost = flags.p + 4;
   w.cand_valid = ctx->cstate.p;
   w.cnt = cnt.p; w.start = start.p; w.bin_of = bin_of.p; w.bcount = bcount.p; w.bstart = bstart.p;
-  w.bfill = bfill.p; w.items = items.p; w.scan_tmp = scan_tmp.p; w.xref = xref.p;
+  w.bfill = bfill.p; w.items = items.p; w.bpos = bpos.p; w.scan_tmp = scan_tmp.p; w.xref = xref.p;
   EPH_HIP(this, hipMemcpyAsync(pinned, ctx->list_bad.p, sizeof(int), hipMemcpyDeviceToHost, s));
   EPH_HIP(this, hipStreamSynchronize(s));
   if (pinned[0]) return fail(EPH_ERR_STATE, "pair list refused on the device (index or row width)");

@@ -268,6 +268,39 @@ __global__ __launch_bounds__(kBlock) void k_nb_lists(int nlocal, const double4* 
   if (l.cand) l.ncand[i] = nc < l.cap_f ? nc : l.cap_f;
 }
 
+// bitonic sort of one wave's 64 E keys, ascending: element n = lane E + s
+template <int E>
+__device__ __forceinline__ void bitonic_wave(uint32_t (&key)[E], const int lane) {
+  constexpr int N = 64 * E;
+#pragma unroll
+  for (int k = 2; k <= N; k <<= 1) {
+#pragma unroll
+    for (int d = k >> 1; d > 0; d >>= 1) {
+      if (d < E) {
+#pragma unroll
+        for (int s = 0; s < E; ++s) {
+          const int ps = s ^ d;
+          if (ps > s) {
+            const bool up = ((lane * E + s) & k) == 0;
+            const uint32_t lo = min(key[s], key[ps]), hi = max(key[s], key[ps]);
+            key[s] = up ? lo : hi;
+            key[ps] = up ? hi : lo;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int s = 0; s < E; ++s) {
+          const int n = lane * E + s;
+          const uint32_t mine = key[s];
+          const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(mine), d / E));
+          const bool keep_min = ((n & d) == 0) == ((n & k) == 0);
+          key[s] = keep_min ? min(mine, other) : max(mine, other);
+        }
+      }
+    }
+  }
+}
+
 // Each atom's fix list into (q(r^2), found position) order, and its
 // candidates (the entries with r^2 < cand2, in list order) rewritten to
 // match: one wave per atom, a bitonic sort of N = 64 E 32-bit keys q x 2^9 + t
@@ -291,34 +324,7 @@ __device__ __forceinline__ void nb_sort_atom(const int i, const int lane, const 
       key[s] = (list_sort_q(ex * ex + ey * ey + ez * ez, l.sort_scale) << 9) | static_cast<uint32_t>(n);
     }
   }
-  constexpr int N = 64 * E;
-#pragma unroll
-  for (int k = 2; k <= N; k <<= 1) {
-#pragma unroll
-    for (int d = k >> 1; d > 0; d >>= 1) {
-      if (d < E) {  // both elements of a pair in this lane
-#pragma unroll
-        for (int s = 0; s < E; ++s) {
-          const int ps = s ^ d;
-          if (ps > s) {
-            const bool up = ((lane * E + s) & k) == 0;
-            const uint32_t lo = min(key[s], key[ps]), hi = max(key[s], key[ps]);
-            key[s] = up ? lo : hi;
-            key[ps] = up ? hi : lo;
-          }
-        }
-      } else {  // the partner element sits in lane ^ (d / E), same slot
-#pragma unroll
-        for (int s = 0; s < E; ++s) {
-          const int n = lane * E + s;
-          const uint32_t mine = key[s];
-          const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(mine), d / E));
-          const bool keep_min = ((n & d) == 0) == ((n & k) == 0);
-          key[s] = keep_min ? min(mine, other) : max(mine, other);
-        }
-      }
-    }
-  }
+  bitonic_wave<E>(key, lane);
   // the indices of the sorted entries, all read before any is written
   int jv[E];
 #pragma unroll
@@ -358,122 +364,6 @@ __device__ __forceinline__ void nb_sort_atom(const int i, const int lane, const 
     }
   }
   if (lane == 63) l.ncand[i] = incl < l.cap_f ? incl : l.cap_f;
-}
-
-// The sort network of nb_sort_atom on one wave's E keys per lane
-template <int E>
-__device__ __forceinline__ void bitonic_wave(uint32_t (&key)[E], const int lane) {
-  constexpr int N = 64 * E;
-#pragma unroll
-  for (int k = 2; k <= N; k <<= 1) {
-#pragma unroll
-    for (int d = k >> 1; d > 0; d >>= 1) {
-      if (d < E) {
-#pragma unroll
-        for (int s = 0; s < E; ++s) {
-          const int ps = s ^ d;
-          if (ps > s) {
-            const bool up = ((lane * E + s) & k) == 0;
-            const uint32_t lo = min(key[s], key[ps]), hi = max(key[s], key[ps]);
-            key[s] = up ? lo : hi;
-            key[ps] = up ? hi : lo;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int s = 0; s < E; ++s) {
-          const int n = lane * E + s;
-          const uint32_t mine = key[s];
-          const uint32_t other = static_cast<uint32_t>(__shfl_xor(static_cast<int>(mine), d / E));
-          const bool keep_min = ((n & d) == 0) == ((n & k) == 0);
-          key[s] = keep_min ? min(mine, other) : max(mine, other);
-        }
-      }
-    }
-  }
-}
-
-// The same sort for lists of at most 256 entries, 64 atoms per block: the
-// list rows of the block's atoms are read and written whole (coalesced)
-// through an LDS tile, and each of the 4 waves sorts 16 of the atoms from it.
-// Rows are padded by one word so that a row-wise and a column-wise pass both
-// avoid bank conflicts.
-template <int E>
-__global__ __launch_bounds__(kBlock) void k_nb_sort_tile(int nlocal, const double4* __restrict__ pos,
-                                                         NbLists l, const int* go) {
-  constexpr int R = 64 * E + 1;
-  __shared__ int s_j[64 * R];        // the block's lists: found order, then sorted
-  __shared__ int s_c[64 * R];        // their candidates
-  __shared__ unsigned char s_cf[64 * 64 * E];  // candidate flag per found position
-  __shared__ int s_nf[64], s_nc[64];
-  if (!*go) return;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int i0 = blockIdx.x * 64; i0 < nlocal; i0 += gridDim.x * 64) {
-    if (threadIdx.x < 64) s_nf[lane] = i0 + lane < nlocal ? l.nn_f[i0 + lane] : 0;
-    __syncthreads();
-    int mx = s_nf[lane];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o));
-    for (int k = wv; k < mx; k += 4)
-      if (k < s_nf[lane]) s_j[lane * R + k] = l.nbr_f[k * l.stride + i0 + lane];
-    __syncthreads();
-    for (int a = wv; a < 64; a += 4) {
-      const int nf = s_nf[a];  // the same for the whole wave
-      if (nf == 0) {
-        if (lane == 0) s_nc[a] = 0;
-        continue;
-      }
-      const int i = i0 + a;
-      const double4 pi = pos[i];
-      uint32_t key[E];
-#pragma unroll
-      for (int s = 0; s < E; ++s) {
-        const int n = lane * E + s;
-        key[s] = ~0u;
-        if (n < nf) {
-          const double4 pj = pos[s_j[a * R + n]];
-          const double ex = pj.x - pi.x, ey = pj.y - pi.y, ez = pj.z - pi.z;
-          const double r2 = ex * ex + ey * ey + ez * ez;
-          key[s] = (list_sort_q(r2, l.sort_scale) << 9) | static_cast<uint32_t>(n);
-          s_cf[a * 64 * E + n] = r2 < l.cand2 ? 1 : 0;
-        }
-      }
-      bitonic_wave<E>(key, lane);
-      int jv[E];
-      int mine = 0;
-#pragma unroll
-      for (int s = 0; s < E; ++s) {
-        const int t = static_cast<int>(key[s] & 511u);
-        const bool in = lane * E + s < nf;
-        jv[s] = in ? s_j[a * R + t] : 0;
-        mine |= (in && s_cf[a * 64 * E + t] ? 1 : 0) << s;
-      }
-      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): every read of row a is back
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int s = 0; s < E; ++s)
-        if (lane * E + s < nf) s_j[a * R + lane * E + s] = jv[s];
-      const int cnt = __builtin_popcount(mine);
-      int incl = cnt;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o);
-        if (lane >= o) incl += v;
-      }
-      int at = incl - cnt;
-#pragma unroll
-      for (int s = 0; s < E; ++s)
-        if ((mine >> s) & 1) s_c[a * R + at++] = jv[s];
-      if (lane == 63) s_nc[a] = incl;
-    }
-    __syncthreads();
-    for (int k = wv; k < mx; k += 4) {
-      if (k < s_nf[lane]) l.nbr_f[k * l.stride + i0 + lane] = s_j[lane * R + k];
-      if (l.cand && k < s_nc[lane]) l.cand[k * l.stride + i0 + lane] = s_c[lane * R + k];
-    }
-    if (l.cand && threadIdx.x < 64 && i0 + lane < nlocal) l.ncand[i0 + lane] = s_nc[lane];
-    __syncthreads();
-  }
 }
 
 constexpr int kSortBlocks = 2048;
@@ -586,6 +476,226 @@ __global__ __launch_bounds__(kSB) void k_nb_scan_apply(const int* in, int n, con
   }
 }
 
+// the atoms' positions in bin order, the index in .w
+__global__ __launch_bounds__(kBlock) void k_nb_bin_pos(int cap, int nlocal, const int* nghost,
+                                                       const double4* __restrict__ pos,
+                                                       const int* __restrict__ items,
+                                                       double4* __restrict__ bpos, const int* go) {
+  if (!*go) return;
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= cap || k >= nlocal + *nghost) return;
+  const int j = items[k];
+  const double4 p = pos[j];
+  bpos[k] = make_double4(p.x, p.y, p.z, __longlong_as_double(j));
+}
+
+// Both lists of TA atoms per block, the fix lists sorted, candidates and all:
+// a wave takes one atom at a time.  The atom's 5 x 5 x 5 stencil is 25 runs of
+// bins that are adjacent in x and so adjacent in bpos; the lanes take the runs'
+// atoms 64 at a time (in the found order of the serial scan), and ballots give
+// each entry its place.  The fix entries' keys are sorted in registers, the
+// rows are collected in LDS and written whole.  (One thread per atom walked
+// the bins' scattered positions and stored one row per lane, and a sort read
+// and wrote the fix rows again.)  A whole rebuild, before and after: 2048
+// atoms 0.60 -> 0.17 ms, 32,000 0.63 -> 0.23, 256,000 1.44 -> 0.77, 2,048,000
+// 9.2 -> 5.0.  Bound by instruction issue: 992 VALU and 128 LDS instructions
+// per atom (counters), 4.6 ms of the 5.0; tiles of 32 atoms, with twice the
+// waves per CU, take the same time.
+// LDS: rows of the pair list, the fix list and the candidates per atom (padded
+// to an odd length), and per wave the keys, their indices and the runs.
+constexpr int kTileWaves = 16, kTileKeys = 256, kTileBlocks = 512;
+struct NbTile {
+  int rl, rf;  // row lengths
+};
+__host__ __device__ inline NbTile nb_tile(const NbLists& l) { return {l.cap_l | 1, l.cap_f | 1}; }
+static size_t nb_tile_lds(const NbLists& l, int ta) {
+  const NbTile t = nb_tile(l);
+  return sizeof(int) * (static_cast<size_t>(ta) * (t.rl + 2 * t.rf + 3) + kTileWaves * (2 * l.cap_f + 64));
+}
+
+template <int E>
+__device__ __forceinline__ int nb_tile_sort(const int nf, const int lane, const uint32_t* key_in,
+                                            const int* jt, int* row_f, int* row_c) {
+  uint32_t key[E];
+#pragma unroll
+  for (int s = 0; s < E; ++s) {
+    const int n = lane * E + s;
+    key[s] = n < nf ? key_in[n] : ~0u;
+  }
+  bitonic_wave<E>(key, lane);
+  int jv[E], mine = 0;
+#pragma unroll
+  for (int s = 0; s < E; ++s) {
+    const bool in = lane * E + s < nf;
+    jv[s] = in ? jt[key[s] & 511u] : 0;
+    mine |= (jv[s] < 0 ? 1 : 0) << s;  // the top bit marks a candidate
+    jv[s] &= 0x7fffffff;
+    if (in) row_f[lane * E + s] = jv[s];
+  }
+  const int cnt = __builtin_popcount(mine);
+  int incl = cnt;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o);
+    if (lane >= o) incl += v;
+  }
+  int at = incl - cnt;
+#pragma unroll
+  for (int s = 0; s < E; ++s)
+    if ((mine >> s) & 1) row_c[at++] = jv[s];
+  return __shfl(incl, 63);
+}
+
+template <int TA>
+__global__ __launch_bounds__(64 * kTileWaves) void k_nb_lists_tile(
+    int nlocal, const double4* __restrict__ pos, const int* __restrict__ rep, NbBoxes b,
+    const int* __restrict__ bstart, const double4* __restrict__ bpos, NbLists l, int* overflow,
+    const int* go) {
+  if (!*go) return;
+  extern __shared__ int s_nb[];
+  const NbTile tl = nb_tile(l);
+  int* s_l = s_nb;
+  int* s_f = s_l + TA * tl.rl;
+  int* s_c = s_f + TA * tl.rf;
+  int* s_n = s_c + TA * tl.rf;  // [3][TA] row counts: pair, fix, candidates
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  int* mine = s_n + 3 * TA + wv * (2 * l.cap_f + 64);
+  uint32_t* s_key = reinterpret_cast<uint32_t*>(mine);
+  int* s_jt = mine + l.cap_f;
+  int* s_pre = s_jt + l.cap_f;  // [32] atoms before each run, [32] where the run starts less that
+  int* s_beg = s_pre + 32;
+  const double reach2 = b.cg * b.cg * (1.0 + 1e-9);
+  // A fixed grid walks the tiles, so that a step without a rebuild costs one
+  // flag read per resident block; the tiles of XCD x form one range.
+  const int ntiles = (nlocal + TA - 1) / TA, x8 = blockIdx.x % 8;
+  const int last = static_cast<int>(static_cast<long>(ntiles) * (x8 + 1) / 8);
+  for (int tile = static_cast<int>(static_cast<long>(ntiles) * x8 / 8) + blockIdx.x / 8; tile < last;
+       tile += gridDim.x / 8) {
+    const int i0 = tile * TA;
+    for (int a = wv; a < TA; a += kTileWaves) {
+      const int i = i0 + a;
+      int nf = 0, nl = 0, nc = 0;
+      if (i < nlocal) {
+        const int r = rep[i];
+        const double4 pi = pos[i];
+        const int* nb = b.nb + 3 * r;
+        const double* glo = b.glo + 3 * r;
+        const int bc[3] = {bin_coord(pi.x, glo[0], b.bs, nb[0]), bin_coord(pi.y, glo[1], b.bs, nb[1]),
+                           bin_coord(pi.z, glo[2], b.bs, nb[2])};
+        // Squared distance from the atom to a bin slab; edge bins also hold the
+        // atoms clamped into them and count as near.
+        auto slab2 = [&](double x, int d, int c) {
+          const double lo = glo[d] + c * b.bs, hi = lo + b.bs;
+          const double g = (c <= 0 || c >= nb[d] - 1) ? 0.0 : (x < lo ? lo - x : (x > hi ? x - hi : 0.0));
+          return g * g;
+        };
+        // lane 5 (dz + 2) + (dy + 2): the run of x bins within reach (between
+        // the first and the last of them; bins farther than reach hold no entry)
+        int beg = 0, len = 0;
+        const int z = bc[2] + lane / 5 - 2, y = bc[1] + lane % 5 - 2;
+        if (lane < 25 && z >= 0 && z < nb[2] && y >= 0 && y < nb[1]) {
+          const double yz = slab2(pi.y, 1, y) + slab2(pi.z, 2, z);
+          int x0 = 1 << 30, x1 = -1;
+          for (int x = max(bc[0] - 2, 0); x <= min(bc[0] + 2, nb[0] - 1); ++x)
+            if (slab2(pi.x, 0, x) + yz <= reach2) {
+              x0 = min(x0, x);
+              x1 = x;
+            }
+          if (x1 >= 0) {
+            const int bin = b.bin_base[r] + nb[0] * (y + nb[1] * z);
+            beg = bstart[bin + x0];
+            len = bstart[bin + x1 + 1] - beg;
+          }
+        }
+        int incl = len;
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) {
+          const int v = __shfl_up(incl, o);
+          if (lane >= o) incl += v;
+        }
+        const int total = __shfl(incl, 31);
+        if (lane < 32) {
+          s_pre[lane] = incl - len;
+          s_beg[lane] = beg - (incl - len);
+        }
+        __builtin_amdgcn_wave_barrier();
+        int* row_l = s_l + a * tl.rl;
+        // four rounds of 64 atoms at a time: their loads travel together
+        constexpr int U = 4;
+        for (int f0 = 0; f0 < total; f0 += 64 * U) {
+          int run[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) run[u] = 0;
+#pragma unroll
+          for (int step = 16; step > 0; step >>= 1)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (s_pre[run[u] + step] <= f0 + 64 * u + lane) run[u] += step;
+          double4 q[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int f = f0 + 64 * u + lane;
+            q[u] = bpos[f < total ? s_beg[run[u]] + f : 0];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            if (f0 + 64 * u >= total) break;
+            const int j = static_cast<int>(__double_as_longlong(q[u].w));
+            const double ex = q[u].x - pi.x, ey = q[u].y - pi.y, ez = q[u].z - pi.z;
+            const double r2 = ex * ex + ey * ey + ez * ez;
+            const bool other = f0 + 64 * u + lane < total && j != i;
+            const bool inl = other && r2 < l.cl2, inf = other && r2 < l.cf2;
+            const unsigned long long bl = __ballot(inl), bf = __ballot(inf);
+            const unsigned long long below = (1ull << lane) - 1ull;
+            if (inl) {
+              const int k = nl + __popcll(bl & below);
+              if (k < l.cap_l) row_l[k] = j;
+            }
+            if (inf) {
+              const int k = nf + __popcll(bf & below);
+              if (k < l.cap_f) {
+                s_key[k] = (list_sort_q(r2, l.sort_scale) << 9) | static_cast<uint32_t>(k);
+                s_jt[k] = j | (r2 < l.cand2 ? 0x80000000 : 0);
+              }
+            }
+            nl += __popcll(bl);
+            nf += __popcll(bf);
+          }
+        }
+        if ((nf > l.cap_f || nl > l.cap_l) && lane == 0) atomicOr(overflow, 2);
+        nf = min(nf, l.cap_f);
+        nl = min(nl, l.cap_l);
+        __builtin_amdgcn_wave_barrier();
+        nc = nf <= 128 ? nb_tile_sort<2>(nf, lane, s_key, s_jt, s_f + a * tl.rf, s_c + a * tl.rf)
+                       : nb_tile_sort<4>(nf, lane, s_key, s_jt, s_f + a * tl.rf, s_c + a * tl.rf);
+        __builtin_amdgcn_wave_barrier();
+      }
+      if (lane == 0) {
+        s_n[a] = nl;
+        s_n[TA + a] = nf;
+        s_n[2 * TA + a] = nc;
+      }
+    }
+    __syncthreads();
+    // whole rows: entry k of the block's atoms by consecutive lanes
+    constexpr int kRows = 64 * kTileWaves / TA;
+    const int at = threadIdx.x % TA, k0 = threadIdx.x / TA;
+    const int i = i0 + at;
+    const int nl = s_n[at], nf = s_n[TA + at], nc = s_n[2 * TA + at];
+    for (int k = k0; k < nl; k += kRows) l.nbr_l[k * l.stride + i] = s_l[at * tl.rl + k];
+    for (int k = k0; k < nf; k += kRows) l.nbr_f[k * l.stride + i] = s_f[at * tl.rf + k];
+    if (l.cand)
+      for (int k = k0; k < nc; k += kRows) l.cand[k * l.stride + i] = s_c[at * tl.rf + k];
+    if (k0 == 0 && i < nlocal) {
+      l.nn_l[i] = nl;
+      l.nn_f[i] = nf;
+      if (l.cand) l.ncand[i] = nc;
+    }
+    __syncthreads();
+  }
+}
+
 static inline int nbk(long n, int b = kBlock) { return static_cast<int>((n + b - 1) / b); }
 
 static hipError_t scan(const int* in, int n, int* out, int* tmp, const int* go, hipStream_t s) {
@@ -639,17 +749,29 @@ hipError_t launch_nb_build(const NbBuild& w, hipStream_t s) {
   k_nb_bin_scatter<<<nbk(cap), kBlock, 0, s>>>(cap, w.nlocal, ng, w.bin_of, w.bstart, w.bfill,
                                                w.items, go);
   k_nb_bin_sort<<<nbk(w.nbins), kBlock, 0, s>>>(w.nbins, w.bstart, w.items, go);
-  NbLists found = w.lists;
-  found.cand = nullptr;  // the candidates are written in the sorted order by k_nb_sort
-  k_nb_lists<<<nbk(w.nlocal), kBlock, 0, s>>>(w.nlocal, w.at.pos, w.at.rep, w.box, w.bstart,
-                                              w.items, found, w.overflow, go);
-  const int ek = w.lists.cap_f <= 128 ? 2 : (w.lists.cap_f <= 256 ? 4 : (w.lists.cap_f <= kListSortMax ? 8 : 0));
-  if (ek == 0) return hipErrorInvalidValue;  // more fix-list entries per atom than the sort takes
-  const int sb = std::min(kSortBlocks, nbk(w.nlocal, kBlock / 64));
-  const int tb = std::min(kSortBlocks, nbk(w.nlocal, 64));
-  if (ek == 2) k_nb_sort_tile<2><<<tb, kBlock, 0, s>>>(w.nlocal, w.at.pos, w.lists, go);
-  else if (ek == 4) k_nb_sort_tile<4><<<tb, kBlock, 0, s>>>(w.nlocal, w.at.pos, w.lists, go);
-  else k_nb_sort<8><<<sb, kBlock, 0, s>>>(w.nlocal, w.at.pos, w.lists, go);
+  // lists of at most kTileKeys fix entries whose rows fit the LDS: the tiled
+  // build, 64 atoms per block where they do
+  constexpr size_t kLdsMax = 160 * 1024 - 1024;
+  const int ta = w.lists.cap_f > kTileKeys ? 0 : nb_tile_lds(w.lists, 64) <= kLdsMax ? 64
+               : nb_tile_lds(w.lists, 32) <= kLdsMax ? 32 : 0;
+  if (ta) {
+    k_nb_bin_pos<<<nbk(cap), kBlock, 0, s>>>(cap, w.nlocal, ng, w.at.pos, w.items, w.bpos, go);
+    const size_t lds = nb_tile_lds(w.lists, ta);
+    auto kern = ta == 64 ? k_nb_lists_tile<64> : k_nb_lists_tile<32>;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (e != hipSuccess) return e;
+    kern<<<std::min((nbk(w.nlocal, ta) + 7) / 8 * 8, kTileBlocks), 64 * kTileWaves, lds, s>>>(w.nlocal, w.at.pos, w.at.rep, w.box, w.bstart,
+                                                         w.bpos, w.lists, w.overflow, go);
+  } else {
+    if (w.lists.cap_f > kListSortMax) return hipErrorInvalidValue;  // more fix-list entries per atom than the sort takes
+    NbLists found = w.lists;
+    found.cand = nullptr;  // the candidates are written in the sorted order by k_nb_sort
+    k_nb_lists<<<nbk(w.nlocal), kBlock, 0, s>>>(w.nlocal, w.at.pos, w.at.rep, w.box, w.bstart,
+                                                w.items, found, w.overflow, go);
+    const int sb = std::min(kSortBlocks, nbk(w.nlocal, kBlock / 64));
+    k_nb_sort<8><<<sb, kBlock, 0, s>>>(w.nlocal, w.at.pos, w.lists, go);
+  }
   const bool cw = w.lists.cand && w.cref && w.cand_valid;
   k_nb_finish<<<nbk(cw ? cap : w.nlocal), kBlock, 0, s>>>(w.nlocal, ng, w.at.pos, w.xref, w.go,
                                                           w.nrebuild, w.cand_valid, w.cref, cw);

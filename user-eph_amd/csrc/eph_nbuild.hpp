@@ -79,6 +79,7 @@ struct NbBuild {
   int* bstart = nullptr;    // [nbins + 1]
   int* bfill = nullptr;     // [nbins + 1]
   int* items = nullptr;     // [nlocal + ghost_cap]
+  double4* bpos = nullptr;  // [nlocal + ghost_cap] positions in bin order
   int* scan_tmp = nullptr;  // [(nlocal + ghost_cap + nbins) / 4096 + 2]
   double4* xref = nullptr;  // [nlocal]
 };
