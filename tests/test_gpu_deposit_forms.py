@@ -28,3 +28,64 @@ def test_cell_sums_match_serial_order(oracle, counts):
         for k in range(len(cell)):
             o.insert_energy(x[k], y[k], z[k], E[k])
     assert np.array_equal(g.get("dT"), o.get("dT"))
+
+
+# the fix's own deposit: atoms per grid cell from 0.5 to 256 (16 slots a cell and a thread, 32 to 256
+# slots and a wave, then the counted form), with a hot corner so that cells differ
+@pytest.mark.parametrize("cells,grid", [(4, 8), (5, 5), (6, 5), (6, 4), (6, 3), (7, 3), (6, 2), (8, 2),
+                                        (4, 1), (5, (2, 7, 3))])
+def test_deposit_forms_match_oracle(oracle, tmp_path, cells, grid):
+    import copy
+
+    import eph_amd as ea
+    from eph_amd import inputs
+    path = str(tmp_path / "b.beta")
+    names = inputs.workload_beta(path, 1)
+    dims = grid if isinstance(grid, tuple) else (grid,) * 3
+    md = ea.MD(cells, seed=4, T=900.0, disp_sigma=0.2)
+    inf = md.info()
+    args = inputs.fix_args(path, names, seed=3, flags="7", grid=dims)
+    cons = (args, 1, inf["boxlo"], inf["boxhi"], 1e-3, inputs.BOLTZ, inputs.FTM2V)
+    ora = oracle.Fix(*cons, masses=[inputs.MASS_CU])
+    gpu = ea.FixEPH(*cons, masses=[inputs.MASS_CU])
+    gpu.init()
+    a = md.snapshot()
+    md.lj(a)
+    b = copy.deepcopy(a)
+    gpu.set_atoms(b)
+    for n in (1, 2):
+        for fix, s in ((ora, a), (gpu, b)):
+            fix.post_force(s, step=n)
+            fix.final_integrate(s)
+            fix.end_of_step(s, n)
+        assert np.array_equal(a.v[:a.nlocal], b.v[:b.nlocal])
+        assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))
+
+
+# a quarter of the box's cells hold all atoms but a few, one cell far more than its bucket
+def test_crowded_cells_match_oracle(oracle, tmp_path):
+    import copy
+
+    import eph_amd as ea
+    from eph_amd import inputs
+    path = str(tmp_path / "b.beta")
+    names = inputs.workload_beta(path, 1)
+    md = ea.MD(6, seed=9, T=900.0)
+    inf = md.info()
+    args = inputs.fix_args(path, names, seed=3, flags="7", grid=(4, 4, 4))
+    cons = (args, 1, inf["boxlo"], inf["boxhi"], 1e-3, inputs.BOLTZ, inputs.FTM2V)
+    ora = oracle.Fix(*cons, masses=[inputs.MASS_CU])
+    gpu = ea.FixEPH(*cons, masses=[inputs.MASS_CU])
+    gpu.init()
+    a = md.snapshot()
+    md.lj(a)
+    b = copy.deepcopy(a)
+    gpu.set_atoms(b)
+    ora.post_force(a, step=1)
+    gpu.post_force(b, step=1)
+    for s in (a, b):  # the deposit sees these positions only
+        s.x[:s.nlocal] = np.random.default_rng(1).uniform(0.0, 0.5, (s.nlocal, 3)) * inf["boxhi"][0]
+        s.x[:300] *= 0.4
+    ora.end_of_step(a, 1)
+    gpu.end_of_step(b, 1)
+    assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))

@@ -658,19 +658,18 @@ int eph_context::end_of_step_after_deposit(long long ntimestep) {
   return EPH_OK;
 }
 
-int eph_grid::bucket_bytes_ok(size_t G) {
+int eph_grid::bucket_bytes_ok(size_t G, int cap) {
   EPH_HIP(this, bcount.reserve(G));  // zero-filled when first made
-  EPH_HIP(this, bitems.reserve(G * kBucket));
+  EPH_HIP(this, bitems.reserve(G * cap));
   EPH_HIP(this, bqueue.reserve(G));
   EPH_HIP(this, bnq.reserve(1));
   return EPH_OK;
 }
 
-// the deposit goes through per-cell buckets when there is one and the grid
-// holds a few atoms per cell on average
-bool eph_context::bucket_deposit() const {
-  return (flags & (EPH_FRICTION | EPH_RANDOM)) &&
-         static_cast<double>(nlocal) <= 6.0 * static_cast<double>(grid->h.ntotal());
+// slots per cell where the deposit goes through per-cell buckets, else 0
+int eph_context::bucket_deposit() const {
+  if (!(flags & (EPH_FRICTION | EPH_RANDOM))) return 0;
+  return bucket_slots(static_cast<double>(nlocal), static_cast<double>(grid->h.ntotal()));
 }
 
 // the deposit half of end_of_step (fix_eph.cpp:364-404): dT_e and the tally.
@@ -685,12 +684,13 @@ int eph_context::dev_deposit(bool kick, bool* kicked_out) {
   const int nb = nblocks_of(nlocal);
   const size_t G = grid->h.ntotal();
   hipEvent_t e;
-  // a few atoms per cell on average: per-cell buckets (three launches)
-  if (bucket_deposit()) {
+  // per-cell buckets (three launches)
+  if (const int cap = bucket_deposit()) {
     EPH_HIP(this, grid->dep.reserve(nlocal, 0, nb));
-    if (int rc = grid->bucket_bytes_ok(G)) return fail(rc, grid->err);
+    if (int rc = grid->bucket_bytes_ok(G, cap)) return fail(rc, grid->err);
     DepositView d = grid->dep.view(true);
     BucketView b;
+    b.cap = cap;
     b.count = grid->bcount.p; b.items = grid->bitems.p; b.queue = grid->bqueue.p; b.nqueue = grid->bnq.p;
     timed_begin("deposit", &e);
     EPH_HIP(this, launch_deposit_bucket(atoms_view(), grid->v, step_params(), work_view(), d, b, fric, rnd,

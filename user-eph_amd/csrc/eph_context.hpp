@@ -53,7 +53,7 @@ struct eph_grid {
   eph::DepositBuffers dep;
   // per-cell buckets of the deposit (count kept at zero between steps)
   eph::DevArray<int> bcount, bitems, bqueue, bnq;
-  int bucket_bytes_ok(size_t G);  // reserves the buckets; 0 when they are ready
+  int bucket_bytes_ok(size_t G, int cap);  // reserves buckets of cap slots; 0 when they are ready
   bool any_tdyn = false;
   bool minmax_valid = false;  // cmin, rmin, kmax and uniform describe h
   bool uniform = false;       // every cell dynamic and of one material
@@ -165,7 +165,7 @@ struct eph_context {
   int dev_final_integrate_end_of_step(long long ntimestep);
   int end_of_step_after_deposit(long long ntimestep);
   int dev_deposit(bool kick, bool* kicked);
-  bool bucket_deposit() const;
+  int bucket_deposit() const;
   int autotune(int* forms, double* ms);
   int grow_filter_state(size_t nall);
   int check_flags();

@@ -159,13 +159,24 @@ struct DepositView {
   int* maxcount = nullptr;    // [1]
 };
 
-// Per-cell buckets of the deposit for grids with a few atoms per cell
-// (launch_deposit_bucket): count and kBucket atom slots per cell, and the
-// queue of cells that received more atoms than that.
-constexpr int kBucket = 16;
+// Per-cell buckets of the deposit (launch_deposit_bucket): count and cap atom
+// slots per cell, and the queue of cells that received more atoms than that.
+constexpr int kBucket = 16, kBucketMax = 256;
+// Slots per cell for n atoms in G cells, 0: no buckets.  At least four times
+// the average: a cell beyond its bucket costs a scan over all atoms, so a box
+// that is three quarters empty still has to fit.  Up to 6 atoms per cell 16
+// slots, which one thread sorts; more than kBucketMax (64 atoms per cell) would
+// not fit a wave's registers.
+inline int bucket_slots(double n, double G) {
+  if (n <= 6.0 * G) return kBucket;
+  int cap = 32;
+  while (cap < 4.0 * n / G) cap <<= 1;
+  return cap <= kBucketMax ? cap : 0;
+}
 struct BucketView {
+  int cap = kBucket;
   int* count = nullptr;   // [G], zero between steps
-  int* items = nullptr;   // [G][kBucket]
+  int* items = nullptr;   // [G][cap]
   int* queue = nullptr;   // [G]
   int* nqueue = nullptr;  // [1]
 };

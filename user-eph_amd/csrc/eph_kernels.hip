@@ -1598,6 +1598,22 @@ static __device__ __forceinline__ void cell_ranks(const int* __restrict__ items,
     }
 }
 
+// the ordered sums of a cell's n <= kWaveCellMax items into dT_e[c], by one wave
+static __device__ __forceinline__ void cell_sum_wave(const GridView& g, const DepositView& d, const int c,
+                                                     const int* __restrict__ items, const int n,
+                                                     const int lane, double* s1, double* s2) {
+  if (n <= 64) cell_ranks<1>(items, n, lane, d, s1, s2);
+  else if (n <= 128) cell_ranks<2>(items, n, lane, d, s1, s2);
+  else cell_ranks<4>(items, n, lane, d, s1, s2);
+  wave_lds_sync();
+  double acc = g.dT[c];
+  if (d.v1)
+    for (int b = 0; b < n; b += 64) acc = add_lanes(acc, b + lane < n ? s1[b + lane] : 0.0, n - b < 64 ? n - b : 64);
+  if (d.v2)
+    for (int b = 0; b < n; b += 64) acc = add_lanes(acc, b + lane < n ? s2[b + lane] : 0.0, n - b < 64 ? n - b : 64);
+  if (lane == 0) g.dT[c] = acc;
+}
+
 __global__ __launch_bounds__(kBlock) void k_cell_sum_wave(GridView g, DepositView d, int ncell,
                                                           int* queue, int* qn) {
   __shared__ double s_val[kBlock / 64][2][kWaveCellMax];
@@ -1611,18 +1627,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_sum_wave(GridView g, DepositVie
     if (lane == 0) queue[atomicAdd(qn, 1)] = c;
     return;
   }
-  double* s1 = s_val[wv][0];
-  double* s2 = s_val[wv][1];
-  if (n <= 64) cell_ranks<1>(d.items + s, n, lane, d, s1, s2);
-  else if (n <= 128) cell_ranks<2>(d.items + s, n, lane, d, s1, s2);
-  else cell_ranks<4>(d.items + s, n, lane, d, s1, s2);
-  wave_lds_sync();
-  double acc = g.dT[c];
-  if (d.v1)
-    for (int b = 0; b < n; b += 64) acc = add_lanes(acc, b + lane < n ? s1[b + lane] : 0.0, n - b < 64 ? n - b : 64);
-  if (d.v2)
-    for (int b = 0; b < n; b += 64) acc = add_lanes(acc, b + lane < n ? s2[b + lane] : 0.0, n - b < 64 ? n - b : 64);
-  if (lane == 0) g.dT[c] = acc;
+  cell_sum_wave(g, d, c, d.items + s, n, lane, s_val[wv][0], s_val[wv][1]);
 }
 
 constexpr int kMedBlock = 1024;
@@ -1730,14 +1735,17 @@ __global__ __launch_bounds__(1024) void k_energy_reduce(const double* partial, i
 }
 
 // ----------------------------------------------- bucketed deposit
-// The same deposit for grids with a few atoms per cell (fcc at one cell per
-// unit cell holds 4 on average, at most 14 while every atom stays within
-// half a cell of its site).  Each cell collects its atoms in a bucket of
-// kBucket slots as they are counted; one thread per cell then sorts its
-// bucket and adds the values in ascending atom order, friction then random,
-// the serial order of fix_eph.cpp:364-390.  A cell that receives more atoms
-// than its bucket holds is queued and summed by k_deposit_finish from an
-// ordered scan of every atom's cell.  Three launches in all.
+// The same deposit without the count, scan and scatter passes.  Each cell
+// collects its atoms in a bucket of cap slots as they are counted; one thread
+// per cell (up to 6 atoms per cell on average: fcc at one cell per unit cell
+// holds 4, at most 14 while every atom stays within half a cell of its site)
+// or one wave per cell then sorts its bucket and adds the values in ascending
+// atom order, friction then random, the serial order of fix_eph.cpp:364-390.
+// A cell that receives more atoms than its bucket holds is queued and summed
+// by k_deposit_finish from an ordered scan of every atom's cell.  Three
+// launches in all: with 32 atoms per cell (32,000 atoms) 24 us with the final
+// kick inside, against 64 us for the twelve launches of the counted deposit
+// and 5 us for the kick.
 // one atom of the bucketed deposit at end-of-step velocity v: its energies
 // into the bucket of its cell and the values the cell sums read
 template <bool FRIC, bool RAND>
@@ -1767,7 +1775,7 @@ __device__ __forceinline__ void deposit_bucket_atom(const int i, const double4& 
     v2 = dE / prescale;
   }
   const int slot = atomicAdd(&b.count[c], 1);
-  if (slot < kBucket) b.items[static_cast<size_t>(c) * kBucket + slot] = i;
+  if (slot < b.cap) b.items[static_cast<size_t>(c) * b.cap + slot] = i;
   if (FRIC) d.v1[i] = v1;
   if (RAND) d.v2[i] = v2;
 }
@@ -1852,6 +1860,24 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket_cells(GridView g, Dep
       if (e < n) acc += d.v2[k[e]];
   }
   g.dT[c] = acc;
+}
+
+// buckets of more than kBucket slots: a wave per cell (see cell_ranks)
+__global__ __launch_bounds__(kBlock) void k_deposit_bucket_wave(GridView g, DepositView d, BucketView b,
+                                                                int ncell) {
+  __shared__ double s_val[kBlock / 64][2][kWaveCellMax];
+  const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  const int c = blockIdx.x * (kBlock / 64) + wv;
+  if (c >= ncell) return;
+  const int n = b.count[c];
+  if (n == 0) return;
+  if (lane == 0) {
+    b.count[c] = 0;
+    if (n > b.cap) b.queue[atomicAdd(b.nqueue, 1)] = c;
+  }
+  if (n > b.cap) return;
+  cell_sum_wave(g, d, c, b.items + static_cast<size_t>(c) * b.cap, n, lane, s_val[wv][0], s_val[wv][1]);
 }
 
 // block 0: E_local and Ee from the block partial sums (as k_energy_reduce);
@@ -2776,7 +2802,8 @@ hipError_t launch_deposit_bucket(const AtomsView& a, const GridView& g, const St
   DepositView dc = d;
   if (!fric) dc.v1 = nullptr;
   if (!rand) dc.v2 = nullptr;
-  k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, dc, b, G);
+  if (b.cap == kBucket) k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, dc, b, G);
+  else k_deposit_bucket_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, dc, b, G);
   k_deposit_finish<<<1 + 16, 1024, 0, s>>>(a, g, dc, b, a.nlocal > 0 ? nb : 0, E_local, Ee);
   return hipGetLastError();
 }
