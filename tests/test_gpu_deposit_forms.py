@@ -62,17 +62,19 @@ def test_deposit_forms_match_oracle(oracle, tmp_path, cells, grid):
         assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))
 
 
-# a quarter of the box's cells hold all atoms but a few, one cell far more than its bucket
-def test_crowded_cells_match_oracle(oracle, tmp_path):
+# an eighth of the box holds all atoms, one cell far more than its bucket; the larger boxes overflow so many
+# cells (of 16 and of 256 slots) that the deposits after the first are counted ones
+@pytest.mark.parametrize("cells,n", [(6, 4), (20, 24), (20, 8)])
+def test_crowded_cells_match_oracle(oracle, tmp_path, cells, n):
     import copy
 
     import eph_amd as ea
     from eph_amd import inputs
     path = str(tmp_path / "b.beta")
     names = inputs.workload_beta(path, 1)
-    md = ea.MD(6, seed=9, T=900.0)
+    md = ea.MD(cells, seed=9, T=900.0)
     inf = md.info()
-    args = inputs.fix_args(path, names, seed=3, flags="7", grid=(4, 4, 4))
+    args = inputs.fix_args(path, names, seed=3, flags="7", grid=(n, n, n))
     cons = (args, 1, inf["boxlo"], inf["boxhi"], 1e-3, inputs.BOLTZ, inputs.FTM2V)
     ora = oracle.Fix(*cons, masses=[inputs.MASS_CU])
     gpu = ea.FixEPH(*cons, masses=[inputs.MASS_CU])
@@ -86,6 +88,7 @@ def test_crowded_cells_match_oracle(oracle, tmp_path):
     for s in (a, b):  # the deposit sees these positions only
         s.x[:s.nlocal] = np.random.default_rng(1).uniform(0.0, 0.5, (s.nlocal, 3)) * inf["boxhi"][0]
         s.x[:300] *= 0.4
-    ora.end_of_step(a, 1)
-    gpu.end_of_step(b, 1)
-    assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))
+    for step in (1, 2, 3):
+        ora.end_of_step(a, step)
+        gpu.end_of_step(b, step)
+        assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))

@@ -619,21 +619,14 @@ int eph_context::dev_final_integrate_end_of_step(long long ntimestep) {
     int rc = dev_final_integrate();
     return rc != EPH_OK ? rc : dev_end_of_step(ntimestep);
   }
-  int rc;
-  if (bucket_deposit() && !(flags & EPH_NOINT)) {
-    bool kicked = false;
-    if ((rc = dev_deposit(true, &kicked)) != EPH_OK) return rc;
-    if (!kicked) return fail(EPH_ERR_STATE, "the fused final kick did not run");
-  } else {
-    if ((rc = dev_final_integrate()) != EPH_OK) return rc;
-    if ((rc = dev_deposit(false, nullptr)) != EPH_OK) return rc;
-  }
+  int rc = dev_deposit(true);
+  if (rc != EPH_OK) return rc;
   return end_of_step_after_deposit(ntimestep);
 }
 
 int eph_context::dev_end_of_step(long long ntimestep) {
   if (atomic()) return eph::atomic_end_of_step(this);
-  int rc = dev_deposit(false, nullptr);
+  int rc = dev_deposit(false);
   if (rc != EPH_OK) return rc;
   return end_of_step_after_deposit(ntimestep);
 }
@@ -663,41 +656,47 @@ int eph_grid::bucket_bytes_ok(size_t G, int cap) {
   EPH_HIP(this, bitems.reserve(G * cap));
   EPH_HIP(this, bqueue.reserve(G));
   EPH_HIP(this, bnq.reserve(1));
+  if (!crowded) {
+    EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&crowded), sizeof(int), hipHostMallocDefault));
+    *crowded = 0;
+  }
   return EPH_OK;
 }
 
 // slots per cell where the deposit goes through per-cell buckets, else 0
 int eph_context::bucket_deposit() const {
   if (!(flags & (EPH_FRICTION | EPH_RANDOM))) return 0;
+  if (grid->crowded && *static_cast<volatile int*>(grid->crowded)) return 0;
   return bucket_slots(static_cast<double>(nlocal), static_cast<double>(grid->h.ntotal()));
 }
 
 // the deposit half of end_of_step (fix_eph.cpp:364-404): dT_e and the tally.
-// kick: apply final_integrate's kick in the same pass where the bucketed
-// deposit runs (*kicked tells whether it did)
-int eph_context::dev_deposit(bool kick, bool* kicked_out) {
+// kick: final_integrate's kick first, in the same pass where the bucketed
+// deposit runs
+int eph_context::dev_deposit(bool kick) {
   if (!have_atoms) return fail(EPH_ERR_STATE, "no atoms");
-  bool kicked = false;
-  if (kicked_out) *kicked_out = false;
   if (flags & EPH_NOINT) kick = false;
+  const int cap = bucket_deposit();
+  if (kick && !cap)
+    if (int rc = dev_final_integrate()) return rc;
   const bool fric = flags & EPH_FRICTION, rnd = flags & EPH_RANDOM;
   const int nb = nblocks_of(nlocal);
   const size_t G = grid->h.ntotal();
   hipEvent_t e;
   // per-cell buckets (three launches)
-  if (const int cap = bucket_deposit()) {
-    EPH_HIP(this, grid->dep.reserve(nlocal, 0, nb));
+  if (cap) {
+    EPH_HIP(this, grid->dep.reserve(nlocal, G, nb));  // also what a counted deposit needs
     if (int rc = grid->bucket_bytes_ok(G, cap)) return fail(rc, grid->err);
     DepositView d = grid->dep.view(true);
     BucketView b;
     b.cap = cap;
     b.count = grid->bcount.p; b.items = grid->bitems.p; b.queue = grid->bqueue.p; b.nqueue = grid->bnq.p;
+    b.limit = queue_limit(nlocal);
+    b.crowded = grid->crowded;
     timed_begin("deposit", &e);
     EPH_HIP(this, launch_deposit_bucket(atoms_view(), grid->v, step_params(), work_view(), d, b, fric, rnd,
                                         kick, scal.p, scal.p + (defer_tally ? 2 : 1), stream));
     timed_end(kick ? "final_integrate+deposit" : "deposit", e);
-    kicked = kick;
-    if (kicked_out) *kicked_out = kicked;
     return EPH_OK;
   }
   if (fric || rnd) {
@@ -1186,7 +1185,7 @@ int eph_end_of_step_local(eph_context* ctx, const double* x, const double* v, do
   if ((rc = upload_rows(ctx, x, ctx->nlocal, ctx->pos.p))) return rc;
   if ((rc = upload_rows(ctx, v, ctx->nlocal, ctx->vel.p))) return rc;
   ctx->defer_tally = true;
-  rc = ctx->dev_deposit(false, nullptr);
+  rc = ctx->dev_deposit(false);
   ctx->defer_tally = false;
   if (rc) return rc;
   std::vector<double> d;
@@ -1568,6 +1567,7 @@ void eph_grid_destroy(eph_grid* g) {
   if (!g) return;
   if (g->stream) (void)hipStreamSynchronize(g->stream);
   hipStream_t s = g->own_stream ? g->stream : nullptr;
+  if (g->crowded) (void)hipHostFree(g->crowded);
   delete g;
   if (s) (void)hipStreamDestroy(s);
 }

@@ -53,6 +53,10 @@ struct eph_grid {
   eph::DepositBuffers dep;
   // per-cell buckets of the deposit (count kept at zero between steps)
   eph::DevArray<int> bcount, bitems, bqueue, bnq;
+  // Pinned: the device sets [0] once more cells overflowed their buckets than
+  // queue_limit allows; the deposits from then on are counted ones.  A plan
+  // only, both forms give the same bits, so it is read without a wait.
+  int* crowded = nullptr;
   int bucket_bytes_ok(size_t G, int cap);  // reserves buckets of cap slots; 0 when they are ready
   bool any_tdyn = false;
   bool minmax_valid = false;  // cmin, rmin, kmax and uniform describe h
@@ -164,7 +168,7 @@ struct eph_context {
   int dev_end_of_step(long long ntimestep);
   int dev_final_integrate_end_of_step(long long ntimestep);
   int end_of_step_after_deposit(long long ntimestep);
-  int dev_deposit(bool kick, bool* kicked);
+  int dev_deposit(bool kick);
   int bucket_deposit() const;
   int autotune(int* forms, double* ms);
   int grow_filter_state(size_t nall);

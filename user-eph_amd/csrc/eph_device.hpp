@@ -162,23 +162,30 @@ struct DepositView {
 // Per-cell buckets of the deposit (launch_deposit_bucket): count and cap atom
 // slots per cell, and the queue of cells that received more atoms than that.
 constexpr int kBucket = 16, kBucketMax = 256;
-// Slots per cell for n atoms in G cells, 0: no buckets.  At least four times
-// the average: a cell beyond its bucket costs a scan over all atoms, so a box
-// that is three quarters empty still has to fit.  Up to 6 atoms per cell 16
-// slots, which one thread sorts; more than kBucketMax (64 atoms per cell) would
-// not fit a wave's registers.
+// Slots per cell for n atoms in G cells, 0: no buckets.  Eight times the
+// average, so that a box that is mostly empty still fits, as far as
+// kBucketMax, what a wave's registers hold, and from 64 atoms per cell on the
+// counted form.  Up to 6 atoms per cell 16 slots, which one thread sorts.
 inline int bucket_slots(double n, double G) {
   if (n <= 6.0 * G) return kBucket;
-  int cap = 32;
-  while (cap < 4.0 * n / G) cap <<= 1;
-  return cap <= kBucketMax ? cap : 0;
+  if (n > 64.0 * G) return 0;
+  int cap = 64;
+  while (cap < kBucketMax && cap < 8.0 * n / G) cap <<= 1;
+  return cap;
 }
+// A cell beyond its bucket costs a scan over all atoms (1.5 us per 1024 of
+// them), shared by kQueueBlocks workgroups.  Beyond this many such cells the
+// counted form (some 45 us more than the bucketed one) is the faster.
+constexpr int kQueueBlocks = 16;
+inline int queue_limit(int n) { return kQueueBlocks * (1 + 32768 / (n > 0 ? n : 1)); }
 struct BucketView {
   int cap = kBucket;
   int* count = nullptr;   // [G], zero between steps
   int* items = nullptr;   // [G][cap]
   int* queue = nullptr;   // [G]
   int* nqueue = nullptr;  // [1]
+  int limit = 0;          // queued cells beyond which *crowded is set
+  int* crowded = nullptr; // pinned host memory
 };
 
 constexpr int kBlock = 256;

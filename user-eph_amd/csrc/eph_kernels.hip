@@ -1742,8 +1742,8 @@ __global__ __launch_bounds__(1024) void k_energy_reduce(const double* partial, i
 // or one wave per cell then sorts its bucket and adds the values in ascending
 // atom order, friction then random, the serial order of fix_eph.cpp:364-390.
 // A cell that receives more atoms than its bucket holds is queued and summed
-// by k_deposit_finish from an ordered scan of every atom's cell.  Three
-// launches in all: with 32 atoms per cell (32,000 atoms) 24 us with the final
+// by k_deposit_finish from an ordered scan of every atom's cell; once many
+// are, the steps that follow take the counted form.  Three launches in all: with 32 atoms per cell (32,000 atoms) 24 us with the final
 // kick inside, against 64 us for the twelve launches of the counted deposit
 // and 5 us for the kick.
 // one atom of the bucketed deposit at end-of-step velocity v: its energies
@@ -1892,6 +1892,7 @@ __global__ __launch_bounds__(1024) void k_deposit_finish(AtomsView a, GridView g
   __shared__ unsigned long long hits[16];
   if (blockIdx.x == 0) {
     energy_reduce(d.partial, nblocks, E_local, Ee, sh);
+    if (threadIdx.x == 0 && *b.nqueue > b.limit) *b.crowded = 1;
     return;
   }
   const int nq = *b.nqueue;
@@ -2804,7 +2805,7 @@ hipError_t launch_deposit_bucket(const AtomsView& a, const GridView& g, const St
   if (!rand) dc.v2 = nullptr;
   if (b.cap == kBucket) k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, dc, b, G);
   else k_deposit_bucket_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, dc, b, G);
-  k_deposit_finish<<<1 + 16, 1024, 0, s>>>(a, g, dc, b, a.nlocal > 0 ? nb : 0, E_local, Ee);
+  k_deposit_finish<<<1 + kQueueBlocks, 1024, 0, s>>>(a, g, dc, b, a.nlocal > 0 ? nb : 0, E_local, Ee);
   return hipGetLastError();
 }
 
