@@ -11,7 +11,9 @@ kappa = 0.1, dt = 0.1 fs, FP64, full model (friction + random + FDM).
 
 A step is one MD step; the timed quantity is the fix's own work per step
 (initial_integrate + post_force + final_integrate + end_of_step, measured
-with HIP events on the fix's stream), as the reference's "Modify" time is.
+with the device's wall clock at the hooks' boundaries; a kernel that also does
+some of the harness's work counts by the bytes each side moves), as the
+reference's "Modify" time is.
 value = atoms x steps / fix seconds.  The pair force, ghost update and
 neighbour rebuilds run in the same loop on the device (rebuilds through the
 host) and are reported separately.
@@ -451,8 +453,9 @@ def main():
     # both kernel forms of each sweep timed on the live system; the faster is kept
     tuned = fix.autotune() if not args.no_autotune else None
     log(f"sweep forms: {tuned}")
-    # the value: K steps as the product runs them, events only at the hook
-    # boundaries (an event between two kernels holds the second back ~10 us)
+    # the value: K steps as the product runs them, with device times taken inside
+    # the kernels at the hook boundaries (an event between two kernels holds the
+    # second back ~10 us)
     md.checkpoint_save(fix)  # kept in host memory
     step0 = step
     res = advance(args.steps, True)

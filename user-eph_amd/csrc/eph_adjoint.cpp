@@ -219,9 +219,8 @@ int eph_adjoint::step(long long n, Rec* r) {
   hipStream_t s = ctx->stream;
   int rc;
   ctx->step = n;
-  if ((rc = ctx->dev_initial_integrate())) return fail(rc, ctx->err);
   bool rebuilt = false, overflow = false;
-  if ((rc = md->neighbours_and_pair(ctx, false, nullptr, &rebuilt, &overflow))) return fail(rc, md->err);
+  if ((rc = md->kick_and_pair(ctx, false, nullptr, &rebuilt, &overflow))) return fail(rc, md->err);
   if (overflow) return fail(EPH_ERR_STATE, "neighbour capacity exceeded during the trajectory");
   if ((rc = ctx->dev_post_force())) return fail(rc, ctx->err);
   if ((rc = ctx->dev_final_integrate())) return fail(rc, ctx->err);

@@ -122,7 +122,7 @@ void eph_grid::substeps(double* r_out, unsigned* steps_out, double* inner_out) c
 }
 
 // EPH_FDM::solve (eph_fdm.h:267-400) on the device
-int eph_grid::solve(int* substeps_out) {
+int eph_grid::solve(int* substeps_out, const DepositTail* tail) {
   if (any_tdyn) {
     EPH_HIP(this, launch_grid_tdyn_update(v, stream));
     EPH_HIP(this, launch_grid_minmax(v, minmax.p, nullptr, stream));
@@ -139,7 +139,7 @@ int eph_grid::solve(int* substeps_out) {
   last_r = r;
   const FdmMaterial mat{h.kappa[0], h.S[0], h.rho[0], h.C[0]};
   EPH_HIP(this, launch_fdm_solve(v, T.p, Tn.p, inner_dt, (int)new_steps,
-                                 !any_tdyn && uniform ? &mat : nullptr, any_tdyn, nonfinite.p, stream));
+                                 !any_tdyn && uniform ? &mat : nullptr, any_tdyn, nonfinite.p, stream, tail));
   v.T = T.p;
   v.Tn = Tn.p;
   last_steps = (int)new_steps;
@@ -443,12 +443,15 @@ int eph_context::resolve_timing() {
   return EPH_OK;
 }
 
-int eph_context::dev_initial_integrate() {
+int eph_context::dev_initial_integrate(const StepExtras* x) {
   if (!have_atoms) return fail(EPH_ERR_STATE, "no atoms");
-  if (flags & EPH_NOINT) return EPH_OK;
+  if (flags & EPH_NOINT) {
+    if (x) EPH_HIP(this, launch_integrate(atoms_view(), step_params(), false, stream, x));
+    return EPH_OK;
+  }
   hipEvent_t a;
   timed_begin("integrate", &a);
-  EPH_HIP(this, launch_integrate(atoms_view(), step_params(), true, stream));
+  EPH_HIP(this, launch_integrate(atoms_view(), step_params(), true, stream, x));
   timed_end("integrate", a);
   return EPH_OK;
 }
@@ -460,6 +463,15 @@ int eph_context::dev_final_integrate() {
   timed_begin("integrate", &a);
   EPH_HIP(this, launch_integrate(atoms_view(), step_params(), false, stream));
   timed_end("integrate", a);
+  return EPH_OK;
+}
+
+int eph_context::dev_ghosts(unsigned long long* t) {
+  const AtomsView a = atoms_view();
+  const WorkView w = work_view();
+  // with timing on the check keeps its own launch and line in the report
+  cand_checked = !timing && !atomic() && w.rcand2 > 0.0 && density_walks_candidates(a, tabs, form_density);
+  EPH_HIP(this, launch_ghost_check(a, w, cand_checked, t, stream));
   return EPH_OK;
 }
 
@@ -488,7 +500,11 @@ int eph_context::dev_post_force() {
   StepParams p = step_params();
   p.xi_mode = (flags & EPH_RANDOM) ? (xi_mode_next ? 1 : 2) : 0;
   const AtomsView a = atoms_view();
-  const WorkView w = work_view();
+  WorkView w = work_view();
+  w.cand_checked = cand_checked;
+  cand_checked = false;
+  w.defer_flags = !timing && model == 4 && nghost > 0 && w.rcand2 > 0.0 &&
+                  density_walks_candidates(a, tabs, form_density);
   hipEvent_t e;
   if (colour == 3 && (flags & EPH_FRICTION)) EPH_HIP(this, launch_colour_v(a, p, w, stream));
   if (!pv_fresh || !a.pv) {
@@ -619,25 +635,27 @@ int eph_context::dev_final_integrate_end_of_step(long long ntimestep) {
     int rc = dev_final_integrate();
     return rc != EPH_OK ? rc : dev_end_of_step(ntimestep);
   }
-  int rc = dev_deposit(true);
+  DepositTail tail;
+  int rc = dev_deposit(true, &tail);
   if (rc != EPH_OK) return rc;
-  return end_of_step_after_deposit(ntimestep);
+  return end_of_step_after_deposit(ntimestep, &tail);
 }
 
 int eph_context::dev_end_of_step(long long ntimestep) {
   if (atomic()) return eph::atomic_end_of_step(this);
-  int rc = dev_deposit(false);
+  DepositTail tail;
+  int rc = dev_deposit(false, &tail);
   if (rc != EPH_OK) return rc;
-  return end_of_step_after_deposit(ntimestep);
+  return end_of_step_after_deposit(ntimestep, &tail);
 }
 
 // the FDM solve and the heat-map output of end_of_step (fix_eph.cpp:392-399)
-int eph_context::end_of_step_after_deposit(long long ntimestep) {
+int eph_context::end_of_step_after_deposit(long long ntimestep, const DepositTail* tail) {
   int rc = EPH_OK;
   hipEvent_t e;
   if (flags & EPH_FDM) {
     timed_begin("fdm_solve", &e);
-    rc = grid->solve(nullptr);
+    rc = grid->solve(nullptr, tail && tail->E_local ? tail : nullptr);
     if (rc != EPH_OK) return fail(rc, grid->err);
     timed_end("fdm_solve", e);
   }
@@ -673,7 +691,7 @@ int eph_context::bucket_deposit() const {
 // the deposit half of end_of_step (fix_eph.cpp:364-404): dT_e and the tally.
 // kick: final_integrate's kick first, in the same pass where the bucketed
 // deposit runs
-int eph_context::dev_deposit(bool kick) {
+int eph_context::dev_deposit(bool kick, DepositTail* tail) {
   if (!have_atoms) return fail(EPH_ERR_STATE, "no atoms");
   if (flags & EPH_NOINT) kick = false;
   const int cap = bucket_deposit();
@@ -695,7 +713,8 @@ int eph_context::dev_deposit(bool kick) {
     b.crowded = grid->crowded;
     timed_begin("deposit", &e);
     EPH_HIP(this, launch_deposit_bucket(atoms_view(), grid->v, step_params(), work_view(), d, b, fric, rnd,
-                                        kick, scal.p, scal.p + (defer_tally ? 2 : 1), stream));
+                                        kick, scal.p, scal.p + (defer_tally ? 2 : 1), stream,
+                                        tail && (flags & EPH_FDM) && !timing ? tail : nullptr));
     timed_end(kick ? "final_integrate+deposit" : "deposit", e);
     return EPH_OK;
   }
@@ -1061,6 +1080,7 @@ int eph_context::d2h(void* dst, const void* src, size_t bytes) {
 
 static int upload_rows(eph_context* c, const double* rows, int n, double4* dst) {
   c->pv_fresh = false;  // positions or velocities written behind the packed records
+  c->cand_checked = false;
   if (n == 0) return EPH_OK;
   if (int rc = c->h2d(c->stage.p, rows, 3 * (size_t)n * sizeof(double))) return rc;
   EPH_HIP(c, launch_rows_into_d4(c->stage.p, n, dst, c->stream));
@@ -1210,7 +1230,7 @@ int eph_end_of_step_reduced(eph_context* ctx, const double* dT, double E, long l
   EPH_HIP(ctx, hipMemcpyAsync(ctx->scal.p, sc, 2 * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
   if (int rc = ctx->h2d(g->dT.p, dT, G * sizeof(double))) return rc;
   ctx->write_output = write_output != 0;
-  const int rc = ctx->end_of_step_after_deposit(ntimestep);
+  const int rc = ctx->end_of_step_after_deposit(ntimestep, nullptr);
   ctx->write_output = true;
   if (rc) return rc;
   EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -72,7 +72,8 @@ struct eph_grid {
   }
   int upload();            // host description -> device (all arrays)
   void refresh_minmax();   // host min/max of the stability estimate
-  int solve(int* substeps);
+  // tail: the deposit's remainder, run before the first sub-step
+  int solve(int* substeps, const eph::DepositTail* tail = nullptr);
   void substeps(double* r, unsigned* steps, double* inner_dt) const;
   int insert_points(int n, const double* x, const double* y, const double* z, const double* E);
   int download(int which, std::vector<double>& out);
@@ -125,6 +126,7 @@ struct eph_context {
   // that move atoms keep them so; anything else that writes pos or vel
   // (uploads, restores) clears this and the next post_force repacks
   bool pv_fresh = false;
+  bool cand_checked = false;  // dev_ghosts made the check of the coming post_force
   // the multi-rank hooks: the deposit leaves Ee alone (the caller adds the
   // sum over ranks), and only the rank that writes files writes the heat map
   bool defer_tally = false, write_output = true;
@@ -160,15 +162,19 @@ struct eph_context {
                 const int* tg);
   int set_ghost_map(int ng, const int* owner, const double* shift);
   int set_neighbors(int nl, const int* off, const int* idx, int neighmask);
-  int dev_initial_integrate();
+  int dev_initial_integrate(const eph::StepExtras* x = nullptr);
   int dev_post_force();
   int dev_post_force_local();   // post_force up to the ghost exchange
   int dev_post_force_ghosts();  // the rest, with the ghosts' halo values in place
   int dev_final_integrate();
   int dev_end_of_step(long long ntimestep);
   int dev_final_integrate_end_of_step(long long ntimestep);
-  int end_of_step_after_deposit(long long ntimestep);
-  int dev_deposit(bool kick);
+  int end_of_step_after_deposit(long long ntimestep, const eph::DepositTail* tail);
+  // tail: may receive the deposit's remainder (E_local set) for the solve to do
+  int dev_deposit(bool kick, eph::DepositTail* tail = nullptr);
+  // ghost positions and velocities, with the density sweep's candidate check
+  // where it is due (the harness's step); t: device time at its start
+  int dev_ghosts(unsigned long long* t);
   int bucket_deposit() const;
   int autotune(int* forms, double* ms);
   int grow_filter_state(size_t nall);

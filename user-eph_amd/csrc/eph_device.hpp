@@ -135,6 +135,8 @@ struct WorkView {
   // [0] candidates valid, [1] waves that scanned the full list, [2] moved
   // count; [3], [4] the same two of the last sweep, [5] 1 if it retook them
   int* cstate = nullptr;
+  bool cand_checked = false;  // the check of this step ran with the ghost update
+  bool defer_flags = false;   // the ghost records' kernel does the state update after the sweep
   double rcand2 = 0.0;
   double half_delta2 = 0.0;     // (0.45 delta)^2
   double reach = 0.0;           // rc + 0.1 delta
@@ -188,6 +190,29 @@ struct BucketView {
   int* crowded = nullptr; // pinned host memory
 };
 
+// What is left of the bucketed deposit after the cells' sums: the tally from
+// the block partials, and the overfull cells
+struct DepositTail {
+  AtomsView a;
+  DepositView d;
+  BucketView b;
+  int nblocks = 0;
+  double* E_local = nullptr;  // null: no tail
+  double* Ee = nullptr;
+};
+
+// Extras of a step of the harness, whose kernels follow each other: the list
+// check in the kernel that moves the atoms, and device times (wall_clock64) in
+// place of events between kernels, each of which costs the device and the
+// host some 6 us.  t: [0] start, [1] end of the initial kick, [2] start of
+// the ghost update, [3] and [4] start and end of the pair force.
+struct StepExtras {
+  const double4* xref = nullptr;  // positions of the last list build
+  double lim = 0.0;
+  int* want = nullptr;            // pinned host memory: 1 when an atom moved farther than lim
+  unsigned long long* t = nullptr;
+};
+
 constexpr int kBlock = 256;
 constexpr int kCellConstant = 0, kCellDynamic = 1, kCellZeroDerivative = 2;
 constexpr int kMaxSortInCell = 64;
@@ -212,6 +237,12 @@ struct Chunk {
 
 // ---- launch wrappers (eph_kernels.hip) ----
 hipError_t launch_ghost_xv(const AtomsView& a, const int* owner, const double4* shift, hipStream_t s);
+// the ghost update and, with check, the density sweep's candidate check of all
+// atoms (w.cand_checked then says so to the sweep)
+hipError_t launch_ghost_check(const AtomsView& a, const WorkView& w, bool check, unsigned long long* t,
+                              hipStream_t s);
+// whether the density sweep in this form walks candidates (w.rcand2 given)
+bool density_walks_candidates(const AtomsView& a, const TablesView& t, int form);
 // indices outside [0, nall) set bit 0 of *bad (and are stored as 0); a row
 // with more than `width` entries sets bit 1 and is stored empty
 hipError_t launch_csr_to_ell(int nlocal, const int* off, const int* idx, int neighmask, int nall,
@@ -234,7 +265,9 @@ hipError_t launch_ghost_halo(const AtomsView& a, const TablesView& t, const Work
                              const double* in, hipStream_t s);
 hipError_t launch_prl_forces(const AtomsView& a, const TablesView& t, const GridView& g,
                              const StepParams& p, const WorkView& w, hipStream_t s, int form = -1);
-hipError_t launch_integrate(const AtomsView& a, const StepParams& p, bool initial, hipStream_t s);
+hipError_t launch_integrate(const AtomsView& a, const StepParams& p, bool initial, hipStream_t s,
+                            const StepExtras* x = nullptr);
+hipError_t launch_stamp(unsigned long long* t, hipStream_t s);
 // models 1 (TTM) and 2 (PRB) of fix eph, after the density sweep
 hipError_t launch_ttm_forces(const AtomsView& a, const TablesView& t, const GridView& g,
                              const StepParams& p, const WorkView& w, hipStream_t s);
@@ -256,11 +289,13 @@ hipError_t launch_deposit_cells(const GridView& g, const DepositView& d, int n_i
                                 hipStream_t s);
 // the whole deposit and tally through per-cell buckets (fric / rand: which
 // parts); with kick, the final velocity-Verlet kick of the group's atoms
-// first, in the same pass.  b.count must be zero on entry and is left zero
+// first, in the same pass.  b.count must be zero on entry and is left zero.
+// tail given: its work is left to launch_deposit_tail or launch_fdm_solve
 hipError_t launch_deposit_bucket(const AtomsView& a, const GridView& g, const StepParams& p,
                                  const WorkView& w, const DepositView& d, const BucketView& b,
                                  bool fric, bool rand, bool kick, double* E_local, double* Ee,
-                                 hipStream_t s);
+                                 hipStream_t s, DepositTail* tail = nullptr);
+hipError_t launch_deposit_tail(const GridView& g, const DepositTail& tail, hipStream_t s);
 hipError_t launch_energy_reduce(const DepositView& d, int nblocks, double* E_local, double* Ee,
                                 hipStream_t s);
 // grid
@@ -275,9 +310,10 @@ struct FdmMaterial {
 // the nsub sub-steps of one solve (eph_fdm.hip): T holds the result on return
 // (T and Tn may have been swapped), dT is cleared, and bit 1 of *nonfinite is
 // set when T holds a non-finite value.  uniform: every cell is a dynamic cell
-// of this material (null: values per cell)
+// of this material (null: values per cell); tail: the deposit's remainder, first
 hipError_t launch_fdm_solve(const GridView& g, double*& T, double*& Tn, double inner_dt, int nsub,
-                            const FdmMaterial* uniform, bool any_tdyn, int* nonfinite, hipStream_t s);
+                            const FdmMaterial* uniform, bool any_tdyn, int* nonfinite, hipStream_t s,
+                            const DepositTail* tail = nullptr);
 hipError_t launch_grid_lookup(const GridView& g, int n, const double* x, const double* y,
                               const double* z, int* idx, double* T, hipStream_t s);
 hipError_t launch_sum(const double* v, int n, double* out, double* scratch, hipStream_t s);
@@ -297,7 +333,7 @@ hipError_t launch_d4_component(const double4* in, int n, int comp, double* out, 
                                int stride4 = 1);
 // harness
 hipError_t launch_lj(const AtomsView& a, const int* nbr, const int* nn, int stride, double eps,
-                     double sigma, double rc2, hipStream_t s);
+                     double sigma, double rc2, hipStream_t s, unsigned long long* t = nullptr);
 hipError_t launch_max_disp2(const AtomsView& a, const double4* ref, double* partial, int nblocks,
                             hipStream_t s);
 hipError_t launch_copy_probe(double4* dst, const double4* src, long n, hipStream_t s);

@@ -10,6 +10,7 @@
 //   10^3 cells 118 -> 35 us, 16^3 118 -> 66 (one workgroup)
 //   20^3 117 -> 78, 40^3 119 -> 80 (8 x 8 x 4 tiles, 3 sub-steps a launch)
 //   64^3 144 -> 117 (16 x 8 x 8 tiles, 2), 80^3 226 -> 148 (16 x 16 x 8, 2)
+#include "eph_deposit.hpp"
 #include "eph_fdm.hpp"
 
 namespace eph {
@@ -30,9 +31,18 @@ struct FdmArgs {
 
 template <int MODE, int NC>
 __global__ __launch_bounds__(kFdmThreads) void k_fdm_block(GridView g, FdmArgs u, double* __restrict__ T,
-                                                           int nsub, int G, int* nonfinite) {
+                                                           int nsub, int G, int* nonfinite,
+                                                           DepositTail tail) {
   extern __shared__ double s_fdm[];
   __shared__ int s_slow;
+  if (tail.E_local) {  // the deposit's remainder, which completes dT_e
+    __shared__ double sh[kFdmThreads];
+    __shared__ unsigned long long hits[kFdmThreads / 64];
+    energy_reduce(tail.d.partial, tail.nblocks, tail.E_local, tail.Ee, sh);
+    if (threadIdx.x == 0 && *tail.b.nqueue > tail.b.limit / kQueueBlocks) *tail.b.crowded = 1;
+    deposit_queued(tail, g, 0, 1, hits);
+    __syncthreads();
+  }
   double* cur = s_fdm;
   double* nxt = s_fdm + G;
   if (threadIdx.x == 0) s_slow = 0;
@@ -195,12 +205,12 @@ static hipError_t allow_lds(Kern k, size_t bytes) {
 
 template <int MODE, int NC>
 static hipError_t block_solve(const GridView& g, const FdmArgs& u, double* T, int nsub, int* nonfinite,
-                              hipStream_t s) {
+                              const DepositTail& tail, hipStream_t s) {
   const int G = g.nx * g.ny * g.nz;
   const size_t lds = static_cast<size_t>(G) * (MODE != 0 ? 24 : 16);
   auto k = k_fdm_block<MODE, NC>;
   if (hipError_t e = allow_lds(k, lds); e != hipSuccess) return e;
-  k<<<1, kFdmThreads, lds, s>>>(g, u, T, nsub, G, nonfinite);
+  k<<<1, kFdmThreads, lds, s>>>(g, u, T, nsub, G, nonfinite, tail);
   return hipGetLastError();
 }
 
@@ -241,14 +251,15 @@ constexpr int kFdmMinTiles = 200;
 
 template <int MODE>
 static hipError_t solve_any(const GridView& g, const FdmArgs& u, double*& T, double*& Tn, int nsub,
-                            int* nonfinite, hipStream_t s) {
+                            int* nonfinite, const DepositTail& tail, hipStream_t s) {
   const int G = g.nx * g.ny * g.nz;
   if (G <= (MODE == 0 ? kFdmBlockUniform : kFdmBlockCells)) {
-    if (G <= kFdmThreads) return block_solve<MODE, 1>(g, u, T, nsub, nonfinite, s);
-    if (G <= 2 * kFdmThreads) return block_solve<MODE, 2>(g, u, T, nsub, nonfinite, s);
-    if constexpr (MODE == 0) return block_solve<MODE, 4>(g, u, T, nsub, nonfinite, s);
+    if (G <= kFdmThreads) return block_solve<MODE, 1>(g, u, T, nsub, nonfinite, tail, s);
+    if (G <= 2 * kFdmThreads) return block_solve<MODE, 2>(g, u, T, nsub, nonfinite, tail, s);
+    if constexpr (MODE == 0) return block_solve<MODE, 4>(g, u, T, nsub, nonfinite, tail, s);
   }
-  hipError_t e = hipSuccess;
+  hipError_t e = tail.E_local ? launch_deposit_tail(g, tail, s) : hipSuccess;
+  if (e != hipSuccess) return e;
   if constexpr (MODE == 0) {
     if (G >= kFdmMinTiles * 2048) e = tile_solve<16, 16, 8, 2>(g, u, T, Tn, nsub, s);
     else if (G >= kFdmMinTiles * 1024) e = tile_solve<16, 8, 8, 2>(g, u, T, Tn, nsub, s);
@@ -265,7 +276,9 @@ static hipError_t solve_any(const GridView& g, const FdmArgs& u, double*& T, dou
 }
 
 hipError_t launch_fdm_solve(const GridView& g, double*& T, double*& Tn, double inner_dt, int nsub,
-                            const FdmMaterial* uniform, bool any_tdyn, int* nonfinite, hipStream_t s) {
+                            const FdmMaterial* uniform, bool any_tdyn, int* nonfinite, hipStream_t s,
+                            const DepositTail* tail) {
+  const DepositTail rest = tail ? *tail : DepositTail();
   FdmArgs u;
   u.inner_dt = inner_dt;
   u.d3[0] = divisor(g.dx); u.d3[1] = divisor(g.dy); u.d3[2] = divisor(g.dz);
@@ -276,10 +289,10 @@ hipError_t launch_fdm_solve(const GridView& g, double*& T, double*& Tn, double i
     u.uni.div = divisor(uniform->rho * uniform->C);
     u.uni.flag = kCellDynamic;
     u.uni.flat = true;
-    return solve_any<0>(g, u, T, Tn, nsub, nonfinite, s);
+    return solve_any<0>(g, u, T, Tn, nsub, nonfinite, rest, s);
   }
-  return any_tdyn ? solve_any<2>(g, u, T, Tn, nsub, nonfinite, s)
-                  : solve_any<1>(g, u, T, Tn, nsub, nonfinite, s);
+  return any_tdyn ? solve_any<2>(g, u, T, Tn, nsub, nonfinite, rest, s)
+                  : solve_any<1>(g, u, T, Tn, nsub, nonfinite, rest, s);
 }
 
 }  // namespace eph

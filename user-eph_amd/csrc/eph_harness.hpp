@@ -40,6 +40,7 @@ struct eph_md {
   eph::DevArray<int> rep, flags, cnt, start, bin_of, bcount, bstart, bfill, items, scan_tmp, nbi;
   eph::DevArray<double> box_d;
   eph::NbBuild nbw;
+  eph::DevArray<unsigned long long> times;  // [5 nsteps + 1] of a run
   int* pinned = nullptr;  // [0..7] copy of flags, [8] the neighbour check's answer
   hipEvent_t checked = nullptr;
   std::vector<char> ckpt;  // eph_md_checkpoint_save(md, ctx, NULL) keeps it here
@@ -63,10 +64,10 @@ struct eph_md {
     x_build.assign(x.begin(), x.begin() + 3 * (size_t)nlocal);
   }
   int upload(eph_context* ctx);
-  // Ghost update and pair force of one step on device lists, the lists rebuilt
-  // first where an atom moved more than skin/2 (or force).  ev (optional): ev[2],
-  // ev[3] recorded around ghost update and pair force.  *overflow: the rebuild
-  // does not fit and the host has to do it (no ghost update, no pair force then).
-  int neighbours_and_pair(eph_context* ctx, bool force, hipEvent_t* ev, bool* rebuilt, bool* overflow);
-  int ghosts_and_pair(eph_context* ctx, hipEvent_t* ev);
+  // One step's initial kick, ghost update and pair force on device lists, the
+  // lists rebuilt in between where an atom moved more than skin/2 (or force).
+  // t (optional): device times, as in StepExtras.  *overflow: the rebuild does
+  // not fit and the host has to do it (no ghost update, no pair force then).
+  int kick_and_pair(eph_context* ctx, bool force, unsigned long long* t, bool* rebuilt, bool* overflow);
+  int ghosts_and_pair(eph_context* ctx, unsigned long long* t);
 };

@@ -8,6 +8,7 @@
 // the cooperative forms a wavefront fetches its atoms' neighbour records
 // together through LDS; the sums themselves stay one thread per atom.
 #include "eph_devfn.hpp"
+#include "eph_deposit.hpp"
 #include "eph_fdm.hpp"
 #include "eph_rng.hpp"
 
@@ -627,6 +628,44 @@ __global__ __launch_bounds__(kBlock) void k_cand_check(int nall, const double4* 
   }
 }
 
+// The ghost update (k_ghost_xv) and, with check, the candidate check of all
+// atoms at the positions it leaves
+__global__ __launch_bounds__(kBlock) void k_ghost_check(AtomsView a, WorkView w, int check,
+                                                        unsigned long long* t) {
+  const int i = (check ? 0 : a.nlocal) + blockIdx.x * kBlock + threadIdx.x;
+  if (t && blockIdx.x == 0 && threadIdx.x == 0) *t = wall_clock64();
+  if (i >= a.nlocal + a.nghost) return;
+  double4 x;
+  if (i >= a.nlocal) {
+    const int g = i - a.nlocal, o = w.ghost_owner[g];
+    const double4 p = a.pos[o];
+    const double4 s = w.ghost_shift[g];
+    x = make_double4(p.x + s.x, p.y + s.y, p.z + s.z, p.w);
+    const double4 v = a.vel[o];
+    a.pos[i] = x;
+    a.vel[i] = v;
+    if (a.pv) {
+      PosVel q;
+      q.p = x;
+      q.v = v;
+      a.pv[i] = q;
+    }
+  } else {
+    x = a.pos[i];
+  }
+  if (!check) return;
+  if (w.cstate[0] == 0) {
+    w.cref[i] = x;
+    return;
+  }
+  const double4 r = w.cref[i];
+  const double dx = x.x - r.x, dy = x.y - r.y, dz = x.z - r.z;
+  if (!(dx * dx + dy * dy + dz * dz < w.half_delta2)) {
+    const int k = atomicAdd(w.cstate + 2, 1);
+    if (k < w.moved_cap) w.moved[k] = x;
+  }
+}
+
 // the same check for a batch of replicas, with the ghost count read on the
 // device (the ensemble's recorded steps, whose ghost count changes between
 // replays; the grid covers nlocal + the ghost capacity); a moved atom's entry
@@ -655,8 +694,7 @@ __global__ __launch_bounds__(kBlock) void k_cand_check_dev(int nlocal, const int
 // when the candidates were taken, so the next check takes new reference
 // positions and the next sweep retakes the candidates.  The moved list starts
 // empty at the next check.
-__global__ void k_cand_flags(int* cstate, int moved_cap) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ __forceinline__ void cand_flags(int* cstate, int moved_cap) {
   const int retake = cstate[0] == 0;
   cstate[3] = cstate[1];
   cstate[4] = cstate[2];
@@ -664,6 +702,10 @@ __global__ void k_cand_flags(int* cstate, int moved_cap) {
   cstate[0] = retake || cstate[2] <= moved_cap ? 1 : 0;
   cstate[1] = 0;
   cstate[2] = 0;
+}
+
+__global__ void k_cand_flags(int* cstate, int moved_cap) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) cand_flags(cstate, moved_cap);
 }
 
 // the split form: 16 atoms per block
@@ -776,6 +818,7 @@ __global__ __launch_bounds__(kBlock) void k_ghost_halo(AtomsView a, TablesView t
 __global__ __launch_bounds__(kBlock) void k_ghost_rec(AtomsView a, WorkView w) {
   const int g = blockIdx.x * kBlock + threadIdx.x;
   if (g < a.nghost) ghost_rec(g, a, w);
+  if (g == 0 && w.defer_flags) cand_flags(w.cstate, w.moved_cap);
 }
 
 // positions and velocities of all atoms, packed for the w sweep
@@ -1344,10 +1387,7 @@ __global__ __launch_bounds__(kBlock) void k_colour_v_ghost(AtomsView a, WorkView
 // --------------------------------------------------------- integrator
 // FixEPH::initial_integrate / final_integrate (fix_eph.cpp:305-348)
 template <bool INITIAL>
-__global__ __launch_bounds__(kBlock) void k_integrate(AtomsView a, StepParams p) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= a.nlocal) return;
-  if (!(a.mask[i] & a.groupbit)) return;
+__device__ __forceinline__ double4 integrate_atom(const int i, const AtomsView& a, const StepParams& p) {
   const int fs = a.fstride;
   const double dtfm = p.dtf / p.mass[a.type[i]];
   double4 v = a.vel[i];
@@ -1355,8 +1395,9 @@ __global__ __launch_bounds__(kBlock) void k_integrate(AtomsView a, StepParams p)
   v.y += dtfm * a.f[fs + i];
   v.z += dtfm * a.f[2 * fs + i];
   a.vel[i] = v;
+  double4 x = v;
   if (INITIAL) {
-    double4 x = a.pos[i];
+    x = a.pos[i];
     x.x += p.dtv * v.x;
     x.y += p.dtv * v.y;
     x.z += p.dtv * v.z;
@@ -1371,6 +1412,41 @@ __global__ __launch_bounds__(kBlock) void k_integrate(AtomsView a, StepParams p)
   // the final kick leaves the records at (x', v_half) of this step's
   // post_force (what the trajectory adjoint reads back); the next initial
   // kick rewrites them before any sweep reads them
+  return x;
+}
+
+template <bool INITIAL>
+__global__ __launch_bounds__(kBlock) void k_integrate(AtomsView a, StepParams p) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i >= a.nlocal) return;
+  if (!(a.mask[i] & a.groupbit)) return;
+  integrate_atom<INITIAL>(i, a, p);
+}
+
+// the time at which block `of` and every 64th before it end, the latest of them
+__device__ __forceinline__ void stamp_end(unsigned long long* t) {
+  if (t && threadIdx.x == 0 && (gridDim.x - 1 - blockIdx.x) % 64 == 0)
+    atomicMax(t, static_cast<unsigned long long>(wall_clock64()));
+}
+
+__global__ void k_stamp(unsigned long long* t) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) *t = wall_clock64();
+}
+
+// the initial kick and the neighbour check of every local atom (the harness's
+// step); move = 0: the check alone
+__global__ __launch_bounds__(kBlock) void k_integrate_check(AtomsView a, StepParams p, StepExtras e,
+                                                            int move) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (e.t && i == 0) e.t[0] = wall_clock64();
+  if (i < a.nlocal) {
+    const bool moves = move && (a.mask[i] & a.groupbit);
+    const double4 x = moves ? integrate_atom<true>(i, a, p) : a.pos[i];
+    const double4 r = e.xref[i];
+    const double dx = x.x - r.x, dy = x.y - r.y, dz = x.z - r.z;
+    if (dx * dx + dy * dy + dz * dz > e.lim) *e.want = 1;
+  }
+  if (e.t) stamp_end(e.t + 1);
 }
 
 __global__ void k_fill_int(int* p, int n, int v) {
@@ -1711,23 +1787,6 @@ __global__ __launch_bounds__(kBlock) void k_cell_sum_huge(GridView g, DepositVie
   }
 }
 
-// E_local = sum of friction then random energies; Ee += E_local
-__device__ __forceinline__ void energy_reduce(const double* partial, int nb, double* E_local,
-                                              double* Ee, double* sh) {
-  double sF = 0.0, sR = 0.0;
-  for (int b = threadIdx.x; b < nb; b += 1024) {
-    sF += partial[2 * b];
-    sR += partial[2 * b + 1];
-  }
-  sF = block_sum(sF, sh);
-  sR = block_sum(sR, sh);
-  if (threadIdx.x == 0) {
-    const double E = sF + sR;
-    *E_local = E;
-    *Ee += E;
-  }
-}
-
 __global__ __launch_bounds__(1024) void k_energy_reduce(const double* partial, int nb,
                                                         double* E_local, double* Ee) {
   __shared__ double sh[1024];
@@ -1881,46 +1940,15 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket_wave(GridView g, Depo
 }
 
 // block 0: E_local and Ee from the block partial sums (as k_energy_reduce);
-// blocks 1..: the queued cells, each by an ordered scan over all atoms:
-// every wave ballots the atoms of the cell among its 64, and thread 0 adds
-// their values in ascending order
-__global__ __launch_bounds__(1024) void k_deposit_finish(AtomsView a, GridView g, DepositView d,
-                                                         BucketView b, int nblocks, double* E_local,
-                                                         double* Ee) {
-  const int n_items = a.nlocal;
+// blocks 1..: the queued cells
+__global__ __launch_bounds__(1024) void k_deposit_finish(DepositTail t, GridView g) {
   __shared__ double sh[1024];
   __shared__ unsigned long long hits[16];
   if (blockIdx.x == 0) {
-    energy_reduce(d.partial, nblocks, E_local, Ee, sh);
-    if (threadIdx.x == 0 && *b.nqueue > b.limit) *b.crowded = 1;
-    return;
-  }
-  const int nq = *b.nqueue;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int q = blockIdx.x - 1; q < nq; q += gridDim.x - 1) {
-    const int c = b.queue[q];
-    double acc = g.dT[c];  // meaningful in thread 0 only
-    for (int pass = 0; pass < 2; ++pass) {
-      const double* v = pass == 0 ? d.v1 : d.v2;
-      if (!v) continue;
-      for (int base = 0; base < n_items; base += 1024) {
-        const int i = base + threadIdx.x;
-        bool in = false;
-        if (i < n_items && (a.mask[i] & a.groupbit)) {
-          const double4 x = a.pos[i];
-          in = cell_of(g, x.x, x.y, x.z) == c;
-        }
-        const unsigned long long m = __ballot(in);
-        if (lane == 0) hits[wv] = m;
-        __syncthreads();
-        if (threadIdx.x == 0)
-          for (int w2 = 0; w2 < 16; ++w2)
-            for (unsigned long long bits = hits[w2]; bits; bits &= bits - 1)
-              acc += v[base + 64 * w2 + __builtin_ctzll(bits)];
-        __syncthreads();
-      }
-    }
-    if (threadIdx.x == 0) g.dT[c] = acc;
+    energy_reduce(t.d.partial, t.nblocks, t.E_local, t.Ee, sh);
+    if (threadIdx.x == 0 && *t.b.nqueue > t.b.limit) *t.b.crowded = 1;
+  } else {
+    deposit_queued(t, g, blockIdx.x - 1, gridDim.x - 1, hits);
   }
 }
 
@@ -2025,9 +2053,11 @@ __global__ __launch_bounds__(kBlock) void k_peratom(AtomsView a, TablesView t, W
 // path (140 entries, 78 of them inside the cutoff).
 template <int S, int U>
 __global__ __launch_bounds__(kBlock) void k_lj(AtomsView a, const int* __restrict__ nbr,
-                                                     const int* __restrict__ nn, int stride,
-                                                     double lj1, double lj2, double rc2) {
+                                               const int* __restrict__ nn, int stride,
+                                               double lj1, double lj2, double rc2,
+                                               unsigned long long* t) {
   __shared__ double2 s_split[(kBlock / 64) * split_stage_lj(U)];
+  if (t && blockIdx.x == 0 && threadIdx.x == 0) *t = wall_clock64();
   const int wv = threadIdx.x >> 6;
   double2* stage = s_split + wv * split_stage_lj(U);
   double* terms = reinterpret_cast<double*>(stage);
@@ -2085,6 +2115,7 @@ __global__ __launch_bounds__(kBlock) void k_lj(AtomsView a, const int* __restric
     split_round_end();
   }
   if (valid && s < 3) a.f[s * a.fstride + i] = acc;
+  if (t) stamp_end(t + 1);
 }
 
 __global__ __launch_bounds__(kBlock) void k_max_disp2(AtomsView a, const double4* ref,
@@ -2488,6 +2519,14 @@ hipError_t launch_ghost_xv(const AtomsView& a, const int* owner, const double4* 
   return hipGetLastError();
 }
 
+hipError_t launch_ghost_check(const AtomsView& a, const WorkView& w, bool check, unsigned long long* t,
+                              hipStream_t s) {
+  const int n = (check ? a.nlocal : 0) + a.nghost;
+  if (n > 0) k_ghost_check<<<nblk(n), kBlock, 0, s>>>(a, w, check ? 1 : 0, t);
+  else if (t) k_stamp<<<1, 64, 0, s>>>(t);
+  return hipGetLastError();
+}
+
 hipError_t launch_csr_to_ell(int nlocal, const int* off, const int* idx, int neighmask, int nall,
                              int* ell, int* nn, int stride, int width, int* bad, hipStream_t s) {
   if (nlocal == 0) return hipSuccess;
@@ -2545,6 +2584,11 @@ static int resolve_form(const AtomsView& a, const TablesView& t, int form, int d
   return form;
 }
 
+bool density_walks_candidates(const AtomsView& a, const TablesView& t, int form) {
+  const int f = resolve_form(a, t, form, 0);
+  return f == 0 || f >= kChunkOcc4;
+}
+
 // LDS request of a cache-table launch: the staging its waves use, or more
 // so that at most 4, 3 or 2 blocks share a CU (160 KB of LDS per CU)
 static size_t chunk_lds(int form, size_t need) {
@@ -2597,7 +2641,7 @@ hipError_t launch_density_w(const AtomsView& a, const TablesView& t, const StepP
   const bool keep = w.rcand2 > 0.0 && w.cstate;
   WorkView wc = w;
   if (!keep) wc.rcand2 = 0.0;
-  if (keep) k_cand_check<<<nblk(a.nlocal + a.nghost), kBlock, 0, s>>>(a.nlocal + a.nghost, a.pos, wc);
+  if (keep && !w.cand_checked) k_cand_check<<<nblk(a.nlocal + a.nghost), kBlock, 0, s>>>(a.nlocal + a.nghost, a.pos, wc);
   if (ev) (void)hipEventRecord(ev[0], s);  // the sweep alone, without the candidate check
   const size_t dl = chunk_lds(f, kDensityStageBytes);
 #define EPH_DW(XI, F, M)                                                                       \
@@ -2615,7 +2659,7 @@ hipError_t launch_density_w(const AtomsView& a, const TablesView& t, const StepP
 #undef EPH_DW_M
 #undef EPH_DW
   if (ev) (void)hipEventRecord(ev[1], s);
-  if (keep) k_cand_flags<<<1, 64, 0, s>>>(w.cstate, w.moved_cap);
+  if (keep && !w.defer_flags) k_cand_flags<<<1, 64, 0, s>>>(w.cstate, w.moved_cap);
   return hipGetLastError();
 }
 
@@ -2719,8 +2763,18 @@ hipError_t launch_colour_v(const AtomsView& a, const StepParams& p, const WorkVi
   return hipGetLastError();
 }
 
-hipError_t launch_integrate(const AtomsView& a, const StepParams& p, bool initial, hipStream_t s) {
+hipError_t launch_stamp(unsigned long long* t, hipStream_t s) {
+  k_stamp<<<1, 64, 0, s>>>(t);
+  return hipGetLastError();
+}
+
+hipError_t launch_integrate(const AtomsView& a, const StepParams& p, bool initial, hipStream_t s,
+                            const StepExtras* x) {
   if (a.nlocal == 0) return hipSuccess;
+  if (x) {
+    k_integrate_check<<<nblk(a.nlocal), kBlock, 0, s>>>(a, p, *x, initial ? 1 : 0);
+    return hipGetLastError();
+  }
   if (initial) k_integrate<true><<<nblk(a.nlocal), kBlock, 0, s>>>(a, p);
   else k_integrate<false><<<nblk(a.nlocal), kBlock, 0, s>>>(a, p);
   return hipGetLastError();
@@ -2787,7 +2841,7 @@ hipError_t launch_deposit_cells(const GridView& g, const DepositView& d, int n_i
 hipError_t launch_deposit_bucket(const AtomsView& a, const GridView& g, const StepParams& p,
                                  const WorkView& w, const DepositView& d, const BucketView& b,
                                  bool fric, bool rand, bool kick, double* E_local, double* Ee,
-                                 hipStream_t s) {
+                                 hipStream_t s, DepositTail* tail) {
   const int G = g.nx * g.ny * g.nz;
   const int nb = nblk(a.nlocal);
   if (a.nlocal > 0) {
@@ -2805,7 +2859,17 @@ hipError_t launch_deposit_bucket(const AtomsView& a, const GridView& g, const St
   if (!rand) dc.v2 = nullptr;
   if (b.cap == kBucket) k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, dc, b, G);
   else k_deposit_bucket_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, dc, b, G);
-  k_deposit_finish<<<1 + kQueueBlocks, 1024, 0, s>>>(a, g, dc, b, a.nlocal > 0 ? nb : 0, E_local, Ee);
+  DepositTail t;
+  t.a = a; t.d = dc; t.b = b; t.nblocks = a.nlocal > 0 ? nb : 0; t.E_local = E_local; t.Ee = Ee;
+  if (tail) {
+    *tail = t;
+    return hipGetLastError();
+  }
+  return launch_deposit_tail(g, t, s);
+}
+
+hipError_t launch_deposit_tail(const GridView& g, const DepositTail& tail, hipStream_t s) {
+  k_deposit_finish<<<1 + kQueueBlocks, 1024, 0, s>>>(tail, g);
   return hipGetLastError();
 }
 
@@ -2854,14 +2918,14 @@ hipError_t launch_peratom(const AtomsView& a, const TablesView& t, const WorkVie
 }
 
 hipError_t launch_lj(const AtomsView& a, const int* nbr, const int* nn, int stride, double eps,
-                     double sigma, double rc2, hipStream_t s) {
+                     double sigma, double rc2, hipStream_t s, unsigned long long* t) {
   if (a.nlocal == 0) return hipSuccess;
   const double s6 = sigma * sigma * sigma * sigma * sigma * sigma;
   const double lj1 = 48.0 * eps * s6 * s6, lj2 = 24.0 * eps * s6;
   if (a.nlocal <= kSplitLj16)
-    k_lj<16, 3><<<nblk(a.nlocal, kBlock / 16), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2);
+    k_lj<16, 3><<<nblk(a.nlocal, kBlock / 16), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2, t);
   else
-    k_lj<8, 3><<<nblk(a.nlocal, kBlock / 8), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2);
+    k_lj<8, 3><<<nblk(a.nlocal, kBlock / 8), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2, t);
   return hipGetLastError();
 }
 

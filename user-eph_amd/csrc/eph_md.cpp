@@ -267,42 +267,41 @@ int eph_md::upload(eph_context* ctx) {
   return EPH_OK;
 }
 
-int eph_md::ghosts_and_pair(eph_context* ctx, hipEvent_t* ev) {
-  hipStream_t s = ctx->stream;
-  if (ev) EPH_HIP(this, hipEventRecord(ev[2], s));
-  EPH_HIP(this, launch_ghost_xv(ctx->atoms_view(), ctx->ghost_owner.p, ctx->ghost_shift.p, s));
+int eph_md::ghosts_and_pair(eph_context* ctx, unsigned long long* t) {
+  if (int rc = ctx->dev_ghosts(t ? t + 2 : nullptr)) return fail(rc, ctx->err);
   EPH_HIP(this, launch_lj(ctx->atoms_view(), lj_nbr.p, lj_nn.p, lj_stride, cfg.lj_eps, cfg.lj_sigma,
-                          cfg.cut_lj * cfg.cut_lj, s));
-  if (ev) EPH_HIP(this, hipEventRecord(ev[3], s));
+                          cfg.cut_lj * cfg.cut_lj, ctx->stream, t ? t + 3 : nullptr));
   return EPH_OK;
 }
 
 // Up to this many atoms the ghost update and the pair force are queued behind
 // the check before the host has its answer, so that the device has work while
 // the host waits (about 10 us); a rebuild then runs them again.  Above, the
-// pair force run in vain (37 us at 32,000 atoms, 145 at 256,000) costs more
+// pair force run in vain (20 us at 32,000 atoms, 125 at 256,000) costs more
 // than the waits it covers once lists are rebuilt every few steps.
 constexpr int kSpeculateAtoms = 65536;
 
-int eph_md::neighbours_and_pair(eph_context* ctx, bool force, hipEvent_t* ev, bool* rebuilt,
-                                bool* overflow) {
+int eph_md::kick_and_pair(eph_context* ctx, bool force, unsigned long long* t, bool* rebuilt,
+                          bool* overflow) {
   hipStream_t s = ctx->stream;
   *rebuilt = *overflow = false;
   volatile int* want = pinned + 8;
   const bool ahead = !force && nlocal <= kSpeculateAtoms;
-  *want = force ? 1 : 0;
-  if (!force) {
-    const double lim = 0.25 * cfg.skin * cfg.skin;
-    EPH_HIP(this, launch_nb_want(nlocal, ctx->pos.p, xref.p, lim, pinned + 8, s));
-    if (ahead) {
-      EPH_HIP(this, hipEventRecord(checked, s));
-      if (int rc = ghosts_and_pair(ctx, ev)) return rc;
-      EPH_HIP(this, hipEventSynchronize(checked));
-    } else {
-      EPH_HIP(this, hipStreamSynchronize(s));
-    }
+  *want = 0;
+  StepExtras x;
+  x.xref = xref.p;
+  x.lim = 0.25 * cfg.skin * cfg.skin;
+  x.want = pinned + 8;
+  x.t = t;
+  if (int rc = ctx->dev_initial_integrate(&x)) return fail(rc, ctx->err);
+  if (ahead) {
+    EPH_HIP(this, hipEventRecord(checked, s));
+    if (int rc = ghosts_and_pair(ctx, t)) return rc;
+    EPH_HIP(this, hipEventSynchronize(checked));
+  } else {
+    EPH_HIP(this, hipStreamSynchronize(s));
   }
-  if (*want) {
+  if (*want || force) {
     EPH_HIP(this, launch_nb_force(nbw.go, s));
     EPH_HIP(this, launch_nb_build(nbw, s));
     EPH_HIP(this, hipMemcpyAsync(pinned, flags.p, 8 * sizeof(int), hipMemcpyDeviceToHost, s));
@@ -317,7 +316,7 @@ int eph_md::neighbours_and_pair(eph_context* ctx, bool force, hipEvent_t* ev, bo
     *rebuilt = true;
   }
   if (ahead && !*rebuilt) return EPH_OK;
-  return ghosts_and_pair(ctx, ev);
+  return ghosts_and_pair(ctx, t);
 }
 
 // copy the device-built system back into the host arrays (for checking)
@@ -615,11 +614,12 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
                int* nrebuild) {
   if (!md || !ctx || nsteps < 0) return EPH_ERR_ARGS;
   hipStream_t s = ctx->stream;
-  // five events per step, read after the last step: no step waits for the
-  // previous one to finish, so each step's first kernels are queued behind it
-  std::vector<hipEvent_t> evs(5 * static_cast<size_t>(nsteps));
-  std::vector<char> host_rebuilt(nsteps, 0);
-  for (auto& e : evs) EPH_HIP(md, hipEventCreate(&e));
+  // five device times per step, read after the last step: no step waits for
+  // the previous one to finish, so each step's first kernels are queued behind it
+  const size_t nt = 5 * static_cast<size_t>(nsteps) + 1;
+  EPH_HIP(md, md->times.reserve(nt));
+  EPH_HIP(md, launch_fill_double(reinterpret_cast<double*>(md->times.p), static_cast<long>(nt), 0.0, s));
+  std::vector<char> host_rebuilt(nsteps, 0), checked(nsteps, 0);
   double t_fix = 0, t_total = 0, t_pair = 0, t_rebuild = 0;
   int nreb = 0;
   const double lim = 0.25 * md->cfg.skin * md->cfg.skin;  // (host rebuilds)
@@ -629,12 +629,7 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
   for (int st = 0; st < nsteps && rc == EPH_OK; ++st) {
     const long long step = first_step + st;
     ctx->step = step;
-    hipEvent_t* ev = evs.data() + 5 * static_cast<size_t>(st);
-    // a step starts where the previous one ended: the previous step's end
-    // event serves as this step's start (one event less between two kernels)
-    if (st == 0) EPH_HIP(md, hipEventRecord(ev[0], s));
-    if ((rc = ctx->dev_initial_integrate())) break;
-    EPH_HIP(md, hipEventRecord(ev[1], s));
+    unsigned long long* tt = md->times.p + 5 * static_cast<size_t>(st);
     bool host_rebuild = false;
     if (md->device_rebuild) {
       // neighbour check and, when an atom moved more than skin/2, the device
@@ -648,7 +643,7 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
       const bool force = md->force_next;
       md->force_next = false;
       bool rebuilt = false;
-      rc = md->neighbours_and_pair(ctx, force, ev, &rebuilt, &host_rebuild);
+      rc = md->kick_and_pair(ctx, force, tt, &rebuilt, &host_rebuild);
       // the candidate buffers belong to this step's launch only (the
       // context may reallocate them before the next)
       md->nbw.lists.cand = nullptr;
@@ -657,6 +652,9 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
       if (rc) break;
       if (rebuilt) ++nreb;
     } else {
+      EPH_HIP(md, launch_stamp(tt, s));
+      if ((rc = ctx->dev_initial_integrate())) break;
+      EPH_HIP(md, launch_stamp(tt + 1, s));
       EPH_HIP(md, launch_max_disp2(ctx->atoms_view(), md->xref.p, md->partial.p, nbp, s));
       EPH_HIP(md, hipMemcpyAsync(part.data(), md->partial.p, nbp * sizeof(double), hipMemcpyDeviceToHost, s));
       EPH_HIP(md, hipStreamSynchronize(s));
@@ -674,31 +672,41 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
       ++nreb;
       t_rebuild += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     }
-    if ((!md->device_rebuild || host_rebuild) && (rc = md->ghosts_and_pair(ctx, ev))) break;
+    if ((!md->device_rebuild || host_rebuild) && (rc = md->ghosts_and_pair(ctx, tt))) break;
+    checked[st] = ctx->cand_checked ? 1 : 0;
     if ((rc = ctx->dev_post_force())) break;
     // nothing runs between the two hooks here: one pass where the deposit allows
     if ((rc = ctx->dev_final_integrate_end_of_step(step))) break;
-    EPH_HIP(md, hipEventRecord(ev[4], s));
     host_rebuilt[st] = host_rebuild ? 1 : 0;
   }
   if (rc == EPH_OK && nsteps > 0) {
-    EPH_HIP(md, hipEventSynchronize(evs[5 * static_cast<size_t>(nsteps) - 1]));
+    EPH_HIP(md, launch_stamp(md->times.p + nt - 1, s));
+    std::vector<unsigned long long> th(nt);
+    EPH_HIP(md, hipMemcpyAsync(th.data(), md->times.p, nt * sizeof(th[0]), hipMemcpyDeviceToHost, s));
+    EPH_HIP(md, hipStreamSynchronize(s));
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device) != hipSuccess || khz <= 0)
+      khz = 100000;
+    auto ms = [&](unsigned long long a, unsigned long long b) { return b > a ? (b - a) / (double)khz : 0.0; };
     for (int st = 0; st < nsteps; ++st) {
-      const hipEvent_t* ev = evs.data() + 5 * static_cast<size_t>(st);
-      const hipEvent_t start = st == 0 ? ev[0] : ev[-1];
-      float a = 0, b = 0, c = 0, d = 0, e = 0;
-      EPH_HIP(md, hipEventElapsedTime(&a, start, ev[1]));
-      EPH_HIP(md, hipEventElapsedTime(&b, ev[3], ev[4]));
-      EPH_HIP(md, hipEventElapsedTime(&c, ev[2], ev[3]));
-      EPH_HIP(md, hipEventElapsedTime(&d, start, ev[4]));
-      if (!host_rebuilt[st]) EPH_HIP(md, hipEventElapsedTime(&e, ev[1], ev[2]));
-      t_fix += a + b;
-      t_pair += c;
-      t_total += d;
-      t_rebuild += e;  // device neighbour check / rebuild
+      const unsigned long long* q = th.data() + 5 * static_cast<size_t>(st);
+      const unsigned long long kicked = std::max(q[0], q[1]), next = q[5];
+      // Two kernels serve both sides and count by the bytes that each moves:
+      // the kick (224 B an atom) with the check of the lists (32), and the
+      // ghost update (228 B a ghost) with the candidate check (64 an atom).
+      const double kick = ms(q[0], kicked), ghosts = ms(q[2], q[3]);
+      const double kick_fix = md->device_rebuild ? 224.0 / 256.0 : 1.0;
+      const double check_bytes = checked[st] ? 64.0 * (md->nlocal + md->nghost) : 0.0;
+      const double ghosts_fix = check_bytes > 0.0 ? check_bytes / (check_bytes + 228.0 * md->nghost) : 0.0;
+      t_fix += kick * kick_fix + ghosts * ghosts_fix;
+      t_rebuild += kick * (1.0 - kick_fix);
+      t_pair += ghosts * (1.0 - ghosts_fix);
+      t_fix += ms(q[4], next);
+      t_pair += ms(q[3], q[4]);
+      t_total += ms(q[0], next);
+      if (!host_rebuilt[st]) t_rebuild += ms(kicked, q[2]);  // device neighbour check / rebuild
     }
   }
-  for (auto& e : evs) (void)hipEventDestroy(e);
   if (rc != EPH_OK) {
     if (md->err.empty()) md->err = ctx->err;
     return rc;

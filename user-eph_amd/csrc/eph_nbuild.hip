@@ -41,18 +41,6 @@ __global__ __launch_bounds__(kBlock) void k_nb_check(int nlocal, const double4* 
   if (dx * dx + dy * dy + dz * dz > lim) atomicOr(go, 1);
 }
 
-// the same into host memory (a flag that the host cleared): a plain store, the
-// same value from every thread that makes one
-__global__ __launch_bounds__(kBlock) void k_nb_want(int nlocal, const double4* __restrict__ pos,
-                                                    const double4* __restrict__ ref, double lim,
-                                                    int* want) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nlocal) return;
-  const double4 p = pos[i], q = ref[i];
-  const double dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-  if (dx * dx + dy * dy + dz * dz > lim) *want = 1;
-}
-
 // Domain::remap of the locals
 __global__ __launch_bounds__(kBlock) void k_nb_wrap(int nlocal, double4* pos, PosVel* pv,
                                                     const int* rep, NbBoxes b, const int* go) {
@@ -389,7 +377,10 @@ __global__ __launch_bounds__(kBlock) void k_nb_finish(int nlocal, const int* ng,
   // of this rebuild (locals and the ghosts just made); otherwise the next
   // density sweep retakes them
   if (cand_written && i < nlocal + *ng) cref[i] = pos[i];
-  if (i == 0 && cand_valid) *cand_valid = cand_written ? 1 : 0;
+  if (i == 0 && cand_valid) {
+    cand_valid[0] = cand_written ? 1 : 0;
+    cand_valid[2] = 0;  // atoms that a check before this rebuild found moved
+  }
   // the last block clears the flag only after every block has read it: the
   // flag is cleared by the next step's k_nb_reset instead
   if (i == 0) atomicAdd(nreb, 1);
@@ -711,12 +702,6 @@ hipError_t launch_nb_check(int nlocal, const double4* pos, const double4* ref, d
                            hipStream_t s) {
   k_nb_reset<<<1, 64, 0, s>>>(go);
   if (nlocal > 0) k_nb_check<<<nbk(nlocal), kBlock, 0, s>>>(nlocal, pos, ref, lim, go);
-  return hipGetLastError();
-}
-
-hipError_t launch_nb_want(int nlocal, const double4* pos, const double4* ref, double lim, int* want,
-                          hipStream_t s) {
-  if (nlocal > 0) k_nb_want<<<nbk(nlocal), kBlock, 0, s>>>(nlocal, pos, ref, lim, want);
   return hipGetLastError();
 }
 

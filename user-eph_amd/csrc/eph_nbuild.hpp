@@ -69,7 +69,7 @@ struct NbBuild {
   int* nrebuild = nullptr;  // [1] count of device rebuilds
   // [1] the density sweep's candidate state: a rebuild that writes the
   // candidates (lists.cand) marks them valid with cref = the positions of the
-  // rebuild; one that does not clears it
+  // rebuild; one that does not clears it.  [2], the moved atoms, is emptied
   int* cand_valid = nullptr;
   double4* cref = nullptr;  // [nlocal + ghost_cap]
   int* cnt = nullptr;       // [nlocal + ghost_cap]
@@ -86,9 +86,6 @@ struct NbBuild {
 
 hipError_t launch_nb_check(int nlocal, const double4* pos, const double4* ref, double lim, int* go,
                            hipStream_t s);
-// *want (pinned host memory, cleared by the host) = 1 when an atom moved too far
-hipError_t launch_nb_want(int nlocal, const double4* pos, const double4* ref, double lim, int* want,
-                          hipStream_t s);
 hipError_t launch_nb_force(int* go, hipStream_t s);
 hipError_t launch_nb_build(const NbBuild& w, hipStream_t s);
 
