@@ -23,39 +23,43 @@ __device__ __forceinline__ void energy_reduce(const double* partial, int nb, dou
   }
 }
 
-// The queued cells q0, q0 + step, ...: each by an ordered scan over all atoms
-// by a block of 1024 threads; every wave ballots the atoms of the cell among
-// its 64, and thread 0 adds their values in ascending order.
+// One overfull cell c of grid g: dT_e plus the values of its atoms among
+// [i0, i1), by an ordered scan of a block of 1024 threads; every wave ballots
+// the atoms of the cell among its 64, and thread 0 adds their values in
+// ascending order.
+__device__ __forceinline__ void queued_cell(const AtomsView& a, const DepositView& d, const GridView& g,
+                                            const int c, const int i0, const int i1,
+                                            unsigned long long* hits) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double acc = g.dT[c];  // meaningful in thread 0 only
+  for (int pass = 0; pass < 2; ++pass) {
+    const double* v = pass == 0 ? d.v1 : d.v2;
+    if (!v) continue;
+    for (int base = i0; base < i1; base += 1024) {
+      const int i = base + threadIdx.x;
+      bool in = false;
+      if (i < i1 && (a.mask[i] & a.groupbit)) {
+        const double4 x = a.pos[i];
+        in = cell_of(g, x.x, x.y, x.z) == c;
+      }
+      const unsigned long long m = __ballot(in);
+      if (lane == 0) hits[wv] = m;
+      __syncthreads();
+      if (threadIdx.x == 0)
+        for (int w2 = 0; w2 < 16; ++w2)
+          for (unsigned long long bits = hits[w2]; bits; bits &= bits - 1)
+            acc += v[base + 64 * w2 + __builtin_ctzll(bits)];
+      __syncthreads();
+    }
+  }
+  if (threadIdx.x == 0) g.dT[c] = acc;
+}
+
+// the queued cells q0, q0 + step, ... of a single grid
 __device__ __forceinline__ void deposit_queued(const DepositTail& t, const GridView& g, const int q0,
                                                const int step, unsigned long long* hits) {
-  const int n_items = t.a.nlocal;
   const int nq = *t.b.nqueue;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int q = q0; q < nq; q += step) {
-    const int c = t.b.queue[q];
-    double acc = g.dT[c];  // meaningful in thread 0 only
-    for (int pass = 0; pass < 2; ++pass) {
-      const double* v = pass == 0 ? t.d.v1 : t.d.v2;
-      if (!v) continue;
-      for (int base = 0; base < n_items; base += 1024) {
-        const int i = base + threadIdx.x;
-        bool in = false;
-        if (i < n_items && (t.a.mask[i] & t.a.groupbit)) {
-          const double4 x = t.a.pos[i];
-          in = cell_of(g, x.x, x.y, x.z) == c;
-        }
-        const unsigned long long m = __ballot(in);
-        if (lane == 0) hits[wv] = m;
-        __syncthreads();
-        if (threadIdx.x == 0)
-          for (int w2 = 0; w2 < 16; ++w2)
-            for (unsigned long long bits = hits[w2]; bits; bits &= bits - 1)
-              acc += v[base + 64 * w2 + __builtin_ctzll(bits)];
-        __syncthreads();
-      }
-    }
-    if (threadIdx.x == 0) g.dT[c] = acc;
-  }
+  for (int q = q0; q < nq; q += step) queued_cell(t.a, t.d, g, t.b.queue[q], 0, t.a.nlocal, hits);
 }
 
 }  // namespace eph

@@ -356,6 +356,23 @@ hipError_t launch_prl_forces_batch(const AtomsView& a, const TablesView& t, cons
 hipError_t launch_deposit_atoms_batch(const AtomsView& a, const GridView* grids, const int* cell_off,
                                       const StepParams& p, const WorkView& w, const DepositView& d,
                                       const Chunk* chunks, int nchunks, hipStream_t s);
+// the bucketed deposit of a batch, with the final kick if asked; all: the
+// replicas' cells as one flat grid; the tallies per replica
+hipError_t launch_deposit_bucket_batch(const AtomsView& a, const GridView* grids, const int* cell_off,
+                                       const int* cell_rep, const GridView& all, const StepParams& p,
+                                       const WorkView& w, const DepositView& d, const BucketView& b,
+                                       const Chunk* chunks, int nchunk, const int* chunk0,
+                                       const int* nchunks, int nrep, bool kick, double* E_local,
+                                       double* Ee, hipStream_t s);
+// The T_e solve of a batch with one workgroup per replica, in place (as
+// launch_fdm_solve).  fdm_batch_args fills a replica's entry of
+// fdm_batch_args_size() bytes; fits: the largest grid has no more cells than a
+// workgroup holds.  uniform: every replica's cells are of one material.
+size_t fdm_batch_args_size();
+void fdm_batch_args(void* entry, const GridView& g, double inner_dt, const FdmMaterial* uniform);
+bool fdm_batch_fits(int max_cells, bool uniform);
+hipError_t launch_fdm_batch(const GridView* grids, const void* args, const int* nsub, int nrep, int max_cells,
+                            bool uniform, int* nonfinite, hipStream_t s);
 hipError_t launch_energy_reduce_batch(const double* partial, const int* chunk0, const int* nchunks,
                                       int nrep, double* E_local, double* Ee, hipStream_t s);
 hipError_t launch_fdm_substep_batch(const GridView* grids, const int* cell_rep, const int* cell_off,

@@ -67,11 +67,22 @@ struct eph_ensemble {
   DevArray<int> grid_steps, max_sub_dev;
   int* max_sub_host = nullptr;  // pinned
   DepositBuffers dep;
+  // bucketed deposit: slots per cell (0: counted), the buckets, and the pinned
+  // flag that the device sets when too many cells overflowed theirs
+  int slots = 0;
+  DevArray<int> bk_count, bk_items, bk_queue, bk_nq;
+  int* crowded = nullptr;
+  bool bucketed() const { return slots > 0 && !*static_cast<volatile int*>(crowded); }
+  // the T_e solve with a workgroup per replica
+  bool fdm_block = false, fdm_uniform = false;
+  int max_cells = 0;
+  DevArray<char> fdm_args;
   GridView gall;  // the concatenated grid as one flat array (deposit, clears)
   // recorded step
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int graph_nlog = -1;
+  bool graph_bucketed = false;
   int var_density = 0, var_force = 0;  // kernel forms chosen by autotune()
 
   int fail(int code, const std::string& m) { err = m; return code; }
@@ -87,6 +98,7 @@ struct eph_ensemble {
       eph_md_destroy(r.md);
     }
     if (max_sub_host) (void)hipHostFree(max_sub_host);
+    if (crowded) (void)hipHostFree(crowded);
     eph_destroy(sys);
   }
   int setup(long long first);
@@ -306,6 +318,32 @@ int eph_ensemble::setup(long long first) {
   EPH_HIP(this, launch_fill_double(Ee.p, R, 0.0, s));
   EPH_HIP(this, launch_fill_int(nonfinite.p, 1, 0, s));
   EPH_HIP(this, dep.reserve(nl, G, nchunk));
+  if (sys->flags & (EPH_FRICTION | EPH_RANDOM)) slots = bucket_slots(nl, G);
+  if (slots) {
+    EPH_HIP(this, bk_count.reserve(G));  // zero-filled
+    EPH_HIP(this, bk_items.reserve(static_cast<size_t>(G) * slots));
+    EPH_HIP(this, bk_queue.reserve(G));
+    EPH_HIP(this, bk_nq.reserve(1));
+    if (!crowded) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&crowded), sizeof(int), hipHostMallocDefault));
+    *crowded = 0;
+  }
+  fdm_uniform = true;
+  max_cells = 0;
+  for (const Replica& p : reps) {
+    fdm_uniform = fdm_uniform && p.fix->grid->uniform;
+    max_cells = std::max(max_cells, p.ncells);
+  }
+  fdm_block = !any_tdyn && fdm_batch_fits(max_cells, fdm_uniform);
+  std::vector<char> fa(R * fdm_batch_args_size());
+  if (fdm_block) {
+    for (int r = 0; r < R; ++r) {
+      const auto& h = reps[r].fix->grid->h;
+      const FdmMaterial mat{h.kappa[0], h.S[0], h.rho[0], h.C[0]};
+      fdm_batch_args(fa.data() + r * fdm_batch_args_size(), gv[r], reps[r].inner_dt, fdm_uniform ? &mat : nullptr);
+    }
+    EPH_HIP(this, fdm_args.reserve(fa.size()));
+    EPH_HIP(this, hipMemcpyAsync(fdm_args.p, fa.data(), fa.size(), hipMemcpyHostToDevice, s));
+  }
   EPH_HIP(this, hipStreamSynchronize(s));
   step0 = first;
   next_step = first;
@@ -341,11 +379,21 @@ int eph_ensemble::enqueue_step(int nlog) {
   if (sys->model == 4)
     EPH_HIP(this, launch_prl_forces_batch(a, sys->tabs, gviews.p, p, w, chunks.p, nchunk, s,
                                           var_force));
-  if ((rc = sys->dev_final_integrate())) return fail(rc, sys->err);
-  // end_of_step (fix_eph.cpp:350-429) and EPH_FDM::solve per replica
+  // final_integrate and end_of_step (fix_eph.cpp:350-429), EPH_FDM::solve per replica
   const bool fric = sys->flags & EPH_FRICTION, rnd = sys->flags & EPH_RANDOM;
+  const bool buckets = (fric || rnd) && bucketed();
+  if (!buckets && (rc = sys->dev_final_integrate())) return fail(rc, sys->err);
   const int R = static_cast<int>(reps.size());
-  if (fric || rnd) {
+  if (buckets) {
+    BucketView b;
+    b.cap = slots;
+    b.count = bk_count.p; b.items = bk_items.p; b.queue = bk_queue.p; b.nqueue = bk_nq.p;
+    b.limit = queue_limit(nl / R);
+    b.crowded = crowded;
+    EPH_HIP(this, launch_deposit_bucket_batch(a, gviews.p, cell_off.p, cell_rep.p, gall, p, w, dep.view(true), b,
+                                              chunks.p, nchunk, chunk0.p, nchunks.p, R,
+                                              !(sys->flags & EPH_NOINT), E_local.p, Ee.p, s));
+  } else if (fric || rnd) {
     DepositView d = dep.view(true);
     EPH_HIP(this, launch_fill_int(d.count, G + 1, 0, s));
     EPH_HIP(this, launch_deposit_atoms_batch(a, gviews.p, cell_off.p, p, w, d, chunks.p, nchunk, s));
@@ -370,10 +418,16 @@ int eph_ensemble::enqueue_step(int nlog) {
   return EPH_OK;
 }
 
-// the stencil sub-steps of every replica: nsub launches, replicas with fewer
-// sub-steps copy in the extra ones; then dT_e is cleared for the next step
+// the stencil sub-steps of every replica: one workgroup each where the grids
+// fit, else nsub launches, in which replicas with fewer sub-steps copy in the
+// extra ones; dT_e is cleared for the next step
 int eph_ensemble::enqueue_fdm(int nsub) {
   hipStream_t s = sys->stream;
+  if (fdm_block) {
+    EPH_HIP(this, launch_fdm_batch(gviews.p, fdm_args.p, sub_n.p, static_cast<int>(reps.size()), max_cells,
+                                   fdm_uniform, nonfinite.p, s));
+    return EPH_OK;
+  }
   for (int n = 0; n < nsub; ++n) {
     const double* in = (n % 2 == 0) ? T.p : Tn.p;
     double* out = (n % 2 == 0) ? Tn.p : T.p;
@@ -466,11 +520,12 @@ int eph_ensemble::autotune(double* ms) {
 }
 
 int eph_ensemble::record(int nlog) {
-  if (exec && graph_nlog == nlog) return EPH_OK;
+  if (exec && graph_nlog == nlog && graph_bucketed == bucketed()) return EPH_OK;
   if (exec) { (void)hipGraphExecDestroy(exec); exec = nullptr; }
   if (graph) { (void)hipGraphDestroy(graph); graph = nullptr; }
   hipStream_t s = sys->stream;
   EPH_HIP(this, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+  const bool was = bucketed();
   int rc = enqueue_step(nlog);
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(s, &g);
@@ -482,6 +537,7 @@ int eph_ensemble::record(int nlog) {
   graph = g;
   EPH_HIP(this, hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
   graph_nlog = nlog;
+  graph_bucketed = was;
   return EPH_OK;
 }
 

@@ -10,6 +10,8 @@
 //   10^3 cells 118 -> 35 us, 16^3 118 -> 66 (one workgroup)
 //   20^3 117 -> 78, 40^3 119 -> 80 (8 x 8 x 4 tiles, 3 sub-steps a launch)
 //   64^3 144 -> 117 (16 x 8 x 8 tiles, 2), 80^3 226 -> 148 (16 x 16 x 8, 2)
+#include <cstring>
+
 #include "eph_deposit.hpp"
 #include "eph_fdm.hpp"
 
@@ -30,19 +32,9 @@ struct FdmArgs {
 };
 
 template <int MODE, int NC>
-__global__ __launch_bounds__(kFdmThreads) void k_fdm_block(GridView g, FdmArgs u, double* __restrict__ T,
-                                                           int nsub, int G, int* nonfinite,
-                                                           DepositTail tail) {
-  extern __shared__ double s_fdm[];
+__device__ __forceinline__ void fdm_block(const GridView& g, const FdmArgs& u, double* __restrict__ T, int nsub,
+                                          int G, int* nonfinite, double* s_fdm) {
   __shared__ int s_slow;
-  if (tail.E_local) {  // the deposit's remainder, which completes dT_e
-    __shared__ double sh[kFdmThreads];
-    __shared__ unsigned long long hits[kFdmThreads / 64];
-    energy_reduce(tail.d.partial, tail.nblocks, tail.E_local, tail.Ee, sh);
-    if (threadIdx.x == 0 && *tail.b.nqueue > tail.b.limit / kQueueBlocks) *tail.b.crowded = 1;
-    deposit_queued(tail, g, 0, 1, hits);
-    __syncthreads();
-  }
   double* cur = s_fdm;
   double* nxt = s_fdm + G;
   if (threadIdx.x == 0) s_slow = 0;
@@ -99,6 +91,36 @@ __global__ __launch_bounds__(kFdmThreads) void k_fdm_block(GridView g, FdmArgs u
     }
   }
   if (bad) atomicOr(nonfinite, 2);
+}
+
+template <int MODE, int NC>
+__global__ __launch_bounds__(kFdmThreads) void k_fdm_block(GridView g, FdmArgs u, double* __restrict__ T,
+                                                           int nsub, int G, int* nonfinite,
+                                                           DepositTail tail) {
+  extern __shared__ double s_fdm[];
+  if (tail.E_local) {  // the deposit's remainder, which completes dT_e
+    __shared__ double sh[kFdmThreads];
+    __shared__ unsigned long long hits[kFdmThreads / 64];
+    energy_reduce(tail.d.partial, tail.nblocks, tail.E_local, tail.Ee, sh);
+    if (threadIdx.x == 0 && *tail.b.nqueue > tail.b.limit / kQueueBlocks) *tail.b.crowded = 1;
+    deposit_queued(tail, g, 0, 1, hits);
+    __syncthreads();
+  }
+  fdm_block<MODE, NC>(g, u, T, nsub, G, nonfinite, s_fdm);
+}
+
+// A workgroup per replica of a batch, in place of a launch per sub-step (5 us
+// each) and two or three (4 us each) for the copy, the clearing of dT_e and
+// the scan for non-finite values.
+template <int MODE, int NC>
+__global__ __launch_bounds__(kFdmThreads) void k_fdm_block_batch(const GridView* __restrict__ grids,
+                                                                 const FdmArgs* __restrict__ args,
+                                                                 const int* __restrict__ nsub,
+                                                                 int* nonfinite) {
+  extern __shared__ double s_fdm[];
+  const GridView g = grids[blockIdx.x];
+  const FdmArgs u = args[blockIdx.x];
+  fdm_block<MODE, NC>(g, u, g.T, nsub[blockIdx.x], g.nx * g.ny * g.nz, nonfinite, s_fdm);
 }
 
 // ---- K sub-steps per launch on tiles, one material in every cell
@@ -275,10 +297,7 @@ static hipError_t solve_any(const GridView& g, const FdmArgs& u, double*& T, dou
   return hipGetLastError();
 }
 
-hipError_t launch_fdm_solve(const GridView& g, double*& T, double*& Tn, double inner_dt, int nsub,
-                            const FdmMaterial* uniform, bool any_tdyn, int* nonfinite, hipStream_t s,
-                            const DepositTail* tail) {
-  const DepositTail rest = tail ? *tail : DepositTail();
+static FdmArgs fdm_args(const GridView& g, double inner_dt, const FdmMaterial* uniform) {
   FdmArgs u;
   u.inner_dt = inner_dt;
   u.d3[0] = divisor(g.dx); u.d3[1] = divisor(g.dy); u.d3[2] = divisor(g.dz);
@@ -289,8 +308,50 @@ hipError_t launch_fdm_solve(const GridView& g, double*& T, double*& Tn, double i
     u.uni.div = divisor(uniform->rho * uniform->C);
     u.uni.flag = kCellDynamic;
     u.uni.flat = true;
-    return solve_any<0>(g, u, T, Tn, nsub, nonfinite, rest, s);
   }
+  return u;
+}
+
+size_t fdm_batch_args_size() { return sizeof(FdmArgs); }
+
+void fdm_batch_args(void* entry, const GridView& g, double inner_dt, const FdmMaterial* uniform) {
+  const FdmArgs u = fdm_args(g, inner_dt, uniform);
+  std::memcpy(entry, &u, sizeof u);
+}
+
+bool fdm_batch_fits(int max_cells, bool uniform) {
+  return max_cells <= (uniform ? kFdmBlockUniform : kFdmBlockCells);
+}
+
+template <int MODE, int NC>
+static hipError_t block_batch(const GridView* grids, const void* args, const int* nsub, int nrep, int max_cells,
+                              int* nonfinite, hipStream_t s) {
+  const size_t lds = static_cast<size_t>(max_cells) * (MODE != 0 ? 24 : 16);
+  auto k = k_fdm_block_batch<MODE, NC>;
+  if (hipError_t e = allow_lds(k, lds); e != hipSuccess) return e;
+  k<<<nrep, kFdmThreads, lds, s>>>(grids, static_cast<const FdmArgs*>(args), nsub, nonfinite);
+  return hipGetLastError();
+}
+
+hipError_t launch_fdm_batch(const GridView* grids, const void* args, const int* nsub, int nrep, int max_cells,
+                            bool uniform, int* nonfinite, hipStream_t s) {
+  if (nrep == 0) return hipSuccess;
+  if (!fdm_batch_fits(max_cells, uniform)) return hipErrorInvalidValue;
+  const int nc = (max_cells + kFdmThreads - 1) / kFdmThreads;
+  if (uniform)
+    return nc <= 1 ? block_batch<0, 1>(grids, args, nsub, nrep, max_cells, nonfinite, s)
+           : nc == 2 ? block_batch<0, 2>(grids, args, nsub, nrep, max_cells, nonfinite, s)
+                     : block_batch<0, 4>(grids, args, nsub, nrep, max_cells, nonfinite, s);
+  return nc <= 1 ? block_batch<1, 1>(grids, args, nsub, nrep, max_cells, nonfinite, s)
+                 : block_batch<1, 2>(grids, args, nsub, nrep, max_cells, nonfinite, s);
+}
+
+hipError_t launch_fdm_solve(const GridView& g, double*& T, double*& Tn, double inner_dt, int nsub,
+                            const FdmMaterial* uniform, bool any_tdyn, int* nonfinite, hipStream_t s,
+                            const DepositTail* tail) {
+  const DepositTail rest = tail ? *tail : DepositTail();
+  const FdmArgs u = fdm_args(g, inner_dt, uniform);
+  if (uniform) return solve_any<0>(g, u, T, Tn, nsub, nonfinite, rest, s);
   return any_tdyn ? solve_any<2>(g, u, T, Tn, nsub, nonfinite, rest, s)
                   : solve_any<1>(g, u, T, Tn, nsub, nonfinite, rest, s);
 }

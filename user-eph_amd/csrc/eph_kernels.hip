@@ -1843,14 +1843,14 @@ __device__ __forceinline__ void deposit_bucket_atom(const int i, const double4& 
 // kick (k_integrate<false>'s expressions), so that one pass serves
 // final_integrate and the deposit of end_of_step when nothing runs between
 template <bool FRIC, bool RAND, bool KICK>
-__global__ __launch_bounds__(kBlock) void k_deposit_bucket(AtomsView a, GridView g, StepParams p,
-                                                           WorkView w, DepositView d,
-                                                           BucketView b) {
+__device__ __forceinline__ void deposit_bucket_block(const int i, const bool in, const AtomsView& a,
+                                                     const GridView& g, const StepParams& p,
+                                                     const WorkView& w, const DepositView& d,
+                                                     const BucketView& b) {
   __shared__ double sh[kBlock];
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i == 0) *b.nqueue = 0;  // the queue of this step starts empty
+  if (blockIdx.x == 0 && threadIdx.x == 0) *b.nqueue = 0;  // the queue of this step starts empty
   double eF = 0.0, eR = 0.0;
-  if (i < a.nlocal && (a.mask[i] & a.groupbit)) {
+  if (in && (a.mask[i] & a.groupbit)) {
     double4 v = a.vel[i];
     if (KICK) {
       const int fs = a.fstride;
@@ -1868,6 +1868,29 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket(AtomsView a, GridView
     d.partial[2 * blockIdx.x] = sF;
     d.partial[2 * blockIdx.x + 1] = sR;
   }
+}
+
+template <bool FRIC, bool RAND, bool KICK>
+__global__ __launch_bounds__(kBlock) void k_deposit_bucket(AtomsView a, GridView g, StepParams p,
+                                                           WorkView w, DepositView d,
+                                                           BucketView b) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  deposit_bucket_block<FRIC, RAND, KICK>(i, i < a.nlocal, a, g, p, w, d, b);
+}
+
+// the same for a batch of replicas: the chunk's atoms into its replica's cells
+template <bool FRIC, bool RAND, bool KICK>
+__global__ __launch_bounds__(kBlock) void k_deposit_bucket_batch(AtomsView a,
+                                                                 const GridView* __restrict__ grids,
+                                                                 const int* __restrict__ cell_off,
+                                                                 StepParams p, WorkView w, DepositView d,
+                                                                 BucketView b,
+                                                                 const Chunk* __restrict__ chunks) {
+  const Chunk c = chunks[blockIdx.x];
+  b.count += cell_off[c.rep];
+  b.items += static_cast<size_t>(cell_off[c.rep]) * b.cap;
+  deposit_bucket_block<FRIC, RAND, KICK>(c.start + threadIdx.x, static_cast<int>(threadIdx.x) < c.count, a,
+                                         grids[c.rep], p, w, d, b);
 }
 
 // compare-exchange of a fixed-size register array (indices known after
@@ -2302,6 +2325,30 @@ __global__ __launch_bounds__(kBlock) void k_deposit_atoms_batch(AtomsView a,
   if (threadIdx.x == 0) {
     d.partial[2 * blockIdx.x] = sF;
     d.partial[2 * blockIdx.x + 1] = sR;
+  }
+}
+
+// k_deposit_finish for a batch: blocks 0..nrep - 1 the replicas' tallies, the
+// others the queued cells, each by a scan of its own replica's atoms
+__global__ __launch_bounds__(1024) void k_deposit_finish_batch(DepositTail t, const GridView* __restrict__ grids,
+                                                               const int* __restrict__ cell_off,
+                                                               const int* __restrict__ cell_rep,
+                                                               const Chunk* __restrict__ chunks,
+                                                               const int* __restrict__ chunk0,
+                                                               const int* __restrict__ nchunks, int nrep) {
+  __shared__ double sh[1024];
+  __shared__ unsigned long long hits[16];
+  const int nq = *t.b.nqueue;
+  if (static_cast<int>(blockIdx.x) < nrep) {
+    const int r = blockIdx.x;
+    energy_reduce(t.d.partial + 2 * chunk0[r], nchunks[r], t.E_local + r, t.Ee + r, sh);
+    if (r == 0 && threadIdx.x == 0 && nq > t.b.limit) *t.b.crowded = 1;
+    return;
+  }
+  for (int q = blockIdx.x - nrep; q < nq; q += gridDim.x - nrep) {
+    const int c = t.b.queue[q], r = cell_rep[c];
+    const Chunk first = chunks[chunk0[r]], last = chunks[chunk0[r] + nchunks[r] - 1];
+    queued_cell(t.a, t.d, grids[r], c - cell_off[r], first.start, last.start + last.count, hits);
   }
 }
 
@@ -2838,6 +2885,12 @@ hipError_t launch_deposit_cells(const GridView& g, const DepositView& d, int n_i
   return hipGetLastError();
 }
 
+// the cells' sums of the bucketed deposit (g: the grid, or a batch's as one)
+static void bucket_cells(const GridView& g, const DepositView& d, const BucketView& b, int G, hipStream_t s) {
+  if (b.cap == kBucket) k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, d, b, G);
+  else k_deposit_bucket_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, d, b, G);
+}
+
 hipError_t launch_deposit_bucket(const AtomsView& a, const GridView& g, const StepParams& p,
                                  const WorkView& w, const DepositView& d, const BucketView& b,
                                  bool fric, bool rand, bool kick, double* E_local, double* Ee,
@@ -2857,8 +2910,7 @@ hipError_t launch_deposit_bucket(const AtomsView& a, const GridView& g, const St
   DepositView dc = d;
   if (!fric) dc.v1 = nullptr;
   if (!rand) dc.v2 = nullptr;
-  if (b.cap == kBucket) k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, dc, b, G);
-  else k_deposit_bucket_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, dc, b, G);
+  bucket_cells(g, dc, b, G, s);
   DepositTail t;
   t.a = a; t.d = dc; t.b = b; t.nblocks = a.nlocal > 0 ? nb : 0; t.E_local = E_local; t.Ee = Ee;
   if (tail) {
@@ -3109,6 +3161,31 @@ hipError_t launch_deposit_atoms_batch(const AtomsView& a, const GridView* grids,
   else if (fric) k_deposit_atoms_batch<true, false><<<nchunks, kBlock, 0, s>>>(a, grids, cell_off, p, w, d, chunks);
   else if (rnd) k_deposit_atoms_batch<false, true><<<nchunks, kBlock, 0, s>>>(a, grids, cell_off, p, w, d, chunks);
   else k_deposit_atoms_batch<false, false><<<nchunks, kBlock, 0, s>>>(a, grids, cell_off, p, w, d, chunks);
+  return hipGetLastError();
+}
+
+hipError_t launch_deposit_bucket_batch(const AtomsView& a, const GridView* grids, const int* cell_off,
+                                       const int* cell_rep, const GridView& all, const StepParams& p,
+                                       const WorkView& w, const DepositView& d, const BucketView& b,
+                                       const Chunk* chunks, int nchunk, const int* chunk0,
+                                       const int* nchunks, int nrep, bool kick, double* E_local,
+                                       double* Ee, hipStream_t s) {
+  const bool fric = p.flags & 0x01, rnd = p.flags & 0x02;
+  if (nchunk == 0 || nrep == 0) return hipSuccess;
+#define EPH_DBB(F, R)                                                                               \
+  if (kick) k_deposit_bucket_batch<F, R, true><<<nchunk, kBlock, 0, s>>>(a, grids, cell_off, p, w, d, b, chunks); \
+  else k_deposit_bucket_batch<F, R, false><<<nchunk, kBlock, 0, s>>>(a, grids, cell_off, p, w, d, b, chunks)
+  if (fric && rnd) { EPH_DBB(true, true); }
+  else if (fric) { EPH_DBB(true, false); }
+  else { EPH_DBB(false, true); }
+#undef EPH_DBB
+  DepositTail t;
+  t.a = a; t.d = d; t.b = b; t.E_local = E_local; t.Ee = Ee;
+  if (!fric) t.d.v1 = nullptr;
+  if (!rnd) t.d.v2 = nullptr;
+  bucket_cells(all, t.d, b, all.nx, s);
+  k_deposit_finish_batch<<<nrep + kQueueBlocks, 1024, 0, s>>>(t, grids, cell_off, cell_rep, chunks, chunk0,
+                                                              nchunks, nrep);
   return hipGetLastError();
 }
 
