@@ -210,6 +210,7 @@ struct StepExtras {
   const double4* xref = nullptr;  // positions of the last list build
   double lim = 0.0;
   int* want = nullptr;            // pinned host memory: 1 when an atom moved farther than lim
+  uint64_t* step = nullptr;       // advanced by one (a batch's step number)
   unsigned long long* t = nullptr;
 };
 
@@ -384,13 +385,16 @@ hipError_t launch_fdm_substeps_batch(const GridView* grids, const int8_t* rep_td
                                      const int* grid_steps, int* sub_n, double* inner_dt, int* max_sub,
                                      int R, hipStream_t s);
 hipError_t launch_copy_double(const double* src, double* dst, int n, hipStream_t s);
-hipError_t launch_ghost_xv_dev(const AtomsView& a, const int* owner, const double4* shift,
-                               const int* ng, int cap, hipStream_t s);
+// the ghost update of a batch (ng ghosts of at most a.nghost) and, with check,
+// the density sweep's candidate check of all atoms, as launch_ghost_check
+hipError_t launch_ghost_check_dev(const AtomsView& a, const WorkView& w, const int* rep, const int* ng,
+                                  bool check, hipStream_t s);
+// whether launch_density_w_batch walks candidates in this form
+bool density_batch_walks_candidates(const TablesView& t, const WorkView& w, int variant);
 hipError_t launch_pack_pv_dev(const AtomsView& a, const WorkView& w, const int* ng, int cap,
                               hipStream_t s);
 hipError_t launch_ghost_rec_dev(const AtomsView& a, const WorkView& w, const int* ng, int cap,
                                 hipStream_t s);
-hipError_t launch_step_advance(uint64_t* step, hipStream_t s);
 hipError_t launch_step_log(const int* flag, const uint64_t* step, const uint64_t* first, int* log,
                            int nlog, hipStream_t s);
 

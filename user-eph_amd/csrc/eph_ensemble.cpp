@@ -65,7 +65,7 @@ struct eph_ensemble {
   DevArray<int8_t> rep_tdyn;
   DevArray<double> grid_dt;
   DevArray<int> grid_steps, max_sub_dev;
-  int* max_sub_host = nullptr;  // pinned
+  int* pinned = nullptr;  // [0] largest sub-step count, [1] lists to be rebuilt
   DepositBuffers dep;
   // bucketed deposit: slots per cell (0: counted), the buckets, and the pinned
   // flag that the device sets when too many cells overflowed theirs
@@ -81,7 +81,6 @@ struct eph_ensemble {
   // recorded step
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  int graph_nlog = -1;
   bool graph_bucketed = false;
   int var_density = 0, var_force = 0;  // kernel forms chosen by autotune()
 
@@ -97,15 +96,16 @@ struct eph_ensemble {
       eph_destroy(r.fix);
       eph_md_destroy(r.md);
     }
-    if (max_sub_host) (void)hipHostFree(max_sub_host);
+    if (pinned) (void)hipHostFree(pinned);
     if (crowded) (void)hipHostFree(crowded);
     eph_destroy(sys);
   }
   int setup(long long first);
-  int enqueue_step(int nlog);
+  int step_front(int nlog);
+  int enqueue_step();
   int enqueue_fdm(int nsub);
   int fdm_after_counts();
-  int record(int nlog);
+  int record();
   int autotune(double* ms);
 };
 
@@ -213,7 +213,7 @@ int eph_ensemble::setup(long long first) {
   EPH_HIP(this, scan_tmp.reserve((cap + nbins) / 4096 + 4));
   NbBuild& w = nbw;
   w.nlocal = nl; w.ghost_cap = ghost_cap; w.nbins = nbins;
-  w.at.pos = sys->pos.p; w.at.vel = sys->vel.p; w.at.type = sys->type.p; w.at.mask = sys->mask.p;
+  w.at.pos = sys->pos.p; w.at.vel = sys->vel.p; w.at.pv = sys->atoms_view().pv; w.at.type = sys->type.p; w.at.mask = sys->mask.p;
   w.at.tag = sys->tag.p; w.at.rep = rep.p; w.at.owner = sys->ghost_owner.p; w.at.shift = sys->ghost_shift.p;
   w.box.lo = box_d.p; w.box.hi = box_d.p + 3 * R; w.box.L = box_d.p + 6 * R; w.box.glo = box_d.p + 9 * R;
   w.box.nb = nbi.p; w.box.bin_base = nbi.p + 3 * R; w.box.bs = bs; w.box.cg = cmax;
@@ -298,8 +298,8 @@ int eph_ensemble::setup(long long first) {
   EPH_HIP(this, nonfinite.reserve(1));
   EPH_HIP(this, rep_tdyn.reserve(R)); EPH_HIP(this, grid_dt.reserve(R));
   EPH_HIP(this, grid_steps.reserve(R)); EPH_HIP(this, max_sub_dev.reserve(1));
-  if (!max_sub_host) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&max_sub_host), sizeof(int)));
-  *max_sub_host = max_sub;
+  if (!pinned) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&pinned), 2 * sizeof(int)));
+  *pinned = max_sub;
   EPH_HIP(this, hipMemcpyAsync(rep_tdyn.p, rtd.data(), R * sizeof(int8_t), hipMemcpyHostToDevice, s));
   EPH_HIP(this, hipMemcpyAsync(grid_dt.p, gdt.data(), R * sizeof(double), hipMemcpyHostToDevice, s));
   EPH_HIP(this, hipMemcpyAsync(grid_steps.p, gsteps.data(), R * sizeof(int), hipMemcpyHostToDevice, s));
@@ -351,28 +351,45 @@ int eph_ensemble::setup(long long first) {
   return EPH_OK;
 }
 
-// one Verlet step of every replica (the step order of eph_md_run)
-int eph_ensemble::enqueue_step(int nlog) {
+// One Verlet step of every replica (the step order of eph_md_run): the kick
+// and the check of the lists, whose answer the host waits for; the rebuild
+// where it is due; then the rest, which can be a recorded graph.  (A rebuild
+// gated on the device costs 26 launches that find nothing to do, 70 us a step.)
+int eph_ensemble::step_front(int nlog) {
+  hipStream_t s = sys->stream;
+  volatile int* want = pinned + 1;
+  *want = 0;
+  StepExtras x;
+  x.xref = xref.p;
+  x.lim = 0.25 * cfg0.skin * cfg0.skin;
+  x.want = pinned + 1;
+  x.step = step_dev.p;
+  if (int rc = sys->dev_initial_integrate(&x)) return fail(rc, sys->err);
+  EPH_HIP(this, hipStreamSynchronize(s));
+  if (!*want) return EPH_OK;
+  EPH_HIP(this, launch_nb_force(nbw.go, s));
+  EPH_HIP(this, launch_nb_build(nbw, s));
+  if (nlog > 0) EPH_HIP(this, launch_step_log(nbw.go, step_dev.p, step_dev.p + 1, rlog.p, nlog, s));
+  return EPH_OK;
+}
+
+int eph_ensemble::enqueue_step() {
   hipStream_t s = sys->stream;
   const int st = sys->stride;
   const int* ng = flags.p + 7;
   int rc;
-  EPH_HIP(this, launch_step_advance(step_dev.p, s));
-  if ((rc = sys->dev_initial_integrate())) return fail(rc, sys->err);
-  const double lim = 0.25 * cfg0.skin * cfg0.skin;
-  EPH_HIP(this, launch_nb_check(nl, sys->pos.p, xref.p, lim, nbw.go, s));
-  EPH_HIP(this, launch_nb_build(nbw, s));
-  if (nlog > 0) EPH_HIP(this, launch_step_log(nbw.go, step_dev.p, step_dev.p + 1, rlog.p, nlog, s));
   AtomsView a = sys->atoms_view();
   a.nghost = ghost_cap;  // the ghost kernels below read the count on the device
-  const WorkView w = sys->work_view();
-  EPH_HIP(this, launch_ghost_xv_dev(a, sys->ghost_owner.p, sys->ghost_shift.p, ng, ghost_cap, s));
+  WorkView w = sys->work_view();
+  w.cand_checked = density_batch_walks_candidates(sys->tabs, w, var_density);
+  w.defer_flags = w.cand_checked && ghost_cap > 0;
+  EPH_HIP(this, launch_ghost_check_dev(a, w, rep.p, ng, w.cand_checked, s));
   EPH_HIP(this, launch_lj(a, lj_nbr.p, lj_nn.p, st, cfg0.lj_eps, cfg0.lj_sigma,
                           cfg0.cut_lj * cfg0.cut_lj, s));
   // post_force (fix_eph.cpp:841-907)
   StepParams p = sys->step_params();
   p.xi_mode = (sys->flags & EPH_RANDOM) ? 2 : 0;
-  EPH_HIP(this, launch_pack_pv_dev(a, w, ng, ghost_cap, s));
+  if (!a.pv) EPH_HIP(this, launch_pack_pv_dev(a, w, ng, ghost_cap, s));
   EPH_HIP(this, launch_density_w_batch(a, sys->tabs, p, w, chunks.p, nchunk, seeds.p, step_dev.p, s,
                                        var_density, ng, rep.p));
   EPH_HIP(this, launch_ghost_rec_dev(a, w, ng, ghost_cap, s));
@@ -413,7 +430,7 @@ int eph_ensemble::enqueue_step(int nlog) {
     EPH_HIP(this, launch_fill_int(max_sub_dev.p, 1, 0, s));
     EPH_HIP(this, launch_fdm_substeps_batch(gviews.p, rep_tdyn.p, grid_dt.p, grid_steps.p, sub_n.p,
                                             inner_dt.p, max_sub_dev.p, R, s));
-    EPH_HIP(this, hipMemcpyAsync(max_sub_host, max_sub_dev.p, sizeof(int), hipMemcpyDeviceToHost, s));
+    EPH_HIP(this, hipMemcpyAsync(pinned, max_sub_dev.p, sizeof(int), hipMemcpyDeviceToHost, s));
   }
   return EPH_OK;
 }
@@ -445,7 +462,7 @@ int eph_ensemble::enqueue_fdm(int nsub) {
 int eph_ensemble::fdm_after_counts() {
   if (!any_tdyn || !(sys->flags & EPH_FDM)) return EPH_OK;
   EPH_HIP(this, hipStreamSynchronize(sys->stream));
-  const int n = *max_sub_host;
+  const int n = *pinned;
   if (n < 1 || n > (1 << 22))
     return fail(EPH_ERR_NONFINITE, "T_e sub-step count out of range (" + std::to_string(n) +
                                        "): C_e, rho_e or kappa of a grid is not usable");
@@ -515,18 +532,17 @@ int eph_ensemble::autotune(double* ms) {
   // a recorded step holds the old forms
   if (exec) { (void)hipGraphExecDestroy(exec); exec = nullptr; }
   if (graph) { (void)hipGraphDestroy(graph); graph = nullptr; }
-  graph_nlog = -1;
   return EPH_OK;
 }
 
-int eph_ensemble::record(int nlog) {
-  if (exec && graph_nlog == nlog && graph_bucketed == bucketed()) return EPH_OK;
+int eph_ensemble::record() {
+  if (exec && graph_bucketed == bucketed()) return EPH_OK;
   if (exec) { (void)hipGraphExecDestroy(exec); exec = nullptr; }
   if (graph) { (void)hipGraphDestroy(graph); graph = nullptr; }
   hipStream_t s = sys->stream;
   EPH_HIP(this, hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   const bool was = bucketed();
-  int rc = enqueue_step(nlog);
+  int rc = enqueue_step();
   hipGraph_t g = nullptr;
   const hipError_t e = hipStreamEndCapture(s, &g);
   if (rc != EPH_OK) {
@@ -536,7 +552,6 @@ int eph_ensemble::record(int nlog) {
   if (e != hipSuccess) return fail_hip(e, "hipStreamEndCapture");
   graph = g;
   EPH_HIP(this, hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-  graph_nlog = nlog;
   graph_bucketed = was;
   return EPH_OK;
 }
@@ -645,15 +660,24 @@ int eph_ensemble_run(eph_ensemble* e, int nsteps, int use_graph, double* ms, int
   e->log_first = static_cast<uint64_t>(e->step0);
   EPH_HIP(e, hipMemcpyAsync(e->step_dev.p + 1, &e->log_first, sizeof(uint64_t), hipMemcpyHostToDevice, s));
   int rc;
-  if (use_graph && (rc = e->record(nlog))) return rc;
+  if (use_graph && (rc = e->record())) return rc;
+  // the records of position and velocity, which the steps then keep current
+  // (but not those of a filtered velocity)
+  {
+    AtomsView av = e->sys->atoms_view();
+    av.nghost = e->ghost_cap;
+    if (av.pv)
+      EPH_HIP(e, launch_pack_pv_dev(av, e->sys->work_view(), e->flags.p + 7, e->ghost_cap, s));
+  }
   hipEvent_t a, b;
   EPH_HIP(e, hipEventCreate(&a));
   EPH_HIP(e, hipEventCreate(&b));
   EPH_HIP(e, hipEventRecord(a, s));
   for (int k = 0; k < nsteps; ++k) {
+    if ((rc = e->step_front(nlog))) return rc;
     if (use_graph) {
       EPH_HIP(e, hipGraphLaunch(e->exec, s));
-    } else if ((rc = e->enqueue_step(nlog))) {
+    } else if ((rc = e->enqueue_step())) {
       return rc;
     }
     if ((rc = e->fdm_after_counts())) return rc;
@@ -694,7 +718,6 @@ int eph_ensemble_set_variants(eph_ensemble* e, int density, int force) {
   e->var_force = force;
   if (e->exec) { (void)hipGraphExecDestroy(e->exec); e->exec = nullptr; }
   if (e->graph) { (void)hipGraphDestroy(e->graph); e->graph = nullptr; }
-  e->graph_nlog = -1;
   return EPH_OK;
 }
 

@@ -612,20 +612,44 @@ __device__ __forceinline__ void density_w_atom_split(const int i_atom, const boo
 // retakes the candidates, the reference positions are the current ones;
 // otherwise every atom 0.45 delta or farther from its reference position (a
 // non-finite distance counts) puts its current position on the moved list.
-__global__ __launch_bounds__(kBlock) void k_cand_check(int nall, const double4* __restrict__ pos,
-                                                       WorkView w) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
+// the ghost update of local or ghost atom i, and its position
+__device__ __forceinline__ double4 ghost_atom(const int i, const AtomsView& a, const WorkView& w) {
+  if (i < a.nlocal) return a.pos[i];
+  const int g = i - a.nlocal, o = w.ghost_owner[g];
+  const double4 p = a.pos[o];
+  const double4 s = w.ghost_shift[g];
+  const double4 x = make_double4(p.x + s.x, p.y + s.y, p.z + s.z, p.w);
+  const double4 v = a.vel[o];
+  a.pos[i] = x;
+  a.vel[i] = v;
+  if (a.pv) {
+    PosVel q;
+    q.p = x;
+    q.v = v;
+    a.pv[i] = q;
+  }
+  return x;
+}
+
+// the candidate check of atom i at x; tag: what .w of its entry holds
+__device__ __forceinline__ void cand_check_atom(const int i, const double4& x, const double tag,
+                                                const WorkView& w) {
   if (w.cstate[0] == 0) {
-    if (i < nall) w.cref[i] = pos[i];
+    w.cref[i] = x;
     return;
   }
-  if (i >= nall) return;
-  const double4 x = pos[i], r = w.cref[i];
+  const double4 r = w.cref[i];
   const double dx = x.x - r.x, dy = x.y - r.y, dz = x.z - r.z;
   if (!(dx * dx + dy * dy + dz * dz < w.half_delta2)) {
     const int k = atomicAdd(w.cstate + 2, 1);
-    if (k < w.moved_cap) w.moved[k] = x;
+    if (k < w.moved_cap) w.moved[k] = make_double4(x.x, x.y, x.z, tag);
   }
+}
+
+__global__ __launch_bounds__(kBlock) void k_cand_check(int nall, const double4* __restrict__ pos,
+                                                       WorkView w) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < nall) cand_check_atom(i, pos[i], pos[i].w, w);
 }
 
 // The ghost update (k_ghost_xv) and, with check, the candidate check of all
@@ -635,35 +659,20 @@ __global__ __launch_bounds__(kBlock) void k_ghost_check(AtomsView a, WorkView w,
   const int i = (check ? 0 : a.nlocal) + blockIdx.x * kBlock + threadIdx.x;
   if (t && blockIdx.x == 0 && threadIdx.x == 0) *t = wall_clock64();
   if (i >= a.nlocal + a.nghost) return;
-  double4 x;
-  if (i >= a.nlocal) {
-    const int g = i - a.nlocal, o = w.ghost_owner[g];
-    const double4 p = a.pos[o];
-    const double4 s = w.ghost_shift[g];
-    x = make_double4(p.x + s.x, p.y + s.y, p.z + s.z, p.w);
-    const double4 v = a.vel[o];
-    a.pos[i] = x;
-    a.vel[i] = v;
-    if (a.pv) {
-      PosVel q;
-      q.p = x;
-      q.v = v;
-      a.pv[i] = q;
-    }
-  } else {
-    x = a.pos[i];
-  }
-  if (!check) return;
-  if (w.cstate[0] == 0) {
-    w.cref[i] = x;
-    return;
-  }
-  const double4 r = w.cref[i];
-  const double dx = x.x - r.x, dy = x.y - r.y, dz = x.z - r.z;
-  if (!(dx * dx + dy * dy + dz * dz < w.half_delta2)) {
-    const int k = atomicAdd(w.cstate + 2, 1);
-    if (k < w.moved_cap) w.moved[k] = x;
-  }
+  const double4 x = ghost_atom(i, a, w);
+  if (check) cand_check_atom(i, x, x.w, w);
+}
+
+// the same for a batch of replicas, with the ghost count read on the device
+// (it changes between replays of a recorded step; the grid covers nlocal + the
+// ghost capacity); a moved atom's entry carries its replica rep[i]
+__global__ __launch_bounds__(kBlock) void k_ghost_check_dev(AtomsView a, WorkView w,
+                                                            const int* __restrict__ rep,
+                                                            const int* __restrict__ ng, int check) {
+  const int i = (check ? 0 : a.nlocal) + blockIdx.x * kBlock + threadIdx.x;
+  if (i >= a.nlocal + *ng) return;
+  const double4 x = ghost_atom(i, a, w);
+  if (check) cand_check_atom(i, x, static_cast<double>(rep[i]), w);
 }
 
 // the same check for a batch of replicas, with the ghost count read on the
@@ -674,18 +683,7 @@ __global__ __launch_bounds__(kBlock) void k_cand_check_dev(int nlocal, const int
                                                            const double4* __restrict__ pos,
                                                            const int* __restrict__ rep, WorkView w) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  const int nall = nlocal + *ng;
-  if (w.cstate[0] == 0) {
-    if (i < nall) w.cref[i] = pos[i];
-    return;
-  }
-  if (i >= nall) return;
-  const double4 x = pos[i], r = w.cref[i];
-  const double dx = x.x - r.x, dy = x.y - r.y, dz = x.z - r.z;
-  if (!(dx * dx + dy * dy + dz * dz < w.half_delta2)) {
-    const int k = atomicAdd(w.cstate + 2, 1);
-    if (k < w.moved_cap) w.moved[k] = make_double4(x.x, x.y, x.z, static_cast<double>(rep[i]));
-  }
+  if (i < nlocal + *ng) cand_check_atom(i, pos[i], static_cast<double>(rep[i]), w);
 }
 
 // After the sweep: a sweep that retook the candidates leaves them valid.  A
@@ -1438,7 +1436,10 @@ __global__ void k_stamp(unsigned long long* t) {
 __global__ __launch_bounds__(kBlock) void k_integrate_check(AtomsView a, StepParams p, StepExtras e,
                                                             int move) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (e.t && i == 0) e.t[0] = wall_clock64();
+  if (i == 0) {
+    if (e.t) e.t[0] = wall_clock64();
+    if (e.step) *e.step += 1;
+  }
   if (i < a.nlocal) {
     const bool moves = move && (a.mask[i] & a.groupbit);
     const double4 x = moves ? integrate_atom<true>(i, a, p) : a.pos[i];
@@ -2223,10 +2224,6 @@ __global__ __launch_bounds__(kBlock) void k_prl_forces_batch_split(AtomsView a, 
 }
 
 // start of a recorded step: step += 1
-__global__ void k_step_advance(uint64_t* step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
-}
-
 // log[step - first] = *flag (which steps rebuilt)
 __global__ void k_step_log(const int* __restrict__ flag, const uint64_t* __restrict__ step,
                            const uint64_t* __restrict__ first, int* log, int nlog) {
@@ -2462,22 +2459,11 @@ __global__ __launch_bounds__(kBlock) void k_copy_double(const double* __restrict
 }
 
 // ghost updates with the ghost count read on the device (graph-capturable)
-__global__ __launch_bounds__(kBlock) void k_ghost_xv_dev(AtomsView a, const int* __restrict__ owner,
-                                                         const double4* __restrict__ shift,
-                                                         const int* __restrict__ ng) {
-  const int g = blockIdx.x * kBlock + threadIdx.x;
-  if (g >= *ng) return;
-  const int o = owner[g];
-  const double4 p = a.pos[o];
-  const double4 s = shift[g];
-  a.pos[a.nlocal + g] = make_double4(p.x + s.x, p.y + s.y, p.z + s.z, p.w);
-  a.vel[a.nlocal + g] = a.vel[o];
-}
-
 __global__ __launch_bounds__(kBlock) void k_ghost_rec_dev(AtomsView a, WorkView w,
                                                           const int* __restrict__ ng) {
   const int g = blockIdx.x * kBlock + threadIdx.x;
   if (g < *ng) ghost_rec(g, a, w);
+  if (g == 0 && w.defer_flags) cand_flags(w.cstate, w.moved_cap);
 }
 
 __global__ __launch_bounds__(kBlock) void k_pack_pv_dev(AtomsView a, WorkView w,
@@ -3048,6 +3034,10 @@ static int batch_lds_block(int form) {
   return form == kLdsForm1024 ? 1024 : form == kLdsForm512 ? 512 : form == kLdsForm256 ? 256 : 0;
 }
 
+bool density_batch_walks_candidates(const TablesView& t, const WorkView& w, int variant) {
+  return !(batch_lds_block(variant) > 0 && batch_lds_possible(t)) && w.rcand2 > 0.0 && w.cstate;
+}
+
 hipError_t launch_density_w_batch(const AtomsView& a, const TablesView& t, const StepParams& p,
                                   const WorkView& w_in, const Chunk* chunks, int nchunks,
                                   const uint32_t* seeds, const uint64_t* step, hipStream_t s,
@@ -3085,7 +3075,7 @@ hipError_t launch_density_w_batch(const AtomsView& a, const TablesView& t, const
   // count and the replica of every atom
   const bool keep = w.rcand2 > 0.0 && w.cstate && ng && rep;
   if (!keep) w.rcand2 = 0.0;
-  if (keep) k_cand_check_dev<<<nblk(a.nlocal + a.nghost), kBlock, 0, s>>>(a.nlocal, ng, a.pos, rep, w);
+  if (keep && !w.cand_checked) k_cand_check_dev<<<nblk(a.nlocal + a.nghost), kBlock, 0, s>>>(a.nlocal, ng, a.pos, rep, w);
   const size_t dl = chunk_lds(variant, kDensityStageBytes);
   const int sp = variant == 0 ? split_density(a.nlocal) : 0;
 #define EPH_DWB_S(S, UR, UW, XI, F, M) \
@@ -3105,7 +3095,7 @@ hipError_t launch_density_w_batch(const AtomsView& a, const TablesView& t, const
 #undef EPH_DWB_M
 #undef EPH_DWB
 #undef EPH_DWB_S
-  if (keep) k_cand_flags<<<1, 64, 0, s>>>(w.cstate, w.moved_cap);
+  if (keep && !w.defer_flags) k_cand_flags<<<1, 64, 0, s>>>(w.cstate, w.moved_cap);
   return hipGetLastError();
 }
 
@@ -3230,10 +3220,10 @@ hipError_t launch_copy_double(const double* src, double* dst, int n, hipStream_t
   return hipGetLastError();
 }
 
-hipError_t launch_ghost_xv_dev(const AtomsView& a, const int* owner, const double4* shift,
-                               const int* ng, int cap, hipStream_t s) {
-  if (cap == 0) return hipSuccess;
-  k_ghost_xv_dev<<<nblk(cap), kBlock, 0, s>>>(a, owner, shift, ng);
+hipError_t launch_ghost_check_dev(const AtomsView& a, const WorkView& w, const int* rep, const int* ng,
+                                  bool check, hipStream_t s) {
+  const int n = (check ? a.nlocal : 0) + a.nghost;
+  if (n > 0) k_ghost_check_dev<<<nblk(n), kBlock, 0, s>>>(a, w, rep, ng, check ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -3249,11 +3239,6 @@ hipError_t launch_ghost_rec_dev(const AtomsView& a, const WorkView& w, const int
                                 hipStream_t s) {
   if (cap == 0) return hipSuccess;
   k_ghost_rec_dev<<<nblk(cap), kBlock, 0, s>>>(a, w, ng);
-  return hipGetLastError();
-}
-
-hipError_t launch_step_advance(uint64_t* step, hipStream_t s) {
-  k_step_advance<<<1, 64, 0, s>>>(step);
   return hipGetLastError();
 }
 

@@ -30,17 +30,6 @@ __device__ __forceinline__ double comp(const double4& p, int d) {
 
 }  // namespace
 
-// max squared displacement since the last build > lim -> go = 1
-__global__ __launch_bounds__(kBlock) void k_nb_check(int nlocal, const double4* __restrict__ pos,
-                                                     const double4* __restrict__ ref, double lim,
-                                                     int* go) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= nlocal) return;
-  const double4 p = pos[i], q = ref[i];
-  const double dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
-  if (dx * dx + dy * dy + dz * dz > lim) atomicOr(go, 1);
-}
-
 // Domain::remap of the locals
 __global__ __launch_bounds__(kBlock) void k_nb_wrap(int nlocal, double4* pos, PosVel* pv,
                                                     const int* rep, NbBoxes b, const int* go) {
@@ -381,13 +370,8 @@ __global__ __launch_bounds__(kBlock) void k_nb_finish(int nlocal, const int* ng,
     cand_valid[0] = cand_written ? 1 : 0;
     cand_valid[2] = 0;  // atoms that a check before this rebuild found moved
   }
-  // the last block clears the flag only after every block has read it: the
-  // flag is cleared by the next step's k_nb_reset instead
+  // (*go stays set: some blocks have yet to read it)
   if (i == 0) atomicAdd(nreb, 1);
-}
-
-__global__ void k_nb_reset(int* go) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *go = 0;
 }
 
 __global__ void k_nb_set(int* p, int v) {
@@ -695,13 +679,6 @@ static hipError_t scan(const int* in, int n, int* out, int* tmp, const int* go, 
   k_nb_scan_reduce<<<nb, kSB, 0, s>>>(in, n, tmp, go);
   k_nb_scan_blocks<<<1, kSB, 0, s>>>(tmp, nb, go);
   k_nb_scan_apply<<<nb, kSB, 0, s>>>(in, n, tmp, out, go);
-  return hipGetLastError();
-}
-
-hipError_t launch_nb_check(int nlocal, const double4* pos, const double4* ref, double lim, int* go,
-                           hipStream_t s) {
-  k_nb_reset<<<1, 64, 0, s>>>(go);
-  if (nlocal > 0) k_nb_check<<<nbk(nlocal), kBlock, 0, s>>>(nlocal, pos, ref, lim, go);
   return hipGetLastError();
 }
 

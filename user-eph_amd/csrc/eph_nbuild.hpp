@@ -84,8 +84,6 @@ struct NbBuild {
   double4* xref = nullptr;  // [nlocal]
 };
 
-hipError_t launch_nb_check(int nlocal, const double4* pos, const double4* ref, double lim, int* go,
-                           hipStream_t s);
 hipError_t launch_nb_force(int* go, hipStream_t s);
 hipError_t launch_nb_build(const NbBuild& w, hipStream_t s);
 
