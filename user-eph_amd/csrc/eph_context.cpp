@@ -127,8 +127,7 @@ int eph_grid::solve(int* substeps_out, const DepositTail* tail) {
     EPH_HIP(this, launch_grid_tdyn_update(v, stream));
     EPH_HIP(this, launch_grid_minmax(v, minmax.p, nullptr, stream));
     double mm[3];
-    EPH_HIP(this, hipMemcpyAsync(mm, minmax.p, sizeof mm, hipMemcpyDeviceToHost, stream));
-    EPH_HIP(this, hipStreamSynchronize(stream));
+    if (int rc = read(minmax.p, mm, sizeof mm)) return rc;
     cmin = mm[0]; rmin = mm[1]; kmax = mm[2];
   } else if (!minmax_valid) {
     refresh_minmax();
@@ -151,29 +150,46 @@ int eph_grid::insert_points(int n, const double* x, const double* y, const doubl
                             const double* E) {
   if (n <= 0) return EPH_OK;
   const size_t G = h.ntotal();
-  EPH_HIP(this, pts.reserve(4 * (size_t)n));
   EPH_HIP(this, dep.reserve(n, G, nblocks_of(n)));
   const size_t b = n * sizeof(double);
-  EPH_HIP(this, hipMemcpyAsync(pts.p, x, b, hipMemcpyHostToDevice, stream));
-  EPH_HIP(this, hipMemcpyAsync(pts.p + n, y, b, hipMemcpyHostToDevice, stream));
-  EPH_HIP(this, hipMemcpyAsync(pts.p + 2 * n, z, b, hipMemcpyHostToDevice, stream));
-  EPH_HIP(this, hipMemcpyAsync(pts.p + 3 * n, E, b, hipMemcpyHostToDevice, stream));
+  const double* src[4] = {x, y, z, E};
+  double* a = arena.take(4 * b);
+  if (!a) EPH_HIP(this, pts.reserve(4 * (size_t)n));
+  for (int k = 0; k < 4; ++k) {
+    if (a) std::memcpy(a + (size_t)k * n, src[k], b);
+    else EPH_HIP(this, hipMemcpyAsync(pts.p + (size_t)k * n, src[k], b, hipMemcpyHostToDevice, stream));
+  }
+  const double* q = a ? a : pts.p;
   DepositView d = dep.view(false);
   EPH_HIP(this, launch_fill_int(d.count, (int)G + 1, 0, stream));
-  EPH_HIP(this, launch_deposit_points(n, pts.p, pts.p + n, pts.p + 2 * n, pts.p + 3 * n, h.dt, v, d, stream));
+  EPH_HIP(this, launch_deposit_points(n, q, q + n, q + 2 * (size_t)n, q + 3 * (size_t)n, h.dt, v, d, stream));
+  if (a) EPH_HIP(this, arena.mark(stream));
   EPH_HIP(this, launch_deposit_cells(v, d, n, dep.qbuf.p, stream));
-  EPH_HIP(this, hipStreamSynchronize(stream));
+  if (!a) EPH_HIP(this, hipStreamSynchronize(stream));
+  return EPH_OK;
+}
+
+// through pinned memory where the result is small; the runtime's own copy into
+// pageable memory otherwise
+static hipError_t read_device(PinnedArena& arena, const void* src, void* dst, size_t bytes, hipStream_t s) {
+  double* p = arena.take(bytes);
+  hipError_t e = hipMemcpyAsync(p ? p : dst, src, bytes, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e == hipSuccess && p) std::memcpy(dst, p, bytes);
+  return e;
+}
+int eph_grid::read(const void* src, void* dst, size_t bytes) {
+  EPH_HIP(this, read_device(arena, src, dst, bytes, stream));
+  return EPH_OK;
+}
+int eph_context::read(const void* src, void* dst, size_t bytes) {
+  EPH_HIP(this, read_device(arena, src, dst, bytes, stream));
   return EPH_OK;
 }
 
 int eph_grid::download(int which, std::vector<double>& out) {
-  const size_t G = h.ntotal();
-  out.resize(G);
-  const double* src = which == 0 ? T.p : which == 1 ? dT.p : which == 2 ? C.p : which == 3 ? rho.p
-                    : which == 4 ? kappa.p : S.p;
-  EPH_HIP(this, hipMemcpyAsync(out.data(), src, G * sizeof(double), hipMemcpyDeviceToHost, stream));
-  EPH_HIP(this, hipStreamSynchronize(stream));
-  return EPH_OK;
+  out.resize(h.ntotal());
+  return read(values(which), out.data(), out.size() * sizeof(double));
 }
 
 int eph_grid::sync_params_from_device() {
@@ -737,10 +753,17 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
 }
 
 int eph_context::check_flags() {
-  int fl = 0, gf = 0;
-  EPH_HIP(this, hipMemcpyAsync(&fl, flags_dev.p, sizeof(int), hipMemcpyDeviceToHost, stream));
-  if (grid) EPH_HIP(this, hipMemcpyAsync(&gf, grid->nonfinite.p, sizeof(int), hipMemcpyDeviceToHost, stream));
-  EPH_HIP(this, hipStreamSynchronize(stream));
+  int gf = 0;
+  int* st = reinterpret_cast<int*>(arena.take(sizeof(double)));
+  if (!grid || st) {
+    if (grid)
+      EPH_HIP(this, launch_hook_out(nullptr, nullptr, 0, nullptr, nullptr, 0, nullptr, 0, nullptr, 0, nullptr,
+                                    grid->nonfinite.p, st, stream));
+    EPH_HIP(this, hipStreamSynchronize(stream));
+    if (grid) gf = st[1];
+  } else if (int rc = read(grid->nonfinite.p, &gf, sizeof gf)) {
+    return rc;
+  }
   if (gf & 2) return fail(EPH_ERR_NONFINITE, "T_e grid became non-finite (FDM instability)");
   return EPH_OK;
 }
@@ -1100,11 +1123,26 @@ static int upload_force(eph_context* c, const double* f) {
   return EPH_OK;
 }
 
+// With timing on the hooks keep the launches that the report names.
+static double* hook_arena(eph_context* c, size_t doubles) {
+  return c->timing ? nullptr : c->arena.take(doubles * sizeof(double));
+}
+
 int eph_initial_integrate(eph_context* ctx, double* x, double* v, const double* f) {
   if (!ctx || !x || !v || !f) return EPH_ERR_ARGS;
   if (!ctx->have_atoms) return ctx->fail(EPH_ERR_STATE, "no atoms");
   if (ctx->flags & EPH_NOINT) return EPH_OK;
   int rc;
+  const size_t n3 = 3 * (size_t)ctx->nlocal, b = n3 * sizeof(double);
+  if (double* p = hook_arena(ctx, 5 * n3)) {
+    ctx->pv_fresh = false;
+    std::memcpy(p, x, b); std::memcpy(p + n3, v, b); std::memcpy(p + 2 * n3, f, b);
+    EPH_HIP(ctx, launch_hook_kick(ctx->atoms_view(), ctx->step_params(), true, p, p + n3, p + 2 * n3,
+                                  p + 3 * n3, p + 4 * n3, ctx->stream));
+    EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(x, p + 3 * n3, b); std::memcpy(v, p + 4 * n3, b);
+    return EPH_OK;
+  }
   if ((rc = upload_rows(ctx, x, ctx->nlocal, ctx->pos.p))) return rc;
   if ((rc = upload_rows(ctx, v, ctx->nlocal, ctx->vel.p))) return rc;
   if ((rc = upload_force(ctx, f))) return rc;
@@ -1121,6 +1159,30 @@ int eph_post_force(eph_context* ctx, const double* x, const double* v, double* f
   if (!ctx->have_atoms) return ctx->fail(EPH_ERR_STATE, "no atoms");
   const int nall = ctx->nlocal + ctx->nghost;
   int rc;
+  const size_t n3 = 3 * (size_t)ctx->nlocal, a3 = 3 * (size_t)nall;
+  if (double* p = nall ? hook_arena(ctx, 2 * a3 + 2 * n3 + 1) : nullptr) {
+    std::memcpy(p, x, a3 * sizeof(double));
+    std::memcpy(p + a3, v, a3 * sizeof(double));
+    std::memcpy(p + 2 * a3, f, n3 * sizeof(double));
+    const AtomsView a = ctx->atoms_view();
+    EPH_HIP(ctx, launch_hook_in(p, p + a3, nall, p + 2 * a3, ctx->nlocal, a.pos, a.vel, a.pv, a.f,
+                                a.fstride, ctx->stream));
+    ctx->pv_fresh = a.pv != nullptr;
+    ctx->cand_checked = false;
+    if ((rc = ctx->dev_post_force())) {
+      (void)hipStreamSynchronize(ctx->stream);  // the arena's readers
+      return rc;
+    }
+    double* fo = p + 2 * a3 + n3;
+    int* status = reinterpret_cast<int*>(fo + n3);
+    EPH_HIP(ctx, launch_hook_out(nullptr, nullptr, 0, nullptr, nullptr, 0, a.f, a.fstride, fo, ctx->nlocal,
+                                 ctx->flags_dev.p, ctx->grid ? ctx->grid->nonfinite.p : nullptr, status,
+                                 ctx->stream));
+    EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(f, fo, n3 * sizeof(double));
+    if (status[1] & 2) return ctx->fail(EPH_ERR_NONFINITE, "T_e grid became non-finite (FDM instability)");
+    return EPH_OK;
+  }
   if ((rc = upload_rows(ctx, x, nall, ctx->pos.p))) return rc;
   if ((rc = upload_rows(ctx, v, nall, ctx->vel.p))) return rc;
   if ((rc = upload_force(ctx, f))) return rc;
@@ -1138,6 +1200,16 @@ int eph_final_integrate(eph_context* ctx, double* v, const double* f) {
   if (!ctx->have_atoms) return ctx->fail(EPH_ERR_STATE, "no atoms");
   if (ctx->flags & EPH_NOINT) return EPH_OK;
   int rc;
+  const size_t n3 = 3 * (size_t)ctx->nlocal, b = n3 * sizeof(double);
+  if (double* p = hook_arena(ctx, 3 * n3)) {
+    ctx->pv_fresh = false;
+    std::memcpy(p, v, b); std::memcpy(p + n3, f, b);
+    EPH_HIP(ctx, launch_hook_kick(ctx->atoms_view(), ctx->step_params(), false, nullptr, p, p + n3,
+                                  nullptr, p + 2 * n3, ctx->stream));
+    EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    std::memcpy(v, p + 2 * n3, b);
+    return EPH_OK;
+  }
   if ((rc = upload_rows(ctx, v, ctx->nlocal, ctx->vel.p))) return rc;
   if ((rc = upload_force(ctx, f))) return rc;
   if ((rc = ctx->dev_final_integrate())) return rc;
@@ -1150,11 +1222,20 @@ int eph_end_of_step(eph_context* ctx, const double* x, const double* v, long lon
   if (!ctx || !x || !v) return EPH_ERR_ARGS;
   if (!ctx->have_atoms) return ctx->fail(EPH_ERR_STATE, "no atoms");
   int rc;
-  if ((rc = upload_rows(ctx, x, ctx->nlocal, ctx->pos.p))) return rc;
-  if ((rc = upload_rows(ctx, v, ctx->nlocal, ctx->vel.p))) return rc;
+  const size_t n3 = 3 * (size_t)ctx->nlocal;
+  if (double* p = n3 ? hook_arena(ctx, 2 * n3) : nullptr) {
+    ctx->pv_fresh = false;
+    std::memcpy(p, x, n3 * sizeof(double));
+    std::memcpy(p + n3, v, n3 * sizeof(double));
+    EPH_HIP(ctx, launch_hook_in(p, p + n3, ctx->nlocal, nullptr, 0, ctx->pos.p, ctx->vel.p, nullptr, nullptr, 0,
+                                ctx->stream));
+    EPH_HIP(ctx, ctx->arena.mark(ctx->stream));
+  } else {
+    if ((rc = upload_rows(ctx, x, ctx->nlocal, ctx->pos.p))) return rc;
+    if ((rc = upload_rows(ctx, v, ctx->nlocal, ctx->vel.p))) return rc;
+  }
   if ((rc = ctx->dev_end_of_step(ntimestep))) return rc;
-  EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return ctx->check_flags();
+  return ctx->check_flags();  // (waits for the step)
 }
 
 int eph_post_force_local(eph_context* ctx, const double* x, const double* v, double* halo) {
@@ -1211,9 +1292,7 @@ int eph_end_of_step_local(eph_context* ctx, const double* x, const double* v, do
   std::vector<double> d;
   if ((rc = ctx->grid->download(1, d))) return ctx->fail(rc, ctx->grid->err);
   std::copy(d.begin(), d.end(), dT);
-  EPH_HIP(ctx, hipMemcpyAsync(E_local, ctx->scal.p, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return EPH_OK;
+  return ctx->read(ctx->scal.p, E_local, sizeof(double));
 }
 
 int eph_end_of_step_reduced(eph_context* ctx, const double* dT, double E, long long ntimestep,
@@ -1255,9 +1334,7 @@ int eph_compute_vector(eph_context* ctx, int i, double* out) {
     return EPH_OK;
   }
   if (i == 1) return eph_grid_T_mean(ctx->grid, out);
-  EPH_HIP(ctx, hipMemcpyAsync(out, ctx->scal.p + 1, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  return EPH_OK;
+  return ctx->read(ctx->scal.p + 1, out, sizeof(double));
 }
 
 int eph_last_energy(eph_context* ctx, double* E_local) {
@@ -1378,6 +1455,17 @@ int eph_dev_get_atoms(eph_context* ctx, double* x, double* v, double* f) {
   if (!ctx) return EPH_ERR_ARGS;
   const int nall = ctx->nlocal + ctx->nghost;
   int rc;
+  const size_t n3 = 3 * (size_t)ctx->nlocal, a3 = 3 * (size_t)nall;
+  if (double* p = nall ? ctx->arena.take((2 * a3 + n3) * sizeof(double)) : nullptr) {
+    EPH_HIP(ctx, launch_hook_out(ctx->pos.p, p, x ? nall : 0, ctx->vel.p, p + a3, v ? nall : 0, ctx->f.p,
+                                 ctx->fstride, p + 2 * a3, f ? ctx->nlocal : 0, nullptr, nullptr, nullptr,
+                                 ctx->stream));
+    EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (x) std::memcpy(x, p, a3 * sizeof(double));
+    if (v) std::memcpy(v, p + a3, a3 * sizeof(double));
+    if (f) std::memcpy(f, p + 2 * a3, n3 * sizeof(double));
+    return EPH_OK;
+  }
   if (x) {
     if ((rc = download_rows(ctx, ctx->pos.p, nall, x))) return rc;
     EPH_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1642,19 +1730,14 @@ int eph_grid_solve(eph_grid* g, int* substeps) {
   int rc = g->solve(substeps);
   if (rc) return rc;
   int fl = 0;
-  EPH_HIP(g, hipMemcpyAsync(&fl, g->nonfinite.p, sizeof(int), hipMemcpyDeviceToHost, g->stream));
-  EPH_HIP(g, hipStreamSynchronize(g->stream));
+  if ((rc = g->read(g->nonfinite.p, &fl, sizeof fl))) return rc;
   if (fl & 2) return g->fail(EPH_ERR_NONFINITE, "T_e grid became non-finite (FDM instability)");
   return EPH_OK;
 }
 
 int eph_grid_get(eph_grid* g, int which, double* out) {
   if (!g || !out || which < 0 || which > 5) return EPH_ERR_ARGS;
-  std::vector<double> tmp;
-  int rc = g->download(which, tmp);
-  if (rc) return rc;
-  std::copy(tmp.begin(), tmp.end(), out);
-  return EPH_OK;
+  return g->read(g->values(which), out, g->h.ntotal() * sizeof(double));
 }
 
 int eph_grid_set(eph_grid* g, int which, const double* in) {
@@ -1713,8 +1796,7 @@ int eph_grid_T_mean(eph_grid* g, double* out) {
   const int G = (int)g->h.ntotal();
   EPH_HIP(g, launch_sum(g->T.p, G, g->sum_tmp.p + 256, g->sum_tmp.p, g->stream));
   double s = 0;
-  EPH_HIP(g, hipMemcpyAsync(&s, g->sum_tmp.p + 256, sizeof(double), hipMemcpyDeviceToHost, g->stream));
-  EPH_HIP(g, hipStreamSynchronize(g->stream));
+  if (int rc = g->read(g->sum_tmp.p + 256, &s, sizeof s)) return rc;
   *out = s / G;
   return EPH_OK;
 }

@@ -58,6 +58,7 @@ struct eph_grid {
   // only, both forms give the same bits, so it is read without a wait.
   int* crowded = nullptr;
   int bucket_bytes_ok(size_t G, int cap);  // reserves buckets of cap slots; 0 when they are ready
+  eph::PinnedArena arena;  // small calls
   bool any_tdyn = false;
   bool minmax_valid = false;  // cmin, rmin, kmax and uniform describe h
   bool uniform = false;       // every cell dynamic and of one material
@@ -77,6 +78,11 @@ struct eph_grid {
   void substeps(double* r, unsigned* steps, double* inner_dt) const;
   int insert_points(int n, const double* x, const double* y, const double* z, const double* E);
   int download(int which, std::vector<double>& out);
+  int read(const void* src, void* dst, size_t bytes);  // device -> host, waits
+  const double* values(int which) const {  // as eph_grid_get numbers them
+    return which == 0 ? T.p : which == 1 ? dT.p : which == 2 ? C.p : which == 3 ? rho.p
+         : which == 4 ? kappa.p : S.p;
+  }
   int sync_params_from_device();  // C, kappa after temperature-dependent updates
 };
 
@@ -138,6 +144,7 @@ struct eph_context {
   // copies of the host-array hooks (pinned chunks, worker threads), made on
   // first use
   std::unique_ptr<eph::HostStager> stager;
+  eph::PinnedArena arena;     // small calls
   bool stage_failed = false;  // no pinned memory: the runtime copies directly
   // optional per-kernel timing
   bool timing = false;
@@ -179,6 +186,7 @@ struct eph_context {
   int autotune(int* forms, double* ms);
   int grow_filter_state(size_t nall);
   int check_flags();
+  int read(const void* src, void* dst, size_t bytes);  // device -> host, waits
   // caller's host memory <-> device buffers on the context's stream: h2d
   // returns once src may be reused, d2h once dst holds the data
   int h2d(void* dst, const void* src, size_t bytes);

@@ -332,6 +332,18 @@ hipError_t launch_rows_into_soa(const double* rows, int n, double* soa, int stri
 hipError_t launch_soa_into_rows(const double* soa, int n, int stride, double* rows, hipStream_t s);
 hipError_t launch_d4_component(const double4* in, int n, int comp, double* out, hipStream_t s,
                                int stride4 = 1);
+// the host-array hooks on pinned memory: LAMMPS rows read and written in place.
+// x, v [n] into positions and velocities (and their records pv), f [nf] into f
+hipError_t launch_hook_in(const double* x, const double* v, int n, const double* f, int nf, double4* pos,
+                          double4* vel, PosVel* pv, double* fdst, int fstride, hipStream_t s);
+// the locals' x, v, f in, their initial or final kick, x and v out (initial) or v out
+hipError_t launch_hook_kick(const AtomsView& a, const StepParams& p, bool initial, const double* x,
+                            const double* v, const double* f, double* xo, double* vo, hipStream_t s);
+// rows of positions [nx], velocities [nv] and forces [nf] (any may be null),
+// and the two status words
+hipError_t launch_hook_out(const double4* pos, double* xo, int nx, const double4* vel, double* vo, int nv,
+                           const double* f, int fstride, double* fo, int nf, const int* flags,
+                           const int* nonfinite, int* status, hipStream_t s);
 // harness
 hipError_t launch_lj(const AtomsView& a, const int* nbr, const int* nn, int stride, double eps,
                      double sigma, double rc2, hipStream_t s, unsigned long long* t = nullptr);

@@ -2530,6 +2530,107 @@ __global__ __launch_bounds__(kBlock) void k_d4_component(const double4* __restri
   out[i] = comp == 0 ? o.x : comp == 1 ? o.y : comp == 2 ? o.z : o.w;
 }
 
+// The host-array hooks on pinned memory.  A block takes 256 rows through LDS,
+// so that every line of the pinned arrays crosses the bus once.
+static __device__ __forceinline__ void rows_load(const double* __restrict__ rows, int base, int n, double* sh) {
+  for (int k = threadIdx.x; k < 3 * min(kBlock, n - base); k += kBlock) sh[k] = rows[3 * base + k];
+}
+static __device__ __forceinline__ void rows_store(double* __restrict__ rows, int base, int n, const double* sh) {
+  for (int k = threadIdx.x; k < 3 * min(kBlock, n - base); k += kBlock) rows[3 * base + k] = sh[k];
+}
+
+__global__ __launch_bounds__(kBlock) void k_hook_in(const double* __restrict__ x, const double* __restrict__ v,
+                                                    int n, const double* __restrict__ f, int nf,
+                                                    double4* pos, double4* vel, PosVel* pv, double* fdst,
+                                                    int fstride) {
+  __shared__ double sx[3 * kBlock], sv[3 * kBlock], sf[3 * kBlock];
+  const int base = blockIdx.x * kBlock, t = threadIdx.x, i = base + t;
+  rows_load(x, base, n, sx);
+  rows_load(v, base, n, sv);
+  if (base < nf) rows_load(f, base, nf, sf);
+  __syncthreads();
+  if (i >= n) return;
+  PosVel q;
+  q.p = make_double4(sx[3 * t], sx[3 * t + 1], sx[3 * t + 2], pos[i].w);
+  q.v = make_double4(sv[3 * t], sv[3 * t + 1], sv[3 * t + 2], vel[i].w);
+  pos[i] = q.p;
+  vel[i] = q.v;
+  if (pv) pv[i] = q;
+  if (i < nf) {
+    fdst[i] = sf[3 * t]; fdst[fstride + i] = sf[3 * t + 1]; fdst[2 * fstride + i] = sf[3 * t + 2];
+  }
+}
+
+template <bool INITIAL>
+__global__ __launch_bounds__(kBlock) void k_hook_kick(AtomsView a, StepParams p, const double* __restrict__ x,
+                                                      const double* __restrict__ v,
+                                                      const double* __restrict__ f, double* xo, double* vo) {
+  __shared__ double sx[3 * kBlock], sv[3 * kBlock], sf[3 * kBlock];
+  const int base = blockIdx.x * kBlock, t = threadIdx.x, i = base + t, n = a.nlocal;
+  if (INITIAL) rows_load(x, base, n, sx);
+  rows_load(v, base, n, sv);
+  rows_load(f, base, n, sf);
+  __syncthreads();
+  if (i < n) {
+    const int fs = a.fstride;
+    a.f[i] = sf[3 * t]; a.f[fs + i] = sf[3 * t + 1]; a.f[2 * fs + i] = sf[3 * t + 2];
+    double4 w = make_double4(sv[3 * t], sv[3 * t + 1], sv[3 * t + 2], a.vel[i].w);
+    double4 q = w;
+    if (INITIAL) q = make_double4(sx[3 * t], sx[3 * t + 1], sx[3 * t + 2], a.pos[i].w);
+    if (a.mask[i] & a.groupbit) {  // k_integrate's expressions
+      const double dtfm = p.dtf / p.mass[a.type[i]];
+      w.x += dtfm * sf[3 * t];
+      w.y += dtfm * sf[3 * t + 1];
+      w.z += dtfm * sf[3 * t + 2];
+      if (INITIAL) {
+        q.x += p.dtv * w.x;
+        q.y += p.dtv * w.y;
+        q.z += p.dtv * w.z;
+      }
+    }
+    a.vel[i] = w;
+    sv[3 * t] = w.x; sv[3 * t + 1] = w.y; sv[3 * t + 2] = w.z;
+    if (INITIAL) {
+      a.pos[i] = q;
+      sx[3 * t] = q.x; sx[3 * t + 1] = q.y; sx[3 * t + 2] = q.z;
+    }
+  }
+  __syncthreads();
+  if (INITIAL) rows_store(xo, base, n, sx);
+  rows_store(vo, base, n, sv);
+}
+
+__global__ __launch_bounds__(kBlock) void k_hook_out(const double4* __restrict__ pos, double* xo, int nx,
+                                                     const double4* __restrict__ vel, double* vo, int nv,
+                                                     const double* __restrict__ f, int fstride, double* fo,
+                                                     int nf, const int* flags, const int* nonfinite,
+                                                     int* status) {
+  __shared__ double sh[3 * kBlock];
+  const int base = blockIdx.x * kBlock, t = threadIdx.x, i = base + t;
+  if (status && i == 0) {
+    status[0] = flags ? *flags : 0;
+    status[1] = nonfinite ? *nonfinite : 0;
+  }
+  auto put = [&](double ax, double ay, double az, double* rows, int n) {
+    sh[3 * t] = ax; sh[3 * t + 1] = ay; sh[3 * t + 2] = az;
+    __syncthreads();
+    rows_store(rows, base, n, sh);
+    __syncthreads();
+  };
+  if (base < nx) {
+    const double4 q = pos[i < nx ? i : base];
+    put(q.x, q.y, q.z, xo, nx);
+  }
+  if (base < nv) {
+    const double4 q = vel[i < nv ? i : base];
+    put(q.x, q.y, q.z, vo, nv);
+  }
+  if (base < nf) {
+    const int j = i < nf ? i : base;
+    put(f[j], f[fstride + j], f[2 * fstride + j], fo, nf);
+  }
+}
+
 // ================================================================ wrappers
 static inline int nblk(long n, int b = kBlock) { return static_cast<int>((n + b - 1) / b); }
 
@@ -3018,6 +3119,30 @@ hipError_t launch_d4_component(const double4* in, int n, int comp, double* out, 
   return hipGetLastError();
 }
 
+
+hipError_t launch_hook_in(const double* x, const double* v, int n, const double* f, int nf, double4* pos,
+                          double4* vel, PosVel* pv, double* fdst, int fstride, hipStream_t s) {
+  if (n > 0) k_hook_in<<<nblk(n), kBlock, 0, s>>>(x, v, n, f, nf, pos, vel, pv, fdst, fstride);
+  return hipGetLastError();
+}
+
+hipError_t launch_hook_kick(const AtomsView& a, const StepParams& p, bool initial, const double* x,
+                            const double* v, const double* f, double* xo, double* vo, hipStream_t s) {
+  if (a.nlocal == 0) return hipSuccess;
+  if (initial) k_hook_kick<true><<<nblk(a.nlocal), kBlock, 0, s>>>(a, p, x, v, f, xo, vo);
+  else k_hook_kick<false><<<nblk(a.nlocal), kBlock, 0, s>>>(a, p, x, v, f, xo, vo);
+  return hipGetLastError();
+}
+
+hipError_t launch_hook_out(const double4* pos, double* xo, int nx, const double4* vel, double* vo, int nv,
+                           const double* f, int fstride, double* fo, int nf, const int* flags,
+                           const int* nonfinite, int* status, hipStream_t s) {
+  const int n = nx > nv ? (nx > nf ? nx : nf) : (nv > nf ? nv : nf);
+  if (n > 0 || status)
+    k_hook_out<<<nblk(n > 0 ? n : 1), kBlock, 0, s>>>(pos, xo, nx, vel, vo, nv, f, fstride, fo, nf, flags,
+                                                      nonfinite, status);
+  return hipGetLastError();
+}
 
 // ---------------------------------------------------------- batched wrappers
 bool batch_lds_possible(const TablesView& t) {

@@ -18,6 +18,41 @@ void range_of(size_t n, int parts, int k, size_t* a, size_t* b) {
 }
 }  // namespace
 
+PinnedArena::~PinnedArena() {
+  if (busy_) (void)hipEventSynchronize(ev_);
+  if (ev_) (void)hipEventDestroy(ev_);
+  if (p_) (void)hipHostFree(p_);
+}
+
+double* PinnedArena::take(size_t bytes) {
+  if (bytes > kMax || failed_) return nullptr;
+  if (busy_ && hipEventSynchronize(ev_) != hipSuccess) return nullptr;
+  busy_ = false;
+  if (bytes > n_) {
+    if (p_) (void)hipHostFree(p_);
+    p_ = nullptr;
+    n_ = 0;
+    size_t want = size_t(1) << 16;
+    while (want < bytes) want <<= 1;
+    hipError_t e = ev_ ? hipSuccess : hipEventCreateWithFlags(&ev_, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&p_), want, hipHostMallocDefault);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      p_ = nullptr;
+      failed_ = true;
+      return nullptr;
+    }
+    n_ = want;
+  }
+  return reinterpret_cast<double*>(p_);
+}
+
+hipError_t PinnedArena::mark(hipStream_t s) {
+  const hipError_t e = hipEventRecord(ev_, s);
+  busy_ = e == hipSuccess;
+  return e;
+}
+
 int HostStager::default_threads() {
   int t = 4;
   if (const char* e = std::getenv("EPH_HOST_THREADS")) {
