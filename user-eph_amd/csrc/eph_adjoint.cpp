@@ -135,7 +135,8 @@ struct eph_adjoint {
   int backward_step(Rec& r, double* g_beta_unused);
 };
 
-#define HCPY(dst, src, n) EPH_HIP(this, hipMemcpyAsync((dst), (src), (n), hipMemcpyDeviceToDevice, s))
+#define HCPY(dst, src, n) \
+  if (!jobs.add((dst), (src), (n))) return fail(EPH_ERR_STATE, "copy list full")
 
 int eph_adjoint::save(State& st) {
   hipStream_t s = ctx->stream;
@@ -147,6 +148,7 @@ int eph_adjoint::save(State& st) {
   EPH_HIP(this, st.T.reserve(G)); EPH_HIP(this, st.scal.reserve(4));
   EPH_HIP(this, st.nbr.reserve(sf)); EPH_HIP(this, st.nnbr.reserve(ctx->stride));
   EPH_HIP(this, st.lj.reserve(sl)); EPH_HIP(this, st.ljn.reserve(ctx->stride));
+  CopyJobs jobs;
   HCPY(st.pos.p, ctx->pos.p, na * sizeof(double4));
   HCPY(st.vel.p, ctx->vel.p, na * sizeof(double4));
   HCPY(st.shift.p, ctx->ghost_shift.p, gc * sizeof(double4));
@@ -159,6 +161,7 @@ int eph_adjoint::save(State& st) {
   HCPY(st.nnbr.p, ctx->nnbr.p, ctx->stride * sizeof(int));
   HCPY(st.lj.p, md->lj_nbr.p, sl * sizeof(int));
   HCPY(st.ljn.p, md->lj_nn.p, ctx->stride * sizeof(int));
+  EPH_HIP(this, launch_copies(jobs, s));
   st.nghost = ctx->nghost;
   EPH_HIP(this, hipStreamSynchronize(s));
   return EPH_OK;
@@ -168,6 +171,7 @@ int eph_adjoint::restore(const State& st) {
   hipStream_t s = ctx->stream;
   const size_t na = nall_cap(), gc = md->ghost_cap, sf = (size_t)md->cap_f * ctx->stride,
                sl = (size_t)md->cap_l * ctx->stride;
+  CopyJobs jobs;
   HCPY(ctx->pos.p, st.pos.p, na * sizeof(double4));
   HCPY(ctx->vel.p, st.vel.p, na * sizeof(double4));
   HCPY(ctx->ghost_shift.p, st.shift.p, gc * sizeof(double4));
@@ -182,7 +186,8 @@ int eph_adjoint::restore(const State& st) {
   ctx->pv_fresh = false;
   HCPY(md->lj_nbr.p, st.lj.p, sl * sizeof(int));
   HCPY(md->lj_nn.p, st.ljn.p, ctx->stride * sizeof(int));
-  EPH_HIP(this, launch_fill_double(ctx->grid->dT.p, G, 0.0, s));
+  HCPY(ctx->grid->dT.p, nullptr, G * sizeof(double));
+  EPH_HIP(this, launch_copies(jobs, s));
   EPH_HIP(this, launch_fill_int(md->flags.p, 8, 0, s));
   ctx->nghost = st.nghost;
   md->nghost = st.nghost;
@@ -223,15 +228,13 @@ int eph_adjoint::step(long long n, Rec* r) {
   if ((rc = md->kick_and_pair(ctx, false, nullptr, &rebuilt, &overflow))) return fail(rc, md->err);
   if (overflow) return fail(EPH_ERR_STATE, "neighbour capacity exceeded during the trajectory");
   if ((rc = ctx->dev_post_force())) return fail(rc, ctx->err);
-  if ((rc = ctx->dev_final_integrate())) return fail(rc, ctx->err);
-  if (r) HCPY(r->TB.p, ctx->grid->T.p, G * sizeof(double));
-  if ((rc = ctx->dev_deposit(false))) return fail(rc, ctx->err);
-  if (r) HCPY(r->DT.p, ctx->grid->dT.p, G * sizeof(double));
-  if (ctx->flags & EPH_FDM) {
-    if ((rc = ctx->grid->solve(nullptr))) return fail(rc, ctx->grid->err);
-  }
+  DepositTail tail;  // (a recorded step keeps dT_e, so its deposit is finished here)
+  if ((rc = ctx->dev_deposit(true, r ? nullptr : &tail))) return fail(rc, ctx->err);
   if (r) {
     const size_t na = (size_t)nl + ctx->nghost, st = ctx->stride;
+    CopyJobs jobs;
+    HCPY(r->TB.p, ctx->grid->T.p, G * sizeof(double));
+    HCPY(r->DT.p, ctx->grid->dT.p, G * sizeof(double));
     HCPY(r->rec.p, ctx->rec.p, na * sizeof(ForceRec));
     HCPY(r->pv.p, ctx->pv.p, na * sizeof(PosVel));
     HCPY(r->vn.p, ctx->vel.p, nl * sizeof(double4));
@@ -241,8 +244,12 @@ int eph_adjoint::step(long long n, Rec* r) {
     HCPY(r->nact.p, ctx->nact.p, st * sizeof(int));
     HCPY(r->lj.p, md->lj_nbr.p, (size_t)md->cap_l * st * sizeof(int));
     HCPY(r->ljn.p, md->lj_nn.p, st * sizeof(int));
-    if (ctx->nghost) HCPY(r->owner.p, ctx->ghost_owner.p, ctx->nghost * sizeof(int));
+    HCPY(r->owner.p, ctx->ghost_owner.p, ctx->nghost * sizeof(int));
+    EPH_HIP(this, launch_copies(jobs, s));
     r->nghost = ctx->nghost;
+  }
+  if (ctx->flags & EPH_FDM) {
+    if ((rc = ctx->grid->solve(nullptr, tail.E_local ? &tail : nullptr))) return fail(rc, ctx->grid->err);
   }
   return EPH_OK;
 }
@@ -255,12 +262,13 @@ int eph_adjoint::backward_step(Rec& r, double*) {
   AdjBuffers b;
   b.xb = xb.p; b.vhb = vhb.p; b.wb = wb.p; b.vnb = vnb.p; b.fEb = fEb.p; b.fRb = fRb.p;
   b.ftb = ftb.p; b.ab = ab.p; b.rb = rb.p; b.Gb = Gb.p;
-  EPH_HIP(this, launch_fill_double(reinterpret_cast<double*>(wb.p), 4 * (long)na, 0.0, s));
-  EPH_HIP(this, launch_fill_double(reinterpret_cast<double*>(fEb.p), 4 * (long)nl, 0.0, s));
-  EPH_HIP(this, launch_fill_double(reinterpret_cast<double*>(fRb.p), 4 * (long)nl, 0.0, s));
-  EPH_HIP(this, launch_fill_double(ab.p, (long)na, 0.0, s));
-  EPH_HIP(this, launch_fill_double(rb.p, (long)na, 0.0, s));
-  EPH_HIP(this, launch_fill_double(dTb.p, G, 0.0, s));
+  CopyJobs jobs;
+  HCPY(wb.p, nullptr, na * sizeof(double4));
+  HCPY(fEb.p, nullptr, nl * sizeof(double4));
+  HCPY(fRb.p, nullptr, nl * sizeof(double4));
+  HCPY(ab.p, nullptr, na * sizeof(double));
+  HCPY(rb.p, nullptr, na * sizeof(double));
+  HCPY(dTb.p, nullptr, G * sizeof(double));
   // FDM: Tb (after) -> Tb2 (before), dTb
   GridView gv = ctx->grid->v;
   gv.dT = r.DT.p;
@@ -282,24 +290,28 @@ int eph_adjoint::backward_step(Rec& r, double*) {
       EPH_HIP(this, hipStreamSynchronize(s));
       grid->cmin = mm[0]; grid->rmin = mm[1]; grid->kmax = mm[2];
       EPH_HIP(this, kb.reserve(G));
-      EPH_HIP(this, launch_fill_double(kb.p, G, 0.0, s));
+      HCPY(kb.p, nullptr, G * sizeof(double));
     } else {
       grid->refresh_minmax();
     }
     grid->substeps(&rr, &S, &inner);
     EPH_HIP(this, Tsub.reserve((size_t)(S + 1) * G));
+    EPH_HIP(this, Tb2.reserve((size_t)S * G));  // a buffer per sub-step, cleared together
     HCPY(Tsub.p, r.TB.p, G * sizeof(double));
+    HCPY(Tb2.p, nullptr, (size_t)S * G * sizeof(double));
+    EPH_HIP(this, launch_copies(jobs, s));
     for (unsigned k = 0; k < S; ++k)
       EPH_HIP(this, launch_fdm_substep(gv, Tsub.p + (size_t)k * G, Tsub.p + (size_t)(k + 1) * G,
                                        inner, tdyn, s));
-    double* other = Tb2.p;
     for (int k = (int)S - 1; k >= 0; --k) {
-      EPH_HIP(this, launch_fill_double(other, G, 0.0, s));
-      EPH_HIP(this, launch_adj_fdm(gv, Tsub.p + (size_t)k * G, cur, other, dTb.p, tdyn ? kb.p : nullptr,
+      double* before = Tb2.p + (size_t)k * G;
+      EPH_HIP(this, launch_adj_fdm(gv, Tsub.p + (size_t)k * G, cur, before, dTb.p, tdyn ? kb.p : nullptr,
                                    inner, s));
-      std::swap(cur, other);
+      cur = before;
     }
     if (tdyn) EPH_HIP(this, launch_adj_kappa_T(gv, r.TB.p, kb.p, cur, s));
+  } else {
+    EPH_HIP(this, launch_copies(jobs, s));
   }
   b.Tb = cur;  // dL/dT_e before this step's solve; the force sweep adds its part
   AdjStepView sv;
@@ -323,7 +335,8 @@ int eph_adjoint::backward_step(Rec& r, double*) {
   f.ljrc2 = md->cfg.cut_lj * md->cfg.cut_lj;
   EPH_HIP(this, launch_adj_step(sv, a, ctx->tabs, gt, ctx->step_params(), f,
                                 (ctx->flags & EPH_FDM) ? dTb.p : nullptr, b, s));
-  if (cur != Tb.p) HCPY(Tb.p, cur, G * sizeof(double));
+  if (cur != Tb.p)
+    EPH_HIP(this, hipMemcpyAsync(Tb.p, cur, G * sizeof(double), hipMemcpyDeviceToDevice, s));
   return EPH_OK;
 }
 

@@ -277,6 +277,19 @@ hipError_t launch_prb_forces(const AtomsView& a, const TablesView& t, const Grid
 // eph/coloured/exp/v1: zv <- zv (1 - zeta) + zeta v for locals, then ghosts <- owners
 hipError_t launch_colour_v(const AtomsView& a, const StepParams& p, const WorkView& w, hipStream_t s);
 hipError_t launch_fill_int(int* p, int n, int v, hipStream_t s);
+// Up to kCopyJobs copies between 16-byte aligned device arrays in one launch
+// (from null: zeroes), of whole 4-byte words
+constexpr int kCopyJobs = 16;
+struct CopyJobs {
+  const void* src[kCopyJobs];
+  void* dst[kCopyJobs];
+  long words[kCopyJobs];
+  int first[kCopyJobs + 1] = {0};  // block at which job k starts
+  int n = 0;
+  // false: the list is full
+  bool add(void* to, const void* from, size_t bytes);
+};
+hipError_t launch_copies(const CopyJobs& j, hipStream_t s);
 hipError_t launch_fill_double(double* p, long n, double v, hipStream_t s);
 // deposit of the fix (energy of friction / random forces at end of step)
 hipError_t launch_deposit_atoms(const AtomsView& a, const GridView& g, const StepParams& p,
