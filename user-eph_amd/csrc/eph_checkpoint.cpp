@@ -369,6 +369,8 @@ int eph_md_checkpoint_load(eph_md* md, eph_context* fix, const char* path) {
       if ((rc = get_dev(fix, fl, fix->cstate.p, 8)) || (rc = get_dev(fix, fl, fix->ncand.p, fix->ncand.n)) ||
           (rc = get_dev(fix, fl, fix->cand.p, fix->cand.n)) || (rc = get_dev(fix, fl, fix->cref.p, fix->cref.n)))
         return rc;
+      // (the pair force's candidates are not in the file)
+      EPH_HIP(fix, launch_fill_int(fix->cstate.p + 6, 2, 0, fix->stream));
     } else if (!fl.seek((long)(8 + sz[0] + sz[1]) * (long)sizeof(int) + (long)sz[2] * (long)sizeof(double4),
                         SEEK_CUR)) {
       return fix->fail(EPH_ERR_FORMAT, "checkpoint file ends early");

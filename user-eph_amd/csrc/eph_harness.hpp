@@ -17,6 +17,11 @@ struct CSR {
 };
 }  // namespace eph
 
+// the pair force's candidates for launch_lj (cand null: buffers missing, or no
+// check before the pair force in this step)
+eph::LjCands lj_cands_of(const eph_context* ctx, const eph::WorkView& w, bool checked, int* cand, int* ncand,
+                         double cut, const int* rep);
+
 struct eph_md {
   std::string err;
   eph_md_config cfg{};
@@ -70,4 +75,6 @@ struct eph_md {
   // not fit and the host has to do it (no ghost update, no pair force then).
   int kick_and_pair(eph_context* ctx, bool force, unsigned long long* t, bool* rebuilt, bool* overflow);
   int ghosts_and_pair(eph_context* ctx, unsigned long long* t);
+  eph::LjCands lj_cands(eph_context* ctx) const;
+  eph::DevArray<int> lj_cand, lj_ncand;  // without them the pair force walks its full list
 };

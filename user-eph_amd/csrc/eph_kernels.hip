@@ -700,6 +700,11 @@ __device__ __forceinline__ void cand_flags(int* cstate, int moved_cap) {
   cstate[0] = retake || cstate[2] <= moved_cap ? 1 : 0;
   cstate[1] = 0;
   cstate[2] = 0;
+  // the pair force's candidates: taken in this step, or not those of the new
+  // reference positions
+  if (cstate[7]) cstate[6] = 1;
+  else if (retake || cstate[6] == 2) cstate[6] = 0;
+  cstate[7] = 0;
 }
 
 __global__ void k_cand_flags(int* cstate, int moved_cap) {
@@ -2096,12 +2101,40 @@ __global__ __launch_bounds__(kBlock) void k_peratom(AtomsView a, TablesView t, W
 // us up to 32,000 atoms and 156 us for 256,000; with 16 lanes 14 us for 256
 // and 15 for 4000, with 8 lanes 26 for 32,000 and 135 for 256,000 (times with
 // the event pair around them).  Bound by latency, then by the vector memory
-// path (140 entries, 78 of them inside the cutoff).
+// path and FP64 issue: 140 list entries an atom, 78 of them inside the cutoff.
+// Hence the candidates: 125 to 91 us for 256,000 atoms, 124 to 107 for 32
+// replicas of 8,000 with a fast atom each.  They are taken in a step whose
+// check took new reference positions (cstate[0] == 0), or that rebuilt the
+// lists ([6] == 2), and hold while [6] == 1; a wave near an atom on the moved
+// list walks its full list, whose other entries add nothing.
+
+// is an atom on the moved list within reach of one of the wave's 64 / S atoms,
+// whose box grown by reach is tested (replicas r0 to r1 of a batch)
+template <int S>
+__device__ __forceinline__ bool lj_near_moved(const double4& pi, const LjCands& c, const int nm,
+                                              const double r0, const double r1) {
+  double lx = pi.x, ly = pi.y, lz = pi.z, hx = pi.x, hy = pi.y, hz = pi.z;
+#pragma unroll
+  for (int o = S; o < 64; o <<= 1) {
+    lx = fmin(lx, __shfl_xor(lx, o)); ly = fmin(ly, __shfl_xor(ly, o)); lz = fmin(lz, __shfl_xor(lz, o));
+    hx = fmax(hx, __shfl_xor(hx, o)); hy = fmax(hy, __shfl_xor(hy, o)); hz = fmax(hz, __shfl_xor(hz, o));
+  }
+  lx -= c.reach; ly -= c.reach; lz -= c.reach;
+  hx += c.reach; hy += c.reach; hz += c.reach;
+  bool hit = false;
+  for (int m = threadIdx.x & 63; m < nm; m += 64) {
+    const double4 q = c.moved[m];
+    hit = hit || ((!c.rep || (q.w >= r0 && q.w <= r1)) && q.x >= lx && q.x <= hx && q.y >= ly && q.y <= hy &&
+                  q.z >= lz && q.z <= hz);
+  }
+  return __any(hit) != 0;
+}
+
 template <int S, int U>
 __global__ __launch_bounds__(kBlock) void k_lj(AtomsView a, const int* __restrict__ nbr,
                                                const int* __restrict__ nn, int stride,
                                                double lj1, double lj2, double rc2,
-                                               unsigned long long* t) {
+                                               unsigned long long* t, LjCands c) {
   __shared__ double2 s_split[(kBlock / 64) * split_stage_lj(U)];
   if (t && blockIdx.x == 0 && threadIdx.x == 0) *t = wall_clock64();
   const int wv = threadIdx.x >> 6;
@@ -2111,15 +2144,31 @@ __global__ __launch_bounds__(kBlock) void k_lj(AtomsView a, const int* __restric
   if (base >= a.nlocal) return;
   const int lane = threadIdx.x & 63, s = lane & (S - 1), ga = lane / S;
   const bool valid = base + ga < a.nlocal;
-  const int i = valid ? base + ga : 0;
+  const int i = valid ? base + ga : base;
   const double2* __restrict__ pos2 = reinterpret_cast<const double2*>(a.pos);
   const double4 pi = a.pos[i];
-  const int n = valid ? nn[i] : 0;
+  bool use = false, take = false;
+  if (c.cand) {
+    const int nm = c.cstate[2], state = c.cstate[6];
+    take = c.cstate[0] == 0 || state == 2;
+    use = !take && state == 1 && nm <= c.moved_cap;
+    if (use && nm > 0) {
+      const double r0 = c.rep ? c.rep[base] : 0.0;
+      const double r1 = c.rep ? c.rep[min(base + 64 / S, a.nlocal) - 1] : 0.0;
+      use = !lj_near_moved<S>(pi, c, nm, r0, r1);
+    }
+    if (take && base == 0 && lane == 0) c.cstate[7] = 1;
+  } else if (c.cstate && base == 0 && lane == 0 && c.cstate[6] == 2) {
+    c.cstate[6] = 0;
+  }
+  const int* __restrict__ list = use ? c.cand : nbr;
+  const int n = valid ? (use ? c.ncand[i] : nn[i]) : 0;
   const int nmax = wave_max(n);
   double acc = 0.0;
+  int nc = 0;
   int jj[U];
 #pragma unroll
-  for (int u = 0; u < U; ++u) jj[u] = S * u + s < n ? nbr[(S * u + s) * stride + i] : 0;
+  for (int u = 0; u < U; ++u) jj[u] = S * u + s < n ? list[(S * u + s) * stride + i] : 0;
   for (int k0 = 0; k0 < nmax; k0 += U * S) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -2130,23 +2179,30 @@ __global__ __launch_bounds__(kBlock) void k_lj(AtomsView a, const int* __restric
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int k = k0 + S * (U + u) + s;
-      jj[u] = k < n ? nbr[k * stride + i] : 0;
+      jj[u] = k < n ? list[k * stride + i] : 0;
     }
     double tx[U], ty[U], tz[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       tx[u] = ty[u] = tz[u] = 0.0;
       if (k0 + S * u < nmax) {
+        const int k = k0 + S * u + s;
         const double4 q = coop_read_pos(stage + 128 * u, lane);
         const double dx = pi.x - q.x, dy = pi.y - q.y, dz = pi.z - q.z;
         const double r2 = dx * dx + dy * dy + dz * dz;
-        if (k0 + S * u + s < n && r2 < rc2) {
+        if (k < n && r2 < rc2) {
           const double r2inv = 1.0 / r2;
           const double r6inv = r2inv * r2inv * r2inv;
           const double fpair = r6inv * (lj1 * r6inv - lj2) * r2inv;
           tx[u] = dx * fpair;
           ty[u] = dy * fpair;
           tz[u] = dz * fpair;
+        }
+        if (take) {
+          const bool in = k < n && r2 < c.cand2;
+          const unsigned cb = static_cast<unsigned>(__ballot(in) >> (S * ga)) & ((1u << S) - 1u);
+          if (in) c.cand[(nc + __popc(cb & ((1u << s) - 1u))) * stride + i] = nbr[k * stride + i];
+          nc += __popc(cb);
         }
       }
     }
@@ -2161,6 +2217,7 @@ __global__ __launch_bounds__(kBlock) void k_lj(AtomsView a, const int* __restric
     split_round_end();
   }
   if (valid && s < 3) a.f[s * a.fstride + i] = acc;
+  if (take && valid && s == 0) c.ncand[i] = nc;
   if (t) stamp_end(t + 1);
 }
 
@@ -3095,14 +3152,14 @@ hipError_t launch_peratom(const AtomsView& a, const TablesView& t, const WorkVie
 }
 
 hipError_t launch_lj(const AtomsView& a, const int* nbr, const int* nn, int stride, double eps,
-                     double sigma, double rc2, hipStream_t s, unsigned long long* t) {
+                     double sigma, double rc2, hipStream_t s, unsigned long long* t, const LjCands& c) {
   if (a.nlocal == 0) return hipSuccess;
   const double s6 = sigma * sigma * sigma * sigma * sigma * sigma;
   const double lj1 = 48.0 * eps * s6 * s6, lj2 = 24.0 * eps * s6;
   if (a.nlocal <= kSplitLj16)
-    k_lj<16, 3><<<nblk(a.nlocal, kBlock / 16), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2, t);
+    k_lj<16, 3><<<nblk(a.nlocal, kBlock / 16), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2, t, c);
   else
-    k_lj<8, 3><<<nblk(a.nlocal, kBlock / 8), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2, t);
+    k_lj<8, 3><<<nblk(a.nlocal, kBlock / 8), kBlock, 0, s>>>(a, nbr, nn, stride, lj1, lj2, rc2, t, c);
   return hipGetLastError();
 }
 

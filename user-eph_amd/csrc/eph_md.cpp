@@ -204,6 +204,11 @@ int eph_md::upload(eph_context* ctx) {
   hipStream_t s = ctx->stream;
   EPH_HIP(this, lj_nbr.reserve((size_t)std::max(mx, 1) * lj_stride));
   EPH_HIP(this, lj_nn.reserve(lj_stride));
+  if (lj_cand.reserve((size_t)std::max(mx, 1) * lj_stride) != hipSuccess ||
+      lj_ncand.reserve(lj_stride) != hipSuccess) {
+    (void)hipGetLastError();
+    lj_cand.release();
+  }
   EPH_HIP(this, lj_off.reserve(nlocal + 1));
   EPH_HIP(this, lj_idx.reserve(std::max<size_t>(lj.idx.size(), 1)));
   EPH_HIP(this, hipMemcpyAsync(lj_off.p, lj.off.data(), (nlocal + 1) * sizeof(int), hipMemcpyHostToDevice, s));
@@ -267,10 +272,27 @@ int eph_md::upload(eph_context* ctx) {
   return EPH_OK;
 }
 
+LjCands lj_cands_of(const eph_context* ctx, const WorkView& w, bool checked, int* cand, int* ncand,
+                    double cut, const int* rep) {
+  LjCands c;
+  c.cstate = ctx->cstate.p;
+  if (!checked || !cand || !ncand) return c;
+  c.cand = cand; c.ncand = ncand;
+  c.moved = w.moved; c.moved_cap = w.moved_cap;
+  c.cand2 = (cut + w.delta) * (cut + w.delta);
+  c.reach = cut + 0.1 * w.delta;  // as the density sweep's
+  c.rep = rep;
+  return c;
+}
+
+LjCands eph_md::lj_cands(eph_context* ctx) const {
+  return lj_cands_of(ctx, ctx->work_view(), ctx->cand_checked, lj_cand.p, lj_ncand.p, cfg.cut_lj, nullptr);
+}
+
 int eph_md::ghosts_and_pair(eph_context* ctx, unsigned long long* t) {
   if (int rc = ctx->dev_ghosts(t ? t + 2 : nullptr)) return fail(rc, ctx->err);
   EPH_HIP(this, launch_lj(ctx->atoms_view(), lj_nbr.p, lj_nn.p, lj_stride, cfg.lj_eps, cfg.lj_sigma,
-                          cfg.cut_lj * cfg.cut_lj, ctx->stream, t ? t + 3 : nullptr));
+                          cfg.cut_lj * cfg.cut_lj, ctx->stream, t ? t + 3 : nullptr, lj_cands(ctx)));
   return EPH_OK;
 }
 

@@ -369,6 +369,8 @@ __global__ __launch_bounds__(kBlock) void k_nb_finish(int nlocal, const int* ng,
   if (i == 0 && cand_valid) {
     cand_valid[0] = cand_written ? 1 : 0;
     cand_valid[2] = 0;  // atoms that a check before this rebuild found moved
+    cand_valid[6] = cand_written ? 2 : 0;  // the pair force's: to be taken in this step
+    cand_valid[7] = 0;
   }
   // (*go stays set: some blocks have yet to read it)
   if (i == 0) atomicAdd(nreb, 1);

@@ -69,7 +69,8 @@ struct NbBuild {
   int* nrebuild = nullptr;  // [1] count of device rebuilds
   // [1] the density sweep's candidate state: a rebuild that writes the
   // candidates (lists.cand) marks them valid with cref = the positions of the
-  // rebuild; one that does not clears it.  [2], the moved atoms, is emptied
+  // rebuild; one that does not clears it.  [2], the moved atoms, is emptied;
+  // [6] asks the pair force to take its candidates
   int* cand_valid = nullptr;
   double4* cref = nullptr;  // [nlocal + ghost_cap]
   int* cnt = nullptr;       // [nlocal + ghost_cap]
