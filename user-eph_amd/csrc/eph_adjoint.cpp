@@ -112,10 +112,17 @@ struct eph_adjoint {
     DevArray<PosVel> pv;
     DevArray<double4> vn;
     DevArray<double> fE, fR, TB, DT;
-    DevArray<int> act, nact, lj, ljn, owner;
-    int nghost = 0;
+    DevArray<int> act, nact;
+    int nghost = 0, lists = 0;
   };
   std::vector<Rec> seg;
+  // the pair lists and ghost owners of a segment's steps, which change with a
+  // rebuild only
+  struct Lists {
+    DevArray<int> lj, ljn, owner;
+  };
+  std::vector<Lists> lists;
+  int nlists = 0;
 
   // adjoint accumulators
   DevArray<double4> xb, vhb, wb, vnb, fEb, fRb, ftb;
@@ -242,9 +249,18 @@ int eph_adjoint::step(long long n, Rec* r) {
     HCPY(r->fR.p, ctx->fR.p, 3 * (size_t)ctx->fstride * sizeof(double));
     HCPY(r->act.p, ctx->act.p, (size_t)md->cap_f * st * sizeof(int));
     HCPY(r->nact.p, ctx->nact.p, st * sizeof(int));
-    HCPY(r->lj.p, md->lj_nbr.p, (size_t)md->cap_l * st * sizeof(int));
-    HCPY(r->ljn.p, md->lj_nn.p, st * sizeof(int));
-    HCPY(r->owner.p, ctx->ghost_owner.p, ctx->nghost * sizeof(int));
+    if (r == seg.data()) nlists = 0;
+    if (rebuilt || nlists == 0) {
+      if (nlists == (int)lists.size()) lists.emplace_back();
+      Lists& l = lists[nlists++];
+      EPH_HIP(this, l.lj.reserve((size_t)md->cap_l * st));
+      EPH_HIP(this, l.ljn.reserve(st));
+      EPH_HIP(this, l.owner.reserve(md->ghost_cap));
+      HCPY(l.lj.p, md->lj_nbr.p, (size_t)md->cap_l * st * sizeof(int));
+      HCPY(l.ljn.p, md->lj_nn.p, st * sizeof(int));
+      HCPY(l.owner.p, ctx->ghost_owner.p, ctx->nghost * sizeof(int));
+    }
+    r->lists = nlists - 1;
     EPH_HIP(this, launch_copies(jobs, s));
     r->nghost = ctx->nghost;
   }
@@ -316,8 +332,9 @@ int eph_adjoint::backward_step(Rec& r, double*) {
   b.Tb = cur;  // dL/dT_e before this step's solve; the force sweep adds its part
   AdjStepView sv;
   sv.rec = r.rec.p; sv.pv = r.pv.p; sv.vn = r.vn.p; sv.fE = r.fE.p; sv.fR = r.fR.p;
-  sv.fstride = ctx->fstride; sv.act = r.act.p; sv.nact = r.nact.p; sv.lj = r.lj.p; sv.ljn = r.ljn.p;
-  sv.owner = r.owner.p; sv.nghost = r.nghost;
+  sv.fstride = ctx->fstride; sv.act = r.act.p; sv.nact = r.nact.p;
+  const Lists& l = lists[r.lists];
+  sv.lj = l.lj.p; sv.ljn = l.ljn.p; sv.owner = l.owner.p; sv.nghost = r.nghost;
   AtomsView a = ctx->atoms_view();
   a.nghost = r.nghost;
   GridView gt = gv;
@@ -488,15 +505,13 @@ int eph_adjoint_backward(eph_adjoint* a, double* g_beta, double* g_v0) {
   EPH_HIP(a, launch_fill_double(reinterpret_cast<double*>(a->ftb.p), 4 * (long)nl, 0.0, s));
   EPH_HIP(a, launch_fill_double(a->Gb.p, 4 * (long)a->n_elem * a->n_beta, 0.0, s));
   // record buffers for one segment
-  const size_t st = ctx->stride, gc = a->md->ghost_cap;
+  const size_t st = ctx->stride;
   a->seg.resize(a->every);
   for (auto& r : a->seg) {
     EPH_HIP(a, r.rec.reserve(na)); EPH_HIP(a, r.pv.reserve(na)); EPH_HIP(a, r.vn.reserve(nl));
     EPH_HIP(a, r.fE.reserve(3 * (size_t)ctx->fstride)); EPH_HIP(a, r.fR.reserve(3 * (size_t)ctx->fstride));
     EPH_HIP(a, r.TB.reserve(G)); EPH_HIP(a, r.DT.reserve(G));
     EPH_HIP(a, r.act.reserve((size_t)a->md->cap_f * st)); EPH_HIP(a, r.nact.reserve(st));
-    EPH_HIP(a, r.lj.reserve((size_t)a->md->cap_l * st)); EPH_HIP(a, r.ljn.reserve(st));
-    EPH_HIP(a, r.owner.reserve(gc));
   }
   int rc;
   const int nseg = (int)a->ckpt.size();

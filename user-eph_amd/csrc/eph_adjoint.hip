@@ -432,37 +432,58 @@ __global__ __launch_bounds__(kBlock) void k_adj_w(AdjStepView s, AtomsView a, Ta
 // ------------------------------------------------------------ alpha(rho)
 // alpha_i = a + rho (b + rho (c + rho d)) on the interval of rho_i: rho_b +=
 // alpha_b alpha', table gradient Gb[e][k] += alpha_b (1, rho, rho^2, rho^3).
-// The atoms of a wave mostly sit on one or two knots (rho is nearly uniform in
-// a crystal), so the table gradient is summed over the wave per distinct knot
-// first and added with one atomic per knot and wave; all lanes take part.
+// The atoms of a crystal mostly sit on one or two knots, and an atomic on an
+// address that all blocks share takes some 50 ns: 32,000 atoms took 27 us with
+// one per knot and wave (1.5 ms with one per atom).
+
+// rho_b and the four terms of atom i; its knot, -1 for none
+__device__ __forceinline__ int adj_alpha_atom(const int i, const AdjStepView& s, const AtomsView& a,
+                                              const TablesView& t, const AdjBuffers& b, double* g) {
+  if (i >= a.nlocal || !(a.mask[i] & a.groupbit)) return -1;
+  const double rho = s.rec[i].rw.w, ab = b.ab[i];
+  if (!(rho > 0.0) || rho > t.rho_cut || ab == 0.0) return -1;
+  const int e = t.n_elem > 1 ? static_cast<int>(s.rec[i].p.w) : 0;
+  int k = static_cast<int>(rho * t.inv_drho);
+  k = k < 0 ? 0 : (k < t.n_beta - 1 ? k : t.n_beta - 1);
+  const int key = e * t.n_beta + k;
+  const double4 c = t.alpha[key];
+  b.rb[i] += ab * (c.y + rho * (2.0 * c.z + 3.0 * rho * c.w));
+  g[0] = ab; g[1] = ab * rho; g[2] = ab * rho * rho; g[3] = ab * rho * rho * rho;
+  return key;
+}
+
+// Tables whose gradient fits the LDS (9 us for those atoms): a few large blocks sum it there
+// and add each touched coefficient once.
+constexpr int kAlphaThreads = 1024, kAlphaBlocks = 32;
+constexpr size_t kAlphaLds = 64 * 1024;
+__global__ __launch_bounds__(kAlphaThreads) void k_adj_alpha_lds(AdjStepView s, AtomsView a, TablesView t,
+                                                                 AdjBuffers b, int ncoef) {
+  extern __shared__ double s_g[];
+  for (int q = threadIdx.x; q < ncoef; q += kAlphaThreads) s_g[q] = 0.0;
+  __syncthreads();
+  for (int i = blockIdx.x * kAlphaThreads + threadIdx.x; i < a.nlocal; i += gridDim.x * kAlphaThreads) {
+    double g[4];
+    const int key = adj_alpha_atom(i, s, a, t, b, g);
+    if (key >= 0)
+      for (int q = 0; q < 4; ++q) atomicAdd(s_g + 4 * key + q, g[q]);
+  }
+  __syncthreads();
+  for (int q = threadIdx.x; q < ncoef; q += kAlphaThreads)
+    if (s_g[q] != 0.0) atomicAdd(b.Gb + q, s_g[q]);
+}
+
+// any table: summed over the wave per distinct knot, all lanes taking part
 __global__ __launch_bounds__(kBlock) void k_adj_alpha(AdjStepView s, AtomsView a, TablesView t,
                                                       AdjBuffers b) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  bool valid = i < a.nlocal && (a.mask[i] & a.groupbit);
-  double rho = 0.0, ab = 0.0;
-  if (valid) {
-    rho = s.rec[i].rw.w;
-    ab = b.ab[i];
-    valid = rho > 0.0 && !(rho > t.rho_cut) && ab != 0.0;
-  }
-  int key = -1;
-  if (valid) {
-    const int e = t.n_elem > 1 ? static_cast<int>(s.rec[i].p.w) : 0;
-    int k = static_cast<int>(rho * t.inv_drho);
-    k = k < 0 ? 0 : (k < t.n_beta - 1 ? k : t.n_beta - 1);
-    key = e * t.n_beta + k;
-    const double4 c = t.alpha[key];
-    b.rb[i] += ab * (c.y + rho * (2.0 * c.z + 3.0 * rho * c.w));
-  }
-  const double g0 = valid ? ab : 0.0, g1 = valid ? ab * rho : 0.0;
-  const double g2 = valid ? ab * rho * rho : 0.0, g3 = valid ? ab * rho * rho * rho : 0.0;
+  double g[4] = {0.0, 0.0, 0.0, 0.0};
+  const int key = adj_alpha_atom(blockIdx.x * kBlock + threadIdx.x, s, a, t, b, g);
   const int lane = static_cast<int>(threadIdx.x) & (warpSize - 1);
-  unsigned long long left = __ballot(valid);
+  unsigned long long left = __ballot(key >= 0);
   while (left) {
     const int lead = __ffsll(static_cast<long long>(left)) - 1;
     const int k0 = __shfl(key, lead);
-    const bool mine = valid && key == k0;
-    double s0 = mine ? g0 : 0.0, s1 = mine ? g1 : 0.0, s2 = mine ? g2 : 0.0, s3 = mine ? g3 : 0.0;
+    const bool mine = key == k0;
+    double s0 = mine ? g[0] : 0.0, s1 = mine ? g[1] : 0.0, s2 = mine ? g[2] : 0.0, s3 = mine ? g[3] : 0.0;
     for (int off = warpSize / 2; off > 0; off >>= 1) {
       s0 += __shfl_xor(s0, off);
       s1 += __shfl_xor(s1, off);
@@ -564,7 +585,14 @@ hipError_t launch_adj_step(const AdjStepView& sv, const AtomsView& a, const Tabl
     k_adj_force<<<nbl, kBlock, 0, s>>>(sv, a, t, f.fric, f.rnd, b);
   }
   if (f.fric) k_adj_w<<<nbl, kBlock, 0, s>>>(sv, a, t, b);
-  k_adj_alpha<<<nb, kBlock, 0, s>>>(sv, a, t, b);
+  const int ncoef = 4 * t.n_elem * t.n_beta;
+  if (ncoef * sizeof(double) <= kAlphaLds) {
+    const int blocks = static_cast<int>((a.nlocal + kAlphaThreads - 1l) / kAlphaThreads);
+    k_adj_alpha_lds<<<blocks < kAlphaBlocks ? blocks : kAlphaBlocks, kAlphaThreads, ncoef * sizeof(double), s>>>(
+        sv, a, t, b, ncoef);
+  } else {
+    k_adj_alpha<<<nb, kBlock, 0, s>>>(sv, a, t, b);
+  }
   k_adj_rho<<<nbl, kBlock, 0, s>>>(sv, a, t, b);
   k_adj_initial<<<nb, kBlock, 0, s>>>(a, p, f.noint, b);
   return hipGetLastError();
