@@ -30,8 +30,8 @@ def test_cell_sums_match_serial_order(oracle, counts):
     assert np.array_equal(g.get("dT"), o.get("dT"))
 
 
-# the fix's own deposit: atoms per grid cell from 0.5 to 256 (16 slots a cell and a thread, 32 to 256
-# slots and a wave, then the counted form), with a hot corner so that cells differ
+# the fix's own deposit: atoms per grid cell from 0.5 to 256 (a thread per cell, a wave per cell,
+# then the counted form), with a hot corner so that cells differ
 @pytest.mark.parametrize("cells,grid", [(4, 8), (5, 5), (6, 5), (6, 4), (6, 3), (7, 3), (6, 2), (8, 2),
                                         (4, 1), (5, (2, 7, 3))])
 def test_deposit_forms_match_oracle(oracle, tmp_path, cells, grid):
@@ -62,10 +62,12 @@ def test_deposit_forms_match_oracle(oracle, tmp_path, cells, grid):
         assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))
 
 
-# an eighth of the box holds all atoms, one cell far more than its bucket; the larger boxes overflow so many
-# cells (of 16 and of 256 slots) that the deposits after the first are counted ones
-@pytest.mark.parametrize("cells,n", [(6, 4), (20, 24), (20, 8)])
-def test_crowded_cells_match_oracle(oracle, tmp_path, cells, n):
+# a corner of the box holds all atoms, part of it more: queued cells out of the bucket, out of bucket and chain
+# (16 slots a cell), and by a scan (27 cells of 1200 atoms in buckets of 1024); so many, or scans so long, that the
+# deposits after the first are counted ones
+@pytest.mark.parametrize("cells,n,corner", [(6, 4, 0.5), (20, 24, 0.5), (20, 8, 0.5), (20, 30, 0.5), (20, 30, 0.2),
+                                            (20, 10, 0.3), (9, 5, 0.2)])
+def test_crowded_cells_match_oracle(oracle, tmp_path, cells, n, corner):
     import copy
 
     import eph_amd as ea
@@ -86,7 +88,7 @@ def test_crowded_cells_match_oracle(oracle, tmp_path, cells, n):
     ora.post_force(a, step=1)
     gpu.post_force(b, step=1)
     for s in (a, b):  # the deposit sees these positions only
-        s.x[:s.nlocal] = np.random.default_rng(1).uniform(0.0, 0.5, (s.nlocal, 3)) * inf["boxhi"][0]
+        s.x[:s.nlocal] = np.random.default_rng(1).uniform(0.0, corner, (s.nlocal, 3)) * inf["boxhi"][0]
         s.x[:300] *= 0.4
     for step in (1, 2, 3):
         ora.end_of_step(a, step)

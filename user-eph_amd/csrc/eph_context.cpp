@@ -163,9 +163,8 @@ int eph_grid::insert_points(int n, const double* x, const double* y, const doubl
   DepositView d = dep.view(false);
   EPH_HIP(this, launch_fill_int(d.count, (int)G + 1, 0, stream));
   EPH_HIP(this, launch_deposit_points(n, q, q + n, q + 2 * (size_t)n, q + 3 * (size_t)n, h.dt, v, d, stream));
-  if (a) EPH_HIP(this, arena.mark(stream));
   EPH_HIP(this, launch_deposit_cells(v, d, n, dep.qbuf.p, stream));
-  if (!a) EPH_HIP(this, hipStreamSynchronize(stream));
+  EPH_HIP(this, hipStreamSynchronize(stream));
   return EPH_OK;
 }
 
@@ -686,14 +685,16 @@ int eph_context::end_of_step_after_deposit(long long ntimestep, const DepositTai
   return EPH_OK;
 }
 
-int eph_grid::bucket_bytes_ok(size_t G, int cap) {
+int eph_grid::bucket_bytes_ok(size_t G, int cap, int n) {
   EPH_HIP(this, bcount.reserve(G));  // zero-filled when first made
   EPH_HIP(this, bitems.reserve(G * cap));
+  EPH_HIP(this, bhead.reserve(G));
+  EPH_HIP(this, bnext.reserve(n));
   EPH_HIP(this, bqueue.reserve(G));
   EPH_HIP(this, bnq.reserve(1));
-  if (!crowded) {
-    EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&crowded), sizeof(int), hipHostMallocDefault));
-    *crowded = 0;
+  if (!bstate) {
+    EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&bstate), sizeof(int), hipHostMallocDefault));
+    *bstate = 0;
   }
   return EPH_OK;
 }
@@ -701,7 +702,7 @@ int eph_grid::bucket_bytes_ok(size_t G, int cap) {
 // slots per cell where the deposit goes through per-cell buckets, else 0
 int eph_context::bucket_deposit() const {
   if (!(flags & (EPH_FRICTION | EPH_RANDOM))) return 0;
-  if (grid->crowded && *static_cast<volatile int*>(grid->crowded)) return 0;
+  if (grid->bstate && *static_cast<volatile int*>(grid->bstate) == kCrowded) return 0;
   return bucket_slots(static_cast<double>(nlocal), static_cast<double>(grid->h.ntotal()));
 }
 
@@ -721,17 +722,19 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
   // per-cell buckets (three launches)
   if (cap) {
     EPH_HIP(this, grid->dep.reserve(nlocal, G, nb));  // also what a counted deposit needs
-    if (int rc = grid->bucket_bytes_ok(G, cap)) return fail(rc, grid->err);
+    if (int rc = grid->bucket_bytes_ok(G, cap, nlocal)) return fail(rc, grid->err);
     DepositView d = grid->dep.view(true);
     BucketView b;
     b.cap = cap;
+    b.thread = nlocal <= kThreadCells * static_cast<double>(G);
+    b.head = grid->bhead.p; b.next = grid->bnext.p;
     b.count = grid->bcount.p; b.items = grid->bitems.p; b.queue = grid->bqueue.p; b.nqueue = grid->bnq.p;
-    b.limit = queue_limit(nlocal);
-    b.crowded = grid->crowded;
+    b.state = grid->bstate;
+    const bool calm = *static_cast<volatile int*>(grid->bstate) == kCalm;
     timed_begin("deposit", &e);
     EPH_HIP(this, launch_deposit_bucket(atoms_view(), grid->v, step_params(), work_view(), d, b, fric, rnd,
                                         kick, scal.p, scal.p + (defer_tally ? 2 : 1), stream,
-                                        tail && (flags & EPH_FDM) && !timing ? tail : nullptr));
+                                        tail && (flags & EPH_FDM) && !timing && calm ? tail : nullptr));
     timed_end(kick ? "final_integrate+deposit" : "deposit", e);
     return EPH_OK;
   }
@@ -1676,7 +1679,7 @@ void eph_grid_destroy(eph_grid* g) {
   if (!g) return;
   if (g->stream) (void)hipStreamSynchronize(g->stream);
   hipStream_t s = g->own_stream ? g->stream : nullptr;
-  if (g->crowded) (void)hipHostFree(g->crowded);
+  if (g->bstate) (void)hipHostFree(g->bstate);
   delete g;
   if (s) (void)hipStreamDestroy(s);
 }

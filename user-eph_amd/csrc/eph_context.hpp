@@ -52,12 +52,12 @@ struct eph_grid {
   eph::DevArray<int> nonfinite, lookup_idx;
   eph::DepositBuffers dep;
   // per-cell buckets of the deposit (count kept at zero between steps)
-  eph::DevArray<int> bcount, bitems, bqueue, bnq;
-  // Pinned: the device sets [0] once more cells overflowed their buckets than
-  // queue_limit allows; the deposits from then on are counted ones.  A plan
-  // only, both forms give the same bits, so it is read without a wait.
-  int* crowded = nullptr;
-  int bucket_bytes_ok(size_t G, int cap);  // reserves buckets of cap slots; 0 when they are ready
+  eph::DevArray<int> bcount, bitems, bhead, bnext, bqueue, bnq;
+  // Pinned: how the last bucketed deposit went (BucketView::state).  After a
+  // crowded one the deposits are counted ones; a plan only, as both forms give
+  // the same bits, so it is read without a wait.
+  int* bstate = nullptr;
+  int bucket_bytes_ok(size_t G, int cap, int n);  // reserves buckets of cap slots for n atoms; 0 when they are ready
   eph::PinnedArena arena;  // small calls
   bool any_tdyn = false;
   bool minmax_valid = false;  // cmin, rmin, kmax and uniform describe h

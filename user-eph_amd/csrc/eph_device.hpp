@@ -162,33 +162,40 @@ struct DepositView {
   int* maxcount = nullptr;    // [1]
 };
 
-// Per-cell buckets of the deposit (launch_deposit_bucket): count and cap atom
-// slots per cell, and the queue of cells that received more atoms than that.
-constexpr int kBucket = 16, kBucketMax = 256;
-// Slots per cell for n atoms in G cells, 0: no buckets.  Eight times the
-// average, so that a box that is mostly empty still fits, as far as
-// kBucketMax, what a wave's registers hold, and from 64 atoms per cell on the
-// counted form.  Up to 6 atoms per cell 16 slots, which one thread sorts.
+// Per-cell buckets of the deposit (launch_deposit_bucket): a count and cap
+// atom slots per cell, and a chain of the atoms beyond them.
+// The cells' sums take kBucket atoms per thread, or kWaveCellMax per wave
+// (what its registers hold); cells with more are queued for a workgroup each.
+constexpr int kBucket = 16, kWaveCellMax = 256;
+// Up to kThreadCells atoms per cell on average a thread per cell, up to
+// kWaveCells a wave; above, the counted form.
+constexpr double kThreadCells = 6.0, kWaveCells = 64.0;
+// Slots per cell for n atoms in G cells, 0: no buckets.  More than the cells'
+// sums need, so that the queued cells of a crowded box find their atoms in
+// the bucket too, where the buckets are small (up to 64 MB).
 inline int bucket_slots(double n, double G) {
-  if (n <= 6.0 * G) return kBucket;
-  if (n > 64.0 * G) return 0;
-  int cap = 64;
-  while (cap < kBucketMax && cap < 8.0 * n / G) cap <<= 1;
-  return cap;
+  if (n > kWaveCells * G) return 0;
+  const bool small = G <= 16384.0;
+  if (n <= kThreadCells * G) return small ? kWaveCellMax : kBucket;
+  return small ? 4 * kWaveCellMax : kWaveCellMax;
 }
-// A cell beyond its bucket costs a scan over all atoms (1.5 us per 1024 of
-// them), shared by kQueueBlocks workgroups.  Beyond this many such cells the
-// counted form (some 45 us more than the bucketed one) is the faster.
-constexpr int kQueueBlocks = 16;
-inline int queue_limit(int n) { return kQueueBlocks * (1 + 32768 / (n > 0 ? n : 1)); }
+// A queued cell takes a workgroup 5 to 10 us; kQueueBlocks share them.  Beyond
+// kQueueEach of them per block the counted form (some 45 us more than the
+// bucketed one) is the faster, and the device says so in *state.  A
+// one-workgroup T_e solve takes the queue over only after a deposit that left
+// it empty.
+constexpr int kQueueBlocks = 64, kQueueEach = 6;
+constexpr int kCrowded = 1, kCalm = 2;
 struct BucketView {
   int cap = kBucket;
+  bool thread = true;     // a thread per cell
   int* count = nullptr;   // [G], zero between steps
   int* items = nullptr;   // [G][cap]
+  int* head = nullptr;    // [G], 1 + the last atom of the cell's chain; zero between steps
+  int* next = nullptr;    // [atoms], the chain
   int* queue = nullptr;   // [G]
   int* nqueue = nullptr;  // [1]
-  int limit = 0;          // queued cells beyond which *crowded is set
-  int* crowded = nullptr; // pinned host memory
+  int* state = nullptr;   // pinned host memory: kCrowded, kCalm, or 0 at first
 };
 
 // What is left of the bucketed deposit after the cells' sums: the tally from

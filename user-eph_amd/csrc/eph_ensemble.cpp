@@ -70,9 +70,9 @@ struct eph_ensemble {
   // bucketed deposit: slots per cell (0: counted), the buckets, and the pinned
   // flag that the device sets when too many cells overflowed theirs
   int slots = 0;
-  DevArray<int> bk_count, bk_items, bk_queue, bk_nq;
-  int* crowded = nullptr;
-  bool bucketed() const { return slots > 0 && !*static_cast<volatile int*>(crowded); }
+  DevArray<int> bk_count, bk_items, bk_head, bk_next, bk_queue, bk_nq;
+  int* bk_state = nullptr;
+  bool bucketed() const { return slots > 0 && *static_cast<volatile int*>(bk_state) != kCrowded; }
   // the T_e solve with a workgroup per replica
   bool fdm_block = false, fdm_uniform = false;
   int max_cells = 0;
@@ -97,7 +97,7 @@ struct eph_ensemble {
       eph_md_destroy(r.md);
     }
     if (pinned) (void)hipHostFree(pinned);
-    if (crowded) (void)hipHostFree(crowded);
+    if (bk_state) (void)hipHostFree(bk_state);
     eph_destroy(sys);
   }
   int setup(long long first);
@@ -327,10 +327,12 @@ int eph_ensemble::setup(long long first) {
   if (slots) {
     EPH_HIP(this, bk_count.reserve(G));  // zero-filled
     EPH_HIP(this, bk_items.reserve(static_cast<size_t>(G) * slots));
+    EPH_HIP(this, bk_head.reserve(G));   // zero-filled
+    EPH_HIP(this, bk_next.reserve(nl));
     EPH_HIP(this, bk_queue.reserve(G));
     EPH_HIP(this, bk_nq.reserve(1));
-    if (!crowded) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&crowded), sizeof(int), hipHostMallocDefault));
-    *crowded = 0;
+    if (!bk_state) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&bk_state), sizeof(int), hipHostMallocDefault));
+    *bk_state = 0;
   }
   fdm_uniform = true;
   max_cells = 0;
@@ -410,9 +412,10 @@ int eph_ensemble::enqueue_step() {
   if (buckets) {
     BucketView b;
     b.cap = slots;
+    b.thread = nl <= kThreadCells * G;
+    b.head = bk_head.p; b.next = bk_next.p;
     b.count = bk_count.p; b.items = bk_items.p; b.queue = bk_queue.p; b.nqueue = bk_nq.p;
-    b.limit = queue_limit(nl / R);
-    b.crowded = crowded;
+    b.state = bk_state;
     EPH_HIP(this, launch_deposit_bucket_batch(a, gviews.p, cell_off.p, cell_rep.p, gall, p, w, dep.view(true), b,
                                               chunks.p, nchunk, chunk0.p, nchunks.p, R,
                                               !(sys->flags & EPH_NOINT), E_local.p, Ee.p, s));

@@ -100,10 +100,12 @@ __global__ __launch_bounds__(kFdmThreads) void k_fdm_block(GridView g, FdmArgs u
   extern __shared__ double s_fdm[];
   if (tail.E_local) {  // the deposit's remainder, which completes dT_e
     __shared__ double sh[kFdmThreads];
-    __shared__ unsigned long long hits[kFdmThreads / 64];
+    __shared__ QueueShared qs;
     energy_reduce(tail.d.partial, tail.nblocks, tail.E_local, tail.Ee, sh);
-    if (threadIdx.x == 0 && *tail.b.nqueue > tail.b.limit / kQueueBlocks) *tail.b.crowded = 1;
-    deposit_queued(tail, g, 0, 1, hits);
+    const int nq = *tail.b.nqueue;
+    if (threadIdx.x == 0 && nq > kQueueEach) *tail.b.state = kCrowded;
+    for (int q = 0; q < nq; ++q)
+      queued_cell(tail.a, tail.d, tail.b, g, tail.b.queue[q], tail.b.queue[q], 0, tail.a.nlocal, qs);
     __syncthreads();
   }
   fdm_block<MODE, NC>(g, u, T, nsub, G, nonfinite, s_fdm);

@@ -1661,21 +1661,12 @@ __global__ __launch_bounds__(kBlock) void k_cell_sum_small(GridView g, DepositVi
   g.dT[c] = acc;
 }
 
-// acc += the first n lanes' v, in lane order: every lane keeps the same sum
-static __device__ __forceinline__ double add_lanes(double acc, double v, int n) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  for (int k = 0; k < n; ++k)
-    acc += __hiloint2double(__builtin_amdgcn_readlane(hi, k), __builtin_amdgcn_readlane(lo, k));
-  return acc;
-}
-
 // One wave per cell, for grids with several items per cell: the items' ranks
 // by counting (their numbers are distinct), their values through LDS in that
 // order, then the serial sums from registers.  With one thread per cell the
 // insertion sort and the dependent loads of the sums are the time: 191 us for
 // 1000 cells of 32 atoms, all but 4 us of which a wave per cell saves (a
 // 32,000-atom MD step goes from 441 to 254 us).
-constexpr int kWaveCellMax = 256;
 template <int E>
 static __device__ __forceinline__ void cell_ranks(const int* __restrict__ items, int n, int lane,
                                                   const DepositView& d, double* s1, double* s2) {
@@ -1828,9 +1819,9 @@ __global__ __launch_bounds__(1024) void k_energy_reduce(const double* partial, i
 // holds 4, at most 14 while every atom stays within half a cell of its site)
 // or one wave per cell then sorts its bucket and adds the values in ascending
 // atom order, friction then random, the serial order of fix_eph.cpp:364-390.
-// A cell that receives more atoms than its bucket holds is queued and summed
-// by k_deposit_finish from an ordered scan of every atom's cell; once many
-// are, the steps that follow take the counted form.  Three launches in all: with 32 atoms per cell (32,000 atoms) 24 us with the final
+// A cell with more atoms than that is queued and summed by a workgroup of
+// k_deposit_finish (queued_cell); once many are, the steps that follow take the
+// counted form.  Three launches in all: with 32 atoms per cell (32,000 atoms) 24 us with the final
 // kick inside, against 64 us for the twelve launches of the counted deposit
 // and 5 us for the kick.
 // one atom of the bucketed deposit at end-of-step velocity v: its energies
@@ -1863,6 +1854,7 @@ __device__ __forceinline__ void deposit_bucket_atom(const int i, const double4& 
   }
   const int slot = atomicAdd(&b.count[c], 1);
   if (slot < b.cap) b.items[static_cast<size_t>(c) * b.cap + slot] = i;
+  else b.next[i] = atomicExch(&b.head[c], i + 1);
   if (FRIC) d.v1[i] = v1;
   if (RAND) d.v2[i] = v2;
 }
@@ -1917,6 +1909,7 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket_batch(AtomsView a,
   const Chunk c = chunks[blockIdx.x];
   b.count += cell_off[c.rep];
   b.items += static_cast<size_t>(cell_off[c.rep]) * b.cap;
+  b.head += cell_off[c.rep];
   deposit_bucket_block<FRIC, RAND, KICK>(c.start + threadIdx.x, static_cast<int>(threadIdx.x) < c.count, a,
                                          grids[c.rep], p, w, d, b);
 }
@@ -1937,13 +1930,13 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket_cells(GridView g, Dep
   if (c >= ncell) return;
   const int n = b.count[c];
   if (n == 0) return;
-  b.count[c] = 0;
-  if (n > kBucket) {
+  if (n > kBucket) {  // (the count is left to the queue)
     b.queue[atomicAdd(b.nqueue, 1)] = c;
     return;
   }
+  b.count[c] = 0;
   int k[kBucket];
-  const int* src = b.items + static_cast<size_t>(c) * kBucket;
+  const int* src = b.items + static_cast<size_t>(c) * b.cap;
 #pragma unroll
   for (int e = 0; e < kBucket; ++e) k[e] = e < n ? src[e] : 0x7fffffff;
 #pragma unroll
@@ -1972,7 +1965,7 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket_cells(GridView g, Dep
   g.dT[c] = acc;
 }
 
-// buckets of more than kBucket slots: a wave per cell (see cell_ranks)
+// a wave per cell (see cell_ranks)
 __global__ __launch_bounds__(kBlock) void k_deposit_bucket_wave(GridView g, DepositView d, BucketView b,
                                                                 int ncell) {
   __shared__ double s_val[kBlock / 64][2][kWaveCellMax];
@@ -1983,10 +1976,10 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket_wave(GridView g, Depo
   const int n = b.count[c];
   if (n == 0) return;
   if (lane == 0) {
-    b.count[c] = 0;
-    if (n > b.cap) b.queue[atomicAdd(b.nqueue, 1)] = c;
+    if (n > kWaveCellMax) b.queue[atomicAdd(b.nqueue, 1)] = c;  // (the count is left to the queue)
+    else b.count[c] = 0;
   }
-  if (n > b.cap) return;
+  if (n > kWaveCellMax) return;
   cell_sum_wave(g, d, c, b.items + static_cast<size_t>(c) * b.cap, n, lane, s_val[wv][0], s_val[wv][1]);
 }
 
@@ -1994,12 +1987,17 @@ __global__ __launch_bounds__(kBlock) void k_deposit_bucket_wave(GridView g, Depo
 // blocks 1..: the queued cells
 __global__ __launch_bounds__(1024) void k_deposit_finish(DepositTail t, GridView g) {
   __shared__ double sh[1024];
-  __shared__ unsigned long long hits[16];
+  __shared__ QueueShared qs;
+  const int nq = *t.b.nqueue;
   if (blockIdx.x == 0) {
     energy_reduce(t.d.partial, t.nblocks, t.E_local, t.Ee, sh);
-    if (threadIdx.x == 0 && *t.b.nqueue > t.b.limit) *t.b.crowded = 1;
+    if (threadIdx.x == 0) {
+      if (nq > kQueueEach * kQueueBlocks) *t.b.state = kCrowded;
+      else if (nq == 0) *t.b.state = kCalm;
+    }
   } else {
-    deposit_queued(t, g, blockIdx.x - 1, gridDim.x - 1, hits);
+    for (int q = blockIdx.x - 1; q < nq; q += gridDim.x - 1)
+      queued_cell(t.a, t.d, t.b, g, t.b.queue[q], t.b.queue[q], 0, t.a.nlocal, qs);
   }
 }
 
@@ -2413,18 +2411,18 @@ __global__ __launch_bounds__(1024) void k_deposit_finish_batch(DepositTail t, co
                                                                const int* __restrict__ chunk0,
                                                                const int* __restrict__ nchunks, int nrep) {
   __shared__ double sh[1024];
-  __shared__ unsigned long long hits[16];
+  __shared__ QueueShared qs;
   const int nq = *t.b.nqueue;
   if (static_cast<int>(blockIdx.x) < nrep) {
     const int r = blockIdx.x;
     energy_reduce(t.d.partial + 2 * chunk0[r], nchunks[r], t.E_local + r, t.Ee + r, sh);
-    if (r == 0 && threadIdx.x == 0 && nq > t.b.limit) *t.b.crowded = 1;
+    if (r == 0 && threadIdx.x == 0 && nq > kQueueEach * kQueueBlocks) *t.b.state = kCrowded;
     return;
   }
   for (int q = blockIdx.x - nrep; q < nq; q += gridDim.x - nrep) {
     const int c = t.b.queue[q], r = cell_rep[c];
     const Chunk first = chunks[chunk0[r]], last = chunks[chunk0[r] + nchunks[r] - 1];
-    queued_cell(t.a, t.d, grids[r], c - cell_off[r], first.start, last.start + last.count, hits);
+    queued_cell(t.a, t.d, t.b, grids[r], c - cell_off[r], c, first.start, last.start + last.count, qs);
   }
 }
 
@@ -3069,7 +3067,7 @@ hipError_t launch_deposit_cells(const GridView& g, const DepositView& d, int n_i
 
 // the cells' sums of the bucketed deposit (g: the grid, or a batch's as one)
 static void bucket_cells(const GridView& g, const DepositView& d, const BucketView& b, int G, hipStream_t s) {
-  if (b.cap == kBucket) k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, d, b, G);
+  if (b.thread) k_deposit_bucket_cells<<<nblk(G), kBlock, 0, s>>>(g, d, b, G);
   else k_deposit_bucket_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, d, b, G);
 }
 
