@@ -12,10 +12,14 @@ pytestmark = pytest.mark.gpu
 
 
 # deposit: a wave per cell (38 atoms per cell on average), counted (378), a thread per cell; solve: one material
-# in 4096 and 4097+ cells, per-cell materials in 1728 and 2197; no solve, no random part, no kick
+# in 4096 and 4097+ cells, per-cell materials in 1728 and 2197; no solve, no random part, no kick; odd and even
+# numbers of sub-steps that go through both buffers
 @pytest.mark.parametrize("cells,grids,flags,file", [
+    ((4, 4), (17, 17), "7", False), ((4, 5), (17, 18), "7", 18), ((4, 5), (17, 18), "7", 19),
+    ((4, 5), (17, 18), "7", 20),
     ((4, 5, 6), (2, 2, 3), "7", True), ((4, 5), (1, 1), "7", False), ((4, 5), (17, 6), "7", False),
-    ((4, 6), (16, 3), "7", False), ((4, 5), (12, 2), "7", True), ((4, 5), (13, 6), "7", True),
+    ((4, 6), (16, 3), "7", False), ((4, 5), (12, 2), "7", "mixed"), ((4, 5), (13, 6), "7", "mixed"),
+    ((4, 5), (9, 6), "7", "mixed"),
     ((4, 5), (4, 4), "3", True), ((4, 5), (4, 4), "5", True), ((4, 5), (4, 4), "6", True),
     ((4, 5), (4, 4), "15", True)])
 @pytest.mark.parametrize("graph", [True, False])
@@ -23,7 +27,13 @@ def test_batch_forms_match_separate_runs(tmp_path, cells, grids, flags, file, gr
     species, dt, nsteps = 1, 5e-4, 12
     reps = []
     for k, (n, g) in enumerate(zip(cells, grids)):
-        beta, names, tin = workload_files(str(tmp_path), f"r{k}", species, n, A, g, hot_spot=(2000.0, 4.0))
+        beta, names, tin = workload_files(str(tmp_path), f"r{k}", species, n, A, g, hot_spot=(2000.0, 4.0),
+                                          steps=int(file) if isinstance(file, int) and file else 1)
+        if file == "mixed":  # another kappa in every third cell
+            lines = open(tin).read().split("\n")
+            lines[8::3] = [ln.replace(" 0.1 1 0", " 0.05 1 0") for ln in lines[8::3]]
+            assert " 0.05 1 0" in lines[8]
+            open(tin, "w").write("\n".join(lines))
         if k > 0:
             beta = reps[0][1][16]
         kw = dict(T_infile=tin) if file else {}

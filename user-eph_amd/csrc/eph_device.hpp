@@ -245,7 +245,6 @@ struct Chunk {
 };
 
 // ---- launch wrappers (eph_kernels.hip) ----
-hipError_t launch_ghost_xv(const AtomsView& a, const int* owner, const double4* shift, hipStream_t s);
 // the ghost update and, with check, the density sweep's candidate check of all
 // atoms (w.cand_checked then says so to the sweep)
 hipError_t launch_ghost_check(const AtomsView& a, const WorkView& w, bool check, unsigned long long* t,

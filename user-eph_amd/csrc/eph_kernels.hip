@@ -15,26 +15,6 @@
 namespace eph {
 
 
-// ---------------------------------------------------------------- comm
-__global__ __launch_bounds__(kBlock) void k_ghost_xv(AtomsView a, const int* __restrict__ owner,
-                                                     const double4* __restrict__ shift) {
-  const int g = blockIdx.x * kBlock + threadIdx.x;
-  if (g >= a.nghost) return;
-  const int o = owner[g];
-  const double4 p = a.pos[o];
-  const double4 s = shift[g];
-  const double4 x = make_double4(p.x + s.x, p.y + s.y, p.z + s.z, p.w);
-  const double4 v = a.vel[o];
-  a.pos[a.nlocal + g] = x;
-  a.vel[a.nlocal + g] = v;
-  if (a.pv) {
-    PosVel q;
-    q.p = x;
-    q.v = v;
-    a.pv[a.nlocal + g] = q;
-  }
-}
-
 // CSR -> transposed ELL; an index outside [0, nall) raises *bad and is stored
 // as 0, so that the list never addresses outside the atom arrays
 __global__ __launch_bounds__(kBlock) void k_csr_to_ell(int nlocal, const int* __restrict__ off,
@@ -652,7 +632,7 @@ __global__ __launch_bounds__(kBlock) void k_cand_check(int nall, const double4* 
   if (i < nall) cand_check_atom(i, pos[i], pos[i].w, w);
 }
 
-// The ghost update (k_ghost_xv) and, with check, the candidate check of all
+// The ghost update and, with check, the candidate check of all
 // atoms at the positions it leaves
 __global__ __launch_bounds__(kBlock) void k_ghost_check(AtomsView a, WorkView w, int check,
                                                         unsigned long long* t) {
@@ -778,6 +758,7 @@ __global__ __launch_bounds__(BLK) void k_density_w_lds(AtomsView a, TablesView t
   }
 }
 
+// ---------------------------------------------------------------- comm
 // forward communication of rho, w (fix_eph.cpp:743-744, 870-871) and xi
 // (:863-864) on one process: ghost <- owner, next to the ghost's own position
 __device__ __forceinline__ void ghost_rec(const int g, const AtomsView& a, const WorkView& w) {
@@ -2723,12 +2704,6 @@ static inline int nblk(long n, int b = kBlock) { return static_cast<int>((n + b 
 static int split_density(int nlocal) { return nlocal <= 8192 ? 16 : nlocal <= 400000 ? 4 : 0; }
 static int split_force(int nlocal) { return nlocal <= 20000 ? 16 : nlocal <= 50000 ? 8 : 0; }
 constexpr int kSplitLj16 = 16384;
-
-hipError_t launch_ghost_xv(const AtomsView& a, const int* owner, const double4* shift, hipStream_t s) {
-  if (a.nghost == 0) return hipSuccess;
-  k_ghost_xv<<<nblk(a.nghost), kBlock, 0, s>>>(a, owner, shift);
-  return hipGetLastError();
-}
 
 hipError_t launch_ghost_check(const AtomsView& a, const WorkView& w, bool check, unsigned long long* t,
                               hipStream_t s) {
