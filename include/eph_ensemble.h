@@ -13,11 +13,13 @@
  *   - the fix sweeps run over chunks of <= 256 atoms of one replica, so each
  *     replica's noise stream (seed, tag, step), T_e cell lookup and energy
  *     partial sums are those of a separate run;
- *   - the T_e grids are concatenated and advanced by one stencil launch per
- *     sub-step (replicas with fewer sub-steps copy); with temperature-
+ *   - the T_e grids are concatenated and advanced by a workgroup per replica
+ *     (up to 4096 cells each, 2048 of several materials) or one stencil launch
+ *     per sub-step (replicas with fewer sub-steps copy); with temperature-
  *     dependent C_e(T), kappa(T) the counts are found on the device each step
  *     and the host reads the largest before the stencil launches;
- *   - the whole step can be recorded once as a hipGraph and replayed.
+ *   - the step behind the check of the lists can be recorded once as a hipGraph
+ *     and replayed.
  * Neighbour rebuilds are collective: when any atom of any replica has moved
  * more than skin/2, every replica rebuilds (the steps are logged, so a
  * separate run forced to rebuild at the same steps reproduces a replica bit
@@ -52,9 +54,9 @@ int eph_ensemble_add(eph_ensemble* e, const eph_md_config* cfg, int narg, const 
  * initial pair forces.  The first step run is first_step. */
 int eph_ensemble_setup(eph_ensemble* e, long long first_step);
 
-/* nsteps Verlet steps of every replica (use_graph: record the step once as a
- * hipGraph and replay it).  *ms receives the device time of the steps;
- * rebuilt[k] (nsteps entries, may be NULL) is 1 when step first + k rebuilt. */
+/* nsteps Verlet steps of every replica (use_graph: record the step behind the
+ * check of the lists once as a hipGraph and replay it).  *ms receives the
+ * device time of the steps; rebuilt[k] (nsteps entries, may be NULL) is 1 when step first + k rebuilt. */
 int eph_ensemble_run(eph_ensemble* e, int nsteps, int use_graph, double* ms, int* rebuilt);
 
 /* Forms of the density and force sweeps, numbered as eph_set_sweep_forms
