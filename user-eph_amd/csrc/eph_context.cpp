@@ -153,7 +153,8 @@ int eph_grid::insert_points(int n, const double* x, const double* y, const doubl
   EPH_HIP(this, dep.reserve(n, G, nblocks_of(n)));
   const size_t b = n * sizeof(double);
   const double* src[4] = {x, y, z, E};
-  double* a = arena.take(4 * b);
+  const PinnedArena::Use mem = arena.use(4 * b);
+  double* a = mem.get();
   if (!a) EPH_HIP(this, pts.reserve(4 * (size_t)n));
   for (int k = 0; k < 4; ++k) {
     if (a) std::memcpy(a + (size_t)k * n, src[k], b);
@@ -171,7 +172,8 @@ int eph_grid::insert_points(int n, const double* x, const double* y, const doubl
 // through pinned memory where the result is small; the runtime's own copy into
 // pageable memory otherwise
 static hipError_t read_device(PinnedArena& arena, const void* src, void* dst, size_t bytes, hipStream_t s) {
-  double* p = arena.take(bytes);
+  const PinnedArena::Use mem = arena.use(bytes);
+  double* p = mem.get();
   hipError_t e = hipMemcpyAsync(p ? p : dst, src, bytes, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e == hipSuccess && p) std::memcpy(dst, p, bytes);
@@ -758,13 +760,14 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
 
 int eph_context::check_flags() {
   int gf = 0;
-  int* st = reinterpret_cast<int*>(arena.take(sizeof(double)));
-  if (!grid || st) {
-    if (grid)
-      EPH_HIP(this, launch_hook_out(nullptr, nullptr, 0, nullptr, nullptr, 0, nullptr, 0, nullptr, 0, nullptr,
-                                    grid->nonfinite.p, st, stream));
+  if (!grid) {
     EPH_HIP(this, hipStreamSynchronize(stream));
-    if (grid) gf = st[1];
+  } else if (const PinnedArena::Use mem = arena.use(sizeof(double))) {
+    int* st = reinterpret_cast<int*>(mem.get());
+    EPH_HIP(this, launch_hook_out(nullptr, nullptr, 0, nullptr, nullptr, 0, nullptr, 0, nullptr, 0, nullptr,
+                                  grid->nonfinite.p, st, stream));
+    EPH_HIP(this, hipStreamSynchronize(stream));
+    gf = st[1];
   } else if (int rc = read(grid->nonfinite.p, &gf, sizeof gf)) {
     return rc;
   }
@@ -1128,8 +1131,8 @@ static int upload_force(eph_context* c, const double* f) {
 }
 
 // With timing on the hooks keep the launches that the report names.
-static double* hook_arena(eph_context* c, size_t doubles) {
-  return c->timing ? nullptr : c->arena.take(doubles * sizeof(double));
+static PinnedArena::Use hook_arena(eph_context* c, size_t doubles) {
+  return c->timing ? PinnedArena::Use() : c->arena.use(doubles * sizeof(double));
 }
 
 int eph_initial_integrate(eph_context* ctx, double* x, double* v, const double* f) {
@@ -1138,7 +1141,8 @@ int eph_initial_integrate(eph_context* ctx, double* x, double* v, const double* 
   if (ctx->flags & EPH_NOINT) return EPH_OK;
   int rc;
   const size_t n3 = 3 * (size_t)ctx->nlocal, b = n3 * sizeof(double);
-  if (double* p = hook_arena(ctx, 5 * n3)) {
+  if (const auto mem = hook_arena(ctx, 5 * n3)) {
+    double* p = mem.get();
     ctx->pv_fresh = false;
     std::memcpy(p, x, b); std::memcpy(p + n3, v, b); std::memcpy(p + 2 * n3, f, b);
     EPH_HIP(ctx, launch_hook_kick(ctx->atoms_view(), ctx->step_params(), true, p, p + n3, p + 2 * n3,
@@ -1164,7 +1168,8 @@ int eph_post_force(eph_context* ctx, const double* x, const double* v, double* f
   const int nall = ctx->nlocal + ctx->nghost;
   int rc;
   const size_t n3 = 3 * (size_t)ctx->nlocal, a3 = 3 * (size_t)nall;
-  if (double* p = nall ? hook_arena(ctx, 2 * a3 + 2 * n3 + 1) : nullptr) {
+  if (const auto mem = nall ? hook_arena(ctx, 2 * a3 + 2 * n3 + 1) : PinnedArena::Use()) {
+    double* p = mem.get();
     std::memcpy(p, x, a3 * sizeof(double));
     std::memcpy(p + a3, v, a3 * sizeof(double));
     std::memcpy(p + 2 * a3, f, n3 * sizeof(double));
@@ -1205,7 +1210,8 @@ int eph_final_integrate(eph_context* ctx, double* v, const double* f) {
   if (ctx->flags & EPH_NOINT) return EPH_OK;
   int rc;
   const size_t n3 = 3 * (size_t)ctx->nlocal, b = n3 * sizeof(double);
-  if (double* p = hook_arena(ctx, 3 * n3)) {
+  if (const auto mem = hook_arena(ctx, 3 * n3)) {
+    double* p = mem.get();
     ctx->pv_fresh = false;
     std::memcpy(p, v, b); std::memcpy(p + n3, f, b);
     EPH_HIP(ctx, launch_hook_kick(ctx->atoms_view(), ctx->step_params(), false, nullptr, p, p + n3,
@@ -1227,13 +1233,14 @@ int eph_end_of_step(eph_context* ctx, const double* x, const double* v, long lon
   if (!ctx->have_atoms) return ctx->fail(EPH_ERR_STATE, "no atoms");
   int rc;
   const size_t n3 = 3 * (size_t)ctx->nlocal;
-  if (double* p = n3 ? hook_arena(ctx, 2 * n3) : nullptr) {
+  if (const auto mem = hook_arena(ctx, 2 * n3)) {
+    double* p = mem.get();
     ctx->pv_fresh = false;
     std::memcpy(p, x, n3 * sizeof(double));
     std::memcpy(p + n3, v, n3 * sizeof(double));
     EPH_HIP(ctx, launch_hook_in(p, p + n3, ctx->nlocal, nullptr, 0, ctx->pos.p, ctx->vel.p, nullptr, nullptr, 0,
                                 ctx->stream));
-    EPH_HIP(ctx, ctx->arena.mark(ctx->stream));
+    EPH_HIP(ctx, ctx->arena.mark(mem, ctx->stream));
   } else {
     if ((rc = upload_rows(ctx, x, ctx->nlocal, ctx->pos.p))) return rc;
     if ((rc = upload_rows(ctx, v, ctx->nlocal, ctx->vel.p))) return rc;
@@ -1460,7 +1467,8 @@ int eph_dev_get_atoms(eph_context* ctx, double* x, double* v, double* f) {
   const int nall = ctx->nlocal + ctx->nghost;
   int rc;
   const size_t n3 = 3 * (size_t)ctx->nlocal, a3 = 3 * (size_t)nall;
-  if (double* p = nall ? ctx->arena.take((2 * a3 + n3) * sizeof(double)) : nullptr) {
+  if (const auto mem = ctx->arena.use((2 * a3 + n3) * sizeof(double))) {
+    double* p = mem.get();
     EPH_HIP(ctx, launch_hook_out(ctx->pos.p, p, x ? nall : 0, ctx->vel.p, p + a3, v ? nall : 0, ctx->f.p,
                                  ctx->fstride, p + 2 * a3, f ? ctx->nlocal : 0, nullptr, nullptr, nullptr,
                                  ctx->stream));

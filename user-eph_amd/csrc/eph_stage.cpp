@@ -24,9 +24,12 @@ PinnedArena::~PinnedArena() {
   if (p_) (void)hipHostFree(p_);
 }
 
-double* PinnedArena::take(size_t bytes) {
-  if (bytes > kMax || failed_) return nullptr;
-  if (busy_ && hipEventSynchronize(ev_) != hipSuccess) return nullptr;
+PinnedArena::Use PinnedArena::use(size_t bytes) {
+  Use u;
+  if (bytes == 0 || bytes > kMax) return u;
+  std::unique_lock<std::mutex> lock(m_);
+  if (failed_) return u;
+  if (busy_ && hipEventSynchronize(ev_) != hipSuccess) return u;
   busy_ = false;
   if (bytes > n_) {
     if (p_) (void)hipHostFree(p_);
@@ -40,14 +43,16 @@ double* PinnedArena::take(size_t bytes) {
       (void)hipGetLastError();
       p_ = nullptr;
       failed_ = true;
-      return nullptr;
+      return u;
     }
     n_ = want;
   }
-  return reinterpret_cast<double*>(p_);
+  u.lock_ = std::move(lock);
+  u.p_ = reinterpret_cast<double*>(p_);
+  return u;
 }
 
-hipError_t PinnedArena::mark(hipStream_t s) {
+hipError_t PinnedArena::mark(const Use&, hipStream_t s) {
   const hipError_t e = hipEventRecord(ev_, s);
   busy_ = e == hipSuccess;
   return e;

@@ -18,24 +18,37 @@ namespace eph {
 // Pinned host memory for the arrays of small calls.  The kernels read and
 // write it in place, so that a call with several arrays takes one memcpy per
 // array, one launch and one wait instead of a copy operation with a wait of
-// its own per array (15 to 25 us each).  One caller at a time, as the context
-// or grid that owns it.
+// its own per array (15 to 25 us each).  A call holds the arena from use() until
+// its Use goes, so calls of several threads on one context or grid (a monitor
+// that reads values while another thread steps) take turns: without that, one
+// call's copy in would land in another's arrays.
 class PinnedArena {
  public:
-  // Beyond this many bytes the copies dominate and the runtime's or the
-  // stager's DMA is as fast as one thread's memcpy.
+  // Beyond this many bytes the calls take the runtime's or the stager's copies.
   static constexpr size_t kMax = size_t(1) << 20;
+  // memory for one call, free to be written; empty when bytes > kMax or no
+  // pinned memory is to be had
+  class Use {
+   public:
+    Use() = default;
+    double* get() const { return p_; }
+    explicit operator bool() const { return p_ != nullptr; }
+
+   private:
+    friend class PinnedArena;
+    std::unique_lock<std::mutex> lock_;
+    double* p_ = nullptr;
+  };
   PinnedArena() = default;
   PinnedArena(const PinnedArena&) = delete;
   PinnedArena& operator=(const PinnedArena&) = delete;
   ~PinnedArena();
-  // memory for one call, free to be written; null when bytes > kMax or no
-  // pinned memory is to be had
-  double* take(size_t bytes);
-  // the work queued on s so far still reads it after the call returns
-  hipError_t mark(hipStream_t s);
+  Use use(size_t bytes);
+  // the work queued on s so far still reads the memory in use after it is given back
+  hipError_t mark(const Use&, hipStream_t s);
 
  private:
+  std::mutex m_;
   char* p_ = nullptr;
   size_t n_ = 0;
   hipEvent_t ev_ = nullptr;
