@@ -94,3 +94,96 @@ def test_crowded_cells_match_oracle(oracle, tmp_path, cells, n, corner):
         ora.end_of_step(a, step)
         gpu.end_of_step(b, step)
         assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))
+
+
+def _fix_pair(oracle, tmp_path, cells, n):
+    import copy
+
+    import eph_amd as ea
+    from eph_amd import inputs
+    path = str(tmp_path / "b.beta")
+    names = inputs.workload_beta(path, 1)
+    md = ea.MD(cells, seed=9, T=900.0)
+    inf = md.info()
+    args = inputs.fix_args(path, names, seed=3, flags="7", grid=(n, n, n))
+    cons = (args, 1, inf["boxlo"], inf["boxhi"], 1e-3, inputs.BOLTZ, inputs.FTM2V)
+    ora = oracle.Fix(*cons, masses=[inputs.MASS_CU])
+    gpu = ea.FixEPH(*cons, masses=[inputs.MASS_CU])
+    gpu.init()
+    a = md.snapshot()
+    md.lj(a)
+    b = copy.deepcopy(a)
+    gpu.set_atoms(b)
+    ora.post_force(a, step=1)
+    gpu.post_force(b, step=1)
+    return md, ora, gpu, a, b
+
+
+def _fill_cells(x, n, L, counts, seed):
+    """the first atoms of x into some of the n^3 cells, counts[k] of them into the k-th"""
+    rng = np.random.default_rng(seed)
+    out, at = x.copy(), 0
+    for c, m in zip(rng.choice(n ** 3, len(counts), replace=False), counts):
+        lo = np.array([c % n, c // n % n, c // n ** 2]) * (L / n)
+        out[at:at + m] = lo + rng.uniform(0.02, 0.98, (m, 3)) * (L / n)
+        at += m
+    return out
+
+
+# cells that overflow after deposits that left the queue empty, so that the queue is the solve's: inside a one-workgroup
+# solve (up to 4096 cells) or by its own launch before the tiles (beyond); up to 6 queued cells and more; their atoms
+# out of the bucket (256 slots, 1024 with a wave per cell, 16 above 16,384 cells), out of bucket and chain, by a scan
+@pytest.mark.parametrize("cells,n,counts", [
+    (8, 8, [17]), (8, 8, [20, 40, 64, 100, 256, 30]), (8, 8, [18] * 7), (8, 8, [25] * 20),
+    (10, 9, [257, 300, 319]), (10, 9, [330, 700]), (10, 9, [40, 260, 900, 25, 17, 16, 33, 34]),
+    (10, 8, [260, 1000]), (12, 8, [1025, 1080, 1100]), (12, 8, [270] * 8),
+    (12, 17, [17, 40, 300, 900]), (12, 17, [20] * 9), (10, 26, [17, 40, 79, 500]), (10, 16, [20, 300, 500])])
+def test_queue_left_to_the_solve_matches_oracle(oracle, tmp_path, cells, n, counts):
+    md, ora, gpu, a, b = _fix_pair(oracle, tmp_path, cells, n)
+    L, nl = md.info()["boxhi"][0], a.nlocal
+    calm = a.x[:nl].copy()
+    step = 0
+    for x in (calm, calm, "fill", "fill", calm, calm, "fill"):
+        step += 1
+        for s in (a, b):  # the deposit sees these positions only
+            s.x[:nl] = _fill_cells(calm, n, L, counts, step) if isinstance(x, str) else x
+        ora.end_of_step(a, step)
+        gpu.end_of_step(b, step)
+        assert np.array_equal(gpu.grid().get("T"), ora.fdm().get("T"))
+        assert gpu.compute_vector(0) == pytest.approx(ora.compute_vector(0), rel=1e-12)
+
+
+def _forms(md, fix, steps):
+    """in how many of the harness's steps the deposit was bucketed (it then takes the final kick along)"""
+    fix.timing(True)
+    md.run(fix, steps)
+    report = fix.timing_report()
+    fix.timing(False)
+    return report.get("final_integrate+deposit", (0.0, 0))[1]
+
+
+# a crowded deposit (900 cells past their buckets; scans over 32,000 atoms for cells of 400), then atoms that are not:
+# the deposit after the first counted one is bucketed again
+@pytest.mark.parametrize("n,corner", [(24, 0.5), (30, 0.2)])
+def test_buckets_return_after_a_crowded_deposit(oracle, tmp_path, n, corner):
+    md, _, gpu, _, b = _fix_pair(oracle, tmp_path, 20, n)
+    md.attach(gpu)
+    assert _forms(md, gpu, 3) == 3
+    x = np.random.default_rng(1).uniform(0.0, corner, (b.nlocal, 3)) * md.info()["boxhi"][0]
+    x[:300] *= 0.4
+    for step in (1, 2, 3):
+        b.x[:b.nlocal] = x
+        gpu.end_of_step(b, step)
+    md.attach(gpu)
+    assert _forms(md, gpu, 3) == 2
+
+
+# 20 queued cells in a one-workgroup solve do not turn the next deposits to the counted form
+def test_a_few_queued_cells_keep_the_buckets(oracle, tmp_path):
+    md, _, gpu, a, b = _fix_pair(oracle, tmp_path, 8, 8)
+    x = a.x[:a.nlocal].copy()
+    for step in (1, 2, 3):
+        b.x[:b.nlocal] = x if step < 3 else _fill_cells(x, 8, md.info()["boxhi"][0], [25] * 20, 1)
+        gpu.end_of_step(b, step)
+    md.attach(gpu)
+    assert _forms(md, gpu, 2) == 2

@@ -49,3 +49,21 @@ def test_batch_forms_match_separate_runs(tmp_path, cells, grids, flags, file, gr
         assert np.array_equal(ens.get(r, "x"), xs[:n]) and np.array_equal(ens.get(r, "v"), vs[:n])
         assert np.array_equal(ens.get(r, "T"), fix.grid().get("T"))
         assert ens.get(r, "E")[1] == fix.compute_vector(0)
+
+
+# grids finer than the lattice planes: 64 atoms in each of 512 cells and none in most (3 a cell on average), so the
+# first deposits are crowded and the next counted ones; the planes then spread and the buckets serve again
+@pytest.mark.parametrize("graph", [True, False])
+def test_batch_deposit_through_crowded_steps(tmp_path, graph):
+    beta, names, _ = workload_files(str(tmp_path), "c", 1, 8, A, 4)
+    reps = [(dict(cells=8, a=A, ntypes=1, seed=30 + r, T=2000.0),
+             inputs.fix_args(beta, names, seed=50 + r, flags="7", grid=(400, 2, 1), kappa=1e-7)) for r in range(16)]
+    ens = _ensemble(reps, 1, 5e-4)
+    rebuilt = np.concatenate([ens.run(n, graph=graph)["rebuilt"] for n in (2, 8, 30, 30)])
+    for r, (kw, args) in enumerate(reps):
+        md, fix = _separate(kw, args, 1, 5e-4, rebuilt)
+        xs, vs, _ = fix.dev_atoms()
+        n = ens.info(r)["nlocal"]
+        assert np.array_equal(ens.get(r, "x"), xs[:n]) and np.array_equal(ens.get(r, "v"), vs[:n])
+        assert np.array_equal(ens.get(r, "T"), fix.grid().get("T"))
+        assert ens.get(r, "E")[1] == fix.compute_vector(0)

@@ -728,7 +728,7 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
     DepositView d = grid->dep.view(true);
     BucketView b;
     b.cap = cap;
-    b.thread = nlocal <= kThreadCells * static_cast<double>(G);
+    b.thread = bucket_limit(nlocal, static_cast<double>(G)) == kBucket;
     b.head = grid->bhead.p; b.next = grid->bnext.p;
     b.count = grid->bcount.p; b.items = grid->bitems.p; b.queue = grid->bqueue.p; b.nqueue = grid->bnq.p;
     b.state = grid->bstate;
@@ -749,7 +749,15 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
     DepositView dc = d;
     if (!fric) dc.v1 = nullptr;
     if (!rnd) dc.v2 = nullptr;
-    EPH_HIP(this, launch_deposit_cells(grid->v, dc, nlocal, grid->dep.qbuf.p, stream));
+    CrowdCheck cc;
+    if (grid->bstate) {  // buckets were crowded: look whether they still would be
+      cc.cap = bucket_slots(nlocal, static_cast<double>(G));
+      cc.limit = bucket_limit(nlocal, static_cast<double>(G));
+      cc.atoms = nlocal;
+      cc.state = grid->bstate;
+      cc.count = cc.cap ? grid->bnq.p : nullptr;
+    }
+    EPH_HIP(this, launch_deposit_cells(grid->v, dc, nlocal, grid->dep.qbuf.p, stream, cc));
     EPH_HIP(this, launch_energy_reduce(d, nb, scal.p, scal.p + (defer_tally ? 2 : 1), stream));
     timed_end("deposit", e);
   } else {

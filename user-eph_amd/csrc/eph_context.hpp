@@ -53,9 +53,9 @@ struct eph_grid {
   eph::DepositBuffers dep;
   // per-cell buckets of the deposit (count kept at zero between steps)
   eph::DevArray<int> bcount, bitems, bhead, bnext, bqueue, bnq;
-  // Pinned: how the last bucketed deposit went (BucketView::state).  After a
-  // crowded one the deposits are counted ones; a plan only, as both forms give
-  // the same bits, so it is read without a wait.
+  // Pinned: how the last deposit went (BucketView::state).  After a crowded one
+  // the next is a counted one; a plan only, as both forms give the same bits, so
+  // it is read without a wait.
   int* bstate = nullptr;
   int bucket_bytes_ok(size_t G, int cap, int n);  // reserves buckets of cap slots for n atoms; 0 when they are ready
   eph::PinnedArena arena;  // small calls

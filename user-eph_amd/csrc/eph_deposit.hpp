@@ -37,11 +37,13 @@ static __device__ __forceinline__ double add_lanes(double acc, double v, int n) 
 // every 512 atoms (or beyond the LDS) an ordered scan over the atoms [i0, i1) is
 // the faster: every wave ballots the atoms of the cell among its 64, and
 // thread 0 adds their values.  32,000 atoms in an eighth of 24^3 cells, some 900
-// cells queued: 0.6 ms a step with its
-// host calls, 9.7 with a scan each.
+// cells queued: 0.6 ms a step with its host calls, 9.7 with a scan each.
 // A scan of more than kQueueScan atoms (3 us per 1024) costs as much as the counted
 // form does.
 constexpr int kQueueItems = 4096, kQueueScan = 16384;
+static __device__ __forceinline__ bool queue_walks(const int n, const int cap, const int atoms) {
+  return n <= kQueueItems && (n - cap <= 64 || n - cap <= atoms / 512);
+}
 struct QueueShared {
   int key[kQueueItems];
   unsigned long long hits[16];
@@ -52,8 +54,8 @@ __device__ __forceinline__ void queued_cell(const AtomsView& a, const DepositVie
                                             const GridView& g, const int c, const int cb, const int i0,
                                             const int i1, QueueShared& sh) {
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int n = b.count[cb], held = min(n, b.cap), links = n - held;
-  const bool walk = n <= kQueueItems && (links <= 64 || links <= (i1 - i0) / 512);
+  const int n = b.count[cb], held = min(n, b.cap);
+  const bool walk = queue_walks(n, b.cap, i1 - i0);
   __syncthreads();  // count read by all, and the last cell's LDS
   if (threadIdx.x == 0) {
     int j = b.head[cb];

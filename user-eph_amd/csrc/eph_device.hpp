@@ -179,11 +179,14 @@ inline int bucket_slots(double n, double G) {
   if (n <= kThreadCells * G) return small ? kWaveCellMax : kBucket;
   return small ? 4 * kWaveCellMax : kWaveCellMax;
 }
+// atoms up to which the cells' sums take a cell themselves
+inline int bucket_limit(double n, double G) { return n <= kThreadCells * G ? kBucket : kWaveCellMax; }
 // A queued cell takes a workgroup 5 to 10 us; kQueueBlocks share them.  Beyond
 // kQueueEach of them per block the counted form (some 45 us more than the
-// bucketed one) is the faster, and the device says so in *state.  A
-// one-workgroup T_e solve takes the queue over only after a deposit that left
-// it empty.
+// bucketed one) is the faster, and the device says so in *state: every deposit,
+// in whichever form, leaves there what the next one should take.  A one-workgroup
+// T_e solve takes the queue over only after a deposit that left it empty, and
+// gives it back once it found more than kQueueEach cells in it.
 constexpr int kQueueBlocks = 64, kQueueEach = 6;
 constexpr int kCrowded = 1, kCalm = 2;
 struct BucketView {
@@ -195,7 +198,7 @@ struct BucketView {
   int* next = nullptr;    // [atoms], the chain
   int* queue = nullptr;   // [G]
   int* nqueue = nullptr;  // [1]
-  int* state = nullptr;   // pinned host memory: kCrowded, kCalm, or 0 at first
+  int* state = nullptr;   // pinned host memory: kCrowded, kCalm, or 0
 };
 
 // What is left of the bucketed deposit after the cells' sums: the tally from
@@ -243,6 +246,21 @@ constexpr int kLdsMinAtoms = 32768;
 struct Chunk {
   int rep, start, count, pad;
 };
+
+// A counted deposit in place of a crowded bucketed one: what the buckets would
+// have left to the queue is counted, so that *state says when they serve again.
+struct CrowdCheck {
+  int* count = nullptr;  // null: no check.  Cells past limit; kCrowdLong: one of them would be scanned for
+  int* state = nullptr;  // as BucketView's
+  int cap = 0, limit = 0;
+  int atoms = 0;
+  // a batch: the atoms of a cell's replica instead
+  const int* cell_rep = nullptr;
+  const Chunk* chunks = nullptr;
+  const int* chunk0 = nullptr;
+  const int* nchunks = nullptr;
+};
+constexpr int kCrowdLong = 1 << 30;
 
 // ---- launch wrappers (eph_kernels.hip) ----
 // the ghost update and, with check, the density sweep's candidate check of all
@@ -307,7 +325,7 @@ hipError_t launch_deposit_points(int n, const double* x, const double* y, const 
 // qbuf: 2 + 2 G ints of queue space for cells holding more than
 // kMaxSortInCell items.  d.count must hold the per-cell counts.
 hipError_t launch_deposit_cells(const GridView& g, const DepositView& d, int n_items, int* qbuf,
-                                hipStream_t s);
+                                hipStream_t s, const CrowdCheck& cc = CrowdCheck());
 // the whole deposit and tally through per-cell buckets (fric / rand: which
 // parts); with kick, the final velocity-Verlet kick of the group's atoms
 // first, in the same pass.  b.count must be zero on entry and is left zero.

@@ -68,7 +68,7 @@ struct eph_ensemble {
   int* pinned = nullptr;  // [0] largest sub-step count, [1] lists to be rebuilt
   DepositBuffers dep;
   // bucketed deposit: slots per cell (0: counted), the buckets, and the pinned
-  // flag that the device sets when too many cells overflowed theirs
+  // word that says how the last deposit went (BucketView::state)
   int slots = 0;
   DevArray<int> bk_count, bk_items, bk_head, bk_next, bk_queue, bk_nq;
   int* bk_state = nullptr;
@@ -412,7 +412,7 @@ int eph_ensemble::enqueue_step() {
   if (buckets) {
     BucketView b;
     b.cap = slots;
-    b.thread = nl <= kThreadCells * G;
+    b.thread = bucket_limit(nl, G) == kBucket;
     b.head = bk_head.p; b.next = bk_next.p;
     b.count = bk_count.p; b.items = bk_items.p; b.queue = bk_queue.p; b.nqueue = bk_nq.p;
     b.state = bk_state;
@@ -426,7 +426,13 @@ int eph_ensemble::enqueue_step() {
     DepositView dc = d;
     if (!fric) dc.v1 = nullptr;
     if (!rnd) dc.v2 = nullptr;
-    EPH_HIP(this, launch_deposit_cells(gall, dc, nl, dep.qbuf.p, s));
+    CrowdCheck cc;
+    if (slots) {
+      cc.count = bk_nq.p; cc.state = bk_state;
+      cc.cap = slots; cc.limit = bucket_limit(nl, G);
+      cc.cell_rep = cell_rep.p; cc.chunks = chunks.p; cc.chunk0 = chunk0.p; cc.nchunks = nchunks.p;
+    }
+    EPH_HIP(this, launch_deposit_cells(gall, dc, nl, dep.qbuf.p, s, cc));
     EPH_HIP(this, launch_energy_reduce_batch(d.partial, chunk0.p, nchunks.p, R, E_local.p, Ee.p, s));
   } else {
     EPH_HIP(this, launch_fill_double(E_local.p, R, 0.0, s));

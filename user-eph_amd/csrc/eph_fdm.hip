@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kFdmThreads) void k_fdm_block(GridView g, FdmArgs u
     __shared__ QueueShared qs;
     energy_reduce(tail.d.partial, tail.nblocks, tail.E_local, tail.Ee, sh);
     const int nq = *tail.b.nqueue;
-    if (threadIdx.x == 0 && nq > kQueueEach) *tail.b.state = kCrowded;
+    if (threadIdx.x == 0 && nq > kQueueEach) *tail.b.state = 0;  // (a cell below may make it kCrowded)
     for (int q = 0; q < nq; ++q)
       queued_cell(tail.a, tail.d, tail.b, g, tail.b.queue[q], tail.b.queue[q], 0, tail.a.nlocal, qs);
     __syncthreads();

@@ -1607,6 +1607,23 @@ __global__ __launch_bounds__(kBlock) void k_scatter(int n, DepositView d) {
   d.items[slot] = i;
 }
 
+// would the queue scan for the n atoms of cell c, and for too long
+static __device__ __forceinline__ bool crowd_long(const CrowdCheck& cc, const int c, const int n) {
+  if (n <= cc.limit) return false;
+  int atoms = cc.atoms;
+  if (cc.cell_rep) {
+    const int r = cc.cell_rep[c];
+    const Chunk last = cc.chunks[cc.chunk0[r] + cc.nchunks[r] - 1];
+    atoms = last.start + last.count - cc.chunks[cc.chunk0[r]].start;
+  }
+  return atoms > kQueueScan && !queue_walks(n, cc.cap, atoms);
+}
+
+__global__ void k_queue_reset(int* qbuf, int* crowd) {
+  if (threadIdx.x < 2) qbuf[threadIdx.x] = 0;
+  if (threadIdx.x == 2 && crowd) *crowd = 0;
+}
+
 // Per cell: dT_e[c] += v1 of its atoms in ascending atom order, then += v2 in
 // ascending order -- the serial order of the two loops of fix_eph.cpp:364-390.
 // Cells with up to kMaxSortInCell items sort them by insertion in place;
@@ -1614,8 +1631,14 @@ __global__ __launch_bounds__(kBlock) void k_scatter(int n, DepositView d) {
 // all items (huge).  d.count is reused as the queue: count[G] holds the
 // number of queued cells and the queue follows in fill[].
 __global__ __launch_bounds__(kBlock) void k_cell_sum_small(GridView g, DepositView d, int ncell,
-                                                           int* queue, int* qn) {
+                                                           int* queue, int* qn, CrowdCheck cc) {
   const int c = blockIdx.x * kBlock + threadIdx.x;
+  if (cc.count) {
+    const int m = c < ncell ? d.start[c + 1] - d.start[c] : 0;
+    const int past = __popcll(__ballot(m > cc.limit));
+    if (past && (threadIdx.x & 63) == 0) atomicAdd(cc.count, past);
+    if (crowd_long(cc, c, m)) atomicOr(cc.count, kCrowdLong);
+  }
   if (c >= ncell) return;
   const int s = d.start[c], n = d.start[c + 1] - s;
   if (n == 0) return;
@@ -1691,7 +1714,7 @@ static __device__ __forceinline__ void cell_sum_wave(const GridView& g, const De
 }
 
 __global__ __launch_bounds__(kBlock) void k_cell_sum_wave(GridView g, DepositView d, int ncell,
-                                                          int* queue, int* qn) {
+                                                          int* queue, int* qn, CrowdCheck cc) {
   __shared__ double s_val[kBlock / 64][2][kWaveCellMax];
   const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
   const int lane = threadIdx.x & 63;
@@ -1699,6 +1722,10 @@ __global__ __launch_bounds__(kBlock) void k_cell_sum_wave(GridView g, DepositVie
   if (c >= ncell) return;
   const int s = d.start[c], n = d.start[c + 1] - s;
   if (n == 0) return;
+  if (cc.count && lane == 0 && n > cc.limit) {
+    atomicAdd(cc.count, 1);
+    if (crowd_long(cc, c, n)) atomicOr(cc.count, kCrowdLong);
+  }
   if (n > kWaveCellMax) {
     if (lane == 0) queue[atomicAdd(qn, 1)] = c;
     return;
@@ -1712,8 +1739,10 @@ constexpr int kMedMax = 8192;
 // then the ordered sums; larger cells fall through to k_cell_sum_huge
 __global__ __launch_bounds__(kMedBlock) void k_cell_sum_medium(GridView g, DepositView d,
                                                                const int* queue, const int* qn,
-                                                               int* huge, int* hn) {
+                                                               int* huge, int* hn, CrowdCheck cc) {
   __shared__ int key[kMedMax];
+  if (cc.count && blockIdx.x == 0 && threadIdx.x == 0)
+    *cc.state = *cc.count > kQueueEach * kQueueBlocks ? kCrowded : 0;
   const int nq = *qn;
   for (int q = blockIdx.x; q < nq; q += gridDim.x) {
     const int c = queue[q];
@@ -3015,7 +3044,7 @@ hipError_t launch_deposit_points(int n, const double* x, const double* y, const 
 
 // count[] -> start[] -> items[] -> ordered per-cell sums into g.dT
 hipError_t launch_deposit_cells(const GridView& g, const DepositView& d, int n_items, int* qbuf,
-                                hipStream_t s) {
+                                hipStream_t s, const CrowdCheck& cc) {
   const int G = g.nx * g.ny * g.nz;
   const int per = kScanBlock * kScanItems;
   const int nb = (G + per - 1) / per;
@@ -3026,16 +3055,16 @@ hipError_t launch_deposit_cells(const GridView& g, const DepositView& d, int n_i
   // [2 + G ..] huge queue
   int* qn = qbuf;
   int* hn = qbuf + 1;
-  k_fill_int<<<1, 64, 0, s>>>(qbuf, 2, 0);
+  k_queue_reset<<<1, 64, 0, s>>>(qbuf, cc.count);
   k_fill_int<<<nblk(G), kBlock, 0, s>>>(d.fill, G, 0);
   if (n_items > 0) k_scatter<<<nblk(n_items), kBlock, 0, s>>>(n_items, d);
   int* queue = qbuf + 2;
   int* huge = qbuf + 2 + G;
   // a wave per cell from 6 items per cell on (below, most lanes would idle and
   // the cells are many: 491,520 cells of 0.4 items take 11 us a thread each)
-  if (n_items >= 6L * G) k_cell_sum_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, d, G, queue, qn);
-  else k_cell_sum_small<<<nblk(G), kBlock, 0, s>>>(g, d, G, queue, qn);
-  k_cell_sum_medium<<<64, kMedBlock, 0, s>>>(g, d, queue, qn, huge, hn);
+  if (n_items >= 6L * G) k_cell_sum_wave<<<nblk(G, kBlock / 64), kBlock, 0, s>>>(g, d, G, queue, qn, cc);
+  else k_cell_sum_small<<<nblk(G), kBlock, 0, s>>>(g, d, G, queue, qn, cc);
+  k_cell_sum_medium<<<64, kMedBlock, 0, s>>>(g, d, queue, qn, huge, hn, cc);
   k_cell_sum_huge<<<16, kBlock, 0, s>>>(g, d, n_items, huge, hn);
   return hipGetLastError();
 }
