@@ -31,6 +31,63 @@ hipError_t DepositBuffers::reserve(size_t n_items, size_t G, size_t nblocks) {
   return hipSuccess;
 }
 
+BucketBuffers::~BucketBuffers() {
+  if (state_) (void)hipHostFree(state_);
+}
+
+bool BucketBuffers::reserve(size_t cells, int slots, int n) {
+  constexpr size_t pad = 64;
+  const size_t want = 3 * cells + pad + static_cast<size_t>(n) + cells * slots;
+  if (refused_ && want >= refused_) return false;
+  if (want > mem_.n || cells != cells_) {
+    mem_.release();  // (count and head of other cells are not where they were)
+    if (mem_.reserve(want) != hipSuccess) {
+      (void)hipGetLastError();
+      mem_.release();
+      cells_ = 0;
+      refused_ = want;
+      return false;
+    }
+  }
+  if (!state_) {
+    if (hipHostMalloc(reinterpret_cast<void**>(&state_), sizeof(int), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      state_ = nullptr;
+      refused_ = 1;
+      return false;
+    }
+    *state_ = 0;
+  }
+  cells_ = cells;
+  slots_ = slots;
+  return true;
+}
+
+BucketView BucketBuffers::view(int n, double G) const {
+  BucketView b;
+  b.cap = slots_;
+  b.thread = bucket_limit(n, G) == kBucket;
+  b.count = mem_.p;
+  b.head = b.count + cells_;
+  b.queue = b.head + cells_;
+  b.nqueue = b.queue + cells_;
+  b.next = b.nqueue + 1;
+  b.items = b.next + n;
+  b.state = state_;
+  return b;
+}
+
+CrowdCheck BucketBuffers::check(int n, double G) const {
+  CrowdCheck c;
+  c.cap = bucket_slots(n, G);
+  if (!mem_.p || !state_ || !c.cap) return c;
+  c.limit = bucket_limit(n, G);
+  c.atoms = n;
+  c.count = mem_.p + 3 * cells_;
+  c.state = state_;
+  return c;
+}
+
 // ====================================================================== grid
 int eph_grid::upload() {
   const size_t G = h.ntotal();
@@ -353,6 +410,7 @@ int eph_context::set_atoms(int nl, int ng, const double* x, const double* v, con
     if ((rc = h2d(tag.p, t.data(), nall * sizeof(int)))) return rc;
   }
   EPH_HIP(this, hipStreamSynchronize(stream));
+  if (grid) grid->buckets.retry();  // (memory may have been freed)
   have_atoms = true;
   return EPH_OK;
 }
@@ -687,25 +745,13 @@ int eph_context::end_of_step_after_deposit(long long ntimestep, const DepositTai
   return EPH_OK;
 }
 
-int eph_grid::bucket_bytes_ok(size_t G, int cap, int n) {
-  EPH_HIP(this, bcount.reserve(G));  // zero-filled when first made
-  EPH_HIP(this, bitems.reserve(G * cap));
-  EPH_HIP(this, bhead.reserve(G));
-  EPH_HIP(this, bnext.reserve(n));
-  EPH_HIP(this, bqueue.reserve(G));
-  EPH_HIP(this, bnq.reserve(1));
-  if (!bstate) {
-    EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&bstate), sizeof(int), hipHostMallocDefault));
-    *bstate = 0;
-  }
-  return EPH_OK;
-}
-
-// slots per cell where the deposit goes through per-cell buckets, else 0
-int eph_context::bucket_deposit() const {
-  if (!(flags & (EPH_FRICTION | EPH_RANDOM))) return 0;
-  if (grid->bstate && *static_cast<volatile int*>(grid->bstate) == kCrowded) return 0;
-  return bucket_slots(static_cast<double>(nlocal), static_cast<double>(grid->h.ntotal()));
+// slots per cell where the deposit goes through per-cell buckets (which are then
+// there), else 0
+int eph_context::bucket_deposit() {
+  if (!(flags & (EPH_FRICTION | EPH_RANDOM)) || grid->buckets.state() == kCrowded) return 0;
+  const size_t G = grid->h.ntotal();
+  const int cap = bucket_slots(nlocal, static_cast<double>(G));
+  return cap && grid->buckets.reserve(G, cap, nlocal) ? cap : 0;
 }
 
 // the deposit half of end_of_step (fix_eph.cpp:364-404): dT_e and the tally.
@@ -724,15 +770,9 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
   // per-cell buckets (three launches)
   if (cap) {
     EPH_HIP(this, grid->dep.reserve(nlocal, G, nb));  // also what a counted deposit needs
-    if (int rc = grid->bucket_bytes_ok(G, cap, nlocal)) return fail(rc, grid->err);
     DepositView d = grid->dep.view(true);
-    BucketView b;
-    b.cap = cap;
-    b.thread = bucket_limit(nlocal, static_cast<double>(G)) == kBucket;
-    b.head = grid->bhead.p; b.next = grid->bnext.p;
-    b.count = grid->bcount.p; b.items = grid->bitems.p; b.queue = grid->bqueue.p; b.nqueue = grid->bnq.p;
-    b.state = grid->bstate;
-    const bool calm = *static_cast<volatile int*>(grid->bstate) == kCalm;
+    const BucketView b = grid->buckets.view(nlocal, static_cast<double>(G));
+    const bool calm = grid->buckets.state() == kCalm;
     timed_begin("deposit", &e);
     EPH_HIP(this, launch_deposit_bucket(atoms_view(), grid->v, step_params(), work_view(), d, b, fric, rnd,
                                         kick, scal.p, scal.p + (defer_tally ? 2 : 1), stream,
@@ -749,15 +789,8 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
     DepositView dc = d;
     if (!fric) dc.v1 = nullptr;
     if (!rnd) dc.v2 = nullptr;
-    CrowdCheck cc;
-    if (grid->bstate) {  // buckets were crowded: look whether they still would be
-      cc.cap = bucket_slots(nlocal, static_cast<double>(G));
-      cc.limit = bucket_limit(nlocal, static_cast<double>(G));
-      cc.atoms = nlocal;
-      cc.state = grid->bstate;
-      cc.count = cc.cap ? grid->bnq.p : nullptr;
-    }
-    EPH_HIP(this, launch_deposit_cells(grid->v, dc, nlocal, grid->dep.qbuf.p, stream, cc));
+    EPH_HIP(this, launch_deposit_cells(grid->v, dc, nlocal, grid->dep.qbuf.p, stream,
+                                       grid->buckets.check(nlocal, static_cast<double>(G))));
     EPH_HIP(this, launch_energy_reduce(d, nb, scal.p, scal.p + (defer_tally ? 2 : 1), stream));
     timed_end("deposit", e);
   } else {
@@ -1695,7 +1728,6 @@ void eph_grid_destroy(eph_grid* g) {
   if (!g) return;
   if (g->stream) (void)hipStreamSynchronize(g->stream);
   hipStream_t s = g->own_stream ? g->stream : nullptr;
-  if (g->bstate) (void)hipHostFree(g->bstate);
   delete g;
   if (s) (void)hipStreamDestroy(s);
 }

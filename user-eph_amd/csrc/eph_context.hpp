@@ -30,6 +30,34 @@ struct DepositBuffers {
   }
 };
 
+// Per-cell buckets of the deposit (a grid's, or a batch's cells as one), in one
+// allocation: they are there as a whole or not at all.
+struct BucketBuffers {
+  BucketBuffers() = default;
+  BucketBuffers(const BucketBuffers&) = delete;
+  BucketBuffers& operator=(const BucketBuffers&) = delete;
+  ~BucketBuffers();
+  // Room for `slots` atoms in each of `cells` cells, n atoms in all; false when
+  // there is no memory for it.  The deposit then takes the counted form, whose
+  // arrays are a few per cent of these on grids with several atoms a cell; the
+  // same size is not asked for again before retry() (new atoms).
+  bool reserve(size_t cells, int slots, int n);
+  void retry() { refused_ = 0; }
+  BucketView view(int n, double G) const;
+  // How the last deposit went (BucketView::state).  After a crowded one the next
+  // is a counted one; a plan only, as both forms give the same bits, so it is
+  // read without a wait.
+  int state() const { return state_ ? *static_cast<volatile int*>(state_) : 0; }
+  // for the counted deposit of n atoms in place of a crowded one
+  CrowdCheck check(int n, double G) const;
+
+ private:
+  DevArray<int> mem_;  // count, head, queue [cells], nqueue, next [n], items [cells][slots]; count and head zero between steps
+  size_t cells_ = 0, refused_ = 0;
+  int slots_ = 0;
+  int* state_ = nullptr;  // pinned
+};
+
 // Runs the error-returning HIP call and turns a failure into a status.
 #define EPH_HIP(obj, call)                                                        \
   do {                                                                            \
@@ -51,13 +79,7 @@ struct eph_grid {
   eph::DevArray<double4> C_T, kappa_T;
   eph::DevArray<int> nonfinite, lookup_idx;
   eph::DepositBuffers dep;
-  // per-cell buckets of the deposit (count kept at zero between steps)
-  eph::DevArray<int> bcount, bitems, bhead, bnext, bqueue, bnq;
-  // Pinned: how the last deposit went (BucketView::state).  After a crowded one
-  // the next is a counted one; a plan only, as both forms give the same bits, so
-  // it is read without a wait.
-  int* bstate = nullptr;
-  int bucket_bytes_ok(size_t G, int cap, int n);  // reserves buckets of cap slots for n atoms; 0 when they are ready
+  eph::BucketBuffers buckets;
   eph::PinnedArena arena;  // small calls
   bool any_tdyn = false;
   bool minmax_valid = false;  // cmin, rmin, kmax and uniform describe h
@@ -182,7 +204,7 @@ struct eph_context {
   // ghost positions and velocities, with the density sweep's candidate check
   // where it is due (the harness's step); t: device time at its start
   int dev_ghosts(unsigned long long* t);
-  int bucket_deposit() const;
+  int bucket_deposit();
   int autotune(int* forms, double* ms);
   int grow_filter_state(size_t nall);
   int check_flags();

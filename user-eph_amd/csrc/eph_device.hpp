@@ -172,7 +172,9 @@ constexpr int kBucket = 16, kWaveCellMax = 256;
 constexpr double kThreadCells = 6.0, kWaveCells = 64.0;
 // Slots per cell for n atoms in G cells, 0: no buckets.  More than the cells'
 // sums need, so that the queued cells of a crowded box find their atoms in
-// the bucket too, where the buckets are small (up to 64 MB).
+// the bucket too, where the buckets are small (up to 64 MB).  On larger grids of
+// 6 to 64 atoms a cell they hold what a wave takes, 1 KB a cell (268 MB for 64^3
+// cells); without memory for that the deposit is a counted one.
 inline int bucket_slots(double n, double G) {
   if (n > kWaveCells * G) return 0;
   const bool small = G <= 16384.0;

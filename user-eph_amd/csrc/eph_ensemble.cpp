@@ -67,12 +67,9 @@ struct eph_ensemble {
   DevArray<int> grid_steps, max_sub_dev;
   int* pinned = nullptr;  // [0] largest sub-step count, [1] lists to be rebuilt
   DepositBuffers dep;
-  // bucketed deposit: slots per cell (0: counted), the buckets, and the pinned
-  // word that says how the last deposit went (BucketView::state)
-  int slots = 0;
-  DevArray<int> bk_count, bk_items, bk_head, bk_next, bk_queue, bk_nq;
-  int* bk_state = nullptr;
-  bool bucketed() const { return slots > 0 && *static_cast<volatile int*>(bk_state) != kCrowded; }
+  BucketBuffers buckets;  // of the deposit, where there is memory for them
+  bool have_buckets = false;
+  bool bucketed() const { return have_buckets && buckets.state() != kCrowded; }
   // the T_e solve with a workgroup per replica
   bool fdm_block = false, fdm_uniform = false;
   int max_cells = 0;
@@ -97,7 +94,6 @@ struct eph_ensemble {
       eph_md_destroy(r.md);
     }
     if (pinned) (void)hipHostFree(pinned);
-    if (bk_state) (void)hipHostFree(bk_state);
     eph_destroy(sys);
   }
   int setup(long long first);
@@ -323,17 +319,8 @@ int eph_ensemble::setup(long long first) {
   EPH_HIP(this, launch_fill_double(Ee.p, R, 0.0, s));
   EPH_HIP(this, launch_fill_int(nonfinite.p, 1, 0, s));
   EPH_HIP(this, dep.reserve(nl, G, nchunk));
-  if (sys->flags & (EPH_FRICTION | EPH_RANDOM)) slots = bucket_slots(nl, G);
-  if (slots) {
-    EPH_HIP(this, bk_count.reserve(G));  // zero-filled
-    EPH_HIP(this, bk_items.reserve(static_cast<size_t>(G) * slots));
-    EPH_HIP(this, bk_head.reserve(G));   // zero-filled
-    EPH_HIP(this, bk_next.reserve(nl));
-    EPH_HIP(this, bk_queue.reserve(G));
-    EPH_HIP(this, bk_nq.reserve(1));
-    if (!bk_state) EPH_HIP(this, hipHostMalloc(reinterpret_cast<void**>(&bk_state), sizeof(int), hipHostMallocDefault));
-    *bk_state = 0;
-  }
+  const int per_cell = sys->flags & (EPH_FRICTION | EPH_RANDOM) ? bucket_slots(nl, G) : 0;
+  have_buckets = per_cell && buckets.reserve(G, per_cell, nl);
   fdm_uniform = true;
   max_cells = 0;
   for (const Replica& p : reps) {
@@ -406,16 +393,11 @@ int eph_ensemble::enqueue_step() {
                                           var_force));
   // final_integrate and end_of_step (fix_eph.cpp:350-429), EPH_FDM::solve per replica
   const bool fric = sys->flags & EPH_FRICTION, rnd = sys->flags & EPH_RANDOM;
-  const bool buckets = (fric || rnd) && bucketed();
-  if (!buckets && (rc = sys->dev_final_integrate())) return fail(rc, sys->err);
+  const bool in_buckets = (fric || rnd) && bucketed();
+  if (!in_buckets && (rc = sys->dev_final_integrate())) return fail(rc, sys->err);
   const int R = static_cast<int>(reps.size());
-  if (buckets) {
-    BucketView b;
-    b.cap = slots;
-    b.thread = bucket_limit(nl, G) == kBucket;
-    b.head = bk_head.p; b.next = bk_next.p;
-    b.count = bk_count.p; b.items = bk_items.p; b.queue = bk_queue.p; b.nqueue = bk_nq.p;
-    b.state = bk_state;
+  if (in_buckets) {
+    const BucketView b = buckets.view(nl, G);
     EPH_HIP(this, launch_deposit_bucket_batch(a, gviews.p, cell_off.p, cell_rep.p, gall, p, w, dep.view(true), b,
                                               chunks.p, nchunk, chunk0.p, nchunks.p, R,
                                               !(sys->flags & EPH_NOINT), E_local.p, Ee.p, s));
@@ -426,12 +408,8 @@ int eph_ensemble::enqueue_step() {
     DepositView dc = d;
     if (!fric) dc.v1 = nullptr;
     if (!rnd) dc.v2 = nullptr;
-    CrowdCheck cc;
-    if (slots) {
-      cc.count = bk_nq.p; cc.state = bk_state;
-      cc.cap = slots; cc.limit = bucket_limit(nl, G);
-      cc.cell_rep = cell_rep.p; cc.chunks = chunks.p; cc.chunk0 = chunk0.p; cc.nchunks = nchunks.p;
-    }
+    CrowdCheck cc = buckets.check(nl, G);
+    cc.cell_rep = cell_rep.p; cc.chunks = chunks.p; cc.chunk0 = chunk0.p; cc.nchunks = nchunks.p;
     EPH_HIP(this, launch_deposit_cells(gall, dc, nl, dep.qbuf.p, s, cc));
     EPH_HIP(this, launch_energy_reduce_batch(d.partial, chunk0.p, nchunks.p, R, E_local.p, Ee.p, s));
   } else {
