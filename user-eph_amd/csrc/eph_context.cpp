@@ -17,17 +17,29 @@ inline int nblocks_of(long n) { return static_cast<int>((n + kBlock - 1) / kBloc
 
 // =================================================================== deposit
 hipError_t DepositBuffers::reserve(size_t n_items, size_t G, size_t nblocks) {
-  hipError_t e;
-  if ((e = cell.reserve(n_items)) != hipSuccess) return e;
-  if ((e = items.reserve(n_items)) != hipSuccess) return e;
-  if ((e = v1.reserve(n_items)) != hipSuccess) return e;
-  if ((e = v2.reserve(n_items)) != hipSuccess) return e;
-  if ((e = count.reserve(G + 1)) != hipSuccess) return e;
-  if ((e = start.reserve(G + 1)) != hipSuccess) return e;
-  if ((e = fill.reserve(G + 1)) != hipSuccess) return e;
-  if ((e = qbuf.reserve(2 + 2 * G)) != hipSuccess) return e;
-  if ((e = scan_tmp.reserve(G / 4096 + 2)) != hipSuccess) return e;
-  if ((e = partial.reserve(2 * nblocks + 2)) != hipSuccess) return e;
+  if (mem_.p && n_items <= items_ && G <= cells_ && nblocks <= blocks_) return hipSuccess;
+  items_ = std::max(n_items, items_);
+  cells_ = std::max(G, cells_);
+  blocks_ = std::max(nblocks, blocks_);
+  auto pad = [](size_t n) { return (n + 31) / 32 * 32; };
+  const size_t n = pad(items_), g = pad(cells_ + 1), b = pad(2 * blocks_ + 2), q = pad(2 + 2 * cells_),
+               t = pad(cells_ / 4096 + 2);
+  const hipError_t e = mem_.reserve(2 * n + b + (2 * n + 3 * g + q + t) / 2);
+  if (e != hipSuccess) {
+    mem_.release();
+    items_ = cells_ = blocks_ = 0;
+    return e;
+  }
+  v_.v1 = mem_.p;
+  v_.v2 = v_.v1 + n;
+  v_.partial = v_.v2 + n;
+  v_.cell = reinterpret_cast<int*>(v_.partial + b);
+  v_.items = v_.cell + n;
+  v_.count = v_.items + n;
+  v_.start = v_.count + g;
+  v_.fill = v_.start + g;
+  qbuf_ = v_.fill + g;
+  v_.scan_tmp = qbuf_ + q;
   return hipSuccess;
 }
 
@@ -41,7 +53,7 @@ bool BucketBuffers::reserve(size_t cells, int slots, int n) {
   if (refused_ && want >= refused_) return false;
   if (want > mem_.n || cells != cells_) {
     mem_.release();  // (count and head of other cells are not where they were)
-    if (mem_.reserve(want) != hipSuccess) {
+    if (mem_.reserve(want + n / 8) != hipSuccess) {  // (a rank's atoms come and go)
       (void)hipGetLastError();
       mem_.release();
       cells_ = 0;
@@ -210,7 +222,7 @@ int eph_grid::insert_points(int n, const double* x, const double* y, const doubl
   EPH_HIP(this, dep.reserve(n, G, nblocks_of(n)));
   const size_t b = n * sizeof(double);
   const double* src[4] = {x, y, z, E};
-  const PinnedArena::Use mem = arena.use(4 * b);
+  const PinnedArena::Use mem = arena->use(4 * b);
   double* a = mem.get();
   if (!a) EPH_HIP(this, pts.reserve(4 * (size_t)n));
   for (int k = 0; k < 4; ++k) {
@@ -221,7 +233,7 @@ int eph_grid::insert_points(int n, const double* x, const double* y, const doubl
   DepositView d = dep.view(false);
   EPH_HIP(this, launch_fill_int(d.count, (int)G + 1, 0, stream));
   EPH_HIP(this, launch_deposit_points(n, q, q + n, q + 2 * (size_t)n, q + 3 * (size_t)n, h.dt, v, d, stream));
-  EPH_HIP(this, launch_deposit_cells(v, d, n, dep.qbuf.p, stream));
+  EPH_HIP(this, launch_deposit_cells(v, d, n, dep.qbuf(), stream));
   EPH_HIP(this, hipStreamSynchronize(stream));
   return EPH_OK;
 }
@@ -237,7 +249,7 @@ static hipError_t read_device(PinnedArena& arena, const void* src, void* dst, si
   return e;
 }
 int eph_grid::read(const void* src, void* dst, size_t bytes) {
-  EPH_HIP(this, read_device(arena, src, dst, bytes, stream));
+  EPH_HIP(this, read_device(*arena, src, dst, bytes, stream));
   return EPH_OK;
 }
 int eph_context::read(const void* src, void* dst, size_t bytes) {
@@ -413,6 +425,24 @@ int eph_context::set_atoms(int nl, int ng, const double* x, const double* v, con
   if (grid) grid->buckets.retry();  // (memory may have been freed)
   have_atoms = true;
   return EPH_OK;
+}
+
+// What the steps and hooks on these atoms use, made here and not inside the
+// first of them (a hook of 32,000 atoms took 0.3 ms longer for it).  What
+// cannot be had is asked for again, and reported, where it is needed.
+void eph_context::prime() {
+  const size_t nl = nlocal, nall = nl + nghost;
+  size_t most = 1;
+  for (size_t n : {15 * nl, 6 * nall + 6 * nl + 1, 9 * nl, 6 * nl, 6 * nall + 3 * nl, grid ? grid->h.ntotal() : 0})
+    if (n * sizeof(double) <= PinnedArena::kMax) most = std::max(most, n);
+  (void)arena.use(most * sizeof(double));
+  if (!grid || !(flags & (EPH_FRICTION | EPH_RANDOM))) return;
+  const size_t G = bucket_deposit() ? 0 : grid->h.ntotal();
+  if (grid->dep.reserve(nl, G, nblocks_of(nlocal)) != hipSuccess) (void)hipGetLastError();
+}
+
+void eph_grid::prime() {
+  (void)arena->use(std::min(PinnedArena::kMax, h.ntotal() * sizeof(double)));  // at least 256 KB: 8192 points
 }
 
 int eph_context::set_ghost_map(int ng, const int* owner, const double* shift) {
@@ -769,7 +799,7 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
   hipEvent_t e;
   // per-cell buckets (three launches)
   if (cap) {
-    EPH_HIP(this, grid->dep.reserve(nlocal, G, nb));  // also what a counted deposit needs
+    EPH_HIP(this, grid->dep.reserve(nlocal, 0, nb));
     DepositView d = grid->dep.view(true);
     const BucketView b = grid->buckets.view(nlocal, static_cast<double>(G));
     const bool calm = grid->buckets.state() == kCalm;
@@ -789,7 +819,7 @@ int eph_context::dev_deposit(bool kick, DepositTail* tail) {
     DepositView dc = d;
     if (!fric) dc.v1 = nullptr;
     if (!rnd) dc.v2 = nullptr;
-    EPH_HIP(this, launch_deposit_cells(grid->v, dc, nlocal, grid->dep.qbuf.p, stream,
+    EPH_HIP(this, launch_deposit_cells(grid->v, dc, nlocal, grid->dep.qbuf(), stream,
                                        grid->buckets.check(nlocal, static_cast<double>(G))));
     EPH_HIP(this, launch_energy_reduce(d, nb, scal.p, scal.p + (defer_tally ? 2 : 1), stream));
     timed_end("deposit", e);
@@ -917,6 +947,7 @@ int eph_create(eph_context** out, int narg, const char* const* arg, int ntypes,
     return bail(EPH_ERR_HIP, "stream creation failed");
   if (!c->atomic()) {
     c->grid = new eph_grid();
+    c->grid->arena = &c->arena;
     c->grid->h = gh;
     if (int rc = grid_init_device(c->grid, device, c->stream)) return bail(rc, c->grid->err);
   }
@@ -1072,7 +1103,9 @@ int eph_get_params(const eph_context* ctx, int* flags, int* model, int* seed, do
 int eph_set_atoms(eph_context* ctx, int nlocal, int nghost, const double* x, const double* v,
                   const int* type, const int* mask, const int* tag) {
   if (!ctx) return EPH_ERR_ARGS;
-  return ctx->set_atoms(nlocal, nghost, x, v, type, mask, tag);
+  const int rc = ctx->set_atoms(nlocal, nghost, x, v, type, mask, tag);
+  if (rc == EPH_OK) ctx->prime();
+  return rc;
 }
 
 int eph_set_ghost_map(eph_context* ctx, int nghost, const int* owner, const double* shift) {
@@ -1701,6 +1734,7 @@ int eph_grid_create(eph_grid** out, int nx, int ny, int nz, const double box[6],
     eph_grid_destroy(g);
     return rc;
   }
+  g->prime();
   *out = g;
   return EPH_OK;
 }
@@ -1720,6 +1754,7 @@ int eph_grid_load(eph_grid** out, const char* path, int device) {
     eph_grid_destroy(g);
     return rc;
   }
+  g->prime();
   *out = g;
   return EPH_OK;
 }

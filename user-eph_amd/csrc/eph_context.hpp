@@ -17,17 +17,22 @@ extern "C" {
 
 namespace eph {
 
-// Scratch of the ordered deposit (per item and per cell arrays).
+// Scratch of the ordered deposit (per item and per cell arrays), in one
+// allocation.
 struct DepositBuffers {
-  DevArray<int> cell, count, start, fill, items, scan_tmp, qbuf;
-  DevArray<double> v1, v2, partial;
   hipError_t reserve(size_t n_items, size_t G, size_t nblocks);
-  DepositView view(bool with_v2) {
-    DepositView d;
-    d.cell = cell.p; d.count = count.p; d.start = start.p; d.fill = fill.p; d.items = items.p;
-    d.v1 = v1.p; d.v2 = with_v2 ? v2.p : nullptr; d.partial = partial.p; d.scan_tmp = scan_tmp.p;
+  DepositView view(bool with_v2) const {
+    DepositView d = v_;
+    if (!with_v2) d.v2 = nullptr;
     return d;
   }
+  int* qbuf() const { return qbuf_; }
+
+ private:
+  DevArray<double> mem_;
+  DepositView v_;
+  int* qbuf_ = nullptr;
+  size_t items_ = 0, cells_ = 0, blocks_ = 0;
 };
 
 // Per-cell buckets of the deposit (a grid's, or a batch's cells as one), in one
@@ -80,7 +85,8 @@ struct eph_grid {
   eph::DevArray<int> nonfinite, lookup_idx;
   eph::DepositBuffers dep;
   eph::BucketBuffers buckets;
-  eph::PinnedArena arena;  // small calls
+  eph::PinnedArena own_arena;            // small calls
+  eph::PinnedArena* arena = &own_arena;  // a fix's grid: the fix's
   bool any_tdyn = false;
   bool minmax_valid = false;  // cmin, rmin, kmax and uniform describe h
   bool uniform = false;       // every cell dynamic and of one material
@@ -93,6 +99,7 @@ struct eph_grid {
     err = std::string("HIP error ") + hipGetErrorString(e) + " in " + what;
     return e == hipErrorOutOfMemory ? EPH_ERR_OOM : EPH_ERR_HIP;
   }
+  void prime();            // pinned memory of the small calls
   int upload();            // host description -> device (all arrays)
   void refresh_minmax();   // host min/max of the stability estimate
   // tail: the deposit's remainder, run before the first sub-step
@@ -189,6 +196,7 @@ struct eph_context {
   int reserve_atoms(int nl, int ng);
   int set_atoms(int nl, int ng, const double* x, const double* v, const int* ty, const int* mk,
                 const int* tg);
+  void prime();  // once atoms are set: buffers of the steps and hooks
   int set_ghost_map(int ng, const int* owner, const double* shift);
   int set_neighbors(int nl, const int* off, const int* idx, int neighmask);
   int dev_initial_integrate(const eph::StepExtras* x = nullptr);

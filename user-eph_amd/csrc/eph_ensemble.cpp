@@ -410,7 +410,7 @@ int eph_ensemble::enqueue_step() {
     if (!rnd) dc.v2 = nullptr;
     CrowdCheck cc = buckets.check(nl, G);
     cc.cell_rep = cell_rep.p; cc.chunks = chunks.p; cc.chunk0 = chunk0.p; cc.nchunks = nchunks.p;
-    EPH_HIP(this, launch_deposit_cells(gall, dc, nl, dep.qbuf.p, s, cc));
+    EPH_HIP(this, launch_deposit_cells(gall, dc, nl, dep.qbuf(), s, cc));
     EPH_HIP(this, launch_energy_reduce_batch(d.partial, chunk0.p, nchunks.p, R, E_local.p, Ee.p, s));
   } else {
     EPH_HIP(this, launch_fill_double(E_local.p, R, 0.0, s));

@@ -607,6 +607,7 @@ int eph_md_attach(eph_md* md, eph_context* ctx) {
   int rc = md->upload(ctx);
   if (rc) return rc;
   // Verlet::setup: pair forces of the initial configuration
+  ctx->prime();
   hipStream_t s = ctx->stream;
   EPH_HIP(md, launch_ghost_check(ctx->atoms_view(), ctx->work_view(), false, nullptr, s));
   EPH_HIP(md, launch_lj(ctx->atoms_view(), md->lj_nbr.p, md->lj_nn.p, md->lj_stride, md->cfg.lj_eps,

@@ -35,7 +35,7 @@ PinnedArena::Use PinnedArena::use(size_t bytes) {
     if (p_) (void)hipHostFree(p_);
     p_ = nullptr;
     n_ = 0;
-    size_t want = size_t(1) << 16;
+    size_t want = size_t(1) << 18;  // (35 us at any size up to kMax)
     while (want < bytes) want <<= 1;
     hipError_t e = ev_ ? hipSuccess : hipEventCreateWithFlags(&ev_, hipEventDisableTiming);
     if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void**>(&p_), want, hipHostMallocDefault);
