@@ -159,3 +159,46 @@ def test_overflowing_moved_list_then_return_keeps_bits(oracle, tmp_path):
     _same(p, "step 4")
     st = p.gpu.candidate_stats()
     assert not st["retaken"] and st["full_waves"] == 0, st
+
+
+def test_check_of_a_failed_step_is_not_the_next_ones(tmp_path):
+    """A harness step that fails after its candidate check (the fix's list was refused), a new list, atoms moved on the
+    device, forces there (which take candidates), forces at the earlier positions: the atom that went away and came back
+    has moved since the candidates were taken."""
+    from eph_amd import inputs
+
+    path = str(tmp_path / "b.beta")
+    names = inputs.workload_beta(path, 1)
+
+    def fix():
+        f = ea.FixEPH(inputs.fix_args(path, names, seed=3, flags="7", grid=(6, 6, 6)), 1, inf["boxlo"], inf["boxhi"],
+                      1e-3, inputs.BOLTZ, inputs.FTM2V, masses=[inputs.MASS_CU])
+        f.init()
+        return f
+
+    md = ea.MD(6, seed=5, T=300.0, pka_eV=100.0)
+    inf = md.info()
+    gpu = fix()
+    md.attach(gpu)
+    md.run(gpu, 1)
+    s = md.snapshot()
+    bad = s.nbr_idx.copy()
+    bad[0] = s.nlocal + s.nghost
+    lists = (ea.lib().eph_set_neighbors, gpu.h, s.nlocal, ea._i(s.nbr_off))
+    assert lists[0](*lists[1:], ea._i(bad), -1) != 0
+    with pytest.raises(ea.EphError):
+        md.run(gpu, 1, first_step=2)
+    s.x, s.v, _ = gpu.dev_atoms()
+    assert lists[0](*lists[1:], ea._i(s.nbr_idx), -1) == 0
+    for _ in range(10):
+        gpu.dev_initial_integrate()
+    gpu.dev_post_force()
+    moved = np.linalg.norm(gpu.dev_atoms()[0] - s.x, axis=1).max()
+    assert 1.4 < moved < 2.5  # far past the candidates' margin
+    ref = fix()
+    ref.set_candidate_margin(0)
+    ref.set_atoms(s)
+    for f in (gpu, ref):
+        s.f = np.zeros_like(s.x)
+        f.post_force(s, step=9)
+    assert np.array_equal(gpu.get("rho"), ref.get("rho")) and np.array_equal(gpu.get("f_EPH"), ref.get("f_EPH"))

@@ -308,6 +308,7 @@ StepParams eph_context::step_params() {
 }
 
 void eph_context::drop_candidates() {
+  cand_checked = false;
   if (cstate.p) (void)launch_fill_int(cstate.p, 8, 0, stream);
 }
 
@@ -551,6 +552,7 @@ int eph_context::resolve_timing() {
 
 int eph_context::dev_initial_integrate(const StepExtras* x) {
   if (!have_atoms) return fail(EPH_ERR_STATE, "no atoms");
+  cand_checked = false;  // it was made at the positions so far
   if (flags & EPH_NOINT) {
     if (x) EPH_HIP(this, launch_integrate(atoms_view(), step_params(), false, stream, x));
     return EPH_OK;
@@ -601,14 +603,15 @@ int eph_context::timed_density(const AtomsView& a, const StepParams& p, const Wo
 }
 
 int eph_context::dev_post_force() {
+  const bool checked = cand_checked;
+  cand_checked = false;
   if (!have_atoms || !have_list) return fail(EPH_ERR_STATE, "atoms and neighbour list must be set");
   if (atomic()) return eph::atomic_post_force(this);
   StepParams p = step_params();
   p.xi_mode = (flags & EPH_RANDOM) ? (xi_mode_next ? 1 : 2) : 0;
   const AtomsView a = atoms_view();
   WorkView w = work_view();
-  w.cand_checked = cand_checked;
-  cand_checked = false;
+  w.cand_checked = checked;
   w.defer_flags = !timing && model == 4 && nghost > 0 && w.rcand2 > 0.0 &&
                   density_walks_candidates(a, tabs, form_density);
   hipEvent_t e;
@@ -649,6 +652,7 @@ int eph_context::dev_post_force() {
 // their xi, rho and w then go to the other ranks' ghosts (the XI, RHO and WI
 // exchanges of :863-871, which only the later stages read)
 int eph_context::dev_post_force_local() {
+  cand_checked = false;
   if (!have_atoms || !have_list) return fail(EPH_ERR_STATE, "atoms and neighbour list must be set");
   if (atomic() || colour == 3 || model != 4)
     return fail(EPH_ERR_UNSUPPORTED, "the split post_force serves the PRL model of eph, "

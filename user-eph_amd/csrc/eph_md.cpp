@@ -330,6 +330,7 @@ int eph_md::kick_and_pair(eph_context* ctx, bool force, unsigned long long* t, b
     EPH_HIP(this, hipStreamSynchronize(s));
     if (pinned[1]) {  // capacity exceeded
       *overflow = true;
+      ctx->cand_checked = false;
       EPH_HIP(this, launch_fill_int(flags.p + 1, 1, 0, s));
       return EPH_OK;
     }
