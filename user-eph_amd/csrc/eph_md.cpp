@@ -9,6 +9,7 @@
 #include <thread>
 
 #include "eph_harness.hpp"
+#include "eph_shares.hpp"
 #include "eph_rng.hpp"
 
 using namespace eph;
@@ -711,17 +712,16 @@ int eph_md_run(eph_md* md, eph_context* ctx, int nsteps, long long first_step, d
     int khz = 0;
     if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, ctx->device) != hipSuccess || khz <= 0)
       khz = 100000;
+    // (the harness's atoms share one mask: all of them are in the group or none)
+    const bool moves = !(ctx->flags & EPH_NOINT) && md->nlocal > 0 && (md->mask[0] & ctx->groupbit);
     auto ms = [&](unsigned long long a, unsigned long long b) { return b > a ? (b - a) / (double)khz : 0.0; };
     for (int st = 0; st < nsteps; ++st) {
       const unsigned long long* q = th.data() + 5 * static_cast<size_t>(st);
       const unsigned long long kicked = std::max(q[0], q[1]), next = q[5];
-      // Two kernels serve both sides and count by the bytes that each moves:
-      // the kick (224 B an atom) with the check of the lists (32), and the
-      // ghost update (228 B a ghost) with the candidate check (64 an atom).
+      // two kernels serve both sides
       const double kick = ms(q[0], kicked), ghosts = ms(q[2], q[3]);
-      const double kick_fix = md->device_rebuild ? 224.0 / 256.0 : 1.0;
-      const double check_bytes = checked[st] ? 64.0 * (md->nlocal + md->nghost) : 0.0;
-      const double ghosts_fix = check_bytes > 0.0 ? check_bytes / (check_bytes + 228.0 * md->nghost) : 0.0;
+      const double kick_fix = kick_share(md->device_rebuild, moves);
+      const double ghosts_fix = ghosts_share(checked[st], md->nlocal, md->nghost);
       t_fix += kick * kick_fix + ghosts * ghosts_fix;
       t_rebuild += kick * (1.0 - kick_fix);
       t_pair += ghosts * (1.0 - ghosts_fix);
