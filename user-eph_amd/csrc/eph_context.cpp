@@ -13,6 +13,8 @@ namespace {
 thread_local std::string g_create_error;
 
 inline int nblocks_of(long n) { return static_cast<int>((n + kBlock - 1) / kBlock); }
+// the parts of one allocation start at whole cache lines (256 B for ints)
+inline size_t whole(size_t n) { return (n + 63) / 64 * 64; }
 }  // namespace
 
 // =================================================================== deposit
@@ -21,9 +23,8 @@ hipError_t DepositBuffers::reserve(size_t n_items, size_t G, size_t nblocks) {
   items_ = std::max(n_items, items_);
   cells_ = std::max(G, cells_);
   blocks_ = std::max(nblocks, blocks_);
-  auto pad = [](size_t n) { return (n + 31) / 32 * 32; };
-  const size_t n = pad(items_), g = pad(cells_ + 1), b = pad(2 * blocks_ + 2), q = pad(2 + 2 * cells_),
-               t = pad(cells_ / 4096 + 2);
+  const size_t n = whole(items_), g = whole(cells_ + 1), b = whole(2 * blocks_ + 2), q = whole(2 + 2 * cells_),
+               t = whole(cells_ / 4096 + 2);
   const hipError_t e = mem_.reserve(2 * n + b + (2 * n + 3 * g + q + t) / 2);
   if (e != hipSuccess) {
     mem_.release();
@@ -48,8 +49,7 @@ BucketBuffers::~BucketBuffers() {
 }
 
 bool BucketBuffers::reserve(size_t cells, int slots, int n) {
-  constexpr size_t pad = 64;
-  const size_t want = 3 * cells + pad + static_cast<size_t>(n) + cells * slots;
+  const size_t want = 3 * whole(cells) + 64 + whole(n) + cells * slots;
   if (refused_ && want >= refused_) return false;
   if (want > mem_.n || cells != cells_) {
     mem_.release();  // (count and head of other cells are not where they were)
@@ -80,11 +80,11 @@ BucketView BucketBuffers::view(int n, double G) const {
   b.cap = slots_;
   b.thread = bucket_limit(n, G) == kBucket;
   b.count = mem_.p;
-  b.head = b.count + cells_;
-  b.queue = b.head + cells_;
-  b.nqueue = b.queue + cells_;
-  b.next = b.nqueue + 1;
-  b.items = b.next + n;
+  b.head = b.count + whole(cells_);
+  b.queue = b.head + whole(cells_);
+  b.nqueue = b.queue + whole(cells_);
+  b.next = b.nqueue + 64;
+  b.items = b.next + whole(n);
   b.state = state_;
   return b;
 }
@@ -95,7 +95,7 @@ CrowdCheck BucketBuffers::check(int n, double G) const {
   if (!mem_.p || !state_ || !c.cap) return c;
   c.limit = bucket_limit(n, G);
   c.atoms = n;
-  c.count = mem_.p + 3 * cells_;
+  c.count = mem_.p + 3 * whole(cells_);
   c.state = state_;
   return c;
 }
