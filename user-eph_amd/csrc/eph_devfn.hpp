@@ -16,6 +16,15 @@ static __device__ __forceinline__ int xcd_block() {
   return x * per + (x < rem ? x : rem) + local;
 }
 
+// What the lanes of a wave wrote (LDS, or memory of their own wave) before it,
+// all of them read after it: the wave's operations run in order, the fences keep
+// the compiler to that order.
+static __device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 static __device__ __forceinline__ double cubic_at(const double4* __restrict__ tab, int n, double inv,
                                            double x) {
   int i = static_cast<int>(x * inv);

@@ -53,11 +53,6 @@ __global__ __launch_bounds__(kBlock) void k_csr_to_ell(int nlocal, const int* __
 // padding); inside a record the parts are rotated per record so that the
 // per-lane reads are free of bank conflicts.  The whole wave runs these loops
 // (to its longest list), lanes past their own list doing only copies.
-static __device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 constexpr int kCoopStage = 384;  // 16-B units of LDS per wave and force-sweep entry (64 x 96 B)
 constexpr int kCoopF = 1;        // force-sweep entries per iteration

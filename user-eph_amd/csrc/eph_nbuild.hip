@@ -15,6 +15,8 @@
 // the whole sequence can be recorded once and replayed every step.
 #include "eph_nbuild.hpp"
 
+#include "eph_devfn.hpp"
+
 namespace eph {
 
 namespace {
@@ -596,7 +598,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_nb_lists_tile(
           s_pre[lane] = incl - len;
           s_beg[lane] = beg - (incl - len);
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         int* row_l = s_l + a * tl.rl;
         // four rounds of 64 atoms at a time: their loads travel together
         constexpr int U = 4;
@@ -643,10 +645,10 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_nb_lists_tile(
         if ((nf > l.cap_f || nl > l.cap_l) && lane == 0) atomicOr(overflow, 2);
         nf = min(nf, l.cap_f);
         nl = min(nl, l.cap_l);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
         nc = nf <= 128 ? nb_tile_sort<2>(nf, lane, s_key, s_jt, s_f + a * tl.rf, s_c + a * tl.rf)
                        : nb_tile_sort<4>(nf, lane, s_key, s_jt, s_f + a * tl.rf, s_c + a * tl.rf);
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_sync();
       }
       if (lane == 0) {
         s_n[a] = nl;
