@@ -461,7 +461,5 @@ hipError_t launch_pack_pv_dev(const AtomsView& a, const WorkView& w, const int* 
                               hipStream_t s);
 hipError_t launch_ghost_rec_dev(const AtomsView& a, const WorkView& w, const int* ng, int cap,
                                 hipStream_t s);
-hipError_t launch_step_log(const int* flag, const uint64_t* step, const uint64_t* first, int* log,
-                           int nlog, hipStream_t s);
 
 }  // namespace eph

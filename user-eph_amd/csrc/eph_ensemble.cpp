@@ -41,12 +41,11 @@ struct eph_ensemble {
   bool ready = false;
   int nl = 0, G = 0, nchunk = 0, max_sub = 0;
   int ghost_cap = 0, cap_f = 0, cap_l = 0, nbins = 0;
-  long long step0 = 1, next_step = 1;
-  uint64_t log_first = 0;  // host source of the device copy (pinned by lifetime)
+  long long next_step = 1;
   eph_md_config cfg0{};
   // harness
   DevArray<int> rep, flags, cnt, start, bin_of, bcount, bstart, bfill, items, scan_tmp, nbi,
-      lj_nbr, lj_nn, lj_cand, lj_ncand, rlog;
+      lj_nbr, lj_nn, lj_cand, lj_ncand;
   DevArray<double> box_d;
   DevArray<double4> xref, bpos;
   NbBuild nbw;
@@ -97,7 +96,7 @@ struct eph_ensemble {
     eph_destroy(sys);
   }
   int setup(long long first);
-  int step_front(int nlog);
+  int step_front(bool* rebuilt);
   int enqueue_step();
   int enqueue_fdm(int nsub);
   int fdm_after_counts();
@@ -221,7 +220,7 @@ int eph_ensemble::setup(long long first) {
   w.lists.sort_scale = list_sort_scale(w.lists.cf2);
   w.lists.nbr_l = lj_nbr.p; w.lists.nn_l = lj_nn.p; w.lists.cap_l = cap_l; w.lists.cl2 = cl * cl;
   w.lists.stride = st;
-  w.go = flags.p; w.overflow = flags.p + 1; w.nrebuild = flags.p + 2; w.nghost = flags.p + 4;
+  w.overflow = flags.p + 1; w.nrebuild = flags.p + 2; w.nghost = flags.p + 4;
   w.cnt = cnt.p; w.start = start.p; w.bin_of = bin_of.p; w.bcount = bcount.p; w.bstart = bstart.p;
   w.bfill = bfill.p; w.items = items.p; w.bpos = bpos.p; w.scan_tmp = scan_tmp.p; w.xref = xref.p;
   // each rebuild also writes the density sweep's candidate lists, valid at
@@ -237,7 +236,6 @@ int eph_ensemble::setup(long long first) {
   }
   // initial ghosts and lists: a forced device build
   EPH_HIP(this, launch_fill_int(flags.p, 8, 0, s));
-  EPH_HIP(this, launch_nb_force(w.go, s));
   EPH_HIP(this, launch_nb_build(w, s));
   int fl[8];
   EPH_HIP(this, hipMemcpyAsync(fl, flags.p, sizeof fl, hipMemcpyDeviceToHost, s));
@@ -295,7 +293,7 @@ int eph_ensemble::setup(long long first) {
   EPH_HIP(this, gviews.reserve(R)); EPH_HIP(this, cell_rep.reserve(G)); EPH_HIP(this, cell_off.reserve(R));
   EPH_HIP(this, chunk0.reserve(R)); EPH_HIP(this, nchunks.reserve(R)); EPH_HIP(this, sub_n.reserve(R));
   EPH_HIP(this, inner_dt.reserve(R)); EPH_HIP(this, seeds.reserve(R)); EPH_HIP(this, chunks.reserve(nchunk));
-  EPH_HIP(this, E_local.reserve(R)); EPH_HIP(this, Ee.reserve(R)); EPH_HIP(this, step_dev.reserve(2));
+  EPH_HIP(this, E_local.reserve(R)); EPH_HIP(this, Ee.reserve(R)); EPH_HIP(this, step_dev.reserve(1));
   EPH_HIP(this, nonfinite.reserve(1));
   EPH_HIP(this, rep_tdyn.reserve(R)); EPH_HIP(this, grid_dt.reserve(R));
   EPH_HIP(this, grid_steps.reserve(R)); EPH_HIP(this, max_sub_dev.reserve(1));
@@ -339,7 +337,6 @@ int eph_ensemble::setup(long long first) {
     EPH_HIP(this, hipMemcpyAsync(fdm_args.p, fa.data(), fa.size(), hipMemcpyHostToDevice, s));
   }
   EPH_HIP(this, hipStreamSynchronize(s));
-  step0 = first;
   next_step = first;
   ready = true;
   return EPH_OK;
@@ -349,7 +346,7 @@ int eph_ensemble::setup(long long first) {
 // and the check of the lists, whose answer the host waits for; the rebuild
 // where it is due; then the rest, which can be a recorded graph.  (A rebuild
 // gated on the device costs 26 launches that find nothing to do, 70 us a step.)
-int eph_ensemble::step_front(int nlog) {
+int eph_ensemble::step_front(bool* rebuilt) {
   hipStream_t s = sys->stream;
   volatile int* want = pinned + 1;
   *want = 0;
@@ -360,10 +357,9 @@ int eph_ensemble::step_front(int nlog) {
   x.step = step_dev.p;
   if (int rc = sys->dev_initial_integrate(&x)) return fail(rc, sys->err);
   EPH_HIP(this, hipStreamSynchronize(s));
-  if (!*want) return EPH_OK;
-  EPH_HIP(this, launch_nb_force(nbw.go, s));
+  *rebuilt = *want != 0;
+  if (!*rebuilt) return EPH_OK;
   EPH_HIP(this, launch_nb_build(nbw, s));
-  if (nlog > 0) EPH_HIP(this, launch_step_log(nbw.go, step_dev.p, step_dev.p + 1, rlog.p, nlog, s));
   return EPH_OK;
 }
 
@@ -643,15 +639,6 @@ int eph_ensemble_run(eph_ensemble* e, int nsteps, int use_graph, double* ms, int
   if (!e || nsteps < 0) return EPH_ERR_ARGS;
   if (!e->ready) return e->fail(EPH_ERR_STATE, "ensemble not set up");
   hipStream_t s = e->sys->stream;
-  const int nlog = rebuilt ? nsteps : 0;
-  if (nlog > 0) {
-    EPH_HIP(e, e->rlog.reserve(nlog));
-    EPH_HIP(e, launch_fill_int(e->rlog.p, nlog, 0, s));
-  }
-  // the log indexes steps from the first step of this call
-  e->step0 = e->next_step;
-  e->log_first = static_cast<uint64_t>(e->step0);
-  EPH_HIP(e, hipMemcpyAsync(e->step_dev.p + 1, &e->log_first, sizeof(uint64_t), hipMemcpyHostToDevice, s));
   int rc;
   if (use_graph && (rc = e->record())) return rc;
   // the records of position and velocity, which the steps then keep current
@@ -667,7 +654,9 @@ int eph_ensemble_run(eph_ensemble* e, int nsteps, int use_graph, double* ms, int
   EPH_HIP(e, hipEventCreate(&b));
   EPH_HIP(e, hipEventRecord(a, s));
   for (int k = 0; k < nsteps; ++k) {
-    if ((rc = e->step_front(nlog))) return rc;
+    bool built = false;
+    if ((rc = e->step_front(&built))) return rc;
+    if (rebuilt) rebuilt[k] = built ? 1 : 0;
     if (use_graph) {
       EPH_HIP(e, hipGraphLaunch(e->exec, s));
     } else if ((rc = e->enqueue_step())) {
@@ -687,7 +676,6 @@ int eph_ensemble_run(eph_ensemble* e, int nsteps, int use_graph, double* ms, int
   int fl[8], nf = 0;
   EPH_HIP(e, hipMemcpyAsync(fl, e->flags.p, sizeof fl, hipMemcpyDeviceToHost, s));
   EPH_HIP(e, hipMemcpyAsync(&nf, e->nonfinite.p, sizeof nf, hipMemcpyDeviceToHost, s));
-  if (nlog > 0) EPH_HIP(e, hipMemcpyAsync(rebuilt, e->rlog.p, nlog * sizeof(int), hipMemcpyDeviceToHost, s));
   EPH_HIP(e, hipStreamSynchronize(s));
   e->sys->nghost = fl[7];
   if (fl[1]) return e->fail(EPH_ERR_STATE, "ensemble ghost or list capacity exceeded during the run");

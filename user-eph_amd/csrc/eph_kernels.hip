@@ -2305,15 +2305,6 @@ __global__ __launch_bounds__(kBlock) void k_prl_forces_batch_split(AtomsView a, 
                                                  s_split + wv * split_stage_f(U));
 }
 
-// start of a recorded step: step += 1
-// log[step - first] = *flag (which steps rebuilt)
-__global__ void k_step_log(const int* __restrict__ flag, const uint64_t* __restrict__ step,
-                           const uint64_t* __restrict__ first, int* log, int nlog) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  const long k = static_cast<long>(*step - *first);
-  if (k >= 0 && k < nlog) log[k] = *flag;
-}
-
 template <bool FRIC, bool RAND, bool MULTI>
 __global__ __launch_bounds__(kBlock) void k_prl_forces_batch(AtomsView a, TablesView t,
                                                              const GridView* __restrict__ grids,
@@ -3456,12 +3447,6 @@ hipError_t launch_ghost_rec_dev(const AtomsView& a, const WorkView& w, const int
                                 hipStream_t s) {
   if (cap == 0) return hipSuccess;
   k_ghost_rec_dev<<<nblk(cap), kBlock, 0, s>>>(a, w, ng);
-  return hipGetLastError();
-}
-
-hipError_t launch_step_log(const int* flag, const uint64_t* step, const uint64_t* first, int* log,
-                           int nlog, hipStream_t s) {
-  k_step_log<<<1, 64, 0, s>>>(flag, step, first, log, nlog);
   return hipGetLastError();
 }
 

@@ -263,7 +263,7 @@ int eph_md::upload(eph_context* ctx) {
   w.lists.sort_scale = list_sort_scale(w.lists.cf2);
   w.lists.nbr_l = lj_nbr.p; w.lists.nn_l = lj_nn.p; w.lists.cap_l = cap_l; w.lists.cl2 = cl * cl;
   w.lists.stride = ctx->stride;
-  w.go = flags.p; w.overflow = flags.p + 1; w.nrebuild = flags.p + 2; w.nghost = flags.p + 4;
+  w.overflow = flags.p + 1; w.nrebuild = flags.p + 2; w.nghost = flags.p + 4;
   w.cand_valid = ctx->cstate.p;
   w.cnt = cnt.p; w.start = start.p; w.bin_of = bin_of.p; w.bcount = bcount.p; w.bstart = bstart.p;
   w.bfill = bfill.p; w.items = items.p; w.bpos = bpos.p; w.scan_tmp = scan_tmp.p; w.xref = xref.p;
@@ -325,7 +325,6 @@ int eph_md::kick_and_pair(eph_context* ctx, bool force, unsigned long long* t, b
     EPH_HIP(this, hipStreamSynchronize(s));
   }
   if (*want || force) {
-    EPH_HIP(this, launch_nb_force(nbw.go, s));
     EPH_HIP(this, launch_nb_build(nbw, s));
     EPH_HIP(this, hipMemcpyAsync(pinned, flags.p, 8 * sizeof(int), hipMemcpyDeviceToHost, s));
     EPH_HIP(this, hipStreamSynchronize(s));

@@ -11,8 +11,7 @@
 //     order, the fix list is then sorted by list_sort_key (distance, index).
 // Several independent systems ("replicas") can be built at once: atom i of
 // replica rep[i] only images and neighbours atoms of its own replica.
-// Every kernel first reads the device flag `go` and returns when it is 0, so
-// the whole sequence can be recorded once and replayed every step.
+// The host launches the sequence when the check of the lists asks for it.
 #include "eph_nbuild.hpp"
 
 #include "eph_devfn.hpp"
@@ -34,8 +33,7 @@ __device__ __forceinline__ double comp(const double4& p, int d) {
 
 // Domain::remap of the locals
 __global__ __launch_bounds__(kBlock) void k_nb_wrap(int nlocal, double4* pos, PosVel* pv,
-                                                    const int* rep, NbBoxes b, const int* go) {
-  if (!*go) return;
+                                                    const int* rep, NbBoxes b) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= nlocal) return;
   const int r = rep[i];
@@ -58,8 +56,7 @@ __global__ __launch_bounds__(kBlock) void k_nb_ghost_count(int d, int cap, int n
                                                            const int* nghost_in,
                                                            const double4* __restrict__ pos,
                                                            const int* __restrict__ rep, NbBoxes b,
-                                                           int* cnt, const int* go) {
-  if (!*go) return;
+                                                           int* cnt) {
   const int s = blockIdx.x * kBlock + threadIdx.x;
   if (s >= cap) return;
   const int nsrc = nlocal + *nghost_in;
@@ -82,8 +79,7 @@ __global__ __launch_bounds__(kBlock) void k_nb_ghost_write(int d, int cap, int n
                                                            const int* __restrict__ cnt,
                                                            const int* __restrict__ start,
                                                            NbAtoms at, NbBoxes b, int ghost_cap,
-                                                           int* overflow, const int* go) {
-  if (!*go) return;
+                                                           int* overflow) {
   const int s = blockIdx.x * kBlock + threadIdx.x;
   const int ng0 = *nghost_in;
   const int nsrc = nlocal + ng0;
@@ -124,8 +120,7 @@ __global__ __launch_bounds__(kBlock) void k_nb_ghost_write(int d, int cap, int n
 __global__ __launch_bounds__(kBlock) void k_nb_bin(int cap, int nlocal, const int* nghost,
                                                     const double4* __restrict__ pos,
                                                     const int* __restrict__ rep, NbBoxes b,
-                                                    int* bin_of, int* bcount, const int* go) {
-  if (!*go) return;
+                                                    int* bin_of, int* bcount) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= cap || i >= nlocal + *nghost) return;
   const int r = rep[i];
@@ -143,8 +138,7 @@ __global__ __launch_bounds__(kBlock) void k_nb_bin(int cap, int nlocal, const in
 __global__ __launch_bounds__(kBlock) void k_nb_bin_scatter(int cap, int nlocal, const int* nghost,
                                                            const int* __restrict__ bin_of,
                                                            const int* __restrict__ bstart,
-                                                           int* bfill, int* items, const int* go) {
-  if (!*go) return;
+                                                           int* bfill, int* items) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= cap || i >= nlocal + *nghost) return;
   const int bin = bin_of[i];
@@ -153,8 +147,7 @@ __global__ __launch_bounds__(kBlock) void k_nb_bin_scatter(int cap, int nlocal, 
 
 // atoms of each bin in ascending index (insertion sort; bins hold few atoms)
 __global__ __launch_bounds__(kBlock) void k_nb_bin_sort(int nbins, const int* __restrict__ bstart,
-                                                        int* items, const int* go) {
-  if (!*go) return;
+                                                        int* items) {
   const int bin = blockIdx.x * kBlock + threadIdx.x;
   if (bin >= nbins) return;
   int* it = items + bstart[bin];
@@ -175,8 +168,7 @@ __global__ __launch_bounds__(kBlock) void k_nb_lists(int nlocal, const double4* 
                                                      const int* __restrict__ rep, NbBoxes b,
                                                      const int* __restrict__ bstart,
                                                      const int* __restrict__ items, NbLists l,
-                                                     int* overflow, const int* go) {
-  if (!*go) return;
+                                                     int* overflow) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= nlocal) return;
   const int r = rep[i];
@@ -286,7 +278,7 @@ __device__ __forceinline__ void bitonic_wave(uint32_t (&key)[E], const int lane)
 // (element n = lane E + s; padding keys ~0 sort last; nn_f <= cap_f <= N).
 // The found position t in a key gives the entry's index, read back before the
 // sorted list is written over the found one.  A fixed grid of waves walks the
-// atoms, so a step without a rebuild costs one flag read per block.
+// atoms.
 template <int E>
 __device__ __forceinline__ void nb_sort_atom(const int i, const int lane, const double4* __restrict__ pos,
                                              const NbLists& l) {
@@ -347,9 +339,7 @@ __device__ __forceinline__ void nb_sort_atom(const int i, const int lane, const 
 
 constexpr int kSortBlocks = 2048;
 template <int E>
-__global__ __launch_bounds__(kBlock) void k_nb_sort(int nlocal, const double4* __restrict__ pos, NbLists l,
-                                                    const int* go) {
-  if (!*go) return;
+__global__ __launch_bounds__(kBlock) void k_nb_sort(int nlocal, const double4* __restrict__ pos, NbLists l) {
   const int lane = threadIdx.x & 63;
   const int nw = gridDim.x * (kBlock / 64);
   for (int i = blockIdx.x * (kBlock / 64) + static_cast<int>(threadIdx.x >> 6); i < nlocal; i += nw)
@@ -358,11 +348,10 @@ __global__ __launch_bounds__(kBlock) void k_nb_sort(int nlocal, const double4* _
 
 __global__ __launch_bounds__(kBlock) void k_nb_finish(int nlocal, const int* ng,
                                                       const double4* __restrict__ pos,
-                                                      double4* ref, int* go, int* nreb,
+                                                      double4* ref, int* nreb,
                                                       int* cand_valid, double4* cref,
                                                       bool cand_written) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (!*go) return;
   if (i < nlocal) ref[i] = pos[i];
   // the candidates of the new lists, if written, are valid at the positions
   // of this rebuild (locals and the ghosts just made); otherwise the next
@@ -374,24 +363,17 @@ __global__ __launch_bounds__(kBlock) void k_nb_finish(int nlocal, const int* ng,
     cand_valid[6] = cand_written ? 2 : 0;  // the pair force's: to be taken in this step
     cand_valid[7] = 0;
   }
-  // (*go stays set: some blocks have yet to read it)
   if (i == 0) atomicAdd(nreb, 1);
 }
 
-__global__ void k_nb_set(int* p, int v) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
-}
-
-__global__ __launch_bounds__(kBlock) void k_nb_zero(int* p, int n, const int* go) {
-  if (!*go) return;
+__global__ __launch_bounds__(kBlock) void k_nb_zero(int* p, int n) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i < n) p[i] = 0;
 }
 
 // ------------------------------------------------------------------ scan
 constexpr int kSB = 1024, kSI = 4;
-__global__ __launch_bounds__(kSB) void k_nb_scan_reduce(const int* in, int n, int* bsum, const int* go) {
-  if (!*go) return;
+__global__ __launch_bounds__(kSB) void k_nb_scan_reduce(const int* in, int n, int* bsum) {
   __shared__ int sh[kSB];
   const int base = blockIdx.x * kSB * kSI;
   int s = 0;
@@ -408,8 +390,7 @@ __global__ __launch_bounds__(kSB) void k_nb_scan_reduce(const int* in, int n, in
   if (threadIdx.x == 0) bsum[blockIdx.x] = sh[0];
 }
 
-__global__ __launch_bounds__(kSB) void k_nb_scan_blocks(int* bsum, int nb, const int* go) {
-  if (!*go) return;
+__global__ __launch_bounds__(kSB) void k_nb_scan_blocks(int* bsum, int nb) {
   __shared__ int sh[kSB];
   int carry = 0;
   for (int base = 0; base < nb; base += kSB) {
@@ -431,8 +412,7 @@ __global__ __launch_bounds__(kSB) void k_nb_scan_blocks(int* bsum, int nb, const
 }
 
 __global__ __launch_bounds__(kSB) void k_nb_scan_apply(const int* in, int n, const int* boff,
-                                                       int* out, const int* go) {
-  if (!*go) return;
+                                                       int* out) {
   __shared__ int sh[kSB];
   const int base = blockIdx.x * kSB * kSI;
   int carry = boff[blockIdx.x];
@@ -459,8 +439,7 @@ __global__ __launch_bounds__(kSB) void k_nb_scan_apply(const int* in, int n, con
 __global__ __launch_bounds__(kBlock) void k_nb_bin_pos(int cap, int nlocal, const int* nghost,
                                                        const double4* __restrict__ pos,
                                                        const int* __restrict__ items,
-                                                       double4* __restrict__ bpos, const int* go) {
-  if (!*go) return;
+                                                       double4* __restrict__ bpos) {
   const int k = blockIdx.x * kBlock + threadIdx.x;
   if (k >= cap || k >= nlocal + *nghost) return;
   const int j = items[k];
@@ -528,9 +507,7 @@ __device__ __forceinline__ int nb_tile_sort(const int nf, const int lane, const 
 template <int TA>
 __global__ __launch_bounds__(64 * kTileWaves) void k_nb_lists_tile(
     int nlocal, const double4* __restrict__ pos, const int* __restrict__ rep, NbBoxes b,
-    const int* __restrict__ bstart, const double4* __restrict__ bpos, NbLists l, int* overflow,
-    const int* go) {
-  if (!*go) return;
+    const int* __restrict__ bstart, const double4* __restrict__ bpos, NbLists l, int* overflow) {
   extern __shared__ int s_nb[];
   const NbTile tl = nb_tile(l);
   int* s_l = s_nb;
@@ -545,8 +522,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_nb_lists_tile(
   int* s_pre = s_jt + l.cap_f;  // [32] atoms before each run, [32] where the run starts less that
   int* s_beg = s_pre + 32;
   const double reach2 = b.cg * b.cg * (1.0 + 1e-9);
-  // A fixed grid walks the tiles, so that a step without a rebuild costs one
-  // flag read per resident block; the tiles of XCD x form one range.
+  // a fixed grid walks the tiles; those of XCD x form one range
   const int ntiles = (nlocal + TA - 1) / TA, x8 = blockIdx.x % 8;
   const int last = static_cast<int>(static_cast<long>(ntiles) * (x8 + 1) / 8);
   for (int tile = static_cast<int>(static_cast<long>(ntiles) * x8 / 8) + blockIdx.x / 8; tile < last;
@@ -677,69 +653,62 @@ __global__ __launch_bounds__(64 * kTileWaves) void k_nb_lists_tile(
 
 static inline int nbk(long n, int b = kBlock) { return static_cast<int>((n + b - 1) / b); }
 
-static hipError_t scan(const int* in, int n, int* out, int* tmp, const int* go, hipStream_t s) {
+static hipError_t scan(const int* in, int n, int* out, int* tmp, hipStream_t s) {
   const int per = kSB * kSI;
   const int nb = (n + per - 1) / per;
-  k_nb_scan_reduce<<<nb, kSB, 0, s>>>(in, n, tmp, go);
-  k_nb_scan_blocks<<<1, kSB, 0, s>>>(tmp, nb, go);
-  k_nb_scan_apply<<<nb, kSB, 0, s>>>(in, n, tmp, out, go);
+  k_nb_scan_reduce<<<nb, kSB, 0, s>>>(in, n, tmp);
+  k_nb_scan_blocks<<<1, kSB, 0, s>>>(tmp, nb);
+  k_nb_scan_apply<<<nb, kSB, 0, s>>>(in, n, tmp, out);
   return hipGetLastError();
 }
 
-hipError_t launch_nb_force(int* go, hipStream_t s) {
-  k_nb_set<<<1, 64, 0, s>>>(go, 1);
-  return hipGetLastError();
-}
-
-// the rebuild proper, guarded by *go
 hipError_t launch_nb_build(const NbBuild& w, hipStream_t s) {
   const int cap = w.nlocal + w.ghost_cap;
-  const int* go = w.go;
-  k_nb_wrap<<<nbk(w.nlocal), kBlock, 0, s>>>(w.nlocal, w.at.pos, w.at.pv, w.at.rep, w.box, go);
+  k_nb_wrap<<<nbk(w.nlocal), kBlock, 0, s>>>(w.nlocal, w.at.pos, w.at.pv, w.at.rep, w.box);
   // ghost passes: nghost[0] = 0, nghost[d + 1] = after pass d
-  k_nb_zero<<<1, 64, 0, s>>>(w.nghost, 4, go);
+  k_nb_zero<<<1, 64, 0, s>>>(w.nghost, 4);
   for (int d = 0; d < 3; ++d) {
     k_nb_ghost_count<<<nbk(cap), kBlock, 0, s>>>(d, cap, w.nlocal, w.nghost + d, w.at.pos, w.at.rep,
-                                                 w.box, w.cnt, go);
-    (void)scan(w.cnt, cap, w.start, w.scan_tmp, go, s);
+                                                 w.box, w.cnt);
+    (void)scan(w.cnt, cap, w.start, w.scan_tmp, s);
     k_nb_ghost_write<<<nbk(cap), kBlock, 0, s>>>(d, cap, w.nlocal, w.nghost + d, w.nghost + d + 1,
                                                  w.cnt, w.start, w.at, w.box, w.ghost_cap,
-                                                 w.overflow, go);
+                                                 w.overflow);
   }
   const int* ng = w.nghost + 3;
-  k_nb_zero<<<nbk(w.nbins + 1), kBlock, 0, s>>>(w.bcount, w.nbins + 1, go);
-  k_nb_zero<<<nbk(w.nbins + 1), kBlock, 0, s>>>(w.bfill, w.nbins + 1, go);
+  k_nb_zero<<<nbk(w.nbins + 1), kBlock, 0, s>>>(w.bcount, w.nbins + 1);
+  k_nb_zero<<<nbk(w.nbins + 1), kBlock, 0, s>>>(w.bfill, w.nbins + 1);
   k_nb_bin<<<nbk(cap), kBlock, 0, s>>>(cap, w.nlocal, ng, w.at.pos, w.at.rep, w.box, w.bin_of,
-                                       w.bcount, go);
-  (void)scan(w.bcount, w.nbins, w.bstart, w.scan_tmp, go, s);
+                                       w.bcount);
+  (void)scan(w.bcount, w.nbins, w.bstart, w.scan_tmp, s);
   k_nb_bin_scatter<<<nbk(cap), kBlock, 0, s>>>(cap, w.nlocal, ng, w.bin_of, w.bstart, w.bfill,
-                                               w.items, go);
-  k_nb_bin_sort<<<nbk(w.nbins), kBlock, 0, s>>>(w.nbins, w.bstart, w.items, go);
+                                               w.items);
+  k_nb_bin_sort<<<nbk(w.nbins), kBlock, 0, s>>>(w.nbins, w.bstart, w.items);
   // lists of at most kTileKeys fix entries whose rows fit the LDS: the tiled
   // build, 64 atoms per block where they do
   constexpr size_t kLdsMax = 160 * 1024 - 1024;
   const int ta = w.lists.cap_f > kTileKeys ? 0 : nb_tile_lds(w.lists, 64) <= kLdsMax ? 64
                : nb_tile_lds(w.lists, 32) <= kLdsMax ? 32 : 0;
   if (ta) {
-    k_nb_bin_pos<<<nbk(cap), kBlock, 0, s>>>(cap, w.nlocal, ng, w.at.pos, w.items, w.bpos, go);
+    k_nb_bin_pos<<<nbk(cap), kBlock, 0, s>>>(cap, w.nlocal, ng, w.at.pos, w.items, w.bpos);
     const size_t lds = nb_tile_lds(w.lists, ta);
     auto kern = ta == 64 ? k_nb_lists_tile<64> : k_nb_lists_tile<32>;
     const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
     if (e != hipSuccess) return e;
     kern<<<std::min((nbk(w.nlocal, ta) + 7) / 8 * 8, kTileBlocks), 64 * kTileWaves, lds, s>>>(w.nlocal, w.at.pos, w.at.rep, w.box, w.bstart,
-                                                         w.bpos, w.lists, w.overflow, go);
+                                                         w.bpos, w.lists, w.overflow);
   } else {
     if (w.lists.cap_f > kListSortMax) return hipErrorInvalidValue;  // more fix-list entries per atom than the sort takes
     NbLists found = w.lists;
     found.cand = nullptr;  // the candidates are written in the sorted order by k_nb_sort
     k_nb_lists<<<nbk(w.nlocal), kBlock, 0, s>>>(w.nlocal, w.at.pos, w.at.rep, w.box, w.bstart,
-                                                w.items, found, w.overflow, go);
+                                                w.items, found, w.overflow);
     const int sb = std::min(kSortBlocks, nbk(w.nlocal, kBlock / 64));
-    k_nb_sort<8><<<sb, kBlock, 0, s>>>(w.nlocal, w.at.pos, w.lists, go);
+    k_nb_sort<8><<<sb, kBlock, 0, s>>>(w.nlocal, w.at.pos, w.lists);
   }
   const bool cw = w.lists.cand && w.cref && w.cand_valid;
-  k_nb_finish<<<nbk(cw ? cap : w.nlocal), kBlock, 0, s>>>(w.nlocal, ng, w.at.pos, w.xref, w.go,
+  k_nb_finish<<<nbk(cw ? cap : w.nlocal), kBlock, 0, s>>>(w.nlocal, ng, w.at.pos, w.xref,
                                                           w.nrebuild, w.cand_valid, w.cref, cw);
   return hipGetLastError();
 }

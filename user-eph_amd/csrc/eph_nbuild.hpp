@@ -63,7 +63,6 @@ struct NbBuild {
   NbAtoms at;
   NbBoxes box;
   NbLists lists;
-  int* go = nullptr;        // [1] rebuild flag
   int* nghost = nullptr;    // [4] ghosts after each pass; [3] is the result
   int* overflow = nullptr;  // [1] bit 0 ghosts, bit 1 lists
   int* nrebuild = nullptr;  // [1] count of device rebuilds
@@ -85,7 +84,6 @@ struct NbBuild {
   double4* xref = nullptr;  // [nlocal]
 };
 
-hipError_t launch_nb_force(int* go, hipStream_t s);
 hipError_t launch_nb_build(const NbBuild& w, hipStream_t s);
 
 }  // namespace eph
