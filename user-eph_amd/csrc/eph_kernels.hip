@@ -424,7 +424,7 @@ constexpr int split_stage_w(int ur, int uw) { return ur * 128 > uw * 256 ? ur * 
 constexpr int split_stage_f(int u) { return u * kCoopStage; }
 constexpr int split_stage_lj(int u) { return u * 128; }
 
-// Lanes s < NC of each atom's 16 add component s of the round's U x 16 entries
+// Lanes s < NC of each atom's S add component s of the round's U x S entries
 // to acc in order; the terms are laid out [atom][entry][NC].
 template <int S, int U, int NC>
 static __device__ __forceinline__ double split_add(double acc, const double* terms, int grp, int s) {
@@ -521,7 +521,7 @@ __device__ __forceinline__ void density_w_atom_split(const int i_atom, const boo
 #pragma unroll
       for (int u = 0; u < U; ++u) terms[ga * (U * S) + S * u + s] = v[u];
       wave_lds_sync();
-      // all 16 lanes keep the sum
+      // all S lanes keep the sum
       const double* tm = terms + ga * (U * S);
 #pragma unroll
       for (int m = 0; m < U * S; ++m) rho += tm[m];
@@ -583,10 +583,6 @@ __device__ __forceinline__ void density_w_atom_split(const int i_atom, const boo
   if (valid && s == 0) density_finish<XI>(i, grp, pi, rho, alpha, wx, wy, wz, a, p, w);
 }
 
-// Before the sweep, over all nall = nlocal + nghost atoms: on a step that
-// retakes the candidates, the reference positions are the current ones;
-// otherwise every atom 0.45 delta or farther from its reference position (a
-// non-finite distance counts) puts its current position on the moved list.
 // the ghost update of local or ghost atom i, and its position
 __device__ __forceinline__ double4 ghost_atom(const int i, const AtomsView& a, const WorkView& w) {
   if (i < a.nlocal) return a.pos[i];
@@ -606,7 +602,11 @@ __device__ __forceinline__ double4 ghost_atom(const int i, const AtomsView& a, c
   return x;
 }
 
-// the candidate check of atom i at x; tag: what .w of its entry holds
+// The candidate check of atom i at x, made before the sweep for every local and
+// ghost atom: on a step that retakes the candidates, the reference positions are
+// the current ones; otherwise every atom 0.45 delta or farther from its reference
+// position (a non-finite distance counts) puts its current position on the moved
+// list.  tag: what .w of its entry holds
 __device__ __forceinline__ void cand_check_atom(const int i, const double4& x, const double tag,
                                                 const WorkView& w) {
   if (w.cstate[0] == 0) {
@@ -621,14 +621,15 @@ __device__ __forceinline__ void cand_check_atom(const int i, const double4& x, c
   }
 }
 
+// the check in a launch of its own: where no ghost update of the harness made it
 __global__ __launch_bounds__(kBlock) void k_cand_check(int nall, const double4* __restrict__ pos,
                                                        WorkView w) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i < nall) cand_check_atom(i, pos[i], pos[i].w, w);
 }
 
-// The ghost update and, with check, the candidate check of all
-// atoms at the positions it leaves
+// the ghost update and, with check, the candidate check of all atoms at the
+// positions it leaves
 __global__ __launch_bounds__(kBlock) void k_ghost_check(AtomsView a, WorkView w, int check,
                                                         unsigned long long* t) {
   const int i = (check ? 0 : a.nlocal) + blockIdx.x * kBlock + threadIdx.x;
@@ -650,10 +651,7 @@ __global__ __launch_bounds__(kBlock) void k_ghost_check_dev(AtomsView a, WorkVie
   if (check) cand_check_atom(i, x, static_cast<double>(rep[i]), w);
 }
 
-// the same check for a batch of replicas, with the ghost count read on the
-// device (the ensemble's recorded steps, whose ghost count changes between
-// replays; the grid covers nlocal + the ghost capacity); a moved atom's entry
-// carries its replica rep[i] in .w
+// k_cand_check for a batch, as k_ghost_check_dev takes its counts and replicas
 __global__ __launch_bounds__(kBlock) void k_cand_check_dev(int nlocal, const int* __restrict__ ng,
                                                            const double4* __restrict__ pos,
                                                            const int* __restrict__ rep, WorkView w) {
@@ -686,7 +684,7 @@ __global__ void k_cand_flags(int* cstate, int moved_cap) {
   if (threadIdx.x == 0 && blockIdx.x == 0) cand_flags(cstate, moved_cap);
 }
 
-// the split form: 16 atoms per block
+// the split form: kBlock / S atoms per block
 template <int S, int UR, int UW, int XI, bool FRIC, bool MULTI>
 __global__ __launch_bounds__(kBlock) void k_density_w_split(AtomsView a, TablesView t, StepParams p,
                                                             WorkView w) {
@@ -1124,7 +1122,7 @@ __device__ __forceinline__ void prl_forces_atom_coop(const int i_lane, const boo
   if (valid) prl_finish<FRIC, RAND>(i, on, pi, fe, fr, a, g, p, w);
 }
 
-// prl_forces_atom in the split form (see S)
+// prl_forces_atom in the split form, S lanes per atom
 template <int S, int U, bool FRIC, bool RAND, bool MULTI>
 __device__ __forceinline__ void prl_forces_atom_split(const int i_atom, const bool valid,
                                                       const AtomsView& a, const TablesView& t,
@@ -1402,7 +1400,7 @@ __global__ __launch_bounds__(kBlock) void k_integrate(AtomsView a, StepParams p)
   integrate_atom<INITIAL>(i, a, p);
 }
 
-// the time at which block `of` and every 64th before it end, the latest of them
+// the time at which the last block and every 64th before it end, the latest of them
 __device__ __forceinline__ void stamp_end(unsigned long long* t) {
   if (t && threadIdx.x == 0 && (gridDim.x - 1 - blockIdx.x) % 64 == 0)
     atomicMax(t, static_cast<unsigned long long>(wall_clock64()));
@@ -2399,7 +2397,7 @@ __global__ __launch_bounds__(kBlock) void k_deposit_atoms_batch(AtomsView a,
 }
 
 // k_deposit_finish for a batch: blocks 0..nrep - 1 the replicas' tallies, the
-// others the queued cells, each by a scan of its own replica's atoms
+// others the queued cells (queued_cell, over their own replica's atoms)
 __global__ __launch_bounds__(1024) void k_deposit_finish_batch(DepositTail t, const GridView* __restrict__ grids,
                                                                const int* __restrict__ cell_off,
                                                                const int* __restrict__ cell_rep,
@@ -2531,7 +2529,7 @@ __global__ __launch_bounds__(kBlock) void k_copy_double(const double* __restrict
   if (i < n) dst[i] = src[i];
 }
 
-// ghost updates with the ghost count read on the device (graph-capturable)
+// k_ghost_rec with the ghost count read on the device (graph-capturable)
 __global__ __launch_bounds__(kBlock) void k_ghost_rec_dev(AtomsView a, WorkView w,
                                                           const int* __restrict__ ng) {
   const int g = blockIdx.x * kBlock + threadIdx.x;
